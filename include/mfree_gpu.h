@@ -102,10 +102,9 @@ typedef struct {
                          float (src/kernels.cuh:48, src/actions_gpu.cu:50,203,217,420-421,
                          src/interactions_gpu.cu:414-415); 0: full double everywhere */
   int max_neighbours; /* neighbour-list capacity per particle; 0 selects 256 */
-  int pair_pass;      /* MFG_PAIR_LIST (0): one thread per particle gathers its neighbour records;
-                         MFG_PAIR_TILED (1): one wavefront per grid column stages the records of
-                         the column's neighbour cells in LDS.  Same sums, same order. */
-  int pair_strip;     /* list pair pass: particles are visited in strips of this many grid
+  int pair_pass;      /* MFG_PAIR_LIST (0); MFG_PAIR_TILED (1) is accepted and selects the same
+                         kernel (a cell-tiled form existed and was slower at every size) */
+  int pair_strip;     /* pair pass: particles are visited in strips of this many grid
                          columns along y, x-row by x-row inside a strip, which keeps the
                          neighbour records in flight within an XCD's L2; 0 selects 8 (FP64) or
                          16 (FP32 modes), or the sorted order when five x-rows of records fit in
@@ -124,7 +123,7 @@ typedef struct {
                          locked grid's bounds are checked at sorts only, and the neighbour lists
                          and PSE sums differ from the reference's).  Applies to a locked grid that
                          does not move; 0 or 1: every step (the reference's results). */
-  int pair_block;     /* list pair pass: threads per workgroup (64, 128 or 256; 0 selects 256).
+  int pair_block;     /* pair pass: threads per workgroup (64, 128 or 256; 0 selects 256).
                          Each wavefront works alone, so the sums do not depend on it; smaller
                          workgroups spread a small instance over more compute units. */
 } mfg_options;

@@ -1,18 +1,14 @@
 """Autotuner of the step's launch choices, per size bucket (batched and served forms).
 
 Every choice offered leaves results bit-identical, so the tuner only measures time:
-- the pair pass's form (MFG_PAIR_LIST, one thread per particle, or MFG_PAIR_TILED, one
-  wavefront per grid column) and the list pass's visiting order (strip width in grid columns, or
-  the sorted order).  The tiled form is offered in FP64 only: both forms form the same sums in
-  the same order, but in the FP32 modes the two kernels' FMA contraction can differ at rounding
-  level;
+- the pair pass's visiting order (strip width in grid columns, or the sorted order);
 - the neighbour pass's cell tile (consecutive grid cells per wavefront: 1, 2, 4, 8, 16), which
   decides how much an empty cell of a grid with wide margins costs;
-- the list pair pass's workgroup size (64, 128, 256 threads): every wavefront works alone, and
+- the pair pass's workgroup size (64, 128, 256 threads): every wavefront works alone, and
   smaller workgroups spread a small instance over more compute units.
 
 For instances on a stream pool (serve mode "streams"), `tune` picks per (bucket, precision) the
-form and order first, then the cell tile with them, then the pair pass's workgroup size.  For batches (serve mode "batched") the cell
+visiting order first, then the cell tile with them, then the pair pass's workgroup size.  For batches (serve mode "batched") the cell
 tile is a property of the whole launch: `tune_batched` measures a throwaway batch of the first
 requests of each precision with every tile.
 
@@ -38,7 +34,7 @@ from . import api
 
 # (pair pass, strip): 0 the library's default, -1 the sorted order
 CANDIDATES = ((api.MFG_PAIR_LIST, 0), (api.MFG_PAIR_LIST, -1), (api.MFG_PAIR_LIST, 8),
-              (api.MFG_PAIR_LIST, 16), (api.MFG_PAIR_TILED, 0))
+              (api.MFG_PAIR_LIST, 16))
 # cells per wavefront of the neighbour pass; 0 the library's automatic choice
 TILES = (1, 2, 4, 8, 16)
 # threads per workgroup of the list pair pass; 0 the library's default (256)
@@ -48,8 +44,8 @@ DEFAULT = (api.MFG_PAIR_LIST, 0, 0, 0, 0)
 
 
 def candidates_for(precision: int, candidates=CANDIDATES) -> tuple:
-    """The candidates whose results are bit-identical to the default's in `precision`."""
-    return tuple(c for c in candidates if c[0] == api.MFG_PAIR_LIST or precision == api.MFG_FP64)
+    """The candidates whose results are bit-identical to the default's in `precision`: all."""
+    return tuple(candidates)
 
 
 def bucket(n: int) -> int:

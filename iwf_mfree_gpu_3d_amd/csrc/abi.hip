@@ -194,7 +194,7 @@ struct mfg_particles {
   void *rec = nullptr;
   double4 *nl4 = nullptr;
   double2 *pse2 = nullptr;
-  double4 *cs4 = nullptr;  // what the CSPM sum reads of each record, 32 bytes
+  double4 *cs4 = nullptr;  // FP32 modes: what the CSPM sum reads of each record, 32 bytes
   double *sums = nullptr;  // neighbour sums of the pair pass, PAIR_SUM_COUNT x sum_stride (SoA)
   size_t sum_stride = 0;
   int *trav = nullptr;     // visiting order of the list pair pass (N_init)
@@ -562,8 +562,6 @@ int check_counters(mfg_particles *p) {
     return fail(MFG_ERR_CAPACITY, "a particle has %d neighbours, list capacity is %d",
                 p->cnt_h->max_count, p->cap);
   if (p->cnt_h->err_grid) return fail(MFG_ERR_GRID, "unblanked particle outside the grid");
-  if (p->cnt_h->err_list)
-    return fail(MFG_ERR_STATE, "a neighbour list entry lies outside the particle's cell stencil");
   // the reference stops the run here (src/grid_gpu_base.cu:159-163); N is 0 only when every
   // particle was hard-blanked
   if (p->N_host == 0 && p->N_init > 0)
@@ -915,7 +913,7 @@ int mfg_particle_gpu_create(unsigned N, const double *pos4, const double *vel4, 
   p->contact_blocks = p->nblk;
   if (hipMalloc(&p->rec, rec_bytes * n) != hipSuccess || hipMalloc(&p->nl4, sizeof(double4) * n) != hipSuccess ||
       hipMalloc(&p->pse2, sizeof(double2) * n) != hipSuccess ||
-      hipMalloc(&p->cs4, sizeof(double4) * n) != hipSuccess ||
+      (precision != MFG_FP64 && hipMalloc(&p->cs4, sizeof(double4) * n) != hipSuccess) ||
       hipMalloc(&p->sums, sizeof(double) * PAIR_SUM_COUNT * n) != hipSuccess ||
       hipMalloc(&p->trav, sizeof(int) * n) != hipSuccess ||
       hipMalloc(&p->poison, sizeof(int) * n) != hipSuccess ||
@@ -1859,19 +1857,19 @@ int step_impl(mfg_leap_frog *lf, mfg_particles *p, mfg_grid *g, int record,
   int rc = grid_update_geometry(g, p, 2.0, t_current);
   if (rc != MFG_OK) return rc;
   const GridInfo gi = g->info();
-  // visiting order of the list pair pass: strips of 8 grid columns for 192-byte FP64 records,
-  // 16 for 112-byte FP32 records (measured best on the 1M single-grain cut); negative: the
-  // sorted order.  Automatic: the sorted order when its window (the records of about five
-  // x-rows) fits in half an XCD's 4 MB L2, where strips gain nothing and cost two launches.
-  const int tiled = g_lib.opt.pair_pass == MFG_PAIR_TILED ? 1 : 0;
+  // visiting order of the pair pass: strips of 8 grid columns for 192-byte FP64 records, 16 for
+  // 112-byte FP32 records (measured best on the 1M single-grain cut: FP64 0.98 ms against 1.05 for 4
+  // and 16 columns); negative: the sorted order.  Automatic: the sorted order when its window (the
+  // records of about five x-rows) fits in half an XCD's 4 MB L2, where strips gain nothing and cost
+  // two launches.
   const double rec_b = p->precision == MFG_FP64 ? 192. : 112.;
   const bool small = 5. * rec_b * p->N_init / (gi.nx > 0 ? gi.nx : 1) <= 2. * 1024 * 1024;
-  const int strip = g_lib.opt.pair_strip > 0    ? g_lib.opt.pair_strip
-                    : g_lib.opt.pair_strip < 0  ? 0
-                    : small                     ? 0
+  const int strip = g_lib.opt.pair_strip > 0   ? g_lib.opt.pair_strip
+                    : g_lib.opt.pair_strip < 0 ? 0
+                    : small                    ? 0
                     : p->precision == MFG_FP64 ? 8
                                                : 16;
-  const int nseg = (!tiled && strip > 0) ? pair_order_segments(gi, strip) : 0;
+  const int nseg = strip > 0 ? pair_order_segments(gi, strip) : 0;
   int n_exh = 0;
   for (int k = 0; k < n_tools; k++) {
     const mfg_tool *t = tools[k];
@@ -1952,9 +1950,8 @@ int step_impl(mfg_leap_frog *lf, mfg_particles *p, mfg_grid *g, int record,
     ProfScope ps(p->precision == MFG_FP64          ? "pair_fp64"
                  : p->precision == MFG_FP32_KAHAN ? "pair_fp32_kahan"
                                                   : "pair_fp32_wide");
-    launch_pair(s, p->N_init, p->st(), p->rec, p->nbr, p->nl_stride, p->count, c, p->cnt, gi,
-                g->count, p->key_sorted, tiled, p->sums, p->sum_stride, trav, p->cs4,
-                g_lib.opt.pair_block);
+    launch_pair(s, p->N_init, p->st(), p->rec, p->nbr, p->nl_stride, p->count, c, p->cnt,
+                p->sums, p->sum_stride, trav, p->cs4, g_lib.opt.pair_block, !g->locked);
   }
   {
     ProfScope ps("particle_update");
@@ -2094,10 +2091,8 @@ int mfg_interactions_monaghan(mfg_particles *p, mfg_grid *g) {
   if (rc != MFG_OK) return rc;
   rc = run_neighbours(g, p, c, 0);
   if (rc != MFG_OK) return rc;
-  const GridInfo gi = g->info();
   launch_pair(g_lib.stream, p->N_init, p->st(), p->rec, p->nbr, p->nl_stride, p->count, c, p->cnt,
-              gi, g->count, p->key_sorted, 0, p->sums, p->sum_stride, nullptr, p->cs4,
-              g_lib.opt.pair_block);
+              p->sums, p->sum_stride, nullptr, p->cs4, g_lib.opt.pair_block, !g->locked);
   launch_act_sums(g_lib.stream, p->st(), p->N_init, p->cnt, c, aux_of(p), p->sums, p->sum_stride,
                   p->poison);
   HIP_TRY(hipGetLastError());
@@ -2308,7 +2303,7 @@ int batch_build(mfg_batch *b, int record) {
   std::vector<Inst> host(n);
   std::vector<unsigned> maps(N_MAPS * map_len, 0u);
   BatchGrid *grids[N_MAPS] = {&b->L.cells1, &b->L.cells, &b->L.tiles, &b->L.one, &b->L.parts,
-                              &b->L.parts8, &b->L.nbrs8, &b->L.tools, &b->L.search};
+                              &b->L.pairs8, &b->L.nbrs8, &b->L.tools, &b->L.search};
   // cell tile of the batched neighbour pass: by the cells per particle of the whole batch
   long cells = 0, parts = 0;
   for (const mfg_batch::Member &m : b->members) {
@@ -2328,7 +2323,7 @@ int batch_build(mfg_batch *b, int record) {
         (unsigned)host[i].nparts,
         1u,
         nblk,
-        round8(nblk),
+        round8((unsigned)pair_blocks(m.p->N_init, b->precision, 256)),
         round8((unsigned)neighbour_blocks(gi, tile)),
         (unsigned)std::max<size_t>(1, m.tools.size()),
         m.search ? std::min(BATCH_SEARCH_BLOCKS, std::max(1u, nblk)) : 0u};
@@ -2351,6 +2346,9 @@ int batch_build(mfg_batch *b, int record) {
   b->L.precision = b->precision;
   b->L.pse = b->pse;
   b->L.cell_tile = tile;
+  b->L.brook = 0;
+  for (const mfg_batch::Member &m : b->members)
+    if (m.c.heat == MFG_HEAT_BROOKSHAW) b->L.brook = 1;
   b->table_record = record;
   b->dirty = false;
   return MFG_OK;

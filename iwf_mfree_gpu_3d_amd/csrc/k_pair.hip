@@ -16,9 +16,16 @@
 // in registers: Jaumann rate, continuity, momentum, advection, NaN/Inf invalidation, leap-frog
 // correction and the Johnson-Cook radial return (FP64).
 //
-// Precision: FP64 evaluates the reference expressions in the reference order.  FP32 computes
-// the relative position in FP64, the pair arithmetic in FP32 and accumulates every neighbour sum
-// with Kahan compensation; the particle update stays FP64.
+// Precision: FP64 throughout, or (FP32 modes) the relative position in FP64, the pair arithmetic in
+// FP32 and every neighbour sum compensated; the particle update stays FP64.
+//
+// The FP64 pair pass at 1M particles (single-grain cut, about 103 neighbours each): 2.07 -> 0.98 ms
+// against one lane per particle with a walk of its own for B and the
+// reference's order of evaluation (385 vector instructions per neighbour step and 110 of the B walk,
+// now 150 and none); 8,000 particles 198 -> 22 us (125 wavefronts of 100 steps, now 500 of 26).  At
+// 1M it runs at 18 TB/s of record reads from the L2s; vector units busy half of the time, the L1 and
+// LDS paths about two thirds, at two waves per SIMD (45 FP64 sums a lane; compiled for three it
+// spills and is slower).
 #include <type_traits>
 
 #include "mfg_device.hpp"
@@ -27,26 +34,8 @@ namespace mfg {
 
 constexpr int BSP = 256;
 // minimum waves per SIMD the pair kernels are compiled for (register budget)
-#ifndef PAIR32_WAVES
-#define PAIR32_WAVES 2
-#endif
-#ifndef PAIR64_WAVES
-#define PAIR64_WAVES 1
-#endif
-// 1: the FP64 pass gathers each record where it is used (with PAIR64_WAVES 2)
-#ifndef PAIR64_SINGLE
-#define PAIR64_SINGLE 0
-#endif
-// 1: the main loop gathers two neighbours ahead instead of one
-#ifndef PAIR64_DEEP
-#define PAIR64_DEEP 0
-#endif
-#ifndef PAIR32_DEEP
-#define PAIR32_DEEP 0
-#endif
-// 1: the FP64 list pass uses the cooperative gather through LDS (k_pair64_dma)
-#ifndef PAIR64_COOP
-#define PAIR64_COOP 1
+#ifndef PAIR_WAVES
+#define PAIR_WAVES 2
 #endif
 
 // ---------------------------------------------------------------------------------------------
@@ -493,109 +482,6 @@ void dispatch_neighbours(int mode, int cpw, A &&...a) {
 #undef MFG_NB_CPW
 }
 
-// Runs body(load(row[k])) for k = 0 .. n-1 in order.  The neighbour indices are read four at a
-// time, one group ahead, and the gather of neighbour k + 1 is issued before the arithmetic of
-// neighbour k: no gather waits on its own index, and one gather is always in flight.
-// Rows are 16-byte aligned and hold a multiple of 4 (at least 8) entries; the entries past n
-// that the vector reads pick up are never dereferenced.
-// SINGLE: each record is gathered where it is used (fewer registers, no overlap by hand);
-// DEEP: the gathers run two neighbours ahead (three record buffers in flight)
-template <bool SINGLE = false, bool DEEP = false, class Load, class Body>
-__device__ __forceinline__ void gather_loop(const int *row, int n, Load &&load, Body &&body) {
-  if (n <= 0) return;
-  typedef int iv4 __attribute__((ext_vector_type(4)));
-  if (DEEP) {
-    iv4 cur = *(const iv4 *)row;
-    iv4 nxt = n > 4 ? *(const iv4 *)(row + 4) : cur;
-    auto b0 = load(cur.x);
-    decltype(b0) b1, b2, b3;
-    if (n > 1) b1 = load(cur.y);
-    for (int k = 0; k < n; k += 4) {
-      if (k + 2 < n) b2 = load(cur.z);
-      body(b0);
-      if (k + 1 >= n) break;
-      if (k + 3 < n) b3 = load(cur.w);
-      body(b1);
-      if (k + 2 >= n) break;
-      cur = nxt;
-      if (k + 8 < n) nxt = *(const iv4 *)(row + k + 8);
-      if (k + 4 < n) b0 = load(cur.x);
-      body(b2);
-      if (k + 3 >= n) break;
-      if (k + 5 < n) b1 = load(cur.y);
-      body(b3);
-    }
-    return;
-  }
-  if (SINGLE) {
-    iv4 nx = *(const iv4 *)row;
-    for (int k = 0; k < n; k += 4) {
-      const iv4 cu = nx;
-      if (k + 4 < n) nx = *(const iv4 *)(row + k + 4);
-      body(load(cu.x));
-      if (k + 1 < n) body(load(cu.y));
-      if (k + 2 < n) body(load(cu.z));
-      if (k + 3 < n) body(load(cu.w));
-    }
-    return;
-  }
-  iv4 cur = *(const iv4 *)row;
-  iv4 nxt = n > 4 ? *(const iv4 *)(row + 4) : cur;
-  auto ra = load(cur.x);
-  decltype(ra) rb;
-  for (int k = 0; k < n; k += 4) {
-    if (k + 1 < n) rb = load(cur.y);
-    body(ra);
-    if (k + 1 >= n) break;
-    if (k + 2 < n) ra = load(cur.z);
-    body(rb);
-    if (k + 2 >= n) break;
-    if (k + 3 < n) rb = load(cur.w);
-    body(ra);
-    if (k + 3 >= n) break;
-    cur = nxt;
-    if (k + 8 < n) nxt = *(const iv4 *)(row + k + 8);
-    if (k + 4 < n) ra = load(cur.x);
-    body(rb);
-  }
-}
-
-// A 16-byte piece of a record (the unit of the cooperative gathers through LDS below).
-typedef unsigned piece16 __attribute__((ext_vector_type(4)));
-
-// Cooperative gather through registers: groups of G lanes load the P pieces of one record each
-// (one piece per lane and instruction), so every load instruction reads 64 / G whole records
-// from contiguous lines; the pieces then go through LDS to the lane that needs the record.  The
-// LDS slot of a record is S bytes (S / 16 odd multiples of four dwords keep the 16-lane phases of
-// a 16-byte LDS access on distinct banks).
-template <int P, int G, int S>
-struct CoopGather {
-  static_assert(P <= G && (G & (G - 1)) == 0 && G <= 64, "pieces per record");
-  static constexpr int R = 64 / G;  // records per load instruction
-  __device__ static void load(const char *base, size_t rec_bytes, int j, int lane,
-                              piece16 (&v)[G]) {
-    const int p = lane & (G - 1);
-    const int ps = p < P ? p : 0;  // lanes beyond the record's pieces reload piece 0
-#pragma unroll
-    for (int q = 0; q < G; q++) {
-      const int jm = __shfl(j, q * R + lane / G, 64);
-      v[q] = *(const piece16 *)(base + (size_t)jm * rec_bytes + 16 * ps);
-    }
-  }
-  __device__ static void store(char *lds, int lane, const piece16 (&v)[G]) {
-    const int p = lane & (G - 1);
-#pragma unroll
-    for (int q = 0; q < G; q++)
-      if (p < P) *(piece16 *)(lds + (q * R + lane / G) * S + 16 * p) = v[q];
-  }
-};
-
-__device__ __forceinline__ void wave_sync_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ---------------------------------------------------------------------------------------------
 // particle update after the neighbour sums (FP64 for both precisions)
 struct PairSums {
@@ -745,141 +631,216 @@ __global__ void __launch_bounds__(BSP)
 }
 
 // ---------------------------------------------------------------------------------------------
-// Neighbour sums of one particle, FP64: the reference's expressions in its order
-// (src/interactions_gpu.cu:152-471).  The list kernels and the tiled kernel below share it.
-struct Pair64 {
-  typedef Rec64 Rec;
-  // what the CSPM sum reads of a neighbour: (x, y, z, h) and (T, vol, c, tool), the first four
-  // 16-byte pieces of a record
-  struct CRec {
-    double4 p, q;
+// Neighbour sums of the pair pass.
+//
+// The reference walks the stencil twice: for the CSPM matrix B, then for sums of the corrected
+// gradient w = B^-1 w0.  Every sum is linear in w, so the pass walks the list once and sums with
+// the uncorrected gradient w0 instead, one sum per component c of w0; finish_sums applies B^-1
+// (or the identity) once per particle.  The stress sum needs its symmetric 3x3 factor per
+// component of w0 (6 x 3 sums), from which the neighbours' part alone is summed: the particle's own
+// stress and artificial stress multiply sum(w0) and sum(f^4 w0) at the end.  Constant factors of a
+// particle (kernel normalisation, mass, viscosity and XSPH factors) are applied at the end as well.
+struct PairAcc {
+  double W[3], F[3];  // sum w0_c, sum fab w0_c
+  double M[6][3];     // sum (A_j + fab R_j)_ab w0_c
+  double D[3][3];     // sum (v_j - v_i)_a vol_j w0_c
+  double V[3];        // sum Pi_ij w0_c
+  double X[3];        // sum W / (rho_i + rho_j) (v_j - v_i)_a
+  double B[6];        // sum vol_j x_a w0_c (symmetric: w0 is along x)
+  double Q[6];        // sum vol_j (T_i - T_j) / r^2 x_a w0_c (Brookshaw heat)
+};
+
+// the scale of w0 in PairAcc: the sums hold w0 = (dW/dq)(q) x / r without the kernel's
+// normalisation and 1/h (k1), W without the normalisation (fac)
+struct PairScale {
+  double k1, fac, mass, eps;
+};
+
+// adds up the partial sums of the four lanes of a particle; every lane gets the total
+__device__ __forceinline__ double quad_sum(double v) {
+  auto dpp = [](double a, auto ctrl) {
+    const long long b = __builtin_bit_cast(long long, a);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, decltype(ctrl)::value, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
   };
-  static constexpr int CPIECES = 4;
-  __device__ static __forceinline__ int cpiece(int pp) { return pp; }
+  v += dpp(v, std::integral_constant<int, 0xb1>{});  // quad_perm 1,0,3,2
+  v += dpp(v, std::integral_constant<int, 0x4e>{});  // quad_perm 2,3,0,1
+  return v;
+}
 
-  Rec64 ri;
-  bool tool_i, tool_nz, brook;
-  double thermal_alpha, hi, h1, fac, Ti;
-  M3 B, invB;
-  PairSums ps;
-
-  __device__ __forceinline__ Pair64(const Consts &c, const Rec64 &r, uint32_t fl) : ri(r) {
-    tool_i = ri.tool == 1.;
-    tool_nz = (fl & FL_TOOL_NZ) != 0;
-    thermal_alpha = tool_nz ? c.alpha_tool : c.alpha_wp;
-    brook = c.heat == MFG_HEAT_BROOKSHAW && thermal_alpha != 0.;
-    hi = ri.h;
-    h1 = 1 / hi;
-    fac = (INV_PI_D)*h1 * h1 * h1;
-    Ti = brook ? ri.T : 0.;
+// the reference's sums of one particle from its PairAcc: B and its inverse
+// (src/interactions_gpu.cu:262-292), then every sum with the corrected gradient
+// (src/interactions_gpu.cu:294-471).  A, R: the particle's own stress terms and artificial stress.
+template <bool BROOK>
+__device__ __forceinline__ void finish_sums(const Consts &c, const PairAcc &p, const PairScale &k,
+                                            const double A[6], const double R[6], bool tool_nz,
+                                            bool brook, PairSums &ps) {
+  M3 B, inv;
+  constexpr int sym[3][3] = {{0, 3, 5}, {3, 1, 4}, {5, 4, 2}};
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      B.m[a][b] = -(k.k1 * p.B[sym[a][b]]);
+      inv.m[a][b] = a == b ? 1. : 0.;
+    }
+  // tool particles (tool != 0) keep the identity correction
+  if (c.cspm && !tool_nz && det3(B) > 1e-8) inv3(B, inv);
+  auto correct = [&](const double s[3], int b) {
+    return __builtin_fma(s[2], inv.m[2][b], __builtin_fma(s[1], inv.m[1][b], s[0] * inv.m[0][b]));
+  };
+  const double km = k.mass * k.k1;
+#pragma unroll
+  for (int a = 0; a < 3; a++)
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+      const int ab = sym[a][b];
+      ps.vd.m[a][b] = k.k1 * correct(p.D[a], b);
+      double t[3];
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        t[q] = __builtin_fma(A[ab], p.W[q], __builtin_fma(R[ab], p.F[q], p.M[ab][q]));
+      ps.sd.m[a][b] = km * correct(t, b);
+    }
+  const double kx = 2. * k.eps * k.mass * k.fac;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    ps.vt[a] = -(km * correct(p.V, a));
+    ps.xt[a] = kx * p.X[a];
+  }
+  ps.Tl = 0.;
+  if (BROOK && brook) {
+    double s = 0.;
 #pragma unroll
     for (int a = 0; a < 3; a++) {
+      const double q[3] = {p.Q[sym[a][0]], p.Q[sym[a][1]], p.Q[sym[a][2]]};
+      s += correct(q, a);
+    }
+    ps.Tl = 2. * k.k1 * s;
+  }
+}
+
+// 1 / a: the hardware reciprocal (relative error below 2^-24) and one step of third order, which
+// gives the correctly rounded quotient for all but ties (2^24 spread arguments: all equal to 1. / a)
+__device__ __forceinline__ double rcp64(double a) {
+  const double r = __builtin_amdgcn_rcp(a);
+  double d = __builtin_fma(-a, r, 1.);
+  d = __builtin_fma(d, d, d);
+  return __builtin_fma(r, d, r);
+}
+
+// r = sqrt(r2) as the reference's sqrt site evaluates it, and 1 / r.  single: the float root of
+// the float-rounded r2.  From v_rsq_f32 with one residual step it equals the correctly rounded
+// root for every mantissa and both exponent parities (all 2^24 compared with __builtin_sqrtf; r2 in
+// a list is at least 1e-8, far from the denormals).  FP64: the coupled iteration from v_rsq_f64.
+__device__ __forceinline__ void root64(double r2, int single, double &rad, double &rinv) {
+  if (single) {
+    const float x = (float)r2, y = __builtin_amdgcn_rsqf(x);
+    float s = x * y;
+    s = __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
+    rad = (double)s;
+    const double r0 = (double)y;
+    double d = __builtin_fma(-rad, r0, 1.);
+    d = __builtin_fma(d, d, d);
+    rinv = __builtin_fma(r0, d, r0);
+  } else {
+    const double y = __builtin_amdgcn_rsq(r2);
+    double g = r2 * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    rad = __builtin_fma(__builtin_fma(-g, g, r2), h, g);
+    h = 2. * h;
+    rinv = __builtin_fma(h, __builtin_fma(-rad, h, 1.), h);
+  }
+}
+
+// FP64 terms.  The spline as the difference of two truncated powers, W = (2-q)^3/4 - (1-q)_+^3:
+// both branches without a selection.
+template <bool BROOK>
+struct Pair64 {
+  double x, y, z, vx, vy, vz, rho, cs, h, T, h1, kfab;
+  double va, vb, ve;
+  int single;
+
+  __device__ __forceinline__ Pair64(const Consts &c, const Rec64 &r)
+      : x(r.x), y(r.y), z(r.z), vx(r.vx), vy(r.vy), vz(r.vz), rho(r.rho), cs(r.c), h(r.h), T(r.T) {
+    h1 = 1. / h;
+    const double fac = INV_PI_D * h1 * h1 * h1;
+    kfab = c.wdeltap > 0 ? fac / c.wdeltap : 0.;
+    // halves of the pair means folded into the constants: mu = (h_i + h_j) v.x / (2 D),
+    // D = r^2 + eta^2 (h_i + h_j)^2 / 4, Pi = 2 mu (beta mu - alpha (c_i + c_j) / 2) / (rho_i + rho_j)
+    va = c.v_alpha;
+    vb = 2. * c.v_beta;
+    ve = 0.25 * (c.v_eta * c.v_eta);
+    single = c.single_sqrt;
+  }
+  __device__ __forceinline__ PairScale scale(const Consts &c) const {
+    const double fac = INV_PI_D * h1 * h1 * h1;
+    return {fac * h1, fac, c.i_mass, c.xspheps};
+  }
+  __device__ __forceinline__ void term(PairAcc &p, const Rec64 &j, bool mech) const {
+    const double dx = x - j.x, dy = y - j.y, dz = z - j.z;
+    const double r2 = dx * dx + dy * dy + dz * dz;  // rounded as the list's support test rounds it
+    double rad, rinv;
+    root64(r2, single, rad, rinv);
+    const double q = rad * h1;
+    const double a = 2. - q, b = __builtin_fmax(1. - q, 0.);
+    const double a2 = a * a, b2 = b * b;
+    const double val = __builtin_fma(a2, 0.25 * a, -(b2 * b));
+    const double g = __builtin_fma(3., b2, -0.75 * a2) * rinv;
+    const double w0[3] = {g * dx, g * dy, g * dz};
+    const double vol = j.vol;
+    if (BROOK) {
+      const double s = vol * (T - j.T) * rcp64(r2);
+      const double sx = s * dx, sy = s * dy, sz = s * dz;
+      p.Q[0] = __builtin_fma(sx, w0[0], p.Q[0]);
+      p.Q[1] = __builtin_fma(sy, w0[1], p.Q[1]);
+      p.Q[2] = __builtin_fma(sz, w0[2], p.Q[2]);
+      p.Q[3] = __builtin_fma(sx, w0[1], p.Q[3]);
+      p.Q[4] = __builtin_fma(sy, w0[2], p.Q[4]);
+      p.Q[5] = __builtin_fma(sx, w0[2], p.Q[5]);
+    }
+    if (!mech || j.tool == 1.) return;
+    const double vw[3] = {vol * w0[0], vol * w0[1], vol * w0[2]};
+    p.B[0] = __builtin_fma(dx, vw[0], p.B[0]);
+    p.B[1] = __builtin_fma(dy, vw[1], p.B[1]);
+    p.B[2] = __builtin_fma(dz, vw[2], p.B[2]);
+    p.B[3] = __builtin_fma(dx, vw[1], p.B[3]);
+    p.B[4] = __builtin_fma(dy, vw[2], p.B[4]);
+    p.B[5] = __builtin_fma(dx, vw[2], p.B[5]);
+    const double dv[3] = {j.vx - vx, j.vy - vy, j.vz - vz};
+    double fab = val * kfab;
+    fab *= fab;
+    fab *= fab;
 #pragma unroll
-      for (int b = 0; b < 3; b++) {
-        invB.m[a][b] = (a == b) ? 1. : 0.;
-        B.m[a][b] = 0.;
-        ps.vd.m[a][b] = 0.;
-        ps.sd.m[a][b] = 0.;
-      }
-      ps.vt[a] = 0.;
-      ps.xt[a] = 0.;
+    for (int k = 0; k < 3; k++) {
+      p.W[k] += w0[k];
+      p.F[k] = __builtin_fma(fab, w0[k], p.F[k]);
+#pragma unroll
+      for (int e = 0; e < 3; e++) p.D[e][k] = __builtin_fma(dv[e], vw[k], p.D[e][k]);
     }
-    ps.Tl = 0.;
-  }
-  // tool particles (tool != 0) keep the identity correction
-  __device__ __forceinline__ bool cspm_sum() const { return !tool_nz; }
-  __device__ __forceinline__ void cspm_term(const Consts &c, const CRec &g) {
-    if (g.q.w == 1.) return;
-    cspm_add(c, g.p.x, g.p.y, g.p.z, g.q.y);
-  }
-  // the same term from the compact entry (x, y, z, vol), the CSPM_TOOL_BITS pattern marking a
-  // tool particle (tool_particle == 1, src/interactions_gpu.cu:251-254)
-  __device__ __forceinline__ void cspm_term(const Consts &c, const double4 &g) {
-    if (__double_as_longlong(g.w) == CSPM_TOOL_BITS) return;
-    cspm_add(c, g.x, g.y, g.z, g.w);
-  }
-  __device__ __forceinline__ void cspm_add(const Consts &c, double xj, double yj, double zj,
-                                           double volj) {
-    double xij = ri.x - xj, yij = ri.y - yj, zij = ri.z - zj;
-    double rr2 = xij * xij + yij * yij + zij * zij;
-    double w, wx, wy, wz;
-    cubic_spline64(xij, yij, zij, rr2, h1, fac, c.single_sqrt, w, wx, wy, wz);
-    B.m[0][0] -= volj * xij * wx; B.m[1][0] -= volj * xij * wy; B.m[2][0] -= volj * xij * wz;
-    B.m[0][1] -= volj * yij * wx; B.m[1][1] -= volj * yij * wy; B.m[2][1] -= volj * yij * wz;
-    B.m[0][2] -= volj * zij * wx; B.m[1][2] -= volj * zij * wy; B.m[2][2] -= volj * zij * wz;
-  }
-  __device__ __forceinline__ void cspm_end() {
-    if (det3(B) > 1e-8) inv3(B, invB);
-  }
-  __device__ __forceinline__ void term(const Consts &c, const Rec64 &rj) {
-    const double mass = c.i_mass, wdeltap = c.wdeltap, eps = c.xspheps;
-    double xij = ri.x - rj.x, yij = ri.y - rj.y, zij = ri.z - rj.z;
-    double rr2 = xij * xij + yij * yij + zij * zij;
-    double w, wx0, wy0, wz0;
-    cubic_spline64(xij, yij, zij, rr2, h1, fac, c.single_sqrt, w, wx0, wy0, wz0);
-    double w_x, w_y, w_z;
-    if (!c.cspm) {
-      w_x = wx0; w_y = wy0; w_z = wz0;
-    } else {
-      w_x = (wx0 * invB.m[0][0] + wy0 * invB.m[1][0] + wz0 * invB.m[2][0]);
-      w_y = (wx0 * invB.m[0][1] + wy0 * invB.m[1][1] + wz0 * invB.m[2][1]);
-      w_z = (wx0 * invB.m[0][2] + wy0 * invB.m[1][2] + wz0 * invB.m[2][2]);
+#pragma unroll
+    for (int e = 0; e < 6; e++) {
+      const double t = __builtin_fma(fab, j.R[e], j.A[e]);
+#pragma unroll
+      for (int k = 0; k < 3; k++) p.M[e][k] = __builtin_fma(t, w0[k], p.M[e][k]);
     }
-    if (!tool_i && !(rj.tool == 1.)) {
-      const double volj = rj.vol;
-      double dvx = rj.vx - ri.vx, dvy = rj.vy - ri.vy, dvz = rj.vz - ri.vz;
-      ps.vd.m[0][0] += dvx * w_x * volj; ps.vd.m[0][1] += dvx * w_y * volj; ps.vd.m[0][2] += dvx * w_z * volj;
-      ps.vd.m[1][0] += dvy * w_x * volj; ps.vd.m[1][1] += dvy * w_y * volj; ps.vd.m[1][2] += dvy * w_z * volj;
-      ps.vd.m[2][0] += dvz * w_x * volj; ps.vd.m[2][1] += dvz * w_y * volj; ps.vd.m[2][2] += dvz * w_z * volj;
-      double Rxx = 0., Ryy = 0., Rzz = 0., Rxy = 0., Rxz = 0., Ryz = 0.;
-      if (wdeltap > 0) {
-        double fab = w / wdeltap;
-        fab *= fab;
-        fab *= fab;
-        Rxx = fab * (ri.R[0] + rj.R[0]);
-        Rxy = fab * (ri.R[3] + rj.R[3]);
-        Ryy = fab * (ri.R[1] + rj.R[1]);
-        Rxz = fab * (ri.R[5] + rj.R[5]);
-        Ryz = fab * (ri.R[4] + rj.R[4]);
-        Rzz = fab * (ri.R[2] + rj.R[2]);
-      }
-      ps.sd.m[0][0] += mass * (ri.A[0] + rj.A[0] + Rxx) * w_x;
-      ps.sd.m[0][1] += mass * (ri.A[3] + rj.A[3] + Rxy) * w_y;
-      ps.sd.m[0][2] += mass * (ri.A[5] + rj.A[5] + Rxz) * w_z;
-      ps.sd.m[1][0] += mass * (ri.A[3] + rj.A[3] + Rxy) * w_x;
-      ps.sd.m[1][1] += mass * (ri.A[1] + rj.A[1] + Ryy) * w_y;
-      ps.sd.m[1][2] += mass * (ri.A[4] + rj.A[4] + Ryz) * w_z;
-      ps.sd.m[2][0] += mass * (ri.A[5] + rj.A[5] + Rxz) * w_x;
-      ps.sd.m[2][1] += mass * (ri.A[4] + rj.A[4] + Ryz) * w_y;
-      ps.sd.m[2][2] += mass * (ri.A[2] + rj.A[2] + Rzz) * w_z;
-      double vijx = ri.vx - rj.vx, vijy = ri.vy - rj.vy, vijz = ri.vz - rj.vz;
-      double vijposij = vijx * xij + vijy * yij + vijz * zij;
-      double rhoij = 0.5 * (ri.rho + rj.rho);
-      if (vijposij < 0.) {
-        double cij = 0.5 * (ri.c + rj.c);
-        double hij = 0.5 * (hi + rj.h);
-        double r2ij = xij * xij + yij * yij + zij * zij;
-        double muij = (hij * vijposij) / (r2ij + c.v_eta * c.v_eta * hij * hij);
-        double piij = (-c.v_alpha * cij * muij + c.v_beta * muij * muij) / rhoij;
-        ps.vt[0] += -mass * piij * w_x;
-        ps.vt[1] += -mass * piij * w_y;
-        ps.vt[2] += -mass * piij * w_z;
-      }
-      ps.xt[0] += -eps * w * mass / rhoij * vijx;
-      ps.xt[1] += -eps * w * mass / rhoij * vijy;
-      ps.xt[2] += -eps * w * mass / rhoij * vijz;
+    // one reciprocal serves 1 / D and 1 / (rho_i + rho_j)
+    const double vr = -__builtin_fma(dv[2], dz, __builtin_fma(dv[1], dy, dv[0] * dx));
+    const double hs = h + j.h, rs = rho + j.rho;
+    const double d = __builtin_fma(ve * hs, hs, r2);
+    const double inv = rcp64(rs * d);
+    const double irs = inv * d;
+    const double mu = 0.5 * hs * __builtin_fmin(vr, 0.) * (inv * rs);
+    const double pi = mu * __builtin_fma(vb, mu, -va * (cs + j.c)) * irs;
+    const double xw = val * irs;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      p.V[k] = __builtin_fma(pi, w0[k], p.V[k]);
+      p.X[k] = __builtin_fma(xw, dv[k], p.X[k]);
     }
-    if (brook) {
-      double rij = sqrt_rn(xij * xij + yij * yij + zij * zij);
-      if (rij > 1e-8) {
-        double ex = xij / rij, ey = yij / rij, ez = zij / rij;
-        double rij1 = 1. / rij;
-        ps.Tl += 2.0 * (rj.vol) * (Ti - rj.T) * rij1 * (ex * w_x + ey * w_y + ez * w_z);
-      }
-    }
-  }
-  __device__ __forceinline__ void store(double *sums, size_t stride, unsigned i) const {
-    store_sums(sums, stride, i, ps);
   }
 };
 
@@ -916,10 +877,6 @@ struct ToolVol {
 template <class Acc>
 struct Pair32 {
   typedef Rec32 Rec;
-  typedef double4 CRec;  // x, y, z, (tool, vol): the first 32 bytes of a record
-  static constexpr int CPIECES = 2;
-  __device__ static __forceinline__ int cpiece(int pp) { return pp; }
-
   Rec32 ri;
   bool tool_i, tool_nz, brook;
   double thermal_alpha;
@@ -1135,119 +1092,413 @@ __global__ void __launch_bounds__(BSP)
 }
 
 // ---------------------------------------------------------------------------------------------
-// List-gather pair pass: one thread per particle, each neighbour record gathered from memory
-// where it is used (two record buffers in flight, gather_loop); thread t takes particle trav[t]
-// (t itself without a visiting order).
-template <class Body>
-__global__ void __launch_bounds__(BSP, PAIR64_WAVES)
-    k_pair_list(unsigned n_init, State st, const typename Body::Rec *__restrict__ rec,
+// A 16-byte piece of a record (the unit of the cooperative gathers through LDS below).
+typedef unsigned piece16 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ __forceinline__ void wave_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Four lanes (a quad) per particle: lane s of the quad takes neighbours s, s + 4, ... of the list
+// and the quad adds up its four partial sums at the end (quad_sum).  A wavefront holds 16 particles,
+// so 8,000 particles fill 500 wavefronts instead of 125, the longest list of a wavefront is that of
+// 16 particles, not 64, and the four neighbours a quad holds at a time are mostly consecutive
+// records.
+constexpr int PAIR_LANES = 4;
+
+// The gather.  Each lane of a quad needs one record per step; the quad loads its four records
+// together, straight into LDS (buffer_load_dwordx4 ... lds writes lane l's 16 bytes at 16 l of the
+// load's 1 KB block).  Load (r, line) of a step fetches 64-byte line `line` of the record of lane r
+// of every quad, one 64-byte line per quad: one L1 access each, where a lane loading its own record
+// makes one per 16-byte piece.  The index of lane r reaches the quad by a quad permutation, and the
+// buffer descriptor's stride is the record size, so the load unit forms index x stride + offset; an
+// index beyond n_rec reads zeros instead of faulting.  Lane e of the quad fetches piece (e + r) mod 4
+// of the line, so piece p of lane s's record lies in slot (p - s) mod 4 of its quad's 64 bytes in
+// block (s, line): the four lanes of a quad read four different slots, and the 16-byte reads of any
+// two (or four) quads fall on distinct banks.
+template <class Rec, int LINES = sizeof(Rec) / 64>
+struct QuadGather {
+  static constexpr int P = 4 * LINES;  // LINES: lines of a record fetched, from its first
+  static constexpr int AREA = 4 * LINES * 1024;
+  static_assert(sizeof(Rec) % 64 == 0 && (int)sizeof(Rec) >= 64 * LINES, "whole 64-byte lines");
+  struct Pieces {
+    piece16 p[P];
+  };
+  __amdgpu_buffer_rsrc_t rsrc;
+  char *area;
+  int off[4];  // byte offset within a line of the piece this lane fetches, per record r
+  int rd[4];   // LDS offset of piece p of line 0 of this lane's record
+  __device__ __forceinline__ QuadGather(const Rec *rec, unsigned n_rec, char *lds, int lane) : area(lds) {
+    // word 3: the untyped 32-bit data format the load-to-LDS path needs on gfx9-family parts
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)rec, (short)sizeof(Rec), (int)n_rec, 0x00020000);
+    const int s = lane & 3;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      off[r] = 16 * ((s + r) & 3);
+      rd[r] = s * LINES * 1024 + 64 * (lane >> 2) + 16 * ((r - s) & 3);
+    }
+  }
+  // fetches record j of every lane (all lanes active)
+  __device__ __forceinline__ void issue(int j) const {
+    const int jr[4] = {__builtin_amdgcn_mov_dpp(j, 0x00, 0xf, 0xf, true),
+                       __builtin_amdgcn_mov_dpp(j, 0x55, 0xf, 0xf, true),
+                       __builtin_amdgcn_mov_dpp(j, 0xaa, 0xf, 0xf, true),
+                       __builtin_amdgcn_mov_dpp(j, 0xff, 0xf, 0xf, true)};
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int l = 0; l < LINES; l++)
+        __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + (r * LINES + l) * 1024),
+                                                    16, jr[r], off[r], 64 * l, 0, 0);
+  }
+  // this lane's record, once the loads have arrived
+  __device__ __forceinline__ Pieces read() const {
+    Pieces pc;
+#pragma unroll
+    for (int p = 0; p < P; p++) pc.p[p] = *(const piece16 *)(area + rd[p & 3] + (p >> 2) * 1024);
+    return pc;
+  }
+};
+
+template <bool BROOK, int BS>
+__device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_init, const State &st,
+                                          const Rec64 *__restrict__ rec,
+                                          const int *__restrict__ nbr, int stride,
+                                          const int *__restrict__ count, const Consts &c,
+                                          const Counters *cnt, double *__restrict__ sums,
+                                          size_t sstride, const int *__restrict__ trav) {
+  typedef QuadGather<Rec64> Gather;
+  __shared__ __align__(16) char s_area[BS / 64][Gather::AREA];
+  const unsigned t = xcd_map(b, nb) * (BS / PAIR_LANES) + threadIdx.x / PAIR_LANES;
+  const unsigned N = cnt->N;
+  const bool in_range = t < N && t < n_init;
+  const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
+  const uint32_t fl = in_range ? st.flags[i] : FL_BLANKED;
+  const bool act = in_range && !(fl & FL_BLANKED);
+  const unsigned ic = act ? i : 0u;
+  // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = lane & (PAIR_LANES - 1);
+  const int nl = act ? count[i] : 0;
+  int steps = (nl + PAIR_LANES - 1) / PAIR_LANES;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
+  steps = __builtin_amdgcn_readfirstlane(steps);
+  const int *row = nbr + (size_t)ic * stride + s;
+  // neighbour s + 4 k of the list; past its end the particle itself, which is loaded and not used
+  auto index = [&](int k) -> int { return s + 4 * k < nl ? row[4 * k] : (int)ic; };
+  const Pair64<BROOK> P(c, rec[ic]);
+  const bool tool_i = (fl & FL_TOOL) != 0, tool_nz = (fl & FL_TOOL_NZ) != 0;
+  const bool brook = BROOK && c.heat == MFG_HEAT_BROOKSHAW && (tool_nz ? c.alpha_tool : c.alpha_wp) != 0.;
+  PairAcc acc = {};
+  const Gather g(rec, n_init, s_area[w], lane);
+  if (steps > 0) {
+    g.issue(index(0));
+    int jn = steps > 1 ? index(1) : 0;
+    for (int k = 0; k < steps; k++) {
+      __builtin_amdgcn_s_waitcnt(0);  // this step's records are in LDS
+      const Rec64 rj = __builtin_bit_cast(Rec64, g.read());
+      __builtin_amdgcn_s_waitcnt(0);  // every lane's reads are done before the area is refilled
+      wave_sync_lds();
+      if (k + 1 < steps) {
+        g.issue(jn);
+        if (k + 2 < steps) jn = index(k + 2);
+      }
+      if (s + 4 * k < nl) P.term(acc, rj, !tool_i);
+    }
+  }
+  if (!act) return;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    acc.W[k] = quad_sum(acc.W[k]);
+    acc.F[k] = quad_sum(acc.F[k]);
+    acc.V[k] = quad_sum(acc.V[k]);
+    acc.X[k] = quad_sum(acc.X[k]);
+#pragma unroll
+    for (int e = 0; e < 3; e++) acc.D[e][k] = quad_sum(acc.D[e][k]);
+#pragma unroll
+    for (int e = 0; e < 6; e++) acc.M[e][k] = quad_sum(acc.M[e][k]);
+  }
+#pragma unroll
+  for (int e = 0; e < 6; e++) {
+    acc.B[e] = quad_sum(acc.B[e]);
+    if (BROOK) acc.Q[e] = quad_sum(acc.Q[e]);
+  }
+  if (s != 0) return;
+  double A[6], R[6];
+#pragma unroll
+  for (int e = 0; e < 6; e++) {
+    A[e] = rec[i].A[e];
+    R[e] = rec[i].R[e];
+  }
+  PairSums ps;
+  finish_sums<BROOK>(c, acc, P.scale(c), A, R, tool_nz, brook, ps);
+  store_sums(sums, sstride, i, ps);
+}
+// BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
+// depend on it)
+template <bool BROOK, int BS>
+__global__ void __launch_bounds__(BS, PAIR_WAVES)
+    k_pair_sums(unsigned n_init, State st, const Rec64 *__restrict__ rec,
                 const int *__restrict__ nbr, int stride, const int *__restrict__ count, Consts c,
                 const Counters *cnt, double *__restrict__ sums, size_t sstride,
                 const int *__restrict__ trav) {
-  typedef typename Body::Rec Rec;
-  typedef typename Body::CRec CRec;
-  const unsigned t = xcd_block() * BSP + threadIdx.x;
-  const unsigned N = cnt->N;
-  if (t >= N || t >= n_init) return;
-  const unsigned i = trav ? (unsigned)trav[t] : t;
-  const uint32_t fl = st.flags[i];
-  if (fl & FL_BLANKED) return;
-  Body P(c, rec[i], fl);
-  const int n = count[i];
-  const int *row = nbr + (size_t)i * stride;
-  if (c.cspm) {
-    if (P.cspm_sum()) {
-      auto load = [&](int j) {
-        const char *b = (const char *)(rec + j);
-        CRec g;
-        piece16 *d = (piece16 *)&g;
-#pragma unroll
-        for (int pp = 0; pp < Body::CPIECES; pp++) d[pp] = *(const piece16 *)(b + 16 * Body::cpiece(pp));
-        return g;
-      };
-      gather_loop(row, n, load, [&](const CRec &g) { P.cspm_term(c, g); });
-    }
-    P.cspm_end();
-  }
-  gather_loop<PAIR64_SINGLE != 0, PAIR64_DEEP != 0>(row, n, [&](int j) { return rec[j]; },
-                                                    [&](const Rec &rj) { P.term(c, rj); });
-  P.store(sums, sstride, i);
+  pair_sums<BROOK, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
+                       sstride, trav);
 }
 
+// ---------------------------------------------------------------------------------------------
+// The FP64 sums in the reference's own order of evaluation: one lane per particle, one neighbour
+// after the other, B first, every product and division rounded as the reference writes it
+// (src/interactions_gpu.cu:152-471).  An unlocked grid takes its origin and cell size from the
+// particles, to the last bit of the outermost position, so there the positions of every step must
+// round as the reference's do for its cell tables to be the reference's; the sums above differ from
+// these in the last bits.  On a locked grid nothing depends on those bits.
+struct PairOrdered64 {
+  Rec64 ri;
+  bool tool_i, tool_nz, brook;
+  double thermal_alpha, hi, h1, fac, Ti;
+  M3 B, invB;
+  PairSums ps;
 
-// FP64 list pass with a cooperative gather through LDS.  Gathered lane by lane, each 16-byte
-// piece of each neighbour record is its own L1 access, and the L1 serves about one access per
-// cycle: at 16 pieces per pair (CSPM sum and main sum) the per-lane pass is bound there.  Here
-// the wavefront loads the records of a step together, P pieces per record and 64 / P records
-// per load instruction, straight into LDS (global_load_lds_dwordx4: no VGPRs hold them in
-// flight), and every lane then reads its own record from LDS.  The CSPM sum comes first: each
-// lane gathers its neighbours' 32-byte compact entries (x, y, z, vol: cs4), half the bytes of
-// the record line it needs and a quarter of the L2 footprint, so they stay in the L2.  The sums
-// of a particle are those of k_pair_list<Pair64>: same terms, same order.
-//
-// LDS placement.  Load instruction q writes lane l's 16 bytes at DMA_BLOCK q + 16 l.  Each
-// group of four lanes (a quad) loads one 64-byte line of one record, so the L1 serves the quad
-// with one access; which line a quad takes and the order of the four pieces inside it are
-// chosen so that piece p of the records of any 16 consecutive lanes lies on 16 distinct 16-byte
-// bank groups (the lanes of one 16-byte LDS read phase).  With rot(L) = (L >> 2) & 3:
-//   main walk (12 pieces, three lines, 5 records per instruction, 15 of 16 quads): line lam of
-//   record 5 q + rr goes to quad c + 4 k, c = (5 q + rr + lam) & 3 and k the rank of rr among
-//   the records of instruction q with a line of class c; lane e of the quad loads its piece
-//   4 lam + ((e + rot) & 3).
-// Piece p of lane L's record then sits at 64 quad + 16 ((p - rot) & 3) in block L's
-// instruction, on bank group 4 (quad & 3) + ((p - rot) & 3) = 4 ((L + lam) & 3) + ((p - rot) & 3).
-constexpr int DMA_BLOCK = 1280;  // 64 x 16 bytes, 256-byte aligned blocks
-struct MainPlan {
-  typedef Rec64 Rec;
-  static constexpr int P = 12, NI = 13, BLOCK = DMA_BLOCK;
-  // area: NI load blocks, the index window (64 x 16 bytes), the load codes
-  static constexpr int WINDOWS = NI * BLOCK, CODES = WINDOWS + 64 * 16;
-  static constexpr int AREA = CODES + 64 * 4 * ((NI + 1) / 2);
-  // per instruction: the source lane's byte address for ds_bpermute (4 x lane, bits 0-7) and the
-  // piece offset (bits 8-15), two per word, kept in LDS (word m of lane l at codes + 4 (64 m + l))
-  // to spare the registers
-  unsigned *codes_;
-  int lane_;
-  __device__ static int quad(int q, int rr, int lam) {
-    const int c = (5 * q + rr + lam) & 3;
-    const int rb = (c - 5 * q + 1) & 3;  // the one rr (mod 4) with no line of class c
-    return c + 4 * (rr - (rr > rb ? 1 : 0));
-  }
-  __device__ void prepare(char *area, int lane) {
-    codes_ = (unsigned *)(area + CODES);
-    lane_ = lane;
-    const int g = lane >> 2, e = lane & 3, c = g & 3, k = g >> 2;
-    unsigned word = 0;
+  __device__ __forceinline__ PairOrdered64(const Consts &c, const Rec64 &r, uint32_t fl) : ri(r) {
+    tool_i = ri.tool == 1.;
+    tool_nz = (fl & FL_TOOL_NZ) != 0;
+    thermal_alpha = tool_nz ? c.alpha_tool : c.alpha_wp;
+    brook = c.heat == MFG_HEAT_BROOKSHAW && thermal_alpha != 0.;
+    hi = ri.h;
+    h1 = 1 / hi;
+    fac = (INV_PI_D)*h1 * h1 * h1;
+    Ti = brook ? ri.T : 0.;
 #pragma unroll
-    for (int q = 0; q < NI; q++) {
-      const int rb = (c - 5 * q + 1) & 3;
-      const int rr = k + (k >= rb ? 1 : 0);
-      int r = 5 * q + rr;
-      const bool on = k < (rb == 0 ? 3 : 4) && r < 64;
-      const int lam = (c - 5 * q - rr) & 3;
-      int pc = 4 * lam + ((e + ((r >> 2) & 3)) & 3);
-      if (!on) {  // an unused quad: reload piece 0 of the instruction's first record
-        r = 5 * q;
-        pc = 0;
+    for (int a = 0; a < 3; a++) {
+#pragma unroll
+      for (int b = 0; b < 3; b++) {
+        invB.m[a][b] = (a == b) ? 1. : 0.;
+        B.m[a][b] = 0.;
+        ps.vd.m[a][b] = 0.;
+        ps.sd.m[a][b] = 0.;
       }
-      const unsigned code = (unsigned)(4 * r) | ((unsigned)(16 * pc) << 8);
-      if (q & 1) {
-        codes_[64 * (q >> 1) + lane] = word | code << 16;
-      } else {
-        word = code;
-        if (q == NI - 1) codes_[64 * (q >> 1) + lane] = word;
+      ps.vt[a] = 0.;
+      ps.xt[a] = 0.;
+    }
+    ps.Tl = 0.;
+  }
+  // tool particles (tool != 0) keep the identity correction
+  __device__ __forceinline__ bool cspm_sum() const { return !tool_nz; }
+  __device__ __forceinline__ void cspm_add(const Consts &c, double xj, double yj, double zj,
+                                           double volj) {
+    double xij = ri.x - xj, yij = ri.y - yj, zij = ri.z - zj;
+    double rr2 = xij * xij + yij * yij + zij * zij;
+    double w, wx, wy, wz;
+    cubic_spline64(xij, yij, zij, rr2, h1, fac, c.single_sqrt, w, wx, wy, wz);
+    B.m[0][0] -= volj * xij * wx; B.m[1][0] -= volj * xij * wy; B.m[2][0] -= volj * xij * wz;
+    B.m[0][1] -= volj * yij * wx; B.m[1][1] -= volj * yij * wy; B.m[2][1] -= volj * yij * wz;
+    B.m[0][2] -= volj * zij * wx; B.m[1][2] -= volj * zij * wy; B.m[2][2] -= volj * zij * wz;
+  }
+  __device__ __forceinline__ void cspm_end() {
+    if (det3(B) > 1e-8) inv3(B, invB);
+  }
+  __device__ __forceinline__ void term(const Consts &c, const Rec64 &rj) {
+    const double mass = c.i_mass, wdeltap = c.wdeltap, eps = c.xspheps;
+    double xij = ri.x - rj.x, yij = ri.y - rj.y, zij = ri.z - rj.z;
+    double rr2 = xij * xij + yij * yij + zij * zij;
+    double w, wx0, wy0, wz0;
+    cubic_spline64(xij, yij, zij, rr2, h1, fac, c.single_sqrt, w, wx0, wy0, wz0);
+    double w_x, w_y, w_z;
+    if (!c.cspm) {
+      w_x = wx0; w_y = wy0; w_z = wz0;
+    } else {
+      w_x = (wx0 * invB.m[0][0] + wy0 * invB.m[1][0] + wz0 * invB.m[2][0]);
+      w_y = (wx0 * invB.m[0][1] + wy0 * invB.m[1][1] + wz0 * invB.m[2][1]);
+      w_z = (wx0 * invB.m[0][2] + wy0 * invB.m[1][2] + wz0 * invB.m[2][2]);
+    }
+    if (!tool_i && !(rj.tool == 1.)) {
+      const double volj = rj.vol;
+      double dvx = rj.vx - ri.vx, dvy = rj.vy - ri.vy, dvz = rj.vz - ri.vz;
+      ps.vd.m[0][0] += dvx * w_x * volj; ps.vd.m[0][1] += dvx * w_y * volj; ps.vd.m[0][2] += dvx * w_z * volj;
+      ps.vd.m[1][0] += dvy * w_x * volj; ps.vd.m[1][1] += dvy * w_y * volj; ps.vd.m[1][2] += dvy * w_z * volj;
+      ps.vd.m[2][0] += dvz * w_x * volj; ps.vd.m[2][1] += dvz * w_y * volj; ps.vd.m[2][2] += dvz * w_z * volj;
+      double Rxx = 0., Ryy = 0., Rzz = 0., Rxy = 0., Rxz = 0., Ryz = 0.;
+      if (wdeltap > 0) {
+        double fab = w / wdeltap;
+        fab *= fab;
+        fab *= fab;
+        Rxx = fab * (ri.R[0] + rj.R[0]);
+        Rxy = fab * (ri.R[3] + rj.R[3]);
+        Ryy = fab * (ri.R[1] + rj.R[1]);
+        Rxz = fab * (ri.R[5] + rj.R[5]);
+        Ryz = fab * (ri.R[4] + rj.R[4]);
+        Rzz = fab * (ri.R[2] + rj.R[2]);
+      }
+      ps.sd.m[0][0] += mass * (ri.A[0] + rj.A[0] + Rxx) * w_x;
+      ps.sd.m[0][1] += mass * (ri.A[3] + rj.A[3] + Rxy) * w_y;
+      ps.sd.m[0][2] += mass * (ri.A[5] + rj.A[5] + Rxz) * w_z;
+      ps.sd.m[1][0] += mass * (ri.A[3] + rj.A[3] + Rxy) * w_x;
+      ps.sd.m[1][1] += mass * (ri.A[1] + rj.A[1] + Ryy) * w_y;
+      ps.sd.m[1][2] += mass * (ri.A[4] + rj.A[4] + Ryz) * w_z;
+      ps.sd.m[2][0] += mass * (ri.A[5] + rj.A[5] + Rxz) * w_x;
+      ps.sd.m[2][1] += mass * (ri.A[4] + rj.A[4] + Ryz) * w_y;
+      ps.sd.m[2][2] += mass * (ri.A[2] + rj.A[2] + Rzz) * w_z;
+      double vijx = ri.vx - rj.vx, vijy = ri.vy - rj.vy, vijz = ri.vz - rj.vz;
+      double vijposij = vijx * xij + vijy * yij + vijz * zij;
+      double rhoij = 0.5 * (ri.rho + rj.rho);
+      if (vijposij < 0.) {
+        double cij = 0.5 * (ri.c + rj.c);
+        double hij = 0.5 * (hi + rj.h);
+        double r2ij = xij * xij + yij * yij + zij * zij;
+        double muij = (hij * vijposij) / (r2ij + c.v_eta * c.v_eta * hij * hij);
+        double piij = (-c.v_alpha * cij * muij + c.v_beta * muij * muij) / rhoij;
+        ps.vt[0] += -mass * piij * w_x;
+        ps.vt[1] += -mass * piij * w_y;
+        ps.vt[2] += -mass * piij * w_z;
+      }
+      ps.xt[0] += -eps * w * mass / rhoij * vijx;
+      ps.xt[1] += -eps * w * mass / rhoij * vijy;
+      ps.xt[2] += -eps * w * mass / rhoij * vijz;
+    }
+    if (brook) {
+      double rij = sqrt_rn(xij * xij + yij * yij + zij * zij);
+      if (rij > 1e-8) {
+        double ex = xij / rij, ey = yij / rij, ez = zij / rij;
+        double rij1 = 1. / rij;
+        ps.Tl += 2.0 * (rj.vol) * (Ti - rj.T) * rij1 * (ex * w_x + ey * w_y + ez * w_z);
       }
     }
   }
-  __device__ unsigned code(int q) const { return codes_[64 * (q >> 1) + lane_] >> (16 * (q & 1)); }
-  __device__ int src_addr(int q) const { return code(q) & 0xff; }
-  __device__ int off(int q) const { return (code(q) >> 8) & 0xff; }
-  __device__ static int read_pos(int L, int p) {
-    const int q = L / 5, rr = L - 5 * q;
-    return DMA_BLOCK * q + 64 * quad(q, rr, p >> 2) + 16 * ((p - ((L >> 2) & 3)) & 3);
+};
+
+// walks the list of a lane with record gathers of LINES lines; step(k, pieces) for k < nl
+template <int LINES, class Step>
+__device__ __forceinline__ void ordered_walk(const QuadGather<Rec64, LINES> &g, const int *row, int nl,
+                                             int nmax, int ic, Step &&step) {
+  typedef int iv4 __attribute__((ext_vector_type(4)));
+  if (nmax <= 0) return;
+  // indices in windows of four, one window ahead (rows hold a multiple of four entries)
+  iv4 cur = {ic, ic, ic, ic}, nxt = cur;
+  if (nl > 0) cur = *(const iv4 *)row;
+  if (nl > 4) nxt = *(const iv4 *)(row + 4);
+  auto index = [&](int k) -> int {
+    if ((k & 3) == 0 && k > 0) {
+      cur = nxt;
+      if (k + 4 < nl) nxt = *(const iv4 *)(row + k + 4);
+    }
+    const int q = k & 3;
+    return k < nl ? (q == 0 ? cur.x : q == 1 ? cur.y : q == 2 ? cur.z : cur.w) : ic;
+  };
+  g.issue(index(0));
+  for (int k = 0; k < nmax; k++) {
+    __builtin_amdgcn_s_waitcnt(0);  // this step's records are in LDS
+    const auto pc = g.read();
+    __builtin_amdgcn_s_waitcnt(0);  // every lane's reads are done before the area is refilled
+    wave_sync_lds();
+    if (k + 1 < nmax) g.issue(index(k + 1));
+    if (k < nl) step(pc);
+  }
+}
+
+template <int BS>
+__global__ void __launch_bounds__(BS, PAIR_WAVES)
+    k_pair_ordered(unsigned n_init, State st, const Rec64 *__restrict__ rec,
+                   const int *__restrict__ nbr, int stride, const int *__restrict__ count, Consts c,
+                   const Counters *cnt, double *__restrict__ sums, size_t sstride,
+                   const int *__restrict__ trav) {
+  typedef QuadGather<Rec64> Gather;
+  __shared__ __align__(16) char s_area[BS / 64][Gather::AREA];
+  const unsigned t = xcd_map(blockIdx.x, gridDim.x) * BS + threadIdx.x;
+  const bool in_range = t < cnt->N && t < n_init;
+  const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
+  const uint32_t fl = in_range ? st.flags[i] : FL_BLANKED;
+  const bool act = in_range && !(fl & FL_BLANKED);
+  const unsigned ic = act ? i : 0u;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  PairOrdered64 P(c, rec[ic], fl);
+  const int nl = act ? count[i] : 0;
+  const int *row = nbr + (size_t)ic * stride;
+  int nmax = nl;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  if (c.cspm) {
+    // x, y, z, h, T, vol, c, tool: the record's first line
+    ordered_walk(QuadGather<Rec64, 1>(rec, n_init, s_area[w], lane), row, P.cspm_sum() ? nl : 0,
+                 nmax, (int)ic, [&](const auto &pc) {
+                   struct Line {
+                     double x, y, z, h, T, vol, c, tool;
+                   };
+                   const Line j = __builtin_bit_cast(Line, pc);
+                   if (j.tool != 1.) P.cspm_add(c, j.x, j.y, j.z, j.vol);
+                 });
+    P.cspm_end();
+  }
+  ordered_walk(Gather(rec, n_init, s_area[w], lane), row, nl, nmax, (int)ic,
+               [&](const auto &pc) { P.term(c, __builtin_bit_cast(Rec64, pc)); });
+  if (act) store_sums(sums, sstride, i, P.ps);
+}
+
+// ---------------------------------------------------------------------------------------------
+// FP32 pair pass: one lane per particle, B first, then the sums with the corrected gradient, each
+// sum over the list in its order (the Kahan sums depend on it).
+// Runs body(load(row[k])) for k = 0 .. n-1 in order.  The neighbour indices are read four at a
+// time, one group ahead, and the gather of neighbour k + 1 is issued before the arithmetic of
+// neighbour k: no gather waits on its own index, and one gather is always in flight.
+// Rows are 16-byte aligned and hold a multiple of 4 (at least 8) entries; the entries past n
+// that the vector reads pick up are never dereferenced.
+template <class Load, class Body>
+__device__ __forceinline__ void gather_loop(const int *row, int n, Load &&load, Body &&body) {
+  if (n <= 0) return;
+  typedef int iv4 __attribute__((ext_vector_type(4)));
+  iv4 cur = *(const iv4 *)row;
+  iv4 nxt = n > 4 ? *(const iv4 *)(row + 4) : cur;
+  auto ra = load(cur.x);
+  decltype(ra) rb;
+  for (int k = 0; k < n; k += 4) {
+    if (k + 1 < n) rb = load(cur.y);
+    body(ra);
+    if (k + 1 >= n) break;
+    if (k + 2 < n) ra = load(cur.z);
+    body(rb);
+    if (k + 2 >= n) break;
+    if (k + 3 < n) rb = load(cur.w);
+    body(ra);
+    if (k + 3 >= n) break;
+    cur = nxt;
+    if (k + 8 < n) nxt = *(const iv4 *)(row + k + 8);
+    if (k + 4 < n) ra = load(cur.x);
+    body(rb);
+  }
+}
+
+// Cooperative gather through registers: groups of G lanes load the P pieces of one record each
+// (one piece per lane and instruction), so every load instruction reads 64 / G whole records
+// from contiguous lines; the pieces then go through LDS to the lane that needs the record.  The
+// LDS slot of a record is S bytes (S / 16 odd multiples of four dwords keep the 16-lane phases of
+// a 16-byte LDS access on distinct banks).
+template <int P, int G, int S>
+struct CoopGather {
+  static_assert(P <= G && (G & (G - 1)) == 0 && G <= 64, "pieces per record");
+  static constexpr int R = 64 / G;  // records per load instruction
+  __device__ static void load(const char *base, size_t rec_bytes, int j, int lane,
+                              piece16 (&v)[G]) {
+    const int p = lane & (G - 1);
+    const int ps = p < P ? p : 0;  // lanes beyond the record's pieces reload piece 0
+#pragma unroll
+    for (int q = 0; q < G; q++) {
+      const int jm = __shfl(j, q * R + lane / G, 64);
+      v[q] = *(const piece16 *)(base + (size_t)jm * rec_bytes + 16 * ps);
+    }
+  }
+  __device__ static void store(char *lds, int lane, const piece16 (&v)[G]) {
+    const int p = lane & (G - 1);
+#pragma unroll
+    for (int q = 0; q < G; q++)
+      if (p < P) *(piece16 *)(lds + (q * R + lane / G) * S + 16 * p) = v[q];
   }
 };
-constexpr int DMA64_AREA = MainPlan::AREA;
+
 // FP32 records (112 bytes, seven pieces): the step's 64 records lie in LDS one after the other
 // (record L at 112 L), as seven 1 KB blocks: load instruction q fetches piece g = 64 q + lane of
 // that image (record g / 7, piece g mod 7), so every lane loads and no piece is fetched twice.
@@ -1271,11 +1522,6 @@ struct Plan32 {
   __device__ int off(int q) const { return off_[q]; }
   __device__ static int read_pos(int L, int p) { return (int)sizeof(Rec32) * L + 16 * p; }
 };
-#ifndef PAIR64D_WAVES
-#define PAIR64D_WAVES 2
-#endif
-typedef __attribute__((address_space(3))) void lds_void;
-
 // Walks the lists of a wavefront: step k gives each lane with k < nl the first P pieces of its
 // neighbour k.  Step k + 1's records and the index window of steps k + 2 .. k + 5 are loaded
 // while step k's term runs.  The records are read through a buffer descriptor whose stride is
@@ -1512,293 +1758,13 @@ __device__ __forceinline__ void pair32_coop(unsigned b, unsigned nb, unsigned n_
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
 // depend on it).  Small instances spread over more compute units with smaller workgroups.
 template <class Acc, int BS>
-__global__ void __launch_bounds__(BS, PAIR32_WAVES)
+__global__ void __launch_bounds__(BS, PAIR_WAVES)
     k_pair32_coop(unsigned n_init, State st, const Rec32 *__restrict__ rec,
                   const int *__restrict__ nbr, int stride, const int *__restrict__ count,
                   Consts c, const Counters *cnt, double *__restrict__ sums, size_t sstride,
                   const int *__restrict__ trav, const double4 *__restrict__ cs4) {
   pair32_coop<Acc, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
                        sstride, trav, cs4);
-}
-
-template <int BS = BSP>
-__device__ __forceinline__ void pair64_dma(unsigned b, unsigned nb, unsigned n_init,
-                                           const State &st, const Rec64 *__restrict__ rec,
-                                           const int *__restrict__ nbr, int stride,
-                                           const int *__restrict__ count, const Consts &c,
-                                           const Counters *cnt, double *__restrict__ sums,
-                                           size_t sstride, const int *__restrict__ trav,
-                                           const double4 *__restrict__ cs4) {
-  typedef Pair64::CRec CRec;
-  static_assert(sizeof(Rec64) == 192 && sizeof(CRec) == 64, "record pieces");
-  const unsigned t = xcd_map(b, nb) * BS + threadIdx.x;
-  const unsigned N = cnt->N;
-  const bool in_range = t < N && t < n_init;
-  const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
-  const uint32_t fl = in_range ? st.flags[i] : FL_BLANKED;
-  const bool act = in_range && !(fl & FL_BLANKED);
-  const unsigned ic = act ? i : 0u;
-  Pair64 P(c, rec[ic], fl);
-  const int nl = act ? count[i] : 0;
-  const int *row = nbr + (size_t)ic * stride;
-  __shared__ __align__(16) char s_area[BS / 64][DMA64_AREA];
-  // the wave index as a scalar: the LDS destinations of the record loads (M0) are then formed
-  // by the scalar unit
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  char *area = s_area[w];
-  if (c.cspm) {
-    const int nc = P.cspm_sum() ? nl : 0;
-    int ncmax = nc;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ncmax = max(ncmax, __shfl_xor(ncmax, o, 64));
-    static_assert(CSPM_RING <= DMA64_AREA, "the CSPM ring fits the main walk's area");
-    dma_cspm_walk(cs4, n_init, row, nc, ncmax, ic, lane, area,
-                  [&](const double4 &g) { P.cspm_term(c, g); });
-    P.cspm_end();
-  }
-  int nmax = nl;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
-  dma_list_walk<MainPlan>(rec, n_init, row, nl, nmax, ic, lane, area,
-                    [&](const auto &pc) { P.term(c, __builtin_bit_cast(Rec64, pc)); });
-  if (!act) return;
-  P.store(sums, sstride, i);
-}
-// BS: threads per workgroup, as for k_pair32_coop
-template <int BS>
-__global__ void __launch_bounds__(BS, PAIR64D_WAVES)
-    k_pair64_dma(unsigned n_init, State st, const Rec64 *__restrict__ rec,
-                 const int *__restrict__ nbr, int stride, const int *__restrict__ count,
-                 Consts c, const Counters *cnt, double *__restrict__ sums, size_t sstride,
-                 const int *__restrict__ trav, const double4 *__restrict__ cs4) {
-  pair64_dma<BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
-                 sstride, trav, cs4);
-}
-
-// ---------------------------------------------------------------------------------------------
-// Cell-tiled pair pass.  One wavefront per grid column (gi, gj); the column's particles are
-// taken in chunks of at most 64 consecutive particles, one per lane.  Every neighbour of a chunk
-// lies in the 25 stencil columns (gi-2..gi+2, gj-2..gj+2) between cells kz_lo-2 and kz_hi+2 of
-// the chunk's first and last particle; in each stencil column those cells hold ONE contiguous
-// range of particles (a run), and the runs in (ii, jj) order concatenate to the chunk's staging
-// sequence S, ascending in particle index.  A neighbour list is ascending in particle index as
-// well (it follows the same cell order), so each lane walks S forwards.
-//
-// S streams through an LDS ring of NB blocks of B records: the whole wavefront loads a block
-// with 16-byte pieces that are contiguous in memory within a run (each record is read once per
-// chunk instead of once per pair), a block is refilled once no lane needs it any more, and the
-// load of the next block is in flight while the lanes compute.  A lane whose next neighbour is
-// not staged yet sits out a step.  Lanes work through their lists in list order, so every sum
-// has the order of the list pass.
-//
-// Staged records are P pieces of 16 bytes: piece pp of a staged record is the 16-byte piece
-// pofs(pp) of the record in memory (all of a record for the main sum, the CSPM fields for the
-// CSPM sum).
-#ifndef TILE64_B
-#define TILE64_B 16
-#endif
-#ifndef TILE64_NB
-#define TILE64_NB 8
-#endif
-#ifndef TILE32_B
-#define TILE32_B 16
-#endif
-#ifndef TILE32_NB
-#define TILE32_NB 12
-#endif
-#ifndef TILE_WAVES
-#define TILE_WAVES 2
-#endif
-
-struct TileRuns {
-  int rs[32], re[32], rp[32];  // run start / end (particle index), position of the run in S
-};
-
-template <int P, int B, int NB, class PieceOf, class Term>
-__device__ __forceinline__ void tile_stream(const char *__restrict__ base, int rec_bytes,
-                                            char *ring, const TileRuns &tr, int nr, int T,
-                                            const int *row, int nl, int cap, int lane, int &err,
-                                            PieceOf pofs, Term &&term) {
-  typedef int iv4 __attribute__((ext_vector_type(4)));
-  constexpr int RS = 16 * P;              // staged record bytes
-  constexpr int PPL = (P * B + 63) / 64;  // pieces per lane per block
-  static_assert(B <= 64 && (B & (B - 1)) == 0, "block of at most 64 records");
-  const int nblk = (T + B - 1) / B;
-  // this lane's list cursor: entry k, its group of four in win, the next group in nwin, the run
-  // r holding entry k and its position pos in S (rows hold cap >= 8 entries, a multiple of 4)
-  int k = 0, r = 0, pos = INT_MAX;
-  iv4 win = *(const iv4 *)row;
-  iv4 nwin;
-  auto locate = [&]() {
-    pos = INT_MAX;
-    if (k >= nl) return;
-    const int q = k & 3;
-    const int j = q == 0 ? win.x : q == 1 ? win.y : q == 2 ? win.z : win.w;
-    while (r < nr - 1 && j >= tr.re[r]) r++;
-    if (j >= tr.rs[r] && j < tr.re[r]) {
-      pos = j - tr.rs[r] + tr.rp[r];
-    } else {  // not in the chunk's stencil: the lane stops and the error is reported
-      err = 1;
-      k = nl;
-    }
-  };
-  locate();
-  int sum = nl, mp = pos;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    sum += __shfl_xor(sum, o, 64);
-    mp = min(mp, __shfl_xor(mp, o, 64));
-  }
-  if (mp == INT_MAX) return;  // uniform: no lane has a neighbour
-  // particle index of record `lane` of block b (lanes < B and inside S)
-  auto block_index = [&](int b) -> int {
-    const int s = b * B + (lane & (B - 1));
-    int lo = 0, hi = nr - 1;  // last run whose position is <= s (a non-empty one)
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (tr.rp[mid] <= s) lo = mid;
-      else hi = mid - 1;
-    }
-    return tr.rs[lo] + (s - tr.rp[lo]);
-  };
-  // a block's pieces are loaded into registers (contiguous in memory within a run) and written
-  // to its ring slot one step later.  Every lane issues every load (lanes without a piece of the
-  // block reload the block's first piece), so the loads need no branch around them.
-  piece16 v[PPL];
-  auto issue = [&](int b) {
-    const int jl = block_index(b);
-    const int nrec = min(B, T - b * B);
-#pragma unroll
-    for (int m = 0; m < PPL; m++) {
-      const int q = lane + 64 * m;
-      const int rr = q / P, pp = q - rr * P;
-      const bool own = q < P * B && rr < nrec;
-      const int jr = __shfl(jl, own ? rr : 0, 64);
-      v[m] = *(const piece16 *)(base + (size_t)jr * rec_bytes + 16 * pofs(own ? pp : 0));
-    }
-  };
-  // slot NB of the ring takes a block that is not needed (the ring was full when it was loaded)
-  auto land = [&](int b, int slot_idx) {
-    char *slot = ring + slot_idx * (B * RS);
-    const int nrec = min(B, T - b * B);
-#pragma unroll
-    for (int m = 0; m < PPL; m++) {
-      const int q = lane + 64 * m;
-      if (q < P * B && q / P < nrec) *(piece16 *)(slot + 16 * q) = v[m];
-    }
-  };
-  int blo = mp / B, bhi = blo;  // blocks [blo, bhi) are staged
-  issue(bhi);
-  land(bhi, bhi % NB);
-  bhi++;
-  bool pending = false;
-  int loaded = bhi;  // block held in v
-  // Each step issues the same memory operations in the same order, all before its arithmetic:
-  // the lane's next group of neighbour indices, then one block (the next block, or a repeat of
-  // the last one when the ring is full).  The block is the youngest load when it lands at the
-  // start of the next step, and the arithmetic of a whole step covers its latency.
-  // Every step either moves a lane on or stages the block the lowest lane waits for (within two
-  // steps), so 3 steps per list entry and 2 per block bound the loop.
-  const int max_steps = 3 * sum + 2 * nblk + 8;
-  int step = 0;
-  for (; step < max_steps; step++) {
-    land(loaded, pending ? bhi % NB : NB);
-    if (pending) bhi++;
-    while (blo < bhi && __ballot(pos < (blo + 1) * B) == 0) blo++;
-    if (__ballot(pos != INT_MAX) == 0) break;
-    if (blo == bhi) {  // no staged block is needed: go to the first block a lane waits for
-      int m2 = pos;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) m2 = min(m2, __shfl_xor(m2, o, 64));
-      blo = bhi = m2 / B;
-    }
-    pending = bhi < nblk && bhi - blo < NB;
-    loaded = min(bhi, nblk - 1);
-    nwin = *(const iv4 *)(row + min((k & ~3) + 4, cap - 4));
-    issue(loaded);
-    wave_sync_lds();  // the landed block is visible to every lane
-    if (pos < bhi * B) {
-      term(ring + ((pos / B) % NB) * (B * RS) + (pos % B) * RS);
-      k++;
-      if ((k & 3) == 0) win = nwin;
-      locate();
-    }
-  }
-  if (step == max_steps) err = 1;
-  wave_sync_lds();  // every read of the ring has completed before it is restaged
-}
-
-template <class Body, int B, int NB>
-__global__ void __launch_bounds__(64, TILE_WAVES)
-    k_pair_tiled(GridInfo g, const int *__restrict__ off, const int *__restrict__ key_sorted,
-                 State st, const typename Body::Rec *__restrict__ rec,
-                 const int *__restrict__ nbr, int stride, const int *__restrict__ count,
-                 Consts c, Counters *cnt, double *__restrict__ sums, size_t sstride) {
-  typedef typename Body::Rec Rec;
-  typedef typename Body::CRec CRec;
-  constexpr int RS = sizeof(Rec);
-  __shared__ __align__(16) char ring[(NB + 1) * B * RS];
-  __shared__ TileRuns tr;
-  const int lane = threadIdx.x;
-  const long col = xcd_block();
-  if (col >= (long)g.nx * g.ny) return;
-  const int gi = (int)(col / g.ny), gj = (int)(col % g.ny);
-  const long cbase = col * g.nz;
-  const int c0 = off[cbase], c1 = off[cbase + g.nz];
-  const int len = c1 - c0;
-  if (len <= 0) return;
-  const int lo_i = max(gi - 2, 0), hi_i = min(gi + 3, g.nx);
-  const int lo_j = max(gj - 2, 0), hi_j = min(gj + 3, g.ny);
-  const int nj = hi_j - lo_j, nr = (hi_i - lo_i) * nj;
-  const int nch = (len + 63) / 64;
-  int err = 0;
-  for (int ch = 0; ch < nch; ch++) {
-    const int p0 = c0 + (int)((long)ch * len / nch);
-    const int p1 = c0 + (int)((long)(ch + 1) * len / nch);
-    const int kz_lo = max(key_sorted[p0] - (int)cbase - 2, 0);
-    const int kz_hi = min(key_sorted[p1 - 1] - (int)cbase + 2, g.nz - 1);
-    int rs = 0, rl = 0;
-    if (lane < nr) {
-      const int ii = lo_i + lane / nj, jj = lo_j + lane % nj;
-      const long cb = ((long)ii * g.ny + jj) * g.nz;
-      rs = off[cb + kz_lo];
-      rl = off[cb + kz_hi + 1] - rs;
-    }
-    int incl = rl;
-#pragma unroll
-    for (int o = 1; o < 32; o <<= 1) {
-      const int t = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += t;
-    }
-    const int T = __builtin_amdgcn_readfirstlane(__shfl(incl, 31, 64));
-    if (lane < 32) {
-      tr.rs[lane] = rs;
-      tr.re[lane] = rs + rl;
-      tr.rp[lane] = incl - rl;
-    }
-    wave_sync_lds();
-    const unsigned i = (unsigned)(p0 + lane);
-    const bool in = lane < p1 - p0;
-    const uint32_t fl = in ? st.flags[i] : FL_BLANKED;
-    const bool act = in && !(fl & FL_BLANKED);
-    const unsigned ic = act ? i : (unsigned)p0;
-    Body P(c, rec[ic], fl);
-    const int n = act ? count[i] : 0;
-    const int *row = nbr + (size_t)ic * stride;
-    if (c.cspm) {
-      tile_stream<Body::CPIECES, B, NB>(
-          (const char *)rec, RS, ring, tr, nr, T, row, P.cspm_sum() ? n : 0, stride, lane, err,
-          [](int pp) { return Body::cpiece(pp); },
-          [&](const char *s) { P.cspm_term(c, *(const CRec *)s); });
-      P.cspm_end();
-    }
-    tile_stream<RS / 16, B, NB>((const char *)rec, RS, ring, tr, nr, T, row, n, stride, lane, err,
-                                [](int pp) { return pp; },
-                                [&](const char *s) { P.term(c, *(const Rec *)s); });
-    if (act) P.store(sums, sstride, i);
-    wave_sync_lds();  // the next chunk rewrites the runs and the ring
-  }
-  if (__ballot(err) != 0 && lane == 0) atomicOr(&cnt->err_list, 1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1840,51 +1806,43 @@ void launch_neighbours(hipStream_t s, const GridInfo &g, const int *offsets, con
                                         nbr, cap, count, T_t, cnt, stat_part, poison);
 }
 
+int pair_blocks(unsigned n_init, int precision, int block) {
+  return (int)nb((long)n_init * (precision == MFG_FP64 ? PAIR_LANES : 1), block);
+}
+
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
-                 int nl_stride, const int *count, const Consts &c, Counters *cnt,
-                 const GridInfo &g, const int *offsets, const int *key_sorted, int tiled,
-                 double *sums, size_t sstride, const int *trav, const double4 *cs4, int block) {
-  if (tiled) {
-    const dim3 grid((unsigned)((long)g.nx * g.ny)), block(64);
-    if (c.precision == MFG_FP64)
-      hipLaunchKernelGGL((k_pair_tiled<Pair64, TILE64_B, TILE64_NB>), grid, block, 0, s, g,
-                         offsets, key_sorted, st, (const Rec64 *)rec, nbr, nl_stride, count, c,
-                         cnt, sums, sstride);
-    else if (c.precision == MFG_FP32_KAHAN)
-      hipLaunchKernelGGL((k_pair_tiled<Pair32<AccKahan>, TILE32_B, TILE32_NB>), grid, block, 0, s,
-                         g, offsets, key_sorted, st, (const Rec32 *)rec, nbr, nl_stride, count, c,
-                         cnt, sums, sstride);
-    else
-      hipLaunchKernelGGL((k_pair_tiled<Pair32<AccWide>, TILE32_B, TILE32_NB>), grid, block, 0, s,
-                         g, offsets, key_sorted, st, (const Rec32 *)rec, nbr, nl_stride, count, c,
-                         cnt, sums, sstride);
-    return;
-  }
+                 int nl_stride, const int *count, const Consts &c, const Counters *cnt,
+                 double *sums, size_t sstride, const int *trav, const double4 *cs4, int block,
+                 bool ordered) {
   const int bs = block == 64 || block == 128 ? block : BSP;
-  const dim3 grid(nb(n_init, bs)), blk(bs);
+  const dim3 blk(bs), grid1(nb(n_init, bs));  // one lane per particle
+  const bool brook = c.heat == MFG_HEAT_BROOKSHAW;
   auto launch = [&](auto bs_c) {
     constexpr int BS = decltype(bs_c)::value;
-    if (c.precision == MFG_FP64 && PAIR64_COOP)
-      hipLaunchKernelGGL(k_pair64_dma<BS>, grid, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr,
-                         nl_stride, count, c, cnt, sums, sstride, trav, cs4);
-    else if (c.precision == MFG_FP64)
-      hipLaunchKernelGGL((k_pair_list<Pair64>), dim3(nb(n_init, BSP)), dim3(BSP), 0, s, n_init, st,
-                         (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
-    else if (c.precision == MFG_FP32_KAHAN)
-      hipLaunchKernelGGL((k_pair32_coop<AccKahan, BS>), grid, blk, 0, s, n_init, st,
+    if (c.precision == MFG_FP32_KAHAN) {
+      hipLaunchKernelGGL((k_pair32_coop<AccKahan, BS>), grid1, blk, 0, s, n_init, st,
                          (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav,
                          cs4);
-    else
-      hipLaunchKernelGGL((k_pair32_coop<AccWide, BS>), grid, blk, 0, s, n_init, st,
+    } else if (c.precision == MFG_FP32_WIDE) {
+      hipLaunchKernelGGL((k_pair32_coop<AccWide, BS>), grid1, blk, 0, s, n_init, st,
                          (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav,
                          cs4);
+    } else if (ordered) {
+      hipLaunchKernelGGL(k_pair_ordered<BS>, grid1, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr,
+                         nl_stride, count, c, cnt, sums, sstride, trav);
+    } else {
+      const dim3 grid((unsigned)pair_blocks(n_init, c.precision, bs));
+      if (brook)
+        hipLaunchKernelGGL((k_pair_sums<true, BS>), grid, blk, 0, s, n_init, st,
+                           (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
+      else
+        hipLaunchKernelGGL((k_pair_sums<false, BS>), grid, blk, 0, s, n_init, st,
+                           (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
+    }
   };
-  if (bs == 64)
-    launch(std::integral_constant<int, 64>{});
-  else if (bs == 128)
-    launch(std::integral_constant<int, 128>{});
-  else
-    launch(std::integral_constant<int, BSP>{});
+  if (bs == 64) launch(std::integral_constant<int, 64>{});
+  else if (bs == 128) launch(std::integral_constant<int, 128>{});
+  else launch(std::integral_constant<int, BSP>{});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1916,15 +1874,16 @@ struct BatchNeighbours {
   }
 };
 
-__global__ void __launch_bounds__(BSP, PAIR64D_WAVES) kb_pair64_dma(const Inst *in, BatchMap m) {
+template <bool BROOK>
+__global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair_sums(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  pair64_dma(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec64 *)d.rec, d.nbr, d.nl_stride, d.count,
-             d.c, d.cnt, d.sums, d.sum_stride, nullptr, d.cs4);
+  pair_sums<BROOK, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec64 *)d.rec, d.nbr,
+                        d.nl_stride, d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr);
 }
 
 template <class Acc>
-__global__ void __launch_bounds__(BSP, PAIR32_WAVES) kb_pair32_coop(const Inst *in, BatchMap m) {
+__global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair32_coop(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
   pair32_coop<Acc>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
@@ -1937,20 +1896,21 @@ __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchM
   update_body(b, d.n_init, d.buf[d.cur ^ 1], d.sums, d.sum_stride, d.poison, d.c, d.cnt);
 }
 
-// The kernel forms of the single-instance step's defaults (the FP64 cooperative gather when it
-// is compiled in, the FP32 cooperative gather) in the sorted visiting order; the PSE mode as
-// run_neighbours picks it.
+// The kernels of the single-instance step in the sorted visiting order; the PSE mode as
+// run_neighbours picks it.  One Brookshaw instance selects the kernel with its sum for all: the
+// others' sums are the same in both.
 void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
   const int mode = !L.pse ? 0 : L.precision == MFG_FP64 ? 1 : 2;
   dispatch_neighbours<BatchNeighbours>(mode, L.cell_tile, s, L);
-  const dim3 gp(L.parts8.blocks), bp(BSP);
-  static_assert(PAIR64_COOP, "the batched FP64 pair pass is the cooperative form");
-  if (L.precision == MFG_FP64)
-    hipLaunchKernelGGL(kb_pair64_dma, gp, bp, 0, s, L.inst, L.parts8.m);
+  const dim3 gp(L.pairs8.blocks), bp(BSP);
+  if (L.precision == MFG_FP64 && L.brook)
+    hipLaunchKernelGGL(kb_pair_sums<true>, gp, bp, 0, s, L.inst, L.pairs8.m);
+  else if (L.precision == MFG_FP64)
+    hipLaunchKernelGGL(kb_pair_sums<false>, gp, bp, 0, s, L.inst, L.pairs8.m);
   else if (L.precision == MFG_FP32_KAHAN)
-    hipLaunchKernelGGL(kb_pair32_coop<AccKahan>, gp, bp, 0, s, L.inst, L.parts8.m);
+    hipLaunchKernelGGL(kb_pair32_coop<AccKahan>, gp, bp, 0, s, L.inst, L.pairs8.m);
   else
-    hipLaunchKernelGGL(kb_pair32_coop<AccWide>, gp, bp, 0, s, L.inst, L.parts8.m);
+    hipLaunchKernelGGL(kb_pair32_coop<AccWide>, gp, bp, 0, s, L.inst, L.pairs8.m);
   hipLaunchKernelGGL(kb_particle_update, dim3(L.parts.blocks), dim3(BSP), 0, s, L.inst, L.parts.m);
 }
 

@@ -2,7 +2,7 @@
 //
 // The files are compiled with -ffp-contract=off: every expression rounds exactly as written, so
 // the FP64 path evaluates the reference formulas in the reference's operation order; fused
-// multiply-adds are only used where they are spelled out (the FP32 pair arithmetic).
+// multiply-adds are only used where they are spelled out (the pair sums and the PSE exponential).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -8,9 +8,8 @@
 //   half-step records (sorted order, rebuilt every step by the permute/predict kernel):
 //     nl4   : double4 (x, y, z, blanked)          -- candidate filter of the neighbour-list pass
 //     pse2  : double2 (T, rho)                    -- PSE heat pass (only with PSE)
-//     cs4   : double4 (x, y, z, vol; CSPM_TOOL_BITS for a tool particle) FP64; the first 32 bytes of
-//             the record FP32                     -- CSPM sum of the pair pass
 //     rec   : pair record, 192 B (FP64) / 112 B (FP32) -- everything a neighbour contributes
+//     cs4   : FP32 modes: the first 32 bytes of the record -- CSPM sum of the pair pass
 //   neighbour list: int32 nbr[i * cap + k] (row-major), count[i]
 //   neighbour sums: 25 doubles per particle (SoA), written by the pair pass and read by the
 //     per-particle update
@@ -35,9 +34,6 @@ constexpr uint32_t FL_FIXED_ONE = 8u;  // fixed == 1        (src/actions_gpu.cu:
 constexpr uint32_t FL_TOOL_NZ = 16u;   // tool_particle != 0 (src/interactions_gpu.cu:167,230)
 
 constexpr int KEY_BLANK = 0x7fffffff;  // INT_MAX, hash of a hard-blanked particle
-// volume slot of a tool particle's FP64 CSPM entry: a quiet NaN with a payload that no
-// arithmetic result carries (0/0 and inf/inf give the payload-free default NaN)
-constexpr long long CSPM_TOOL_BITS = 0x7ff80000cafe7001ll;
 
 struct State {
   double *x, *y, *z;
@@ -59,16 +55,16 @@ struct State {
 constexpr int STATE_DOUBLES = 3 + 3 + 3 + 6 + 2 + 6 + 3 + 3 + 3 + 2 + 6;
 
 // pair record, FP64: 24 doubles
-struct alignas(16) Rec64 {
+struct alignas(64) Rec64 {
   double x, y, z, h;
-  double T, vol, c, tool;  // with x .. h: what the CSPM sum of the per-lane and tiled forms reads
+  double T, vol, c, tool;
   double vx, vy, vz, rho;
   double A[6];  // (S - p I) / rho^2 for the diagonal, S / rho^2 off the diagonal
   double R[6];  // artificial stress
 };
 
 // pair record, FP32 pair arithmetic: positions stay FP64; the first 32 bytes hold everything
-// the CSPM pass reads (x, y, z, tool, vol)
+// the CSPM sum reads (x, y, z, tool, vol)
 struct alignas(16) Rec32 {
   double x, y, z;
   float tool, vol;
@@ -111,7 +107,6 @@ struct Counters {
   int err_capacity;      // neighbour list overflow
   int err_grid;          // unblanked particle outside the grid
   int max_count;         // largest neighbour count of the last list build
-  int err_list;          // tiled pair pass: a list entry outside the particle's stencil
   unsigned long long candidates;  // candidate pairs visited by the last neighbour pass
   unsigned long long pairs;       // interacting pairs of the last neighbour pass
 };
@@ -193,14 +188,14 @@ void launch_neighbours(hipStream_t s, const GridInfo &g, const int *offsets, con
                        const double2 *pse2, const double *h, const uint32_t *flags,
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
                        int want_pse, unsigned long long *stat_part, int *poison, int cell_tile);
-// pair pass (neighbour sums).  tiled: one wavefront per grid column stages the neighbour
-// records of the column's particles in LDS (offsets and sorted keys of the grid); otherwise one
-// thread per particle gathers them from memory
+// pair pass (neighbour sums); pair_blocks: its workgroups of `block` threads (64, 128 or 256), four
+// lanes per particle in FP64, one in the FP32 modes.  ordered: FP64 sums in the reference's order of
+// evaluation, to the bit (unlocked grids), one lane per particle.  cs4: FP32 modes only
+int pair_blocks(unsigned n_init, int precision, int block);
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
-                 int nl_stride, const int *count, const Consts &c, Counters *cnt,
-                 const GridInfo &g, const int *offsets, const int *key_sorted, int tiled,
-                 double *sums, size_t sum_stride, const int *trav, const double4 *cs4,
-                 int block);
+                 int nl_stride, const int *count, const Consts &c, const Counters *cnt,
+                 double *sums, size_t sum_stride, const int *trav, const double4 *cs4, int block,
+                 bool ordered);
 // visiting order of the list pair pass: strips of `strip` grid columns along y, x-row by x-row
 // inside a strip (trav[t] = particle visited at position t < N); seg_pos holds
 // pair_order_segments(g, strip) ints
@@ -302,13 +297,14 @@ struct BatchLaunch {
   const Inst *inst;  // device array of n descriptors
   int n;
   int precision, pse;
+  int brook;         // an instance conducts heat by Brookshaw's form
   int cell_tile;     // cells per wavefront of the neighbour pass
   BatchGrid cells1;  // num_cell + 1 entries, 256 per workgroup
   BatchGrid cells;   // num_cell entries, 256 per workgroup
   BatchGrid tiles;   // scan tiles of the cell counts
   BatchGrid one;     // one workgroup per instance
   BatchGrid parts;   // N_init particles, 256 per workgroup
-  BatchGrid parts8;  // the same, padded to a multiple of 8 workgroups (XCD-ordered kernels)
+  BatchGrid pairs8;  // pair-pass workgroups, padded to a multiple of 8 (XCD-ordered kernels)
   BatchGrid nbrs8;   // neighbour-pass workgroups, padded to a multiple of 8
   BatchGrid tools;   // one workgroup per tool (at least one per instance)
   BatchGrid search;  // lane-parallel contact search workgroups

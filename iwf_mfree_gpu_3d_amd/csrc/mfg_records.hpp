@@ -6,24 +6,6 @@
 
 namespace mfg {
 
-// what the CSPM sum reads of a neighbour, 32 bytes: FP64 (x, y, z, vol), the volume of a tool
-// particle replaced by the NaN pattern CSPM_TOOL_BITS (no volume m / rho has that payload, so a
-// workpiece particle of negative or non-finite density still counts as the reference counts it);
-// FP32 the record's first 32 bytes (x, y, z, {tool, vol})
-template <class RecT>
-__device__ __forceinline__ double4 cspm_entry(const double *xh, double vol, bool tool);
-template <>
-__device__ __forceinline__ double4 cspm_entry<Rec64>(const double *xh, double vol, bool tool) {
-  return make_double4(xh[0], xh[1], xh[2], tool ? __longlong_as_double(CSPM_TOOL_BITS) : vol);
-}
-template <>
-__device__ __forceinline__ double4 cspm_entry<Rec32>(const double *xh, double vol, bool tool) {
-  struct {
-    float tool, vol;
-  } tv = {tool ? 1.f : 0.f, (float)vol};
-  return make_double4(xh[0], xh[1], xh[2], __builtin_bit_cast(double, tv));
-}
-
 template <class RecT>
 __device__ __forceinline__ void store_rec(RecT *rec, unsigned i, const double *xh, double h,
                                           const double *vh, double rho, const double *A,
@@ -66,7 +48,7 @@ __device__ __forceinline__ void store_rec<Rec32>(Rec32 *rec, unsigned i, const d
 }
 
 // The records of particle i from its half-step (or current) state: the pair record (FP64 or FP32
-// layout), what the CSPM sum reads, the neighbour pass's candidate entry and the PSE entry.
+// layout), what the FP32 CSPM sum reads, the neighbour pass's candidate entry and the PSE entry.
 // p and R: pressure and artificial stress (zero for blanked and tool particles).
 template <class RecT>
 __device__ __forceinline__ void emit_record(unsigned i, const double xh[3], double h,
@@ -80,7 +62,12 @@ __device__ __forceinline__ void emit_record(unsigned i, const double xh[3], doub
   double vol = c.i_mass / rhoh;
   double cs = sqrt_site(c.i_K / rhoh, c.single_sqrt);
   store_rec<RecT>(rec, i, xh, h, vh, rhoh, A, R, Th, vol, cs, tool ? 1.0 : 0.0);
-  cs4[i] = cspm_entry<RecT>(xh, vol, tool);
+  if constexpr (sizeof(RecT) == sizeof(Rec32)) {  // what the FP32 CSPM sum reads of a neighbour
+    struct {
+      float tool, vol;
+    } tv = {tool ? 1.f : 0.f, (float)vol};
+    cs4[i] = make_double4(xh[0], xh[1], xh[2], __builtin_bit_cast(double, tv));
+  }
   // candidate flag of the neighbour pass: 1 blanked, 2 a non-finite value among the fields a
   // neighbour contributes (the reference's loops visit every candidate of the stencil, so
   // 0 * NaN carries such a value into the sums of every particle around it)
