@@ -95,7 +95,8 @@ __constant__ double2 EXP2_J64[64] = {
 // In two halves, so that a wavefront starts the table reads of a whole particle group before it
 // needs the first (waiting on each read where it is issued left the LDS latency exposed: slower
 // than the library routine despite fewer instructions).  exp_reduce: n, r and the table read;
-// exp_finish: the polynomial and the scaling.
+// exp_finish: the polynomial and the scaling.  n is rounded by adding 1.5 2^52, whose low mantissa
+// word then holds it as an integer.
 struct ExpPart {
   double r;
   int n;
@@ -103,10 +104,11 @@ struct ExpPart {
 };
 __device__ __forceinline__ ExpPart exp_reduce(double a, const double2 *tab) {
   a = __builtin_fmax(a, -746.);
-  const double n = __builtin_rint(a * EXP_INV_LN2_64);
+  const double t = __builtin_fma(a, EXP_INV_LN2_64, 0x1.8p52);
+  const double n = t - 0x1.8p52;
   ExpPart e;
   e.r = __builtin_fma(-n, EXP_LN2_64_LO, __builtin_fma(-n, EXP_LN2_64_HI, a));
-  e.n = (int)n;
+  e.n = (int)__builtin_bit_cast(long long, t);
   e.s = tab[e.n & 63];
   return e;
 }
@@ -121,14 +123,18 @@ __device__ __forceinline__ double exp_finish(const ExpPart &e) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// One wavefront per cell.  All particles of a cell share the 25 candidate ranges, so the wave
-// lists the candidates once (in LDS, in the reference's visiting order) and its lanes take
-// candidates: the candidate loads are coalesced.  The cell's particles are taken in groups of up
-// to NB_GROUP; each 64-candidate chunk is loaded once and tested against every particle of the
-// group (their data broadcast from LDS), which amortises the loads and gives the wave
-// independent work to overlap.  For each particle an ordered ballot compaction appends the kept
-// candidates to its row-major list; its PSE sum is a per-lane partial reduced over the wave.
+// One wavefront per cell.  All particles of a cell share the 25 candidate ranges (in the reference's
+// visiting order) and the wave's lanes take candidates: the candidate loads are coalesced.  The
+// cell's particles are taken in groups of up to NB_GROUP; each 64-candidate chunk is loaded once
+// (ahead, while the chunk before it is worked on) and tested against every particle of the group, which
+// amortises the loads and gives the wave independent work to overlap.  For each particle the ballot
+// of the kept candidates appends them in order to its row-major list; its PSE sum is a per-lane
+// partial reduced over the wave.
 //   PSE_MODE 0: no PSE sum; 1: FP64 PSE terms; 2: FP32 PSE terms accumulated in FP64
+// Bound by vector issue (84 % busy at 1M).  1M single-grain cut, FP64 1.27 -> 0.94 ms, FP32 0.92 ->
+// 0.74 ms, 65k FP64 131 -> 99 us: a group of four against 64 candidates took 211 vector instructions
+// and 28 LDS reads with its particles' data in LDS, a branch per particle and the candidates listed
+// in LDS beforehand; now 181 and 2 (+ 4 table reads), the listing included.
 // Cells (wavefronts) per workgroup.  One: cells differ in particles and candidates, and the
 // waves of a larger workgroup wait for its slowest cell at the end (the statistics sum) while
 // holding their slots; measured 12-14 % slower with four.
@@ -137,7 +143,6 @@ __device__ __forceinline__ double exp_finish(const ExpPart &e) {
 #endif
 constexpr int NB_WAVES = NB_WAVES_PER_BLOCK;
 constexpr int NB_BLOCK = 64 * NB_WAVES;
-constexpr int NB_LCAP = 1024;           // candidates listed in LDS per cell (beyond: searched)
 #ifndef NB_GROUP_SIZE
 #define NB_GROUP_SIZE 4
 #endif
@@ -149,14 +154,6 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-struct NbParticle {
-  double x, y, z, fourh2;
-  double Ti, coef, inv_h2;
-  float coef_f, inv_h2_f;  // FP32 copies for PSE_MODE 2
-  int nolist;              // blanked, or its own record holds a non-finite value: no list
-  int pad;
-};
-
 // Candidate q of a cell's list as the neighbour pass needs it: particle index, (x, y, z, flag)
 // and (T, m / rho).
 struct NbCand {
@@ -165,12 +162,73 @@ struct NbCand {
   double2 tr;
 };
 
-// The particles [s, e) of one cell against its T candidates (fetch(q, valid, g0) gives candidate
-// q; lanes with !valid get any readable record, masked off): support test, PSE sum, ordered list
-// write.  pd: this wavefront's LDS slots for a group's particle data.
+// inclusive scan over the wavefront of ints >= 0: sums, or the largest so far
+template <bool MAX>
+__device__ __forceinline__ int wave_scan(int v) {
+  auto step = [&](auto ctrl, auto rows) {
+    const int t = __builtin_amdgcn_update_dpp(0, v, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    v = MAX ? max(v, t) : v + t;
+  };
+  step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{});  // row_shr 1, 2, 4, 8
+  step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+  step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{});
+  step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+  step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{});  // row_bcast 15, 31
+  step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+  return v;
+}
+
+// v of the lane at a fixed distance inside its row of 16
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+
+// exchanges rows of 16 or 32 lanes between two registers and adds them: of 32, lanes 0-31 get
+// a(l) + a(l + 32) and lanes 32-63 b(l - 32) + b(l); of 16, rows 0 and 2 get a's row pairs, rows 1
+// and 3 b's
+template <int ROWS>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  const long long ia = __builtin_bit_cast(long long, a), ib = __builtin_bit_cast(long long, b);
+  auto swap = [](unsigned x, unsigned y) {
+    if constexpr (ROWS == 32) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+  };
+  const auto lo = swap((unsigned)ia, (unsigned)ib), hi = swap((unsigned)(ia >> 32), (unsigned)(ib >> 32));
+  return __builtin_bit_cast(double, (unsigned long long)hi[0] << 32 | lo[0]) +
+         __builtin_bit_cast(double, (unsigned long long)hi[1] << 32 | lo[1]);
+}
+
+// The sums over the wavefront of four values: row r of 16 lanes gets that of a[row_sum_of(r)].  9
+// instructions for the first two halvings of all four and 12 for the last four, against 18 per value.
+constexpr int row_sum_of(int row) { return row == 1 ? 2 : row == 2 ? 1 : row; }
+__device__ __forceinline__ double row_sums(const double a[4]) {
+  double v = swap_add<16>(swap_add<32>(a[0], a[1]), swap_add<32>(a[2], a[3]));
+  v += dpp64<0x128>(v);  // row_ror 8, 4, 2, 1
+  v += dpp64<0x124>(v);
+  v += dpp64<0x122>(v);
+  v += dpp64<0x121>(v);
+  return v;
+}
+
+// lane u's value in every lane, as a scalar
+__device__ __forceinline__ double read_lane(double v, int u) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, u);
+  const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), u);
+  return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+
+// The particles [s, e) of one cell against its T candidates (fetch(b0) gives each lane candidate
+// b0 + lane, or past T any readable record, masked off; b0 ascends by 64 from 0): support test, PSE
+// sum, ordered list write.  A group's
+// particle data are scalars: read from LDS for every chunk of candidates they were two thirds of the
+// LDS traffic, which returns a value per lane also where all lanes read one address.
 template <int PSE_MODE, class Fetch>
-__device__ __forceinline__ void cell_lists(int s, int e, int T, int lane, NbParticle *pd,
-                                           Fetch &&fetch, const double4 *__restrict__ nl4,
+__device__ __forceinline__ void cell_lists(int s, int e, int T, int lane, Fetch &&fetch, const double4 *__restrict__ nl4,
                                            const double2 *__restrict__ pse2,
                                            const double *__restrict__ h,
                                            const uint32_t *__restrict__ flags, const Consts &c,
@@ -178,177 +236,170 @@ __device__ __forceinline__ void cell_lists(int s, int e, int T, int lane, NbPart
                                            double *__restrict__ T_t, Counters *cnt,
                                            int *__restrict__ poison, const double2 *exp_tab,
                                            unsigned long long &n_cand, unsigned long long &n_pair) {
-  for (int g0 = s; g0 < e; g0 += NB_GROUP) {
-    const int gn = min(NB_GROUP, e - g0);
-    if (lane < gn) {
-      const int p = g0 + lane;
-      const double4 pi = nl4[p];
-      const double hi = h[p];
-      NbParticle d;
-      d.x = pi.x; d.y = pi.y; d.z = pi.z;
-      d.fourh2 = 4 * hi * hi;
-      d.nolist = pi.w != 0. ? 1 : 0;
-      d.pad = 0;
-      d.Ti = 0.; d.coef = 0.; d.inv_h2 = 0.;
-      if (PSE_MODE) {
-        d.Ti = pse2[p].x;
-        const double h2 = hi * hi;
-        const double h4 = h2 * h2;
-        const double h5 = hi * h4;
-        d.coef = +4. / (h5 * PI_D * sqrt_rn(PI_D));
-        d.inv_h2 = 1. / h2;
-      }
-      d.coef_f = (float)d.coef;
-      d.inv_h2_f = (float)d.inv_h2;
-      pd[lane] = d;
+  static_assert(NB_GROUP == 4, "row_sums");
+  // a group of GN particles from g0: GN is a compile-time constant, so that the work on one candidate
+  // for all of them is one block of independent chains (behind a branch each, they ran one after the
+  // other)
+  auto group = [&](const int g0, auto gn_c) {
+    constexpr int gn = decltype(gn_c)::value;
+    // lane u: particle u of the group (the others repeat the last)
+    const int pl = g0 + min(lane, gn - 1);
+    const double4 pi = nl4[pl];
+    const double hi = h[pl], h2 = hi * hi;
+    double Tl = 0., il = 0., cl = 0.;
+    if (PSE_MODE) {
+      Tl = pse2[pl].x;
+      il = rcp64(h2);
     }
-    wave_lds_sync();
-    // per particle of the group: list length so far, PSE partial, whether it gets a list, its
-    // row (all wave-uniform but the PSE partial)
-    int np[NB_GROUP];
-    double acc[NB_GROUP];
-    bool listed[NB_GROUP];
-    int *row[NB_GROUP];
+    if (PSE_MODE == 2) cl = +4. / (hi * (h2 * h2) * PI_D * sqrt_rn(PI_D));
+    // squared support; -1 (no candidate is inside) for a particle that gets no list: blanked, or its
+    // own record non-finite
+    const double fl = pi.w == 0. ? 4 * hi * hi : -1.;
+    // per particle of the group (all wave-uniform but the PSE partial): position, squared support,
+    // temperature, 1 / h^2, the FP32 PSE constants, list length so far
+    double px[gn], py[gn], pz[gn], p4h2[gn], pT[gn], pih2[gn];
+    float pc_f[gn], pih2_f[gn];
+    int np[NB_GROUP] = {0, 0, 0, 0};
+    double acc[NB_GROUP] = {0., 0., 0., 0.};
+    int *const rows = nbr + (size_t)g0 * cap;
 #pragma unroll
-    for (int u = 0; u < NB_GROUP; u++) {
-      np[u] = 0;
-      acc[u] = 0.;
-      listed[u] = u < gn && __builtin_amdgcn_readfirstlane(pd[u < gn ? u : 0].nolist) == 0;
-      row[u] = nbr + (size_t)(g0 + u) * cap;
+    for (int u = 0; u < gn; u++) {
+      px[u] = read_lane(pi.x, u);
+      py[u] = read_lane(pi.y, u);
+      pz[u] = read_lane(pi.z, u);
+      p4h2[u] = read_lane(fl, u);
+      pT[u] = read_lane(Tl, u);
+      pih2[u] = read_lane(il, u);
+      pc_f[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, (float)cl), u));
+      pih2_f[u] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, (float)il), u));
     }
     // a non-finite record among the candidates poisons every particle of the group (they share
     // the stencil)
     unsigned long long bad = 0;
     // one chunk of 64 candidates against the group; TAIL: the last chunk, lanes past T masked
-    auto chunk = [&](const int b0, auto tail) {
+    auto chunk = [&](const int b0, const NbCand &cd, auto tail) {
       constexpr bool TAIL = decltype(tail)::value;
-      const int q = b0 + lane;
-      const bool valid = !TAIL || q < T;
-      const NbCand cd = fetch(q, valid, g0);
+      const bool valid = !TAIL || b0 + lane < T;
       const int j = cd.j;
       const double4 pj = cd.pj;
-      const double2 tr = cd.tr;
-      const bool cand_ok = valid && pj.w == 0.;
-      bad |= __builtin_amdgcn_ballot_w64(valid && pj.w == 2.);
+      double2 tr = cd.tr;
+      unsigned long long in_chunk = ~0ull;
+      if (TAIL) in_chunk = __builtin_amdgcn_ballot_w64(valid);
+      const unsigned long long cand_ok = __builtin_amdgcn_ballot_w64(pj.w == 0.) & in_chunk;
+      bad |= __builtin_amdgcn_ballot_w64(pj.w == 2.) & in_chunk;
+      if (PSE_MODE && TAIL) tr.y = valid ? tr.y : 0.;  // masked lanes add zero
       float try_f = 0.f;
       if (PSE_MODE == 2) try_f = (float)tr.y;
       // lapl_pse (src/kernels.cuh:71-92) times (T_j - T_i) m / rho_j
       // (src/interactions_gpu.cu:124-147); r^2 / h^2 as r^2 times 1 / h^2 and m / rho_j from the
-      // record, each within two ulps of the reference's sqrt-square and divisions.  Masked lanes
-      // add zero (adding a zero leaves the sum as it is).  FP64: the exp of every particle of the
+      // record, each within two ulps of the reference's sqrt-square and divisions.  FP64: the kernel's
+      // constant 4 / (h^5 pi sqrt(pi)) multiplies the sum; the exp of every particle of the
       // group is reduced (table reads started) in the first loop and finished in the second.
-      ExpPart ex[NB_GROUP];
+      ExpPart ex[gn];
 #pragma unroll
-      for (int u = 0; u < NB_GROUP; u++) {
-        if (u < gn) {
-          const NbParticle &d = pd[u];
-          const double xij = d.x - pj.x, yij = d.y - pj.y, zij = d.z - pj.z;
-          const double rr2 = xij * xij + yij * yij + zij * zij;
-          const bool inside = !(rr2 >= d.fourh2 || rr2 < 1e-8);  // src/kernels.cuh:41
-          if (PSE_MODE == 1) ex[u] = exp_reduce(-rr2 * d.inv_h2, exp_tab);
-          if (PSE_MODE == 2) {
-            const float w2 = d.coef_f * __expf(-(float)rr2 * d.inv_h2_f);
-            const double t = (double)((float)(tr.x - d.Ti) * w2 * try_f);
-            acc[u] += TAIL ? (valid ? t : 0.) : t;
-          }
-          // ordered compaction: the kept candidates of the chunk go to the row in lane order
-          const bool ok = cand_ok && listed[u] && inside;
-          const unsigned long long m = __builtin_amdgcn_ballot_w64(ok);
-          const unsigned pos =
-              __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-          if (ok && (int)pos < cap - np[u]) row[u][np[u] + (int)pos] = j;
-          np[u] += __popcll(m);
+      for (int u = 0; u < gn; u++) {
+        const double xij = px[u] - pj.x, yij = py[u] - pj.y, zij = pz[u] - pj.z;
+        const double rr2 = xij * xij + yij * yij + zij * zij;
+        if (PSE_MODE == 1) ex[u] = exp_reduce(-rr2 * pih2[u], exp_tab);
+        if (PSE_MODE == 2) {
+          const float w2 = pc_f[u] * __expf(-(float)rr2 * pih2_f[u]);
+          acc[u] += (double)((float)(tr.x - pT[u]) * w2 * try_f);
         }
+        // ordered compaction: the candidates inside the support (src/kernels.cuh:41) go to the row in
+        // lane order
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(rr2 < p4h2[u]) &
+                                     ~__builtin_amdgcn_ballot_w64(rr2 < 1e-8) & cand_ok;
+        const int n = __popcll(m);
+        const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+            (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)(np[u] + u * cap)));
+        if (np[u] + n <= cap) {
+          if (__builtin_amdgcn_inverse_ballot_w64(m)) rows[pos] = j;
+        } else if (__builtin_amdgcn_inverse_ballot_w64(m) && (int)pos < (u + 1) * cap) {
+          rows[pos] = j;
+        }
+        np[u] += n;
       }
       if (PSE_MODE == 1) {
 #pragma unroll
-        for (int u = 0; u < NB_GROUP; u++) {
-          if (u < gn) {
-            const double w2 = pd[u].coef * exp_finish(ex[u]);
-            const double t = (tr.x - pd[u].Ti) * w2 * tr.y;
-            acc[u] += TAIL ? (valid ? t : 0.) : t;
-          }
-        }
+        for (int u = 0; u < gn; u++)
+          acc[u] = __builtin_fma(tr.y * exp_finish(ex[u]), tr.x - pT[u], acc[u]);
       }
     };
+    // the next chunk's candidates are loaded while a chunk is worked on
+    NbCand cd = fetch(0);
     int b0 = 0;
-    for (; b0 + 64 <= T; b0 += 64) chunk(b0, std::false_type{});
-    if (b0 < T) chunk(b0, std::true_type{});
-#pragma unroll
-    for (int u = 0; u < NB_GROUP; u++) {
-      if (u < gn) {
-        double a = acc[u];
-        if (PSE_MODE) {
-#pragma unroll
-          for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    for (; b0 + 64 <= T; b0 += 64) {
+      const NbCand nx = fetch(b0 + 64);
+      chunk(b0, cd, std::false_type{});
+      cd = nx;
+    }
+    if (b0 < T) chunk(b0, cd, std::true_type{});
+    // row r of 16 lanes ends with the sum of particle row_sum_of(r), whose results its first lane
+    // writes
+    double sum = 0.;
+    if (PSE_MODE) sum = row_sums(acc);
+    const int row_id = lane >> 4;
+    const int u = row_sum_of(row_id);
+    const int n_u = u == 0 ? np[0] : u == 1 ? np[1] : u == 2 ? np[2] : np[3];
+    if ((lane & 15) == 0 && u < gn) {
+      const int p = g0 + u;
+      poison[p] = bad != 0 ? 1 : 0;
+      if (n_u > cap) {
+        atomicOr(&cnt->err_capacity, 1);
+        atomicMax(&cnt->max_count, n_u);
+      }
+      count[p] = min(n_u, cap);
+      if (PSE_MODE) {
+        if (PSE_MODE == 1) {
+          const double hi = h[p], h2 = hi * hi;
+          sum *= 4. * rcp64(h2 * h2 * hi * (PI_D * 1.7724538509055160273));  // sqrt(pi)
         }
-        const int p = g0 + u;
-        if (lane == 0) {
-          poison[p] = bad != 0 ? 1 : 0;
-          if (np[u] > cap) {
-            atomicOr(&cnt->err_capacity, 1);
-            atomicMax(&cnt->max_count, np[u]);
-          }
-          count[p] = np[u] > cap ? cap : np[u];
-          if (PSE_MODE) T_t[p] = ((flags[p] & FL_TOOL) ? c.alpha_tool : c.alpha_wp) * a;
-        }
-        n_cand += (unsigned long long)T;
-        n_pair += (unsigned long long)(np[u] > cap ? cap : np[u]);
+        T_t[p] = ((flags[p] & FL_TOOL) ? c.alpha_tool : c.alpha_wp) * sum;
       }
     }
-    wave_lds_sync();  // the next group overwrites pd
+#pragma unroll
+    for (int v = 0; v < gn; v++) {
+      n_cand += (unsigned long long)T;
+      n_pair += (unsigned long long)min(np[v], cap);
+    }
+  };
+  int g0 = s;
+  for (; g0 + NB_GROUP <= e; g0 += NB_GROUP) group(g0, std::integral_constant<int, NB_GROUP>{});
+  switch (e - g0) {
+    case 1: group(g0, std::integral_constant<int, 1>{}); break;
+    case 2: group(g0, std::integral_constant<int, 2>{}); break;
+    case 3: group(g0, std::integral_constant<int, 3>{}); break;
   }
 }
 
 // The candidate ranges of one cell: for stencil column r = lane < nr, the particles of rows
-// [lo_k, hi_k) of grid column (lo_i + r / nj, lo_j + r % nj); T, and the exclusive prefix of the
-// range lengths and each range's first particle in LDS (pref, rst; entries past nr hold T).
+// [lo_k, hi_k) of grid column (lo_i + r / nj, lo_j + r % nj): each lane's first particle st, their
+// number len and the exclusive prefix ex of the lengths; returns their sum T.
 __device__ __forceinline__ int cell_ranges(const GridInfo &g, const int *__restrict__ off, int lane,
                                            int lo_i, int lo_j, int nj, int nr, int lo_k, int hi_k,
-                                           int *pref, int *rst, int &st, int &len) {
+                                           int &st, int &len, int &ex) {
   const int nyz = g.ny * g.nz;
   st = 0;
   len = 0;
   if (lane < nr) {
-    const int ii = lo_i + lane / nj, jj = lo_j + lane % nj;
-    const long cb = (long)ii * nyz + (long)jj * g.nz;
+    const int q = nj == 5 ? (lane * 52) >> 8 : lane / nj;  // lane / 5 for lane < 25
+    const long cb = (long)(lo_i + q) * nyz + (long)(lo_j + lane - q * nj) * g.nz;
     st = off[cb + lo_k];
     len = off[cb + hi_k] - st;
   }
-  int incl = len;
-#pragma unroll
-  for (int o = 1; o < 32; o <<= 1) {
-    const int t = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += t;
-  }
-  const int T = __builtin_amdgcn_readfirstlane(__shfl(incl, 31, 64));
-  if (lane < 32) {
-    pref[lane] = incl - len;
-    rst[lane] = st;
-  }
-  wave_lds_sync();
-  return T;
+  const int incl = wave_scan<false>(len);  // lanes from nr on hold 0
+  ex = incl - len;
+  return __builtin_amdgcn_readlane(incl, 63);
 }
 
-// last stencil column whose prefix is <= q (never an empty one)
-__device__ __forceinline__ int range_of(const int *pref, int nr, int q) {
-  int lo = 0, hi = nr - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (pref[mid] <= q) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
-// minimum waves per SIMD the kernel is compiled for (register budget): FP64 PSE 6 (80 VGPRs, no
-// spill; 7 waves spill and are no faster), the others 8; faster than the 5 / 7 waves the
-// unconstrained register use gives
+// minimum waves per SIMD the kernel is compiled for (register budget): FP64 PSE 6, the others 7;
+// 1M single-grain cut FP64 0.94 ms (5 waves 0.98, 4 waves 0.98), FP32 0.74 (6 waves 0.77, 5 waves
+// 0.76)
 #ifndef NB_WAVES_FP64_PSE
 #define NB_WAVES_FP64_PSE 6
 #endif
 #ifndef NB_WAVES_OTHER
-#define NB_WAVES_OTHER 8
+#define NB_WAVES_OTHER 7
 #endif
 // body of workgroup b of nb (the single-instance kernel and the batched one below); each wavefront
 // takes CPW consecutive cells in turn (the cell tile), so that an empty cell costs two loads
@@ -360,10 +411,7 @@ __device__ __forceinline__ void cell_neighbours(
     const double *__restrict__ h, const uint32_t *__restrict__ flags, const Consts &c,
     int *__restrict__ nbr, int cap, int *__restrict__ count, double *__restrict__ T_t,
     Counters *cnt, unsigned long long *__restrict__ stat_part, int *__restrict__ poison) {
-  __shared__ int s_cand[NB_WAVES][NB_LCAP];
-  __shared__ int s_pref[NB_WAVES][32];
-  __shared__ int s_rst[NB_WAVES][32];
-  __shared__ NbParticle s_pd[NB_WAVES][NB_GROUP];
+  __shared__ int s_start[NB_WAVES][64];
   __shared__ unsigned long long s_stat[NB_WAVES][2];
   __shared__ double2 s_exp[PSE_MODE == 1 ? 64 : 1];
   const int lane = threadIdx.x & 63;
@@ -375,44 +423,39 @@ __device__ __forceinline__ void cell_neighbours(
   const long c0 = ((long)xcd_map(b, nb) * NB_WAVES + w) * CPW;
   unsigned long long n_cand = 0, n_pair = 0;
   // the particles [s, e) of one cell against its stencil's candidates
-  auto do_cell = [&](const long cell, const int s, const int e) {
-    const int nyz = g.ny * g.nz;
-    const int gi = (int)(cell / nyz);
-    const int gj = (int)((cell - (long)gi * nyz) / g.nz);
-    const int gk = (int)(cell % g.nz);
+  auto do_cell = [&](const long c_, const int s, const int e) {
+    const unsigned cell = (unsigned)c_, nyz = (unsigned)(g.ny * g.nz);  // cell hashes are 32-bit
+    const int gi = (int)(cell / nyz), rem = (int)(cell - gi * nyz);
+    const int gj = rem / g.nz, gk = rem - gj * g.nz;
     const int lo_i = gi - 2 < 0 ? 0 : gi - 2, hi_i = gi + 3 > g.nx ? g.nx : gi + 3;
     const int lo_j = gj - 2 < 0 ? 0 : gj - 2, hi_j = gj + 3 > g.ny ? g.ny : gj + 3;
     const int lo_k = gk - 2 < 0 ? 0 : gk - 2, hi_k = gk + 3 > g.nz ? g.nz : gk + 3;
     const int nj = hi_j - lo_j, nr = (hi_i - lo_i) * nj;
-    int st, len;
-    const int T = cell_ranges(g, off, lane, lo_i, lo_j, nj, nr, lo_k, hi_k, s_pref[w], s_rst[w],
-                              st, len);
-    const bool in_lds = T <= NB_LCAP;
-    if (in_lds) {
-      for (int r = 0; r < nr; r++) {
-        const int rs = s_rst[w][r], rp = s_pref[w][r], rl = s_pref[w][r + 1] - rp;
-        for (int t = lane; t < rl; t += 64) s_cand[w][rp + t] = rs + t;
-      }
+    int st, len, ex;
+    const int T = cell_ranges(g, off, lane, lo_i, lo_j, nj, nr, lo_k, hi_k, st, len, ex);
+    // Candidate q of range r is particle q + (st - ex), and st - ex ascends over the non-empty
+    // ranges: of the 64 candidates from b0, those a range starts at get its st - ex from LDS, the rest
+    // by a running maximum (16 instructions, against a loop over the 25 ranges before).
+    int carry = 0;
+    auto fetch = [&](int b0) {
+      if (b0 == 0) carry = 0;
+      s_start[w][lane] = 0;
       wave_lds_sync();
-    }
-    auto fetch = [&](int q, bool valid, int g0) {
+      if (len > 0 && (unsigned)(ex - b0) < 64u) s_start[w][ex - b0] = st - ex;
+      wave_lds_sync();
+      const int d = max(wave_scan<true>(s_start[w][lane]), carry);
+      wave_lds_sync();
+      carry = __builtin_amdgcn_readlane(d, 63);
+      const int q = b0 + lane;
       NbCand cd;
-      int j = g0;
-      if (valid) {
-        if (in_lds) {
-          j = s_cand[w][q];
-        } else {
-          const int r = range_of(s_pref[w], nr, q);
-          j = s_rst[w][r] + (q - s_pref[w][r]);
-        }
-      }
-      cd.j = j;
-      cd.pj = nl4[j];
+      cd.j = q < T ? d + q : s;
+      // byte offsets of 32 bits: a particle takes over 2 KB of device memory, so all are below 2^27
+      cd.pj = *(const double4 *)((const char *)nl4 + (unsigned)cd.j * 32u);
       cd.tr = make_double2(0., 1.);
-      if (PSE_MODE) cd.tr = pse2[j];
+      if (PSE_MODE) cd.tr = *(const double2 *)((const char *)pse2 + (unsigned)cd.j * 16u);
       return cd;
     };
-    cell_lists<PSE_MODE>(s, e, T, lane, s_pd[w], fetch, nl4, pse2, h, flags, c, nbr, cap, count,
+    cell_lists<PSE_MODE>(s, e, T, lane, fetch, nl4, pse2, h, flags, c, nbr, cap, count,
                          T_t, cnt, poison, s_exp, n_cand, n_pair);
   };
   if constexpr (CPW == 1) {
@@ -719,15 +762,6 @@ __device__ __forceinline__ void finish_sums(const Consts &c, const PairAcc &p, c
     }
     ps.Tl = 2. * k.k1 * s;
   }
-}
-
-// 1 / a: the hardware reciprocal (relative error below 2^-24) and one step of third order, which
-// gives the correctly rounded quotient for all but ties (2^24 spread arguments: all equal to 1. / a)
-__device__ __forceinline__ double rcp64(double a) {
-  const double r = __builtin_amdgcn_rcp(a);
-  double d = __builtin_fma(-a, r, 1.);
-  d = __builtin_fma(d, d, d);
-  return __builtin_fma(r, d, r);
 }
 
 // r = sqrt(r2) as the reference's sqrt site evaluates it, and 1 / r.  single: the float root of

@@ -58,6 +58,15 @@ __device__ __forceinline__ double sqrt_site(double a, int single) {
   return single ? (double)sqrt_rn((float)a) : sqrt_rn(a);
 }
 
+// 1 / a: the hardware reciprocal (relative error below 2^-24) and one step of third order, which
+// gives the correctly rounded quotient for all but ties (2^24 spread arguments: all equal to 1. / a)
+__device__ __forceinline__ double rcp64(double a) {
+  const double r = __builtin_amdgcn_rcp(a);
+  double d = __builtin_fma(-a, r, 1.);
+  d = __builtin_fma(d, d, d);
+  return __builtin_fma(r, d, r);
+}
+
 // ---- small symmetric / general 3x3 helpers in GLM storage m[col][row] ------------------------
 struct M3 {
   double m[3][3];
