@@ -216,6 +216,9 @@ struct mfg_particles {
   // leap-frog start-of-step copies (lazily allocated)
   double *vder = nullptr, *sder = nullptr, *nrm = nullptr, *x0 = nullptr;
   int *flag_d = nullptr;
+  double *stage = nullptr;  // pinned host buffer of small downloads (made by the first)
+  size_t stage_bytes = 0;
+  std::mutex stage_use;
   unsigned long long *stat_part = nullptr;  // per-workgroup (candidates, pairs) of the last list build
   int stat_cap = 0, stat_n = 0;
   // lane-parallel exhaustive contact search (lazily sized)
@@ -286,6 +289,8 @@ struct mfg_tool {
 struct mfg_tool_forces {
   unsigned n = 0;
   float *d = nullptr;
+  float *h = nullptr;  // pinned, what get_host reads
+  std::mutex h_use;
 };
 
 struct mfg_leap_frog {
@@ -321,6 +326,7 @@ void free_particles(mfg_particles *p) {
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (p->cnt_h) (void)hipHostFree(p->cnt_h);
+  if (p->stage) (void)hipHostFree(p->stage);
 }
 
 int grid_alloc(mfg_grid *g) {
@@ -554,9 +560,8 @@ int run_neighbours(mfg_grid *g, mfg_particles *p, const Consts &c, int want_pse,
   return MFG_OK;
 }
 
-int check_counters(mfg_particles *p) {
-  HIP_TRY(hipMemcpyAsync(p->cnt_h, p->cnt, sizeof(Counters), hipMemcpyDeviceToHost, g_lib.stream));
-  HIP_TRY(hipStreamSynchronize(g_lib.stream));
+// N and the device's errors from the pinned mirror (its copy has arrived)
+int judge_counters(mfg_particles *p) {
   p->N_host = p->cnt_h->N;
   if (p->cnt_h->err_capacity)
     return fail(MFG_ERR_CAPACITY, "a particle has %d neighbours, list capacity is %d",
@@ -566,6 +571,52 @@ int check_counters(mfg_particles *p) {
   // particle was hard-blanked
   if (p->N_host == 0 && p->N_init > 0)
     return fail(MFG_ERR_ALL_BLANKED, "all particles left bbox due to blanking");
+  return MFG_OK;
+}
+
+int check_counters(mfg_particles *p) {
+  launch_words_to_host(g_lib.stream, p->cnt, p->cnt_h, sizeof(Counters) / 4);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipStreamSynchronize(g_lib.stream));
+  return judge_counters(p);
+}
+
+// A field of every particle to host memory, interleaved by the device.  Fields of up to STAGE_BYTES:
+// the kernel writes them and the counters into the set's pinned buffer, one launch and one wait (a
+// copy command takes 60 us however small: 8,000 positions 394 -> 24 us).  Larger ones go
+// through the pair-sum array (free between two calls: the pair pass writes it and the update of the
+// same call reads it) straight into the caller's memory.
+constexpr size_t STAGE_BYTES = (size_t)1 << 20;
+int download_field(mfg_particles *p, const PackField &f, double *host) {
+  std::lock_guard<std::mutex> lock(p->stage_use);
+  hipStream_t s = g_lib.stream;
+  const size_t bytes = sizeof(double) * f.w * (size_t)p->N_init;
+  if (bytes <= STAGE_BYTES) {
+    if (bytes > p->stage_bytes) {
+      if (p->stage) (void)hipHostFree(p->stage);
+      p->stage = nullptr;
+      p->stage_bytes = 0;
+      const size_t want = std::min(STAGE_BYTES, sizeof(double) * 9 * (size_t)p->N_init);
+      HIP_TRY(hipHostMalloc(&p->stage, want));
+      p->stage_bytes = want;
+    }
+    launch_pack_field(s, f, p->N_init, p->stage, p->cnt, p->cnt_h);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(s));
+    const int rc = judge_counters(p);
+    if (rc == MFG_OK) std::memcpy(host, p->stage, bytes);
+    return rc;
+  }
+  const void *dev = f.src[0];
+  if (f.w != 1 || f.kind != PACK_F64) {
+    launch_pack_field(s, f, p->N_init, p->sums, nullptr, nullptr);
+    HIP_TRY(hipGetLastError());
+    dev = p->sums;
+  }
+  const int rc = check_counters(p);
+  if (rc != MFG_OK) return rc;
+  HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
   return MFG_OK;
 }
 
@@ -1085,58 +1136,21 @@ int mfg_particle_gpu_restore(mfg_particles *p, const void *host) {
 int mfg_particle_gpu_download(mfg_particles *p, int f, double *host) {
   NEED_LIB();
   if (!p || !host) return fail(MFG_ERR_ARG, "null argument");
-  // errors of the queued steps surface here too (the copies below synchronise anyway)
-  const int rc0 = check_counters(p);
-  if (rc0 != MFG_OK) return rc0;
   const unsigned N = p->N_init;
+  const size_t n = padded(N);
   const State &st = p->st();
   hipStream_t s = g_lib.stream;
-  std::vector<double> a(N);
-  auto get = [&](const double *src) -> bool {
-    return hipMemcpyAsync(a.data(), src, sizeof(double) * N, hipMemcpyDeviceToHost, s) == hipSuccess &&
-           hipStreamSynchronize(s) == hipSuccess;
+  // errors of the queued steps surface here too
+  auto put1 = [&](const double *x) { return download_field(p, PackField{{x}, 1, PACK_F64}, host); };
+  auto put3 = [&](const double *x, const double *y, const double *z) {
+    return download_field(p, PackField{{x, y, z}, 3, PACK_F64}, host);
   };
-  auto put3 = [&](const double *x, const double *y, const double *z) -> int {
-    const double *src[3] = {x, y, z};
-    for (int k = 0; k < 3; k++) {
-      if (!get(src[k])) return fail(MFG_ERR_HIP, "download failed");
-      for (unsigned i = 0; i < N; i++) host[3 * (size_t)i + k] = a[i];
-    }
-    return MFG_OK;
+  // GLM storage m[col][row]; symmetric entries mirrored
+  auto put_sym = [&](double *const *S) {
+    return download_field(
+        p, PackField{{S[0], S[3], S[5], S[3], S[1], S[4], S[5], S[4], S[2]}, 9, PACK_F64}, host);
   };
-  auto put_sym = [&](double *const *S6) -> int {
-    // GLM storage m[col][row]; symmetric entries mirrored
-    const int dst_of[6][2] = {{0, 0}, {4, 4}, {8, 8}, {1, 3}, {5, 7}, {2, 6}};
-    for (int k = 0; k < 6; k++) {
-      if (!get(S6[k])) return fail(MFG_ERR_HIP, "download failed");
-      for (unsigned i = 0; i < N; i++) {
-        host[9 * (size_t)i + dst_of[k][0]] = a[i];
-        host[9 * (size_t)i + dst_of[k][1]] = a[i];
-      }
-    }
-    return MFG_OK;
-  };
-  auto put1 = [&](const double *x) -> int {
-    if (!get(x)) return fail(MFG_ERR_HIP, "download failed");
-    std::memcpy(host, a.data(), sizeof(double) * N);
-    return MFG_OK;
-  };
-  auto put_u = [&](const void *src, int kind) -> int {
-    std::vector<uint32_t> u(N);
-    if (hipMemcpyAsync(u.data(), src, sizeof(uint32_t) * N, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
-      return fail(MFG_ERR_HIP, "download failed");
-    for (unsigned i = 0; i < N; i++) {
-      uint32_t v = u[i];
-      switch (kind) {
-        case 0: host[i] = (v & FL_FIXED_ONE) ? 1. : ((v & FL_FIXED) ? 2. : 0.); break;
-        case 1: host[i] = (v & FL_BLANKED) ? 1. : 0.; break;
-        case 2: host[i] = (v & FL_TOOL) ? 1. : ((v & FL_TOOL_NZ) ? 2. : 0.); break;
-        default: host[i] = (double)(int)v; break;
-      }
-    }
-    return MFG_OK;
-  };
+  auto put_u = [&](const void *u, int kind) { return download_field(p, PackField{{u}, 1, kind}, host); };
   switch (f) {
     case MFG_F_POS: return put3(st.x, st.y, st.z);
     case MFG_F_VEL: return put3(st.vx, st.vy, st.vz);
@@ -1154,54 +1168,48 @@ int mfg_particle_gpu_download(mfg_particles *p, int f, double *host) {
     case MFG_F_T: return put1(st.T);
     case MFG_F_RHO_T: return put1(st.rho_t);
     case MFG_F_T_T: return put1(st.T_t);
-    case MFG_F_FIXED: return put_u(st.flags, 0);
-    case MFG_F_BLANKED: return put_u(st.flags, 1);
-    case MFG_F_TOOL: return put_u(st.flags, 2);
-    case MFG_F_ID: return put_u(st.id, 3);
-    case MFG_F_HASH: return put_u(p->key_sorted, 3);
-    case MFG_F_IDX: return put_u(p->order, 3);
+    case MFG_F_FIXED: return put_u(st.flags, PACK_FIXED);
+    case MFG_F_BLANKED: return put_u(st.flags, PACK_BLANKED);
+    case MFG_F_TOOL: return put_u(st.flags, PACK_TOOL);
+    case MFG_F_ID: return put_u(st.id, PACK_I32);
+    case MFG_F_HASH: return put_u(p->key_sorted, PACK_I32);
+    case MFG_F_IDX: return put_u(p->order, PACK_I32);
     case MFG_F_S_DER:
     case MFG_F_V_DER: {
+      const int rc = check_counters(p);
+      if (rc != MFG_OK) return rc;
       const double *m = f == MFG_F_V_DER ? p->vder : p->sder;
       if (!m) return fail(MFG_ERR_STATE, "no velocity gradient / stress divergence yet (interactions_monaghan computes them)");
-      const size_t n = padded(N);
-      for (int k = 0; k < 9; k++) {
-        if (!get(m + k * n)) return fail(MFG_ERR_HIP, "download failed");
-        for (unsigned i = 0; i < N; i++) host[9 * (size_t)i + k] = a[i];
-      }
-      return MFG_OK;
+      PackField pf{{}, 9, PACK_F64};
+      for (int k = 0; k < 9; k++) pf.src[k] = m + k * n;
+      return download_field(p, pf, host);
     }
     case MFG_F_N: {
+      const int rc = check_counters(p);
+      if (rc != MFG_OK) return rc;
       if (!p->nrm) return fail(MFG_ERR_STATE, "no contact normals yet (tool compute_contact_force writes them)");
-      const size_t n = padded(N);
       return put3(p->nrm, p->nrm + n, p->nrm + 2 * n);
     }
     case MFG_F_P:
     case MFG_F_R: {
+      const int rc = check_counters(p);
+      if (rc != MFG_OK) return rc;
       if (!p->p_dbg) {
         // pressure and artificial stress live in the pair records; keep copies from now on
-        if (hipMalloc(&p->p_dbg, sizeof(double) * padded(N)) != hipSuccess ||
-            hipMalloc(&p->R_dbg, sizeof(double) * 6 * padded(N)) != hipSuccess)
+        if (hipMalloc(&p->p_dbg, sizeof(double) * n) != hipSuccess ||
+            hipMalloc(&p->R_dbg, sizeof(double) * 6 * n) != hipSuccess)
           return fail(MFG_ERR_NOMEM, "debug copies");
-        (void)hipMemsetAsync(p->p_dbg, 0, sizeof(double) * padded(N), s);
-        (void)hipMemsetAsync(p->R_dbg, 0, sizeof(double) * 6 * padded(N), s);
+        (void)hipMemsetAsync(p->p_dbg, 0, sizeof(double) * n, s);
+        (void)hipMemsetAsync(p->R_dbg, 0, sizeof(double) * 6 * n, s);
         return fail(MFG_ERR_STATE, "pressure / artificial stress are recorded from the next step on");
       }
       if (f == MFG_F_P) return put1(p->p_dbg);
-      std::vector<double> r(6 * (size_t)N);
-      if (hipMemcpyAsync(r.data(), p->R_dbg, sizeof(double) * 6 * N, hipMemcpyDeviceToHost, s) != hipSuccess ||
-          hipStreamSynchronize(s) != hipSuccess)
-        return fail(MFG_ERR_HIP, "download failed");
-      const int dst_of[6][2] = {{0, 0}, {4, 4}, {8, 8}, {1, 3}, {5, 7}, {2, 6}};
-      for (unsigned i = 0; i < N; i++)
-        for (int k = 0; k < 6; k++) {
-          host[9 * (size_t)i + dst_of[k][0]] = r[6 * (size_t)i + k];
-          host[9 * (size_t)i + dst_of[k][1]] = r[6 * (size_t)i + k];
-        }
-      return MFG_OK;
+      return download_field(p, PackField{{p->R_dbg}, 9, PACK_SYM6}, host);
     }
-    default:
-      return fail(MFG_ERR_ARG, "unknown field %d", f);
+    default: {
+      const int rc = check_counters(p);
+      return rc != MFG_OK ? rc : fail(MFG_ERR_ARG, "unknown field %d", f);
+    }
   }
 }
 
@@ -1728,8 +1736,9 @@ int mfg_tool_forces_create(unsigned n, mfg_tool_forces **out) {
   if (!out || n == 0 || n > MAX_TOOLS) return fail(MFG_ERR_ARG, "tool forces for %u tools (max %d)", n, MAX_TOOLS);
   mfg_tool_forces *f = new mfg_tool_forces();
   f->n = n;
-  if (hipMalloc(&f->d, sizeof(float) * 3 * n) != hipSuccess) {
-    delete f;
+  if (hipMalloc(&f->d, sizeof(float) * 3 * n) != hipSuccess ||
+      hipHostMalloc(&f->h, sizeof(float) * 3 * n) != hipSuccess) {
+    mfg_tool_forces_destroy(f);
     return fail(MFG_ERR_NOMEM, "tool forces");
   }
   (void)hipMemsetAsync(f->d, 0, sizeof(float) * 3 * n, g_lib.stream);
@@ -1739,6 +1748,7 @@ int mfg_tool_forces_create(unsigned n, mfg_tool_forces **out) {
 int mfg_tool_forces_destroy(mfg_tool_forces *f) {
   if (!f) return MFG_OK;
   if (f->d) (void)hipFree(f->d);
+  if (f->h) (void)hipHostFree(f->h);
   delete f;
   return MFG_OK;
 }
@@ -1751,8 +1761,11 @@ int mfg_tool_forces_reset(mfg_tool_forces *f) {
 int mfg_tool_forces_get_host(mfg_tool_forces *f, float *xyz) {
   NEED_LIB();
   if (!f || !xyz) return fail(MFG_ERR_ARG, "null argument");
-  HIP_TRY(hipMemcpyAsync(xyz, f->d, sizeof(float) * 3 * f->n, hipMemcpyDeviceToHost, g_lib.stream));
+  std::lock_guard<std::mutex> lock(f->h_use);
+  launch_words_to_host(g_lib.stream, f->d, f->h, 3 * f->n);
+  HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(g_lib.stream));
+  std::memcpy(xyz, f->h, sizeof(float) * 3 * f->n);
   return MFG_OK;
 }
 

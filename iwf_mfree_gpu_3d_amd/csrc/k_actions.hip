@@ -236,6 +236,42 @@ __global__ void __launch_bounds__(BA) k_act_sums(State st, const Counters *cnt, 
   if (c.heat == MFG_HEAT_BROOKSHAW && alpha != 0.) st.T_t[i] = alpha * sums[24 * stride + i];
 }
 
+// One thread per element of the host's layout.  The host-side interleave that it replaces went over the
+// field once per component (S at 1M particles: 14.5 ms, now the copy's 5).
+template <int W>
+__global__ void __launch_bounds__(BA) k_pack_field(PackField f, unsigned n, double *out,
+                                                   const Counters *cnt, Counters *cnt_h) {
+  if (cnt && blockIdx.x == 0 && threadIdx.x == 0) *cnt_h = *cnt;
+  const size_t e = (size_t)blockIdx.x * BA + threadIdx.x;
+  if (e >= (size_t)n * W) return;
+  const unsigned i = (unsigned)(e / W);
+  const int k = (int)(e - (size_t)i * W);
+  const void *src = f.src[0];
+#pragma unroll
+  for (int q = 1; q < W; q++) src = k == q ? f.src[q] : src;
+  double v;
+  if (f.kind == PACK_F64) {
+    v = ((const double *)src)[i];
+  } else if (f.kind == PACK_SYM6) {
+    constexpr int sym[9] = {0, 3, 5, 3, 1, 4, 5, 4, 2};  // xx yy zz xy yz zx in GLM's 9
+    int q = sym[0];
+#pragma unroll
+    for (int m = 1; m < W; m++) q = k == m ? sym[m] : q;
+    v = ((const double *)f.src[0])[6 * (size_t)i + q];
+  } else {
+    const uint32_t u = ((const uint32_t *)src)[i];
+    v = f.kind == PACK_FIXED     ? (u & FL_FIXED_ONE ? 1. : u & FL_FIXED ? 2. : 0.)
+        : f.kind == PACK_BLANKED ? (u & FL_BLANKED ? 1. : 0.)
+        : f.kind == PACK_TOOL    ? (u & FL_TOOL ? 1. : u & FL_TOOL_NZ ? 2. : 0.)
+                                 : (double)(int)u;
+  }
+  out[e] = v;
+}
+
+__global__ void __launch_bounds__(BA) k_words_to_host(const uint32_t *src, uint32_t *dst, unsigned n) {
+  for (unsigned i = threadIdx.x; i < n; i += BA) dst[i] = src[i];
+}
+
 // ---------------------------------------------------------------------------------------------
 static inline unsigned nba(long n) { return (unsigned)((n + BA - 1) / BA); }
 
@@ -286,6 +322,18 @@ void launch_act_sums(hipStream_t s, const State &st, unsigned n_init, const Coun
                      const int *poison) {
   hipLaunchKernelGGL(k_act_sums, dim3(nba(n_init)), dim3(BA), 0, s, st, cnt, c, a, sums, stride,
                      poison);
+}
+
+void launch_pack_field(hipStream_t s, const PackField &f, unsigned n, double *out, const Counters *cnt,
+                       Counters *cnt_h) {
+  const dim3 g(nba((long)n * f.w)), b(BA);
+  if (f.w == 1) hipLaunchKernelGGL(k_pack_field<1>, g, b, 0, s, f, n, out, cnt, cnt_h);
+  else if (f.w == 3) hipLaunchKernelGGL(k_pack_field<3>, g, b, 0, s, f, n, out, cnt, cnt_h);
+  else hipLaunchKernelGGL(k_pack_field<9>, g, b, 0, s, f, n, out, cnt, cnt_h);
+}
+
+void launch_words_to_host(hipStream_t s, const void *src, void *pinned, unsigned n_words) {
+  hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(BA), 0, s, (const uint32_t *)src, (uint32_t *)pinned, n_words);
 }
 
 }  // namespace mfg

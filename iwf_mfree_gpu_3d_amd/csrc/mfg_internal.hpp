@@ -211,6 +211,19 @@ void launch_particle_update(hipStream_t s, unsigned n_init, const State &st, con
                             size_t sum_stride, const int *poison, const Consts &c,
                             const Counters *cnt);
 
+// A field as the host holds it (w doubles per particle, particle-major) from the device's arrays:
+// element k of particle i is src[k][i], flags and integers turned into doubles
+enum { PACK_F64, PACK_FIXED, PACK_BLANKED, PACK_TOOL, PACK_I32, PACK_SYM6 };  // SYM6: src[0] holds 6 a particle
+struct PackField {
+  const void *src[9];
+  int w, kind;
+};
+// out may be pinned host memory; cnt, if given, goes to cnt_h (pinned) in the same launch
+void launch_pack_field(hipStream_t s, const PackField &f, unsigned n, double *out, const Counters *cnt,
+                       Counters *cnt_h);
+// a few words to pinned host memory: a kernel's store arrives in 6 us, a copy command's in 60
+void launch_words_to_host(hipStream_t s, const void *src, void *pinned, unsigned n_words);
+
 // moves n triangles (and, in the same launch, n2 more of a second array) to time t
 void launch_tool_update(hipStream_t s, Tri *tris, const double *p_init, int n, double t,
                         const double vel[3], Tri *tris2 = nullptr, const double *p_init2 = nullptr,
