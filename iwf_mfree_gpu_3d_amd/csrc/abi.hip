@@ -2336,7 +2336,7 @@ int batch_build(mfg_batch *b, int record) {
         (unsigned)host[i].nparts,
         1u,
         nblk,
-        round8((unsigned)pair_blocks(m.p->N_init, b->precision, 256)),
+        round8((unsigned)pair_blocks(m.p->N_init, 256)),
         round8((unsigned)neighbour_blocks(gi, tile)),
         (unsigned)std::max<size_t>(1, m.tools.size()),
         m.search ? std::min(BATCH_SEARCH_BLOCKS, std::max(1u, nblk)) : 0u};

@@ -904,29 +904,23 @@ struct AccWide {
   __device__ __forceinline__ double val() const { return s; }
 };
 
+// The CSPM entry of a neighbour (cs4): position, tool flag and volume
 struct ToolVol {
   float tool, vol;
 };
 
-template <class Acc>
+// One neighbour's terms of every sum, in FP32.  Where they round is fixed: the Johnson-Cook solve of
+// the update stops at 1e-6, so a sum that differs in its last bit can end it
+// an iteration earlier and move a result by more than its rounding.
+template <bool BROOK>
 struct Pair32 {
-  typedef Rec32 Rec;
   Rec32 ri;
-  bool tool_i, tool_nz, brook;
-  double thermal_alpha;
-  float hi, h1, fac, Ti, mass, inv_wdp, eps, va, vb, ve2;
+  float h1, fac, mass, inv_wdp, eps, va, vb, ve2;
   float iB[9];  // inverse CSPM matrix, [col][row] flattened
-  Acc B[9], vd[9], sd[9], vt[3], xt[3], Tl;
 
-  __device__ __forceinline__ Pair32(const Consts &c, const Rec32 &r, uint32_t fl) : ri(r) {
-    tool_i = ri.tool == 1.f;
-    tool_nz = (fl & FL_TOOL_NZ) != 0;
-    thermal_alpha = tool_nz ? c.alpha_tool : c.alpha_wp;
-    brook = c.heat == MFG_HEAT_BROOKSHAW && thermal_alpha != 0.;
-    hi = ri.h;
-    h1 = __builtin_amdgcn_rcpf(hi);
+  __device__ __forceinline__ Pair32(const Consts &c, const Rec32 &r) : ri(r) {
+    h1 = __builtin_amdgcn_rcpf(ri.h);
     fac = (float)INV_PI_D * h1 * h1 * h1;
-    Ti = brook ? ri.T : 0.f;
     mass = (float)c.i_mass;
     inv_wdp = c.wdeltap > 0 ? (float)(1.0 / c.wdeltap) : 0.f;
     eps = (float)c.xspheps;
@@ -934,43 +928,39 @@ struct Pair32 {
     vb = (float)c.v_beta;
     ve2 = (float)(c.v_eta * c.v_eta);
 #pragma unroll
-    for (int q = 0; q < 9; q++) {
-      iB[q] = (q % 4 == 0) ? 1.f : 0.f;
-      B[q].zero();
-      vd[q].zero();
-      sd[q].zero();
-    }
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      vt[a].zero();
-      xt[a].zero();
-    }
-    Tl.zero();
+    for (int q = 0; q < 9; q++) iB[q] = (q % 4 == 0) ? 1.f : 0.f;
   }
-  __device__ __forceinline__ bool cspm_sum() const { return !tool_nz; }
-  __device__ __forceinline__ void cspm_term(const Consts &, const double4 &g) {
+  // r / h, rounded: never fused into what follows
+  __device__ __forceinline__ float ratio(float rad) const { return rad * h1; }
+  // derivative of the cubic spline over its factor: both branches are x y h1 / r
+  __device__ __forceinline__ float spline_der(float q, float rinv) const {
 #pragma clang fp contract(fast)
-    const ToolVol tv = __builtin_bit_cast(ToolVol, g.w);
-    if (tv.tool == 1.f) return;
+    const bool outer = q > 1.f;
+    const float a = 2.f - q, b = 1.f - 0.75f * q;
+    const float x = outer ? -0.75f * a : -3.0f * q;
+    const float y = outer ? a : b;
+    return x * y * h1 * rinv;
+  }
+  // x_first: r^2 begins with x^2 rounded and y^2 fused on, not the other way round
+  __device__ __forceinline__ void cspm_term(const double4 &g, float vol, bool x_first, float (&b)[9]) const {
+#pragma clang fp contract(fast)
     float xij = (float)(ri.x - g.x), yij = (float)(ri.y - g.y), zij = (float)(ri.z - g.z);
-    float rr2 = xij * xij + yij * yij + zij * zij;
+    const float u = x_first ? xij : yij, v = x_first ? yij : xij;
+    float rr2 = __builtin_fmaf(zij, zij, __builtin_fmaf(v, v, u * u));
     float rad = __builtin_amdgcn_sqrtf(rr2);
     float rinv = __builtin_amdgcn_rcpf(rad);
-    float q = rad * h1;
-    float der = (q > 1.f) ? -0.75f * (2.f - q) * (2.f - q) * h1 * rinv
-                          : -3.0f * q * (1.f - 0.75f * q) * h1 * rinv;
-    float dw = der * fac * tv.vol;
+    float dw = spline_der(ratio(rad), rinv) * fac * vol;
     float gx = dw * xij, gy = dw * yij, gz = dw * zij;
-    B[0].add(-xij * gx); B[3].add(-xij * gy); B[6].add(-xij * gz);
-    B[1].add(-yij * gx); B[4].add(-yij * gy); B[7].add(-yij * gz);
-    B[2].add(-zij * gx); B[5].add(-zij * gy); B[8].add(-zij * gz);
+    b[0] = -xij * gx; b[3] = -xij * gy; b[6] = -xij * gz;
+    b[1] = -yij * gx; b[4] = -yij * gy; b[7] = -yij * gz;
+    b[2] = -zij * gx; b[5] = -zij * gy; b[8] = -zij * gz;
   }
-  __device__ __forceinline__ void cspm_end() {
+  __device__ __forceinline__ void invert(const double (&B)[9]) {
     M3 Bd, inv;
 #pragma unroll
     for (int a = 0; a < 3; a++)
 #pragma unroll
-      for (int b = 0; b < 3; b++) Bd.m[a][b] = B[3 * a + b].val();
+      for (int b = 0; b < 3; b++) Bd.m[a][b] = B[3 * a + b];
     if (det3(Bd) > 1e-8) {
       inv3(Bd, inv);
 #pragma unroll
@@ -979,85 +969,63 @@ struct Pair32 {
         for (int b = 0; b < 3; b++) iB[3 * a + b] = (float)inv.m[a][b];
     }
   }
-  __device__ __forceinline__ void term(const Consts &, const Rec32 &rj) {
+  // v: the 24 mechanical terms by slot (0 .. 8 vd, 9 .. 17 sd, 18 19 23 xt, 20 .. 22 vt); approach: the viscous ones count; heat, hot: the
+  // Brookshaw term and whether it counts
+  __device__ __forceinline__ void term(const Rec32 &rj, float (&v)[24], bool &approach, float &heat,
+                                       bool &hot) const {
 #pragma clang fp contract(fast)
     float xij = (float)(ri.x - rj.x), yij = (float)(ri.y - rj.y), zij = (float)(ri.z - rj.z);
     float rr2 = xij * xij + yij * yij + zij * zij;
     float rad = __builtin_amdgcn_sqrtf(rr2);
     float rinv = __builtin_amdgcn_rcpf(rad);
-    float q = rad * h1;
-    float val, der;
-    if (q > 1.f) {
-      float a = 2.f - q;
-      val = 0.25f * a * a * a;
-      der = -0.75f * a * a * h1 * rinv;
-    } else {
-      val = 1.f - 1.5f * q * q * (1.f - 0.5f * q);
-      der = -3.0f * q * (1.f - 0.75f * q) * h1 * rinv;
-    }
-    float w = val * fac;
-    float d = der * fac;
+    float q = ratio(rad);
+    float a = 2.f - q;
+    float v_out = 0.25f * a * a * a;
+    float v_in = 1.f - 1.5f * q * q * (1.f - 0.5f * q);
+    float w = (q > 1.f ? v_out : v_in) * fac;
+    float d = spline_der(q, rinv) * fac;
     float wx0 = d * xij, wy0 = d * yij, wz0 = d * zij;
     float w_x = wx0 * iB[0] + wy0 * iB[3] + wz0 * iB[6];
     float w_y = wx0 * iB[1] + wy0 * iB[4] + wz0 * iB[7];
     float w_z = wx0 * iB[2] + wy0 * iB[5] + wz0 * iB[8];
-    if (!tool_i && !(rj.tool == 1.f)) {
-      const float volj = rj.vol;
-      float dvx = (rj.vx - ri.vx) * volj, dvy = (rj.vy - ri.vy) * volj, dvz = (rj.vz - ri.vz) * volj;
-      vd[0].add(dvx * w_x); vd[1].add(dvx * w_y); vd[2].add(dvx * w_z);
-      vd[3].add(dvy * w_x); vd[4].add(dvy * w_y); vd[5].add(dvy * w_z);
-      vd[6].add(dvz * w_x); vd[7].add(dvz * w_y); vd[8].add(dvz * w_z);
-      float fab = w * inv_wdp;
-      fab *= fab;
-      fab *= fab;
-      float Rxx = fab * (ri.R[0] + rj.R[0]), Ryy = fab * (ri.R[1] + rj.R[1]);
-      float Rzz = fab * (ri.R[2] + rj.R[2]), Rxy = fab * (ri.R[3] + rj.R[3]);
-      float Ryz = fab * (ri.R[4] + rj.R[4]), Rxz = fab * (ri.R[5] + rj.R[5]);
-      float mx = mass * w_x, my = mass * w_y, mz = mass * w_z;
-      float Txx = ri.A[0] + rj.A[0] + Rxx, Tyy = ri.A[1] + rj.A[1] + Ryy, Tzz = ri.A[2] + rj.A[2] + Rzz;
-      float Txy = ri.A[3] + rj.A[3] + Rxy, Tyz = ri.A[4] + rj.A[4] + Ryz, Txz = ri.A[5] + rj.A[5] + Rxz;
-      sd[0].add(Txx * mx); sd[1].add(Txy * my); sd[2].add(Txz * mz);
-      sd[3].add(Txy * mx); sd[4].add(Tyy * my); sd[5].add(Tyz * mz);
-      sd[6].add(Txz * mx); sd[7].add(Tyz * my); sd[8].add(Tzz * mz);
-      float vijx = ri.vx - rj.vx, vijy = ri.vy - rj.vy, vijz = ri.vz - rj.vz;
-      float vijposij = vijx * xij + vijy * yij + vijz * zij;
-      float rhoij_inv = __builtin_amdgcn_rcpf(0.5f * (ri.rho + rj.rho));
-      if (vijposij < 0.f) {
-        float cij = 0.5f * (ri.c + rj.c);
-        float hij = 0.5f * (hi + rj.h);
-        float muij = (hij * vijposij) * __builtin_amdgcn_rcpf(rr2 + ve2 * hij * hij);
-        float piij = (-va * cij * muij + vb * muij * muij) * rhoij_inv;
-        float f = -mass * piij;
-        vt[0].add(f * w_x);
-        vt[1].add(f * w_y);
-        vt[2].add(f * w_z);
-      }
-      float g = -eps * w * mass * rhoij_inv;
-      xt[0].add(g * vijx);
-      xt[1].add(g * vijy);
-      xt[2].add(g * vijz);
-    }
-    if (brook && rad > 1e-8f) {
+    const float volj = rj.vol;
+    float vijx = ri.vx - rj.vx, vijy = ri.vy - rj.vy, vijz = ri.vz - rj.vz;
+    float dvx = -vijx * volj, dvy = -vijy * volj, dvz = -vijz * volj;
+    v[0] = dvx * w_x; v[1] = dvx * w_y; v[2] = dvx * w_z;
+    v[3] = dvy * w_x; v[4] = dvy * w_y; v[5] = dvy * w_z;
+    v[6] = dvz * w_x; v[7] = dvz * w_y; v[8] = dvz * w_z;
+    float fab = w * inv_wdp;
+    fab *= fab;
+    fab *= fab;
+    float Rxx = fab * (ri.R[0] + rj.R[0]), Ryy = fab * (ri.R[1] + rj.R[1]);
+    float Rzz = fab * (ri.R[2] + rj.R[2]), Rxy = fab * (ri.R[3] + rj.R[3]);
+    float Ryz = fab * (ri.R[4] + rj.R[4]), Rxz = fab * (ri.R[5] + rj.R[5]);
+    float mx = mass * w_x, my = mass * w_y, mz = mass * w_z;
+    float Txx = ri.A[0] + rj.A[0] + Rxx, Tyy = ri.A[1] + rj.A[1] + Ryy, Tzz = ri.A[2] + rj.A[2] + Rzz;
+    float Txy = ri.A[3] + rj.A[3] + Rxy, Tyz = ri.A[4] + rj.A[4] + Ryz, Txz = ri.A[5] + rj.A[5] + Rxz;
+    v[9] = Txx * mx; v[10] = Txy * my; v[11] = Txz * mz;
+    v[12] = Txy * mx; v[13] = Tyy * my; v[14] = Tyz * mz;
+    v[15] = Txz * mx; v[16] = Tyz * my; v[17] = Tzz * mz;
+    float vijposij = vijx * xij + vijy * yij + vijz * zij;
+    float rhoij_inv = __builtin_amdgcn_rcpf(0.5f * (ri.rho + rj.rho));
+    approach = vijposij < 0.f;
+    float cij = 0.5f * (ri.c + rj.c);
+    float hij = 0.5f * (ri.h + rj.h);
+    float muij = (hij * vijposij) * __builtin_amdgcn_rcpf(rr2 + ve2 * hij * hij);
+    float piij = (-va * cij * muij + vb * muij * muij) * rhoij_inv;
+    float f = -mass * piij;
+    v[20] = f * w_x;
+    v[21] = f * w_y;
+    v[22] = f * w_z;
+    float g = -eps * w * mass * rhoij_inv;
+    v[18] = g * vijx;
+    v[19] = g * vijy;
+    v[23] = g * vijz;
+    if (BROOK) {
       float e_w = (xij * w_x + yij * w_y + zij * w_z) * rinv;
-      Tl.add(2.0f * rj.vol * (Ti - rj.T) * rinv * e_w);
+      heat = 2.0f * rj.vol * (ri.T - rj.T) * rinv * e_w;
+      hot = rad > 1e-8f;
     }
-  }
-  __device__ __forceinline__ void store(double *sums, size_t stride, unsigned i) const {
-    PairSums ps;
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-      for (int b = 0; b < 3; b++) {
-        ps.vd.m[a][b] = vd[3 * a + b].val();
-        ps.sd.m[a][b] = sd[3 * a + b].val();
-      }
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-      ps.vt[a] = vt[a].val();
-      ps.xt[a] = xt[a].val();
-    }
-    ps.Tl = Tl.val();
-    store_sums(sums, stride, i, ps);
   }
 };
 
@@ -1474,331 +1442,300 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 }
 
 // ---------------------------------------------------------------------------------------------
-// FP32 pair pass: one lane per particle, B first, then the sums with the corrected gradient, each
-// sum over the list in its order (the Kahan sums depend on it).
-// Runs body(load(row[k])) for k = 0 .. n-1 in order.  The neighbour indices are read four at a
-// time, one group ahead, and the gather of neighbour k + 1 is issued before the arithmetic of
-// neighbour k: no gather waits on its own index, and one gather is always in flight.
-// Rows are 16-byte aligned and hold a multiple of 4 (at least 8) entries; the entries past n
-// that the vector reads pick up are never dereferenced.
-template <class Load, class Body>
-__device__ __forceinline__ void gather_loop(const int *row, int n, Load &&load, Body &&body) {
-  if (n <= 0) return;
-  typedef int iv4 __attribute__((ext_vector_type(4)));
-  iv4 cur = *(const iv4 *)row;
-  iv4 nxt = n > 4 ? *(const iv4 *)(row + 4) : cur;
-  auto ra = load(cur.x);
-  decltype(ra) rb;
-  for (int k = 0; k < n; k += 4) {
-    if (k + 1 < n) rb = load(cur.y);
-    body(ra);
-    if (k + 1 >= n) break;
-    if (k + 2 < n) ra = load(cur.z);
-    body(rb);
-    if (k + 2 >= n) break;
-    if (k + 3 < n) rb = load(cur.w);
-    body(ra);
-    if (k + 3 >= n) break;
-    cur = nxt;
-    if (k + 8 < n) nxt = *(const iv4 *)(row + k + 8);
-    if (k + 4 < n) ra = load(cur.x);
-    body(rb);
+// FP32 pair pass.  Every sum runs over the list in its order (the Kahan sums depend on it), first
+// the nine of B, then the 24 with the corrected gradient; so a sum is one lane's, and a lane per
+// particle would keep 25 of them.  Here a particle has four lanes, one in each row of 16 of its
+// wavefront: in step k the lane of row n forms all terms of neighbour 4 k + n, the rows exchange
+// them (spread: four registers in four instructions), and every lane then adds the four neighbours'
+// terms of its own quarter of the sums, in list order.
+//
+// Against one lane per particle, the same sums to the bit: 19,000 particles 137 -> 59 us (300 wavefronts
+// of 100 steps, now 1,200 of 26), 255k with wide sums 396 -> 324 us, 1M 1.35 -> 1.25 ms.  At 1M the
+// vector units are full: 424 instructions per 64 pairs, the exchanges and the transcendentals counting
+// double and fourfold; one lane per particle needs 345 but runs at the pace of its list reads (each
+// lane walks its own row: 1.42 ms).  115 registers: four waves per SIMD (three: 1.25 ms; five spill).
+// The index of a lane's next neighbour is one 4-byte read two steps ahead: reading them by fours and
+// exchanging them waits longer (1.86 ms).
+constexpr int PAIR32_WAVES = 4;
+
+// rows of 16 lanes: on return v[n] in row r holds what v[r] held in row n
+__device__ __forceinline__ void spread(float (&v)[4]) {
+  unsigned u[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) u[r] = __builtin_bit_cast(unsigned, v[r]);
+  auto a = __builtin_amdgcn_permlane32_swap(u[0], u[2], false, false);
+  auto b = __builtin_amdgcn_permlane32_swap(u[1], u[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  u[0] = c[0]; u[1] = c[1]; u[2] = d[0]; u[3] = d[1];
+#pragma unroll
+  for (int r = 0; r < 4; r++) v[r] = __builtin_bit_cast(float, u[r]);
+}
+// v[n] = x of row n, in every row
+__device__ __forceinline__ void rows_of(float x, float (&v)[4]) {
+  v[0] = v[1] = v[2] = v[3] = x;
+  spread(v);
+}
+__device__ __forceinline__ void rows_of(double x, double (&v)[4]) {
+  const uint64_t w = __builtin_bit_cast(uint64_t, x);
+  const unsigned w0 = (unsigned)w, w1 = (unsigned)(w >> 32);
+  float lo[4], hi[4];
+  rows_of(__builtin_bit_cast(float, w0), lo);
+  rows_of(__builtin_bit_cast(float, w1), hi);
+#pragma unroll
+  for (int n = 0; n < 4; n++)
+    v[n] = __builtin_bit_cast(double, ((uint64_t)__builtin_bit_cast(unsigned, hi[n]) << 32) |
+                                          __builtin_bit_cast(unsigned, lo[n]));
+}
+// the lanes of the 16 particles for which row n's bit of m is set
+__device__ __forceinline__ uint64_t row_mask(uint64_t m, int n) {
+  const uint64_t r = (m >> (16 * n)) & 0xffff;
+  const uint64_t h = r | (r << 16);
+  return h | (h << 32);
+}
+// adds neighbours 0 .. 3 to M sums; m: the lanes whose own neighbour counts.  With all of them in, no
+// masks (a masked sum costs a fifth operation)
+template <int M, class Acc>
+__device__ __forceinline__ void add_rows(Acc (&a)[M], const float (&v)[M][4], uint64_t m) {
+  if (m == ~0ull) {
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+#pragma unroll
+      for (int q = 0; q < M; q++) a[q].add(v[q][n]);
+  } else {
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+      if (__builtin_amdgcn_inverse_ballot_w64(row_mask(m, n))) {
+#pragma unroll
+        for (int q = 0; q < M; q++) a[q].add(v[q][n]);
+      }
   }
 }
 
-// Cooperative gather through registers: groups of G lanes load the P pieces of one record each
-// (one piece per lane and instruction), so every load instruction reads 64 / G whole records
-// from contiguous lines; the pieces then go through LDS to the lane that needs the record.  The
-// LDS slot of a record is S bytes (S / 16 odd multiples of four dwords keep the 16-lane phases of
-// a 16-byte LDS access on distinct banks).
-template <int P, int G, int S>
-struct CoopGather {
-  static_assert(P <= G && (G & (G - 1)) == 0 && G <= 64, "pieces per record");
-  static constexpr int R = 64 / G;  // records per load instruction
-  __device__ static void load(const char *base, size_t rec_bytes, int j, int lane,
-                              piece16 (&v)[G]) {
-    const int p = lane & (G - 1);
-    const int ps = p < P ? p : 0;  // lanes beyond the record's pieces reload piece 0
+// The records of a step: 64 in LDS one after the other (record of lane L at 112 L), as seven 1 KB
+// blocks: load q fetches piece g = 64 q + lane of that image (record g / 7, piece g mod 7), so every
+// lane loads and no piece is fetched twice.  At the 112-byte stride the 16-byte reads of a lane's own
+// record fall on distinct banks for the lanes one read phase serves.  The buffer descriptor's stride
+// is the record size: the load unit forms index x stride + offset, and an index beyond n_rec reads
+// zeros instead of faulting.
+struct RecGather {
+  static constexpr int P = 7, AREA = P * 1024;
+  static_assert(sizeof(Rec32) == 16 * P, "FP32 record image");
+  struct Pieces {
+    piece16 p[P];
+  };
+  __amdgpu_buffer_rsrc_t rsrc;
+  char *area;
+  int src[P], off[P], lane;
+  __device__ __forceinline__ RecGather(const Rec32 *rec, unsigned n_rec, char *lds, int l) : area(lds), lane(l) {
+    // word 3: the untyped 32-bit data format the load-to-LDS path needs on gfx9-family parts
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)rec, (short)sizeof(Rec32), (int)n_rec, 0x00020000);
 #pragma unroll
-    for (int q = 0; q < G; q++) {
-      const int jm = __shfl(j, q * R + lane / G, 64);
-      v[q] = *(const piece16 *)(base + (size_t)jm * rec_bytes + 16 * ps);
-    }
-  }
-  __device__ static void store(char *lds, int lane, const piece16 (&v)[G]) {
-    const int p = lane & (G - 1);
-#pragma unroll
-    for (int q = 0; q < G; q++)
-      if (p < P) *(piece16 *)(lds + (q * R + lane / G) * S + 16 * p) = v[q];
-  }
-};
-
-// FP32 records (112 bytes, seven pieces): the step's 64 records lie in LDS one after the other
-// (record L at 112 L), as seven 1 KB blocks: load instruction q fetches piece g = 64 q + lane of
-// that image (record g / 7, piece g mod 7), so every lane loads and no piece is fetched twice.
-// At the 112-byte record stride the 16-byte reads of a lane's own record fall on distinct banks
-// for the lanes one read phase serves.
-struct Plan32 {
-  typedef Rec32 Rec;
-  static constexpr int P = 7, NI = 7, BLOCK = 64 * 16;
-  static constexpr int WINDOWS = NI * BLOCK, AREA = WINDOWS + 64 * 16;
-  static_assert(sizeof(Rec32) == 16 * P && NI * BLOCK == 64 * (int)sizeof(Rec32), "FP32 record image");
-  int src_[NI], off_[NI];
-  __device__ void prepare(char *, int lane) {
-#pragma unroll
-    for (int q = 0; q < NI; q++) {
+    for (int q = 0; q < P; q++) {
       const int g = 64 * q + lane, r = g / P;
-      src_[q] = 4 * r;
-      off_[q] = 16 * (g - P * r);
+      src[q] = 4 * r;
+      off[q] = 16 * (g - P * r);
     }
   }
-  __device__ int src_addr(int q) const { return src_[q]; }
-  __device__ int off(int q) const { return off_[q]; }
-  __device__ static int read_pos(int L, int p) { return (int)sizeof(Rec32) * L + 16 * p; }
+  __device__ __forceinline__ void issue(int j) const {
+    int jm[P];
+#pragma unroll
+    for (int q = 0; q < P; q++) jm[q] = __builtin_amdgcn_ds_bpermute(src[q], j);
+#pragma unroll
+    for (int q = 0; q < P; q++)
+      __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + 1024 * q), 16, jm[q], off[q], 0,
+                                                  0, 0);
+  }
+  __device__ __forceinline__ Rec32 read() const {
+    Pieces pc;
+#pragma unroll
+    for (int p = 0; p < P; p++) pc.p[p] = *(const piece16 *)(area + (int)sizeof(Rec32) * lane + 16 * p);
+    return __builtin_bit_cast(Rec32, pc);
+  }
 };
-// Walks the lists of a wavefront: step k gives each lane with k < nl the first P pieces of its
-// neighbour k.  Step k + 1's records and the index window of steps k + 2 .. k + 5 are loaded
-// while step k's term runs.  The records are read through a buffer descriptor whose stride is
-// the record size: the load unit forms record index x stride + piece offset (no 64-bit address
-// arithmetic per load), and an index beyond n_rec reads zeros instead of faulting.
-template <class Plan, class Term>
-__device__ __forceinline__ void dma_list_walk(const typename Plan::Rec *__restrict__ rec,
-                                              unsigned n_rec, const int *row, int nl, int nmax,
-                                              unsigned ic, int lane, char *area, Term &&term) {
-  typedef typename Plan::Rec Rec;
-  constexpr int P = Plan::P, NI = Plan::NI;
-  static_assert(NI * Plan::BLOCK <= Plan::WINDOWS, "area");
-  typedef int iv4 __attribute__((ext_vector_type(4)));
-  char *wslot = area + Plan::WINDOWS;
-  Plan plan;
-  plan.prepare(area, lane);
-  iv4 wc = {0, 0, 0, 0};
-  if (nl > 0) wc = *(const iv4 *)row;
-  auto idx_at = [&](int k) -> int {
-    if (k >= nl) return (int)ic;  // past the end of the list: the lane's own record, unused
-    const int q = k & 3;
-    return q == 0 ? wc.x : q == 1 ? wc.y : q == 2 ? wc.z : wc.w;
+// The CSPM entries of a step likewise, 32 bytes a lane in two loads (load q: piece g = 64 q + lane of
+// the 2 KB image, entry g / 2).  The two pieces of an entry swap slots every eight entries, so that the
+// 16-byte reads of 16 consecutive lanes fall on distinct bank groups.  The terms are light, so the
+// walk holds CSPM_BLOCK steps in LDS while the next CSPM_BLOCK load.
+constexpr int CSPM_BLOCK = 2, CSPM_STEP = 64 * 32, CSPM_AREA = 2 * CSPM_BLOCK * CSPM_STEP;
+struct EntryGather {
+  struct Pieces {
+    piece16 p[2];
   };
-  // word 3: the untyped 32-bit data format the load-to-LDS path needs on gfx9-family parts
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void *)rec, (short)sizeof(Rec), (int)n_rec, 0x00020000);
-  auto issue = [&](int k) {
-    const int j = idx_at(k);
-    int jm[NI];
+  __amdgpu_buffer_rsrc_t rsrc;
+  int src[2], off[2], rd[2];
+  __device__ __forceinline__ EntryGather(const double4 *cs4, unsigned n_rec, int lane) {
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)cs4, (short)sizeof(double4), (int)n_rec, 0x00020000);
 #pragma unroll
-    for (int q = 0; q < NI; q++) jm[q] = __builtin_amdgcn_ds_bpermute(plan.src_addr(q), j);
-#pragma unroll
-    for (int q = 0; q < NI; q++)
-      __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + Plan::BLOCK * q), 16,
-                                                  jm[q], plan.off(q), 0, 0, 0);
-  };
-  if (nmax > 0) issue(0);
-  for (int k = 0; k < nmax; k++) {
-    __builtin_amdgcn_s_waitcnt(0);  // this step's records (and a window) are in LDS
-    struct Pieces {
-      piece16 p[P];
-    } pc;
-#pragma unroll
-    for (int p = 0; p < P; p++) pc.p[p] = *(const piece16 *)(area + Plan::read_pos(lane, p));
-    const bool next_window = ((k + 1) & 3) == 0 && k + 1 < nmax;
-    iv4 wl = wc;
-    if (next_window) wl = *(const iv4 *)(wslot + 16 * lane);
-    __builtin_amdgcn_s_waitcnt(0);  // every lane's reads are done before the area is refilled
-    wave_sync_lds();
-    if (k + 1 < nmax) {
-      wc = wl;
-      issue(k + 1);
-      // the window of steps k+2 .. k+5, read at step k+1 (a lane past its list reads its first)
-      if (((k + 2) & 3) == 0 && k + 2 < nmax) {
-        const int *src = k + 2 < nl ? row + k + 2 : row;
-        __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)wslot, 16, 0, 0);
-      }
+    for (int q = 0; q < 2; q++) {
+      const int g = 64 * q + lane, r = g >> 1;
+      src[q] = 4 * r;
+      off[q] = 16 * (((g & 1) + (r >> 3)) & 1);
+      rd[q] = 32 * lane + 16 * (((lane >> 3) + q) & 1);
     }
-    if (k < nl) term(pc);
   }
-  __builtin_amdgcn_s_waitcnt(0);
-  wave_sync_lds();  // the area is free for the next walk
-}
+  __device__ __forceinline__ void issue(int j, char *area) const {
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+      __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + 1024 * q), 16,
+                                                  __builtin_amdgcn_ds_bpermute(src[q], j), off[q], 0, 0, 0);
+  }
+  __device__ __forceinline__ double4 read(const char *area) const {
+    Pieces pc;
+#pragma unroll
+    for (int q = 0; q < 2; q++) pc.p[q] = *(const piece16 *)(area + rd[q]);
+    return __builtin_bit_cast(double4, pc);
+  }
+};
 
-// The CSPM walk through LDS: step k gives each lane with k < nl its neighbour k's 32-byte entry
-// (x, y, z, volume or the tool pattern).  A step's 64 entries are two load instructions straight
-// into LDS (instruction q fetches 16-byte piece g = 64 q + lane of the step's 2 KB image: entry
-// g / 2), through a buffer descriptor of 32-byte stride as in dma_list_walk.  The term is light,
-// so the walk runs in blocks of four steps with the next block's eight loads in flight while a
-// block computes: a ring of two blocks, 16 KB of the area.  The two pieces of an entry swap
-// slots every eight entries, so that the 16-byte reads of 16 consecutive lanes fall on distinct
-// bank groups.  The indices come as each lane's int4 row windows, one block ahead.
-constexpr int CSPM_STEP = 64 * 32;
-constexpr int CSPM_RING = 2 * 4 * CSPM_STEP;
-template <class Term>
-__device__ __forceinline__ void dma_cspm_walk(const double4 *__restrict__ cs4, unsigned n_rec,
-                                              const int *row, int nl, int nmax, unsigned ic,
-                                              int lane, char *area, Term &&term) {
-  typedef int iv4 __attribute__((ext_vector_type(4)));
-  constexpr int S = 4;  // steps per block: one int4 window of indices
-  const int nb = (nmax + S - 1) / S;
-  if (nb == 0) return;
-  int src[2], off[2];
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int g = 64 * q + lane, r = g >> 1;
-    src[q] = 4 * r;
-    off[q] = 16 * (((g & 1) + (r >> 3)) & 1);
-  }
-  const int rd0 = 32 * lane + 16 * ((lane >> 3) & 1);
-  const int rd1 = 32 * lane + 16 * (((lane >> 3) + 1) & 1);
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void *)cs4, (short)sizeof(double4), (int)n_rec, 0x00020000);
-  // the indices of block b (the lane's own record past its list)
-  auto window = [&](int b) -> iv4 {
-    const int k = S * b;
-    iv4 w = {(int)ic, (int)ic, (int)ic, (int)ic};
-    if (k < nl) w = *(const iv4 *)(row + k);
-    return w;
-  };
-  auto issue = [&](int b, const iv4 &w) {
-    char *base = area + (b & 1) * S * CSPM_STEP;
-#pragma unroll
-    for (int s = 0; s < S; s++) {
-      const int j = S * b + s < nl ? w[s] : (int)ic;
-#pragma unroll
-      for (int q = 0; q < 2; q++)
-        __builtin_amdgcn_struct_ptr_buffer_load_lds(
-            rsrc, (lds_void *)(base + s * CSPM_STEP + 1024 * q), 16,
-            __builtin_amdgcn_ds_bpermute(src[q], j), off[q], 0, 0, 0);
-    }
-  };
-  issue(0, window(0));
-  iv4 wn = nb > 1 ? window(1) : iv4{0, 0, 0, 0};
-  for (int b = 0; b < nb; b++) {
-    __builtin_amdgcn_s_waitcnt(0);  // block b's entries (and the next window) have arrived
-    wave_sync_lds();
-    if (b + 1 < nb) issue(b + 1, wn);  // into the half block b - 1 used, read before
-    if (b + 2 < nb) wn = window(b + 2);
-    const char *base = area + (b & 1) * S * CSPM_STEP;
-#pragma unroll
-    for (int s = 0; s < S; s++) {
-      if (S * b + s < nl) {
-        struct Pieces {
-          piece16 p[2];
-        } pc;
-        pc.p[0] = *(const piece16 *)(base + s * CSPM_STEP + rd0);
-        pc.p[1] = *(const piece16 *)(base + s * CSPM_STEP + rd1);
-        term(__builtin_bit_cast(double4, pc));
-      }
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  wave_sync_lds();  // the area is free for the next walk
-}
-
-// FP32 list pass with the cooperative gather for the main sum: the 64 lanes of a wavefront run
-// the pair loop together (inactive lanes with an empty list) because every lane helps load.
-// Loaded lane by lane, every 16-byte piece of every record would be a separate L1 access; here
-// each load instruction reads whole records from contiguous lines straight into LDS (Plan32),
-// and each lane then reads its own record from there.
-template <class Acc, int BS = BSP>
-__device__ __forceinline__ void pair32_coop(unsigned b, unsigned nb, unsigned n_init,
-                                            const State &st, const Rec32 *__restrict__ rec,
-                                            const int *__restrict__ nbr, int stride,
-                                            const int *__restrict__ count, const Consts &c,
-                                            const Counters *cnt, double *__restrict__ sums,
-                                            size_t sstride, const int *__restrict__ trav,
-                                            const double4 *__restrict__ cs4) {
-  const unsigned t = xcd_map(b, nb) * BS + threadIdx.x;
+template <class Acc, bool BROOK, int BS>
+__device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_init, const State &st,
+                                          const Rec32 *__restrict__ rec, const int *__restrict__ nbr,
+                                          int stride, const int *__restrict__ count, const Consts &c,
+                                          const Counters *cnt, double *__restrict__ sums,
+                                          size_t sstride, const int *__restrict__ trav,
+                                          const double4 *__restrict__ cs4) {
+  constexpr int AREA = CSPM_AREA > RecGather::AREA ? CSPM_AREA : RecGather::AREA;
+  __shared__ __align__(16) char s_area[BS / 64][AREA];
+  // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n = lane >> 4;
+  const unsigned t = xcd_map(b, nb) * (BS / PAIR_LANES) + 16 * w + (lane & 15);
   const unsigned N = cnt->N;
   const bool in_range = t < N && t < n_init;
   const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
   const uint32_t fl = in_range ? st.flags[i] : FL_BLANKED;
   const bool act = in_range && !(fl & FL_BLANKED);
   const unsigned ic = act ? i : 0u;
-  Pair32<Acc> P(c, rec[ic], fl);
   const int nl = act ? count[i] : 0;
-  const int *row = nbr + (size_t)ic * stride;
-  // The gathers: straight into LDS (dma_cspm_walk, Plan32) with Kahan sums, per lane and through
-  // registers (CoopGather) with wide sums, the faster of the two for each on the 1M single-grain
-  // cut (Kahan 1.51 -> 1.39 -> 1.29 ms with the direct record, then CSPM-entry loads; wide 1.39
-  // with registers, 1.44 with direct record loads, 1.95 with direct CSPM-entry loads).
-  if constexpr (!std::is_same<Acc, AccWide>::value) {
-    constexpr int AREA = Plan32::AREA > CSPM_RING ? Plan32::AREA : CSPM_RING;
-    __shared__ __align__(16) char s_area[BS / 64][AREA];
-    // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (c.cspm) {
-      const int nc = P.cspm_sum() ? nl : 0;
-      int ncmax = nc;
+  int steps = (nl + PAIR_LANES - 1) / PAIR_LANES;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) ncmax = max(ncmax, __shfl_xor(ncmax, o, 64));
-      dma_cspm_walk(cs4, n_init, row, nc, ncmax, ic, lane, s_area[w],
-                    [&](const double4 &g) { P.cspm_term(c, g); });
-      P.cspm_end();
-    }
-    int nmax = nl;
+  for (int o = 8; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
+  steps = __builtin_amdgcn_readfirstlane(steps);
+  const int *row = nbr + (size_t)ic * stride + n;
+  // neighbour 4 k + n of the list; past its end the particle itself, which is loaded and not used
+  auto index = [&](int k) -> int { return n + 4 * k < nl ? row[4 * k] : (int)ic; };
+  Pair32<BROOK> P(c, rec[ic]);
+  const bool tool_i = P.ri.tool == 1.f, tool_nz = (fl & FL_TOOL_NZ) != 0;
+  char *area = s_area[w];
+  if (c.cspm && steps > 0) {
+    const EntryGather g(cs4, n_init, lane);
+    // the wide sums' terms have always been rounded so for all but every fourth neighbour
+    const bool x_first = std::is_same<Acc, AccWide>::value && n != 0;
+    Acc a2[2], a1[1];  // B[4 m + n] and, in every row, B[8]
+    a2[0].zero();
+    a2[1].zero();
+    a1[0].zero();
+    const int nb = (steps + CSPM_BLOCK - 1) / CSPM_BLOCK;
+    int jn[CSPM_BLOCK];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
-    dma_list_walk<Plan32>(rec, n_init, row, nl, nmax, ic, lane, s_area[w],
-                          [&](const auto &pc) { P.term(c, __builtin_bit_cast(Rec32, pc)); });
-  } else {
-    if (c.cspm) {
-      if (P.cspm_sum())
-        gather_loop(row, nl, [&](int j) { return cs4[j]; },
-                    [&](const double4 &g) { P.cspm_term(c, g); });
-      P.cspm_end();
-    }
-    typedef CoopGather<sizeof(Rec32) / 16, 8, sizeof(Rec32)> CG;
-    __shared__ __align__(16) char s_rec[2][BS / 64][64 * sizeof(Rec32)];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int nmax = nl;
+    for (int s = 0; s < CSPM_BLOCK; s++) g.issue(index(s), area + s * CSPM_STEP);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) nmax = max(nmax, __shfl_xor(nmax, o, 64));
-    typedef int iv4 __attribute__((ext_vector_type(4)));
-    iv4 win = {0, 0, 0, 0};
-    // neighbour of this lane at step k (its own particle past the end of its list); k ascends
-    auto idx_at = [&](int k) -> int {
-      if ((k & 3) == 0 && k < nl) win = *(const iv4 *)(row + k);
-      if (k >= nl) return (int)ic;
-      const int q = k & 3;
-      return q == 0 ? win.x : q == 1 ? win.y : q == 2 ? win.z : win.w;
-    };
-    piece16 v[8];
-    if (nmax > 0) {
-      CG::load((const char *)rec, sizeof(Rec32), idx_at(0), lane, v);
-      CG::store(s_rec[0][w], lane, v);
+    for (int s = 0; s < CSPM_BLOCK; s++) jn[s] = index(CSPM_BLOCK + s);
+    for (int b = 0; b < nb; b++) {
+      __builtin_amdgcn_s_waitcnt(0);  // this block's entries have arrived, and the next indices
       wave_sync_lds();
-    }
-    for (int k = 0; k < nmax; k++) {
-      const bool more = k + 1 < nmax;
-      if (more) CG::load((const char *)rec, sizeof(Rec32), idx_at(k + 1), lane, v);
-      if (k < nl) {
-        // the record as seven 16-byte reads: at the 112-byte slot stride the 8 lanes a 16-byte
-        // read serves per cycle fall on distinct banks, while 4- and 8-byte field reads would put
-        // 4 lanes on each bank
-        struct Pieces {
-          piece16 p[sizeof(Rec32) / 16];
-        } pc;
-        const char *src = s_rec[k & 1][w] + lane * sizeof(Rec32);
+      const char *here = area + (b & 1) * CSPM_BLOCK * CSPM_STEP;
+      if (b + 1 < nb) {  // into the half that block b - 1 used, read before
+        char *next = area + ((b + 1) & 1) * CSPM_BLOCK * CSPM_STEP;
 #pragma unroll
-        for (int q = 0; q < (int)(sizeof(Rec32) / 16); q++)
-          pc.p[q] = *(const piece16 *)(src + 16 * q);
-        P.term(c, __builtin_bit_cast(Rec32, pc));
+        for (int s = 0; s < CSPM_BLOCK; s++) g.issue(jn[s], next + s * CSPM_STEP);
+#pragma unroll
+        for (int s = 0; s < CSPM_BLOCK; s++) jn[s] = index((b + 2) * CSPM_BLOCK + s);
       }
-      if (more) CG::store(s_rec[(k + 1) & 1][w], lane, v);
+#pragma unroll
+      for (int s = 0; s < CSPM_BLOCK; s++) {
+        const double4 e = g.read(here + s * CSPM_STEP);
+        const ToolVol tv = __builtin_bit_cast(ToolVol, e.w);
+        float B[9], v2[2][4], v1[1][4];
+        P.cspm_term(e, tv.vol, x_first, B);
+        const uint64_t m = __builtin_amdgcn_ballot_w64(n + 4 * (b * CSPM_BLOCK + s) < nl && !tool_nz && tv.tool != 1.f);
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) v2[q][r] = B[4 * q + r];
+          spread(v2[q]);
+        }
+        rows_of(B[8], v1[0]);
+        add_rows(a2, v2, m);
+        add_rows(a1, v1, m);
+      }
+    }
+    wave_sync_lds();  // the area is free for the next walk
+    double B[9], r4[4];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+      rows_of(a2[q].val(), r4);
+#pragma unroll
+      for (int r = 0; r < 4; r++) B[4 * q + r] = r4[r];
+    }
+    B[8] = a1[0].val();
+    P.invert(B);
+  }
+  Acc a5[5], av[1], ah[1];
+#pragma unroll
+  for (int q = 0; q < 5; q++) a5[q].zero();
+  av[0].zero();
+  ah[0].zero();
+  const RecGather g(rec, n_init, area, lane);
+  const bool brook = BROOK && (tool_nz ? c.alpha_tool : c.alpha_wp) != 0.;
+  if (steps > 0) {
+    g.issue(index(0));
+    int jn = index(1);
+    for (int k = 0; k < steps; k++) {
+      __builtin_amdgcn_s_waitcnt(0);  // this step's records are in LDS
+      const Rec32 rj = g.read();
+      __builtin_amdgcn_s_waitcnt(0);  // every lane's reads are done before the area is refilled
       wave_sync_lds();
+      if (k + 1 < steps) {
+        g.issue(jn);
+        jn = index(k + 2);
+      }
+      float v[24], v5[5][4], vv[1][4], heat = 0.f;
+      bool approach, hot = false;
+      P.term(rj, v, approach, heat, hot);
+      const bool in_list = n + 4 * k < nl, mech = in_list && !tool_i && !(rj.tool == 1.f);
+      const uint64_t m = __builtin_amdgcn_ballot_w64(mech), mv = __builtin_amdgcn_ballot_w64(mech && approach);
+#pragma unroll
+      for (int q = 0; q < 5; q++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) v5[q][r] = v[4 * q + r];
+        spread(v5[q]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) vv[0][r] = v[20 + r];
+      spread(vv[0]);
+      add_rows(a5, v5, m);
+      // rows 0 .. 2 hold the viscous sums, row 3 one of the velocity smoothing
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const uint64_t keep = (row_mask(mv, q) & 0x0000ffffffffffffull) | (row_mask(m, q) & 0xffff000000000000ull);
+        if (__builtin_amdgcn_inverse_ballot_w64(keep)) av[0].add(vv[0][q]);
+      }
+      if (BROOK) {
+        float vh[1][4];
+        rows_of(heat, vh[0]);
+        add_rows(ah, vh, __builtin_amdgcn_ballot_w64(in_list && brook && hot));
+      }
     }
   }
   if (!act) return;
-  P.store(sums, sstride, i);
+  // slots 4 q + n: vd 0 .. 8, sd 0 .. 8, xt 0, xt 1 | vt 0 .. 2, xt 2
+#pragma unroll
+  for (int q = 0; q < 5; q++) sums[(4 * q + n + (q == 4 && n >= 2 ? 3 : 0)) * sstride + i] = a5[q].val();
+  sums[(n < 3 ? 18 + n : 23) * sstride + i] = av[0].val();
+  if (n == 0) sums[24 * sstride + i] = BROOK ? ah[0].val() : 0.;
 }
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
 // depend on it).  Small instances spread over more compute units with smaller workgroups.
-template <class Acc, int BS>
-__global__ void __launch_bounds__(BS, PAIR_WAVES)
-    k_pair32_coop(unsigned n_init, State st, const Rec32 *__restrict__ rec,
-                  const int *__restrict__ nbr, int stride, const int *__restrict__ count,
-                  Consts c, const Counters *cnt, double *__restrict__ sums, size_t sstride,
-                  const int *__restrict__ trav, const double4 *__restrict__ cs4) {
-  pair32_coop<Acc, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
-                       sstride, trav, cs4);
+template <class Acc, bool BROOK, int BS>
+__global__ void __launch_bounds__(BS, PAIR32_WAVES)
+    k_pair_rows(unsigned n_init, State st, const Rec32 *__restrict__ rec,
+                const int *__restrict__ nbr, int stride, const int *__restrict__ count,
+                Consts c, const Counters *cnt, double *__restrict__ sums, size_t sstride,
+                const int *__restrict__ trav, const double4 *__restrict__ cs4) {
+  pair_rows<Acc, BROOK, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
+                            sstride, trav, cs4);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1840,43 +1777,38 @@ void launch_neighbours(hipStream_t s, const GridInfo &g, const int *offsets, con
                                         nbr, cap, count, T_t, cnt, stat_part, poison);
 }
 
-int pair_blocks(unsigned n_init, int precision, int block) {
-  return (int)nb((long)n_init * (precision == MFG_FP64 ? PAIR_LANES : 1), block);
-}
+int pair_blocks(unsigned n_init, int block) { return (int)nb((long)n_init * PAIR_LANES, block); }
 
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
                  int nl_stride, const int *count, const Consts &c, const Counters *cnt,
                  double *sums, size_t sstride, const int *trav, const double4 *cs4, int block,
                  bool ordered) {
   const int bs = block == 64 || block == 128 ? block : BSP;
-  const dim3 blk(bs), grid1(nb(n_init, bs));  // one lane per particle
+  const dim3 blk(bs), grid((unsigned)pair_blocks(n_init, bs));
   const bool brook = c.heat == MFG_HEAT_BROOKSHAW;
-  auto launch = [&](auto bs_c) {
+  auto launch = [&](auto bs_c, auto brook_c) {
     constexpr int BS = decltype(bs_c)::value;
-    if (c.precision == MFG_FP32_KAHAN) {
-      hipLaunchKernelGGL((k_pair32_coop<AccKahan, BS>), grid1, blk, 0, s, n_init, st,
-                         (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav,
-                         cs4);
-    } else if (c.precision == MFG_FP32_WIDE) {
-      hipLaunchKernelGGL((k_pair32_coop<AccWide, BS>), grid1, blk, 0, s, n_init, st,
-                         (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav,
-                         cs4);
-    } else if (ordered) {
-      hipLaunchKernelGGL(k_pair_ordered<BS>, grid1, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr,
+    constexpr bool BROOK = decltype(brook_c)::value;
+    if (c.precision == MFG_FP32_KAHAN)
+      hipLaunchKernelGGL((k_pair_rows<AccKahan, BROOK, BS>), grid, blk, 0, s, n_init, st, (const Rec32 *)rec,
+                         nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+    else if (c.precision == MFG_FP32_WIDE)
+      hipLaunchKernelGGL((k_pair_rows<AccWide, BROOK, BS>), grid, blk, 0, s, n_init, st, (const Rec32 *)rec,
+                         nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+    else if (ordered)  // one lane per particle
+      hipLaunchKernelGGL(k_pair_ordered<BS>, dim3(nb(n_init, bs)), blk, 0, s, n_init, st, (const Rec64 *)rec,
+                         nbr, nl_stride, count, c, cnt, sums, sstride, trav);
+    else
+      hipLaunchKernelGGL((k_pair_sums<BROOK, BS>), grid, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr,
                          nl_stride, count, c, cnt, sums, sstride, trav);
-    } else {
-      const dim3 grid((unsigned)pair_blocks(n_init, c.precision, bs));
-      if (brook)
-        hipLaunchKernelGGL((k_pair_sums<true, BS>), grid, blk, 0, s, n_init, st,
-                           (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
-      else
-        hipLaunchKernelGGL((k_pair_sums<false, BS>), grid, blk, 0, s, n_init, st,
-                           (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
-    }
   };
-  if (bs == 64) launch(std::integral_constant<int, 64>{});
-  else if (bs == 128) launch(std::integral_constant<int, 128>{});
-  else launch(std::integral_constant<int, BSP>{});
+  auto sized = [&](auto bs_c) {
+    if (brook) launch(bs_c, std::true_type{});
+    else launch(bs_c, std::false_type{});
+  };
+  if (bs == 64) sized(std::integral_constant<int, 64>{});
+  else if (bs == 128) sized(std::integral_constant<int, 128>{});
+  else sized(std::integral_constant<int, BSP>{});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1916,12 +1848,12 @@ __global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair_sums(const Inst *in, 
                         d.nl_stride, d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr);
 }
 
-template <class Acc>
-__global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair32_coop(const Inst *in, BatchMap m) {
+template <class Acc, bool BROOK>
+__global__ void __launch_bounds__(BSP, PAIR32_WAVES) kb_pair_rows(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  pair32_coop<Acc>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
-                   d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, d.cs4);
+  pair_rows<Acc, BROOK, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
+                             d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, d.cs4);
 }
 
 __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchMap m) {
@@ -1937,14 +1869,17 @@ void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
   const int mode = !L.pse ? 0 : L.precision == MFG_FP64 ? 1 : 2;
   dispatch_neighbours<BatchNeighbours>(mode, L.cell_tile, s, L);
   const dim3 gp(L.pairs8.blocks), bp(BSP);
-  if (L.precision == MFG_FP64 && L.brook)
-    hipLaunchKernelGGL(kb_pair_sums<true>, gp, bp, 0, s, L.inst, L.pairs8.m);
-  else if (L.precision == MFG_FP64)
-    hipLaunchKernelGGL(kb_pair_sums<false>, gp, bp, 0, s, L.inst, L.pairs8.m);
-  else if (L.precision == MFG_FP32_KAHAN)
-    hipLaunchKernelGGL(kb_pair32_coop<AccKahan>, gp, bp, 0, s, L.inst, L.pairs8.m);
-  else
-    hipLaunchKernelGGL(kb_pair32_coop<AccWide>, gp, bp, 0, s, L.inst, L.pairs8.m);
+  auto launch = [&](auto brook_c) {
+    constexpr bool BROOK = decltype(brook_c)::value;
+    if (L.precision == MFG_FP64)
+      hipLaunchKernelGGL(kb_pair_sums<BROOK>, gp, bp, 0, s, L.inst, L.pairs8.m);
+    else if (L.precision == MFG_FP32_KAHAN)
+      hipLaunchKernelGGL((kb_pair_rows<AccKahan, BROOK>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    else
+      hipLaunchKernelGGL((kb_pair_rows<AccWide, BROOK>), gp, bp, 0, s, L.inst, L.pairs8.m);
+  };
+  if (L.brook) launch(std::true_type{});
+  else launch(std::false_type{});
   hipLaunchKernelGGL(kb_particle_update, dim3(L.parts.blocks), dim3(BSP), 0, s, L.inst, L.parts.m);
 }
 

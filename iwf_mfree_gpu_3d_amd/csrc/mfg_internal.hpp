@@ -188,10 +188,10 @@ void launch_neighbours(hipStream_t s, const GridInfo &g, const int *offsets, con
                        const double2 *pse2, const double *h, const uint32_t *flags,
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
                        int want_pse, unsigned long long *stat_part, int *poison, int cell_tile);
-// pair pass (neighbour sums); pair_blocks: its workgroups of `block` threads (64, 128 or 256), four
-// lanes per particle in FP64, one in the FP32 modes.  ordered: FP64 sums in the reference's order of
-// evaluation, to the bit (unlocked grids), one lane per particle.  cs4: FP32 modes only
-int pair_blocks(unsigned n_init, int precision, int block);
+// pair pass (neighbour sums), four lanes per particle; pair_blocks: its workgroups of `block` threads
+// (64, 128 or 256).  ordered: FP64 sums in the reference's order of evaluation, to the bit (unlocked
+// grids), one lane per particle.  cs4: FP32 modes only
+int pair_blocks(unsigned n_init, int block);
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
                  int nl_stride, const int *count, const Consts &c, const Counters *cnt,
                  double *sums, size_t sum_stride, const int *trav, const double4 *cs4, int block,
