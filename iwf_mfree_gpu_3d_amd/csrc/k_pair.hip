@@ -641,7 +641,7 @@ __device__ __forceinline__ void update_body(unsigned b, unsigned n_init, const S
                                             const double *__restrict__ sums, size_t stride,
                                             const int *__restrict__ poison, const Consts &c,
                                             const Counters *cnt) {
-  const unsigned i = b * BSP + threadIdx.x;
+  const unsigned i = b * blockDim.x + threadIdx.x;
   if (i >= cnt->N || i >= n_init) return;
   const uint32_t fl = st.flags[i];
   if (fl & FL_BLANKED) return;
@@ -1899,7 +1899,11 @@ void launch_pair_order(hipStream_t s, unsigned n_init, const GridInfo &g, const 
 void launch_particle_update(hipStream_t s, unsigned n_init, const State &st, const double *sums,
                             size_t sstride, const int *poison, const Consts &c,
                             const Counters *cnt) {
-  hipLaunchKernelGGL(k_particle_update, dim3(nb(n_init, BSP)), dim3(BSP), 0, s, n_init, st, sums,
+  // one wavefront per workgroup: the few wavefronts with particles in the Johnson-Cook solve run for
+  // six iterations of 1.6 us and more while the others are done, and hold back only themselves (256
+  // threads: 8,000 particles 25 us, now 19; 19,000 26, 22.5; 1M 172, 156; 64,000 27, 28)
+  constexpr int BS = 64;
+  hipLaunchKernelGGL(k_particle_update, dim3(nb(n_init, BS)), dim3(BS), 0, s, n_init, st, sums,
                      sstride, poison, c, cnt);
 }
 
