@@ -244,7 +244,7 @@ struct mfg_grid {
   double vel_bbox[3] = {0, 0, 0};
   long nx = 0, ny = 0, nz = 0, num_cell = 0, max_cell = 0;
   int *count = nullptr;  // max_cell + 1: counts, then offsets
-  int *fill = nullptr;
+  int *hist = nullptr;
   int *parts = nullptr;
   int nparts_cap = 0;
   double *bbox_part = nullptr;
@@ -331,8 +331,10 @@ void free_particles(mfg_particles *p) {
 
 int grid_alloc(mfg_grid *g) {
   HIP_TRY(hipMalloc(&g->count, sizeof(int) * (g->max_cell + 1)));
-  HIP_TRY(hipMalloc(&g->fill, sizeof(int) * (g->max_cell + 1)));
-  g->nparts_cap = (int)((g->max_cell + 4095) / 4096) + 1;
+  HIP_TRY(hipMalloc(&g->hist, sizeof(int) * (g->max_cell + 1)));
+  HIP_TRY(hipMemsetAsync(g->hist, 0, sizeof(int) * (g->max_cell + 1), g_lib.stream));
+  HIP_TRY(hipStreamSynchronize(g_lib.stream));  // a sort may run on a stream set later
+  g->nparts_cap = scan_tiles(g->max_cell, false) + 1;
   HIP_TRY(hipMalloc(&g->parts, sizeof(int) * g->nparts_cap));
   HIP_TRY(hipMalloc(&g->bbox_part, sizeof(double) * 7 * 1024));
   g->bbox_host.assign(7 * 1024, 0.);
@@ -345,7 +347,8 @@ GridBuffers grid_buffers(mfg_grid *g, mfg_particles *p) {
   gb.key_sorted = p->key_sorted;
   gb.order = p->order;
   gb.count = g->count;
-  gb.fill = g->fill;
+  gb.hist = g->hist;
+  gb.scattered = p->trav;
   gb.blk = p->blk;
   gb.blk2 = g->parts;
   gb.nblk = p->nblk;
@@ -395,7 +398,6 @@ int grid_update_geometry(mfg_grid *g, mfg_particles *p, double kernel_width, dou
   return grid_update_unlocked(g, p, kernel_width);
 }
 
-// hash (+ blanking), scan, scatter, per-cell fix-up: the sort permutation and cell offsets
 // what decides whether the cell tables of a sort still describe a grid: origin, cell size and
 // cells per axis
 void grid_geometry(const mfg_grid *g, double geom[7]) {
@@ -421,7 +423,8 @@ bool keep_last_sort(const mfg_grid *g, const mfg_particles *p) {
   return true;
 }
 
-void sort_keys(mfg_grid *g, mfg_particles *p, const mfg_blanking_state *b) {
+// hash (+ blanking), scan, scatter: the particles by cell and the cell offsets.  ordered: with the order inside the cells, which the permutation of a fused step finds itself
+void sort_keys(mfg_grid *g, mfg_particles *p, const mfg_blanking_state *b, bool ordered = true) {
   GridBuffers gb = grid_buffers(g, p);
   GridInfo gi = g->info();
   double bb[6];
@@ -446,21 +449,24 @@ void sort_keys(mfg_grid *g, mfg_particles *p, const mfg_blanking_state *b) {
     ProfScope ps("scatter");
     launch_scatter(g_lib.stream, p->N_init, gi, gb, p->cnt);
   }
-  {
-    ProfScope ps("cell_fixup");
-    launch_fixup(g_lib.stream, gi, gb);
+  if (ordered) {
+    ProfScope ps("cell_order");
+    launch_order(g_lib.stream, p->N_init, gb);
   }
-  g->scanned = true;
+  g->scanned = ordered;
   g->sorted_for = p;
   p->sorted_grid = g;
   grid_geometry(g, p->sorted_geom);
   p->since_sort = 0;
 }
 
-// identity: the particle order stays (a step between sorts): no gather, keys kept
-void permute(mfg_grid *g, mfg_particles *p, const Consts &c, int predict, bool identity = false) {
+enum PermuteFrom { FROM_ORDER, FROM_SCATTERED, IN_PLACE };
+// FROM_SCATTERED: of a sort that left the order inside the cells open.  IN_PLACE: the particle order
+// stays (a step between sorts): no gather, keys kept
+void permute(mfg_grid *g, mfg_particles *p, const Consts &c, int predict, PermuteFrom from) {
   GridBuffers gb = grid_buffers(g, p);
-  if (identity) gb.order = nullptr;
+  if (from == IN_PLACE) gb.order = nullptr;
+  if (from != FROM_SCATTERED) gb.scattered = nullptr;
   ProfScope ps(predict ? "permute_predict" : "permute");
   int nxt = 1 - p->cur;
   launch_permute_predict_ex(g_lib.stream, p->buf[p->cur], p->buf[nxt], p->N_init, gb, p->cnt, c,
@@ -1338,7 +1344,7 @@ int mfg_grid_create_unlocked(int kind, long max_cell, int num_part, mfg_grid **o
 int mfg_grid_destroy(mfg_grid *g) {
   if (!g) return MFG_OK;
   if (g_lib.ready) (void)hipStreamSynchronize(g_lib.stream);
-  void *ptrs[] = {g->count, g->fill, g->parts, g->bbox_part};
+  void *ptrs[] = {g->count, g->hist, g->parts, g->bbox_part};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   delete g;
@@ -1408,7 +1414,7 @@ int mfg_grid_sort(mfg_grid *g, mfg_particles *p) {
   const int rc = check_counters(p);
   if (rc != MFG_OK) return rc;
   Consts c = make_consts(0., p->precision);
-  permute(g, p, c, 0);
+  permute(g, p, c, 0, FROM_ORDER);
   // the keys now describe the sorted order; a further sort hashes again
   g->scanned = false;
   return MFG_OK;
@@ -1448,6 +1454,7 @@ int mfg_grid_neighbours(mfg_grid *g, mfg_particles *p, int *h_counts, int *h_lis
   // build nl4 from the current state: a permute with the identity order would do; use the
   // predict path with dt = 0 on a copy of the order (half step == current state)
   GridBuffers gb = grid_buffers(g, p);
+  gb.scattered = nullptr;
   std::vector<int> ident(p->N_init);
   for (unsigned i = 0; i < p->N_init; i++) ident[i] = (int)i;
   int *saved_order = nullptr;
@@ -1940,10 +1947,11 @@ int step_impl(mfg_leap_frog *lf, mfg_particles *p, mfg_grid *g, int record,
   }
   if (keep_last_sort(g, p)) {
     p->since_sort++;
-    permute(g, p, c, 1, true);
+    permute(g, p, c, 1, IN_PLACE);
   } else {
-    sort_keys(g, p, blanking);
-    permute(g, p, c, 1);
+    const bool apart = order_apart(p->N_init);
+    sort_keys(g, p, blanking, apart);
+    permute(g, p, c, 1, apart ? FROM_ORDER : FROM_SCATTERED);
   }
   g->scanned = false;  // the permutation is applied: a later mfg_grid_sort hashes again
   // pair pass
@@ -2187,7 +2195,6 @@ struct mfg_batch {
 
 namespace {
 
-constexpr int SCAN_TILE_CELLS = 256 * 16;  // cells per scan tile of the counting sort
 constexpr unsigned BATCH_SEARCH_BLOCKS = 64;
 
 unsigned round8(unsigned n) { return (n + 7u) / 8u * 8u; }
@@ -2211,7 +2218,6 @@ Inst batch_inst(const mfg_batch::Member &m, int record) {
   d.n_init = p->N_init;
   d.g = m.g->info();
   d.gb = grid_buffers(m.g, p);
-  d.nparts = (int)((m.g->num_cell + SCAN_TILE_CELLS - 1) / SCAN_TILE_CELLS);
   d.blanking = m.blanking;
   for (int k = 0; k < 6; k++) d.bb[k] = m.bb[k];
   d.vmax2 = m.vmax2;
@@ -2304,7 +2310,7 @@ int batch_build(mfg_batch *b, int record) {
     HIP_TRY(hipMalloc(&b->d_inst, sizeof(Inst) * (size_t)n));
     b->inst_cap = n;
   }
-  constexpr int N_MAPS = 9;
+  constexpr int N_MAPS = 7;
   const size_t map_len = (size_t)n + 1;
   if (N_MAPS * map_len > b->maps_cap) {
     if (b->d_maps) (void)hipFree(b->d_maps);
@@ -2315,25 +2321,27 @@ int batch_build(mfg_batch *b, int record) {
   }
   std::vector<Inst> host(n);
   std::vector<unsigned> maps(N_MAPS * map_len, 0u);
-  BatchGrid *grids[N_MAPS] = {&b->L.cells1, &b->L.cells, &b->L.tiles, &b->L.one, &b->L.parts,
+  BatchGrid *grids[N_MAPS] = {&b->L.tiles, &b->L.one, &b->L.parts,
                               &b->L.pairs8, &b->L.nbrs8, &b->L.tools, &b->L.search};
   // cell tile of the batched neighbour pass: by the cells per particle of the whole batch
-  long cells = 0, parts = 0;
+  long cells = 0, parts = 0, most = 0;
   for (const mfg_batch::Member &m : b->members) {
     cells += m.g->num_cell;
+    most = std::max(most, (long)m.g->num_cell);
     parts += m.p->N_init;
   }
   const int tile = resolve_cell_tile(b->cell_tile ? b->cell_tile : g_lib.opt.cell_tile, cells,
                                      (unsigned)std::min<long>(parts, 0xffffffffL));
+  b->L.scan_alone = most <= SCAN_ALONE;
+  b->L.ordered = order_apart(parts);
   for (int i = 0; i < n; i++) {
     const mfg_batch::Member &m = b->members[i];
     host[i] = batch_inst(m, record);
+    host[i].ordered = b->L.ordered;
     const GridInfo gi = m.g->info();
     const unsigned nblk = (unsigned)m.p->nblk;
     const unsigned blocks[N_MAPS] = {
-        (unsigned)((gi.num_cell + 1 + 255) / 256),
-        (unsigned)((gi.num_cell + 255) / 256),
-        (unsigned)host[i].nparts,
+        (unsigned)scan_tiles(gi.num_cell, b->L.scan_alone),
         1u,
         nblk,
         round8((unsigned)pair_blocks(m.p->N_init, 256)),

@@ -10,19 +10,27 @@
 //                                                          src/actions_gpu.cu:40-53,70-132
 //
 // Sort: keys are cell hashes < num_cell or INT_MAX.  A counting sort by cell gives the cell
-// offsets directly (exclusive scan of the per-cell counts); particles are placed with an atomic
-// slot inside their cell and each cell is then re-ordered by previous index, which makes the
-// result identical to a stable sort.  INT_MAX keys go to the tail in previous-index order by a
-// block-wise compaction.  Cell start/end of the reference are off[c], off[c+1] for non-empty
-// cells.
+// offsets directly (exclusive scan of the per-cell counts).  The atomic that counts a particle
+// returns its slot inside the cell, in no particular order; the permutation then takes each
+// particle to its place by previous index among its cell's, which makes the result identical to a
+// stable sort.  INT_MAX keys go to the tail in previous-index order by a block-wise compaction.
+// Cell start/end of the reference are off[c], off[c+1] for non-empty cells.
+//
+// Launches bound the sort of small sets and atomics that of large ones.  The counts are an array of
+// their own that the scatter leaves zero for the next sort; the scan is one launch up to SCAN_ALONE
+// cells and two above; the order inside the cells is the permutation's own work for small sets; and a
+// run of particles of one cell is counted by one atomic, which also hands out their slots.  With the
+// permutation: 8,000 particles 44 us in eight launches, now 29 in four; 1M 0.32 ms, now 0.25 (hash 33
+// us, now 17: the particles come in the last sort's order; scatter 40, now 6.4: no atomics; fix-up and
+// zeroing 17, now 7.6).
 #include "mfg_device.hpp"
 #include "mfg_records.hpp"
 
 namespace mfg {
 
-constexpr int BS = 256;          // threads per block of the particle passes
-constexpr int SCAN_ITEMS = 16;   // items per thread of the cell scan
-constexpr int SCAN_TILE = BS * SCAN_ITEMS;
+constexpr int BS = 256;  // threads per block of the particle passes
+constexpr int SCAN_ITEMS = SCAN_TILE / BS;
+constexpr int SCAN_NT = 1024;  // threads of a tile without tile sums
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
   const int lane = threadIdx.x & 63;
@@ -67,26 +75,14 @@ __device__ __forceinline__ bool rates_invalid(const State &st, unsigned i) {
 
 // Each kernel below is a body run by workgroup `b` (blockIdx.x of a single-instance launch, the
 // workgroup inside its instance's range of a batched launch) and a __global__ wrapper.
-__device__ __forceinline__ void zero_cells(unsigned b, int *count, int *fill, long n) {
-  long c = (long)b * BS + threadIdx.x;
-  if (c < n) {
-    count[c] = 0;
-    fill[c] = 0;
-  }
-  if (c == n) count[c] = 0;
-}
-__global__ void __launch_bounds__(BS) k_zero_cells(int *count, int *fill, long n) {
-  zero_cells(blockIdx.x, count, fill, n);
-}
-
 __device__ __forceinline__ void blank_hash_count(unsigned b, const State &st, unsigned n_init,
                                                  const GridInfo &g, int blanking, double b0,
                                                  double b1, double b2, double b3, double b4,
-                                                 double b5, double vmax2, int *key, int *count,
-                                                 int *blk, Counters *cnt) {
+                                                 double b5, double vmax2, int *key, int *hist,
+                                                 int *slot, int *blk, Counters *cnt) {
   __shared__ int lds[BS / 64 + 1];
   const unsigned i = b * BS + threadIdx.x;
-  int blank_key = 0;
+  int blank_key = 0, k = KEY_BLANK;
   if (i < n_init) {
     uint32_t fl = st.flags[i];
     if (blanking) {
@@ -102,7 +98,6 @@ __device__ __forceinline__ void blank_hash_count(unsigned b, const State &st, un
       if (nf != fl) st.flags[i] = nf;
       fl = nf;
     }
-    int k;
     if ((fl & FL_BLANKED) && g.hard_blank) {
       k = KEY_BLANK;
     } else {
@@ -117,9 +112,19 @@ __device__ __forceinline__ void blank_hash_count(unsigned b, const State &st, un
       }
     }
     key[i] = k;
-    if (k != KEY_BLANK) atomicAdd(&count[k], 1);
     blank_key = (k == KEY_BLANK) ? 1 : 0;
   }
+  // one atomic for a run of lanes in the same cell (the particles come in the last sort's order, two
+  // or three to a cell): the first lane adds the run's length, each takes its place in the run
+  const int lane = threadIdx.x & 63;
+  const int k_before = __shfl_up(k, 1, 64);  // by every lane: a lane that sits out gives 0
+  const uint64_t heads = __ballot(lane == 0 || k_before != k);
+  const int head = 63 - __clzll(heads & (~0ull >> (63 - lane)));
+  const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1);
+  int first = 0;
+  if (head == lane && k != KEY_BLANK) first = atomicAdd(&hist[k], later ? __ffsll((unsigned long long)later) : 64 - lane);
+  first = __shfl(first, head, 64);
+  if (k != KEY_BLANK) slot[i] = first + lane - head;
   int total;
   block_excl_scan<BS>(blank_key, lds, total);
   if (threadIdx.x == 0) blk[b] = total;
@@ -127,141 +132,165 @@ __device__ __forceinline__ void blank_hash_count(unsigned b, const State &st, un
 __global__ void __launch_bounds__(BS)
     k_blank_hash_count(State st, unsigned n_init, GridInfo g, int blanking, double b0, double b1,
                        double b2, double b3, double b4, double b5, double vmax2, int *key,
-                       int *count, int *blk, Counters *cnt) {
-  blank_hash_count(blockIdx.x, st, n_init, g, blanking, b0, b1, b2, b3, b4, b5, vmax2, key, count,
-                   blk, cnt);
+                       int *hist, int *slot, int *blk, Counters *cnt) {
+  blank_hash_count(blockIdx.x, st, n_init, g, blanking, b0, b1, b2, b3, b4, b5, vmax2, key, hist,
+                   slot, blk, cnt);
+}
+
+// ITEMS consecutive entries from k on, those beyond n as 0 (k and the array 16-byte aligned)
+template <int ITEMS>
+__device__ __forceinline__ void load_items(const int *a, long k, long n, int (&v)[ITEMS]) {
+  if (k + ITEMS <= n) {
+#pragma unroll
+    for (int q = 0; q < ITEMS; q += 4) {
+      const int4 x = *(const int4 *)(a + k + q);
+      v[q] = x.x; v[q + 1] = x.y; v[q + 2] = x.z; v[q + 3] = x.w;
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < ITEMS; q++) v[q] = k + q < n ? a[k + q] : 0;
+  }
 }
 
 // tile reduction of the cell counts
-__device__ __forceinline__ void scan_reduce(unsigned b, const int *count, long n, int *part) {
+__device__ __forceinline__ void scan_reduce(unsigned b, const int *hist, long n, int *part) {
   __shared__ int lds[BS / 64 + 1];
-  long base = (long)b * SCAN_TILE + (long)threadIdx.x * SCAN_ITEMS;
-  int s = 0;
+  int v[SCAN_ITEMS], s = 0;
+  load_items<SCAN_ITEMS>(hist, (long)b * SCAN_TILE + (long)threadIdx.x * SCAN_ITEMS, n, v);
 #pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; k++)
-    if (base + k < n) s += count[base + k];
+  for (int q = 0; q < SCAN_ITEMS; q++) s += v[q];
   int total;
   block_excl_scan<BS>(s, lds, total);
   if (threadIdx.x == 0) part[b] = total;
 }
-__global__ void __launch_bounds__(BS) k_scan_reduce(const int *count, long n, int *part) {
-  scan_reduce(blockIdx.x, count, n, part);
+__global__ void __launch_bounds__(BS) k_scan_reduce(const int *hist, long n, int *part) {
+  scan_reduce(blockIdx.x, hist, n, part);
 }
 
-// single-block exclusive scan of two small arrays (tile sums of the cells, block blank counts)
-constexpr int SB = 1024;
-__device__ void block_scan_array(int *a, int n, int *lds, int &total) {
-  int per = (n + SB - 1) / SB;
-  int beg = threadIdx.x * per, end = min(beg + per, n);
-  int s = 0;
-  for (int k = beg; k < end; k++) s += a[k];
-  int off = block_excl_scan<SB>(s, lds, total);
-  for (int k = beg; k < end; k++) {
-    int t = a[k];
-    a[k] = off;
-    off += t;
+// The offsets of tile b's cells (NT threads, ITEMS cells each), and with the last tile the totals.  A
+// tile's base is the sum of all before it: of the tile sums, or without them (part null: SCAN_ALONE)
+// of the counts themselves, eight loads of a thread in flight (26,000 cells: 6.7 us, 62,000: 7.4; the
+// two launches 4.6 and 4.8 and the gap between).
+template <int NT, int ITEMS>
+__device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, const int *part, int *off,
+                                           unsigned n_init, Counters *cnt) {
+  __shared__ int lds[NT / 64 + 1];
+  const long base = ((long)b * NT + threadIdx.x) * ITEMS;
+  int v[ITEMS], s = 0, before = 0, total, prefix;
+  load_items<ITEMS>(hist, base, n, v);
+  if (part) {
+    for (unsigned k = threadIdx.x; k < b; k += NT) before += part[k];
+  } else {
+    // b tiles of NT x ITEMS counts: ITEMS / 4 vectors a thread and tile
+    const int4 *h = (const int4 *)hist + threadIdx.x;
+#pragma unroll 8
+    for (unsigned k = 0; k < b * (ITEMS / 4); k++) {
+      const int4 x = h[(size_t)k * NT];
+      before += x.x + x.y + x.z + x.w;
+    }
   }
-  __syncthreads();
-}
-
-__device__ __forceinline__ void scan_top(int *part, int nparts, int *blk, int nblk, int *count,
-                                         long num_cell, Counters *cnt) {
-  __shared__ int lds[SB / 64 + 1];
-  int tot_valid, tot_blank;
-  block_scan_array(part, nparts, lds, tot_valid);
-  block_scan_array(blk, nblk, lds, tot_blank);
-  if (threadIdx.x == 0) {
-    count[num_cell] = tot_valid;
-    cnt->N = (unsigned)tot_valid;
-    cnt->n_blank_key = (unsigned)tot_blank;
+#pragma unroll
+  for (int q = 0; q < ITEMS; q++) s += v[q];
+  block_excl_scan<NT>(before, lds, prefix);
+  int o = prefix + block_excl_scan<NT>(s, lds, total);
+  if (threadIdx.x == 0 && (long)(b + 1) * NT * ITEMS >= n) {  // the last tile
+    off[n] = prefix + total;
+    cnt->N = (unsigned)(prefix + total);
+    cnt->n_blank_key = n_init - (unsigned)(prefix + total);
     cnt->candidates = 0ull;
     cnt->pairs = 0ull;
   }
-}
-__global__ void __launch_bounds__(SB) k_scan_top(int *part, int nparts, int *blk, int nblk,
-                                                 int *count, long num_cell, Counters *cnt) {
-  scan_top(part, nparts, blk, nblk, count, num_cell, cnt);
-}
-
-__device__ __forceinline__ void scan_down(unsigned b, int *count, long n, const int *part) {
-  __shared__ int lds[BS / 64 + 1];
-  long base = (long)b * SCAN_TILE + (long)threadIdx.x * SCAN_ITEMS;
-  int v[SCAN_ITEMS];
-  int s = 0;
+  int w[ITEMS];
 #pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; k++) {
-    v[k] = (base + k < n) ? count[base + k] : 0;
-    s += v[k];
+  for (int q = 0; q < ITEMS; q++) {
+    w[q] = o;
+    o += v[q];
   }
-  int total;
-  int off = block_excl_scan<BS>(s, lds, total) + part[b];
+  if (base + ITEMS <= n) {
 #pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; k++)
-    if (base + k < n) {
-      count[base + k] = off;
-      off += v[k];
-    }
+    for (int q = 0; q < ITEMS; q += 4) *(int4 *)(off + base + q) = make_int4(w[q], w[q + 1], w[q + 2], w[q + 3]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < ITEMS; q++)
+      if (base + q < n) off[base + q] = w[q];
+  }
 }
-__global__ void __launch_bounds__(BS) k_scan_down(int *count, long n, const int *part) {
-  scan_down(blockIdx.x, count, n, part);
+template <int NT, int ITEMS>
+__global__ void __launch_bounds__(NT) k_scan_cells(const int *hist, long n, const int *part, int *off,
+                                                   unsigned n_init, Counters *cnt) {
+  scan_cells<NT, ITEMS>(blockIdx.x, hist, n, part, off, n_init, cnt);
 }
 
-__device__ __forceinline__ void scatter(unsigned b, unsigned n_init, const int *key,
-                                        const int *off, int *fill, const int *blk,
+// particles to their cells (order: an INT_MAX key's particle at its final place, the others in any
+// order within their cell), and the counts back to zero
+__device__ __forceinline__ void scatter(unsigned b, unsigned nb, unsigned n_init, long num_cell, const int *key,
+                                        const int *off, const int *slot, int *hist, const int *blk,
                                         const Counters *cnt, int *order) {
   __shared__ int lds[BS / 64 + 1];
   const unsigned i = b * BS + threadIdx.x;
-  int k = (i < n_init) ? key[i] : 0;
-  int is_blank = (i < n_init && k == KEY_BLANK) ? 1 : 0;
+  const int k = (i < n_init) ? key[i] : 0;
+  const int is_blank = (i < n_init && k == KEY_BLANK) ? 1 : 0;
   int total;
-  int rank = block_excl_scan<BS>(is_blank, lds, total);
-  if (i >= n_init) return;
-  int pos;
-  if (is_blank) pos = (int)cnt->N + blk[b] + rank;
-  else pos = off[k] + atomicAdd(&fill[k], 1);
-  order[pos] = (int)i;
+  const int rank = block_excl_scan<BS>(is_blank, lds, total);
+  if (total > 0) {
+    int before = 0, prefix;
+    for (unsigned q = threadIdx.x; q < b; q += BS) before += blk[q];
+    block_excl_scan<BS>(before, lds, prefix);
+    if (is_blank) order[(int)cnt->N + prefix + rank] = (int)i;
+  }
+  if (i < n_init && !is_blank) order[off[k] + slot[i]] = (int)i;
+  for (long c = (long)i; c < num_cell; c += (long)nb * BS) hist[c] = 0;
 }
-__global__ void __launch_bounds__(BS) k_scatter(unsigned n_init, const int *key, const int *off,
-                                                int *fill, const int *blk, const Counters *cnt,
-                                                int *order) {
-  scatter(blockIdx.x, n_init, key, off, fill, blk, cnt, order);
+__global__ void __launch_bounds__(BS) k_scatter(unsigned n_init, long num_cell, const int *key, const int *off,
+                                                const int *slot, int *hist, const int *blk,
+                                                const Counters *cnt, int *order) {
+  scatter(blockIdx.x, gridDim.x, n_init, num_cell, key, off, slot, hist, blk, cnt, order);
 }
 
-// restore previous-index order inside every cell (stable sort)
-__device__ __forceinline__ void fixup(unsigned wg, const int *off, long num_cell, int *order) {
-  long c = (long)wg * BS + threadIdx.x;
-  if (c >= num_cell) return;
-  int s = off[c], e = off[c + 1];
-  if (e - s < 2) return;
-  for (int a = s + 1; a < e; a++) {
-    int v = order[a];
-    int b = a - 1;
-    while (b >= s && order[b] > v) {
-      order[b + 1] = order[b];
-      b--;
-    }
-    order[b + 1] = v;
-  }
+// The place of the particle at scattered position t: by previous index among its cell's.
+__device__ __forceinline__ unsigned place_in_cell(unsigned t, const int *scattered, const int *off, int particle,
+                                                  int key) {
+  if (key == KEY_BLANK) return t;
+  const int s = off[key], e = off[key + 1];
+  int place = s;
+  for (int q = s; q < e; q++) place += scattered[q] < particle;
+  return (unsigned)place;
 }
-__global__ void __launch_bounds__(BS) k_fixup(const int *off, long num_cell, int *order) {
-  fixup(blockIdx.x, off, num_cell, order);
+__device__ __forceinline__ void order_cells(unsigned b, unsigned n_init, const int *scattered, const int *key,
+                                            const int *off, int *order) {
+  const unsigned t = b * BS + threadIdx.x;
+  if (t >= n_init) return;
+  const int s = scattered[t];
+  order[place_in_cell(t, scattered, off, s, key[s])] = s;
+}
+__global__ void __launch_bounds__(BS) k_order(unsigned n_init, const int *scattered, const int *key,
+                                              const int *off, int *order) {
+  order_cells(blockIdx.x, n_init, scattered, key, off, order);
 }
 
 // gather the persistent state by the sort permutation, then predict the half step and build the
 // pair records (EOS and artificial stress included)
 template <class RecT>
 __device__ __forceinline__ void permute_predict(unsigned b, const State &src, const State &dst,
-                                                unsigned n_init, const int *order,
-                                                const int *key, int *key_sorted,
+                                                unsigned n_init, int *order, const int *scattered,
+                                                const int *off, const int *key, int *key_sorted,
                                                 const Counters *cnt, const Consts &c, int predict,
                                                 RecT *rec, double4 *nl4, double2 *pse2,
                                                 double4 *cs4, double *p_dbg, double *R_dbg) {
-  const unsigned i = b * BS + threadIdx.x;
+  unsigned i = b * BS + threadIdx.x;
   if (i >= n_init) return;
   const unsigned N = cnt->N;
-  // a null order: the particles keep their places (a step between sorts)
-  const int s = order ? order[i] : (int)i;
-  if (order) key_sorted[i] = key[s];
+  // from the scattered particles (the order inside the cells is found here and kept), from a
+  // finished order, or, both null, the particles keep their places (a step between sorts)
+  const int s = scattered ? scattered[i] : order ? order[i] : (int)i;
+  if (scattered || order) {
+    const int k = key[s];
+    if (scattered) {
+      i = place_in_cell(i, scattered, off, s, k);
+      order[i] = s;
+    }
+    key_sorted[i] = k;
+  }
   double x[3] = {src.x[s], src.y[s], src.z[s]};
   double v[3] = {src.vx[s], src.vy[s], src.vz[s]};
   double S[6], St[6];
@@ -333,10 +362,10 @@ __device__ __forceinline__ void permute_predict(unsigned b, const State &src, co
 }
 template <class RecT>
 __global__ void __launch_bounds__(BS)
-    k_permute_predict(State src, State dst, unsigned n_init, const int *order, const int *key,
-                      int *key_sorted, const Counters *cnt, Consts c, int predict, RecT *rec,
+    k_permute_predict(State src, State dst, unsigned n_init, int *order, const int *scattered,
+                      const int *off, const int *key, int *key_sorted, const Counters *cnt, Consts c, int predict, RecT *rec,
                       double4 *nl4, double2 *pse2, double4 *cs4, double *p_dbg, double *R_dbg) {
-  permute_predict<RecT>(blockIdx.x, src, dst, n_init, order, key, key_sorted, cnt, c, predict, rec,
+  permute_predict<RecT>(blockIdx.x, src, dst, n_init, order, scattered, off, key, key_sorted, cnt, c, predict, rec,
                         nl4, pse2, cs4, p_dbg, R_dbg);
 }
 
@@ -392,34 +421,43 @@ static inline unsigned nblocks(long n, int bs) { return (unsigned)((n + bs - 1) 
 void launch_blank_hash_count(hipStream_t s, const State &st, unsigned n_init, const GridInfo &g,
                              int blanking, const double *bb, double vmax2, GridBuffers &gb,
                              Counters *cnt) {
-  hipLaunchKernelGGL(k_zero_cells, dim3(nblocks(g.num_cell + 1, BS)), dim3(BS), 0, s, gb.count,
-                     gb.fill, g.num_cell);
   double z[6] = {0, 0, 0, 0, 0, 0};
   const double *b = bb ? bb : z;
   hipLaunchKernelGGL(k_blank_hash_count, dim3(gb.nblk), dim3(BS), 0, s, st, n_init, g, blanking,
-                     b[0], b[1], b[2], b[3], b[4], b[5], vmax2, gb.key, gb.count, gb.blk, cnt);
+                     b[0], b[1], b[2], b[3], b[4], b[5], vmax2, gb.key, gb.hist, gb.order, gb.blk, cnt);
+}
+
+// The order inside the cells in a launch of its own or by the permutation, whose gathers then wait for
+// four dependent reads more: 8,000 particles 2.5 us and a launch against 1.1 more; 1M 7.6 us against 28
+bool order_apart(long particles) { return particles >= 128 * 1024; }
+
+int scan_tiles(long num_cell, bool alone) {
+  return (int)nblocks(num_cell, alone ? SCAN_TILE_ALONE : SCAN_TILE);
 }
 
 void launch_scan_cells(hipStream_t s, const GridInfo &g, GridBuffers &gb, unsigned n_init,
                        Counters *cnt) {
-  (void)n_init;
-  int nparts = (int)nblocks(g.num_cell, SCAN_TILE);
-  hipLaunchKernelGGL(k_scan_reduce, dim3(nparts), dim3(BS), 0, s, gb.count, g.num_cell, gb.blk2);
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(SB), 0, s, gb.blk2, nparts, gb.blk, gb.nblk,
-                     gb.count, g.num_cell, cnt);
-  hipLaunchKernelGGL(k_scan_down, dim3(nparts), dim3(BS), 0, s, gb.count, g.num_cell, gb.blk2);
+  const bool alone = g.num_cell <= SCAN_ALONE;
+  const dim3 tiles((unsigned)scan_tiles(g.num_cell, alone));
+  if (alone) {
+    hipLaunchKernelGGL((k_scan_cells<SCAN_NT, SCAN_TILE_ALONE / SCAN_NT>), tiles, dim3(SCAN_NT), 0, s, gb.hist, g.num_cell,
+                       (const int *)nullptr, gb.count, n_init, cnt);
+    return;
+  }
+  hipLaunchKernelGGL(k_scan_reduce, tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2);
+  hipLaunchKernelGGL((k_scan_cells<BS, SCAN_ITEMS>), tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2,
+                     gb.count, n_init, cnt);
 }
 
 void launch_scatter(hipStream_t s, unsigned n_init, const GridInfo &g, GridBuffers &gb,
                     Counters *cnt) {
-  (void)g;
-  hipLaunchKernelGGL(k_scatter, dim3(gb.nblk), dim3(BS), 0, s, n_init, gb.key, gb.count, gb.fill,
-                     gb.blk, cnt, gb.order);
+  hipLaunchKernelGGL(k_scatter, dim3(gb.nblk), dim3(BS), 0, s, n_init, g.num_cell, gb.key, gb.count,
+                     gb.order, gb.hist, gb.blk, cnt, gb.scattered);
 }
 
-void launch_fixup(hipStream_t s, const GridInfo &g, GridBuffers &gb) {
-  hipLaunchKernelGGL(k_fixup, dim3(nblocks(g.num_cell, BS)), dim3(BS), 0, s, gb.count, g.num_cell,
-                     gb.order);
+void launch_order(hipStream_t s, unsigned n_init, GridBuffers &gb) {
+  hipLaunchKernelGGL(k_order, dim3(nblocks(n_init, BS)), dim3(BS), 0, s, n_init, gb.scattered, gb.key,
+                     gb.count, gb.order);
 }
 
 void launch_permute_predict_ex(hipStream_t s, const State &src, const State &dst, unsigned n_init,
@@ -428,19 +466,12 @@ void launch_permute_predict_ex(hipStream_t s, const State &src, const State &dst
                                double *p_dbg, double *R_dbg) {
   if (c.precision == MFG_FP64)
     hipLaunchKernelGGL(k_permute_predict<Rec64>, dim3(nblocks(n_init, BS)), dim3(BS), 0, s, src,
-                       dst, n_init, gb.order, gb.key, gb.key_sorted, cnt, c, predict, (Rec64 *)rec,
+                       dst, n_init, gb.order, gb.scattered, gb.count, gb.key, gb.key_sorted, cnt, c, predict, (Rec64 *)rec,
                        nl4, pse2, cs4, p_dbg, R_dbg);
   else
     hipLaunchKernelGGL(k_permute_predict<Rec32>, dim3(nblocks(n_init, BS)), dim3(BS), 0, s, src,
-                       dst, n_init, gb.order, gb.key, gb.key_sorted, cnt, c, predict, (Rec32 *)rec,
+                       dst, n_init, gb.order, gb.scattered, gb.count, gb.key, gb.key_sorted, cnt, c, predict, (Rec32 *)rec,
                        nl4, pse2, cs4, p_dbg, R_dbg);
-}
-
-void launch_permute_predict(hipStream_t s, const State &src, const State &dst, unsigned n_init,
-                            const GridBuffers &gb, const Counters *cnt, const Consts &c,
-                            int predict, void *rec, double4 *nl4, double2 *pse2, double4 *cs4) {
-  launch_permute_predict_ex(s, src, dst, n_init, gb, cnt, c, predict, rec, nl4, pse2, cs4, nullptr,
-                            nullptr);
 }
 
 void launch_cells_to_tables(hipStream_t s, const GridInfo &g, const int *offsets, int rothlin,
@@ -459,68 +490,61 @@ void launch_bbox_reduce(hipStream_t s, const State &st, const Counters *cnt, uns
 // batched launches: the same bodies, arguments from each instance's descriptor.  Before the
 // permutation an instance's state is buf[cur], after it buf[cur ^ 1].
 // ---------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(BS) kb_zero_cells(const Inst *in, BatchMap m) {
-  unsigned b, nb;
-  const Inst &d = in[batch_locate(m, b, nb)];
-  zero_cells(b, d.gb.count, d.gb.fill, d.g.num_cell);
-}
-
 __global__ void __launch_bounds__(BS) kb_blank_hash_count(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
   blank_hash_count(b, d.buf[d.cur], d.n_init, d.g, d.blanking, d.bb[0], d.bb[1], d.bb[2], d.bb[3],
-                   d.bb[4], d.bb[5], d.vmax2, d.gb.key, d.gb.count, d.gb.blk, d.cnt);
+                   d.bb[4], d.bb[5], d.vmax2, d.gb.key, d.gb.hist, d.gb.order, d.gb.blk, d.cnt);
 }
 
 __global__ void __launch_bounds__(BS) kb_scan_reduce(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  scan_reduce(b, d.gb.count, d.g.num_cell, d.gb.blk2);
+  scan_reduce(b, d.gb.hist, d.g.num_cell, d.gb.blk2);
 }
 
-__global__ void __launch_bounds__(SB) kb_scan_top(const Inst *in, BatchMap m) {
+template <int NT, int ITEMS>
+__global__ void __launch_bounds__(NT) kb_scan_cells(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  scan_top(d.gb.blk2, d.nparts, d.gb.blk, d.gb.nblk, d.gb.count, d.g.num_cell, d.cnt);
-}
-
-__global__ void __launch_bounds__(BS) kb_scan_down(const Inst *in, BatchMap m) {
-  unsigned b, nb;
-  const Inst &d = in[batch_locate(m, b, nb)];
-  scan_down(b, d.gb.count, d.g.num_cell, d.gb.blk2);
+  scan_cells<NT, ITEMS>(b, d.gb.hist, d.g.num_cell, NT == BS ? d.gb.blk2 : nullptr, d.gb.count, d.n_init,
+                        d.cnt);
 }
 
 __global__ void __launch_bounds__(BS) kb_scatter(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  scatter(b, d.n_init, d.gb.key, d.gb.count, d.gb.fill, d.gb.blk, d.cnt, d.gb.order);
+  scatter(b, nb, d.n_init, d.g.num_cell, d.gb.key, d.gb.count, d.gb.order, d.gb.hist, d.gb.blk, d.cnt,
+          d.gb.scattered);
 }
 
-__global__ void __launch_bounds__(BS) kb_fixup(const Inst *in, BatchMap m) {
+__global__ void __launch_bounds__(BS) kb_order(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  fixup(b, d.gb.count, d.g.num_cell, d.gb.order);
+  order_cells(b, d.n_init, d.gb.scattered, d.gb.key, d.gb.count, d.gb.order);
 }
 
 template <class RecT>
 __global__ void __launch_bounds__(BS) kb_permute_predict(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  permute_predict<RecT>(b, d.buf[d.cur], d.buf[d.cur ^ 1], d.n_init, d.gb.order, d.gb.key,
-                        d.gb.key_sorted, d.cnt, d.c, 1, (RecT *)d.rec, d.nl4, d.pse2, d.cs4,
+  permute_predict<RecT>(b, d.buf[d.cur], d.buf[d.cur ^ 1], d.n_init, d.gb.order, d.ordered ? nullptr : d.gb.scattered,
+                        d.gb.count, d.gb.key, d.gb.key_sorted, d.cnt, d.c, 1, (RecT *)d.rec, d.nl4, d.pse2, d.cs4,
                         nullptr, nullptr);
 }
 
-// hash + blanking, scan, scatter and fix-up of every instance (the sort permutation and cell
-// offsets), as sort_keys does for one
+// hash + blanking, scan and scatter of every instance, as sort_keys does for one
 void launch_batch_sort(hipStream_t s, const BatchLaunch &L) {
-  hipLaunchKernelGGL(kb_zero_cells, dim3(L.cells1.blocks), dim3(BS), 0, s, L.inst, L.cells1.m);
   hipLaunchKernelGGL(kb_blank_hash_count, dim3(L.parts.blocks), dim3(BS), 0, s, L.inst, L.parts.m);
-  hipLaunchKernelGGL(kb_scan_reduce, dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
-  hipLaunchKernelGGL(kb_scan_top, dim3(L.one.blocks), dim3(SB), 0, s, L.inst, L.one.m);
-  hipLaunchKernelGGL(kb_scan_down, dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
+  if (L.scan_alone) {
+    hipLaunchKernelGGL((kb_scan_cells<SCAN_NT, SCAN_TILE_ALONE / SCAN_NT>), dim3(L.tiles.blocks), dim3(SCAN_NT), 0, s,
+                       L.inst, L.tiles.m);
+  } else {
+    hipLaunchKernelGGL(kb_scan_reduce, dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
+    hipLaunchKernelGGL((kb_scan_cells<BS, SCAN_ITEMS>), dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
+  }
   hipLaunchKernelGGL(kb_scatter, dim3(L.parts.blocks), dim3(BS), 0, s, L.inst, L.parts.m);
-  hipLaunchKernelGGL(kb_fixup, dim3(L.cells.blocks), dim3(BS), 0, s, L.inst, L.cells.m);
+  if (L.ordered) hipLaunchKernelGGL(kb_order, dim3(L.parts.blocks), dim3(BS), 0, s, L.inst, L.parts.m);
 }
 
 void launch_batch_permute(hipStream_t s, const BatchLaunch &L) {

@@ -153,10 +153,12 @@ struct ToolSet {
 struct GridBuffers {
   int *key;          // N_init, unsorted
   int *key_sorted;   // N_init
-  int *order;        // N_init
-  int *count;        // num_cell + 1 (counts, then exclusive offsets)
-  int *fill;         // num_cell
-  int *blk;          // per-block blanked counts / offsets
+  int *order;        // N_init; within a sort the slots inside the cells, until the order is known
+  int *scattered;    // N_init: the particles by cell, in no order inside one (permute: null once
+                     // order is final)
+  int *count;        // num_cell + 1: exclusive offsets of the cells
+  int *hist;         // num_cell particle counts of a sort under way; zero between sorts
+  int *blk;          // per-block blanked counts
   int *blk2;         // scan scratch
   int nblk;          // blocks of the hash kernel
 };
@@ -168,10 +170,12 @@ void launch_scan_cells(hipStream_t s, const GridInfo &g, GridBuffers &gb, unsign
                        Counters *cnt);
 void launch_scatter(hipStream_t s, unsigned n_init, const GridInfo &g, GridBuffers &gb,
                     Counters *cnt);
-void launch_fixup(hipStream_t s, const GridInfo &g, GridBuffers &gb);
-void launch_permute_predict(hipStream_t s, const State &src, const State &dst, unsigned n_init,
-                            const GridBuffers &gb, const Counters *cnt, const Consts &c,
-                            int predict, void *rec, double4 *nl4, double2 *pse2, double4 *cs4);
+void launch_order(hipStream_t s, unsigned n_init, GridBuffers &gb);
+// cells per workgroup of the scan; up to SCAN_ALONE cells it runs without tile sums
+constexpr int SCAN_TILE = 256 * 16, SCAN_TILE_ALONE = 1024 * 4;
+constexpr long SCAN_ALONE = 128 * 1024;
+int scan_tiles(long num_cell, bool alone);
+bool order_apart(long particles);  // whether a step runs launch_order
 void launch_cells_to_tables(hipStream_t s, const GridInfo &g, const int *offsets, int rothlin,
                             int *start, int *end);
 void launch_bbox_reduce(hipStream_t s, const State &st, const Counters *cnt, unsigned n_init,
@@ -279,7 +283,7 @@ struct Inst {
   unsigned n_init;
   GridInfo g;
   GridBuffers gb;
-  int nparts;                 // scan tiles of the cell counts
+  int ordered;                // the sort leaves gb.order final (order_apart)
   int blanking;
   double bb[6], vmax2;        // blanking box and squared speed limit
   Consts c;
@@ -312,8 +316,8 @@ struct BatchLaunch {
   int precision, pse;
   int brook;         // an instance conducts heat by Brookshaw's form
   int cell_tile;     // cells per wavefront of the neighbour pass
-  BatchGrid cells1;  // num_cell + 1 entries, 256 per workgroup
-  BatchGrid cells;   // num_cell entries, 256 per workgroup
+  int ordered;       // order_apart
+  int scan_alone;    // no instance has more than SCAN_ALONE cells
   BatchGrid tiles;   // scan tiles of the cell counts
   BatchGrid one;     // one workgroup per instance
   BatchGrid parts;   // N_init particles, 256 per workgroup
