@@ -29,7 +29,7 @@ namespace mfg {
 void launch_permute_predict_ex(hipStream_t s, const State &src, const State &dst, unsigned n_init,
                                const GridBuffers &gb, const Counters *cnt, const Consts &c,
                                int predict, void *rec, double4 *nl4, double2 *pse2, double4 *cs4,
-                               double *p_dbg, double *R_dbg);
+                               double *p_dbg, double *R_dbg, unsigned *list_n);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -341,6 +341,15 @@ int grid_alloc(mfg_grid *g) {
   return MFG_OK;
 }
 
+// the moving box and clock of a tool whose triangles move to time tc
+void advance_tool(mfg_tool *t, double tc, double dt) {
+  t->mesh_tc = tc;
+  for (int k = 0; k < 3; k++) {
+    t->bbmin[k] += dt * t->vel[k];
+    t->bbmax[k] += dt * t->vel[k];
+  }
+}
+
 GridBuffers grid_buffers(mfg_grid *g, mfg_particles *p) {
   GridBuffers gb;
   gb.key = p->key;
@@ -463,14 +472,16 @@ void sort_keys(mfg_grid *g, mfg_particles *p, const mfg_blanking_state *b, bool 
 enum PermuteFrom { FROM_ORDER, FROM_SCATTERED, IN_PLACE };
 // FROM_SCATTERED: of a sort that left the order inside the cells open.  IN_PLACE: the particle order
 // stays (a step between sorts): no gather, keys kept
-void permute(mfg_grid *g, mfg_particles *p, const Consts &c, int predict, PermuteFrom from) {
+// list_n: a counter to clear in the same launch
+void permute(mfg_grid *g, mfg_particles *p, const Consts &c, int predict, PermuteFrom from,
+             unsigned *list_n = nullptr) {
   GridBuffers gb = grid_buffers(g, p);
   if (from == IN_PLACE) gb.order = nullptr;
   if (from != FROM_SCATTERED) gb.scattered = nullptr;
   ProfScope ps(predict ? "permute_predict" : "permute");
   int nxt = 1 - p->cur;
   launch_permute_predict_ex(g_lib.stream, p->buf[p->cur], p->buf[nxt], p->N_init, gb, p->cnt, c,
-                            predict, p->rec, p->nl4, p->pse2, p->cs4, p->p_dbg, p->R_dbg);
+                            predict, p->rec, p->nl4, p->pse2, p->cs4, p->p_dbg, p->R_dbg, list_n);
   p->cur = nxt;
 }
 
@@ -1467,7 +1478,7 @@ int mfg_grid_neighbours(mfg_grid *g, mfg_particles *p, int *h_counts, int *h_lis
   HIP_TRY(hipMemcpyAsync(p->key, p->key_sorted, sizeof(int) * p->N_init, hipMemcpyDeviceToDevice, g_lib.stream));
   HIP_TRY(hipStreamSynchronize(g_lib.stream));
   launch_permute_predict_ex(g_lib.stream, st, p->buf[1 - p->cur], p->N_init, gb, p->cnt, c, 1,
-                            p->rec, p->nl4, p->pse2, p->cs4, nullptr, nullptr);
+                            p->rec, p->nl4, p->pse2, p->cs4, nullptr, nullptr, nullptr);
   p->cur = 1 - p->cur;
   HIP_TRY(hipMemcpyAsync(p->order, saved_order, sizeof(int) * p->N_init, hipMemcpyDeviceToDevice, g_lib.stream));
   HIP_TRY(hipMemcpyAsync(p->key, saved_keys, sizeof(int) * p->N_init, hipMemcpyDeviceToDevice, g_lib.stream));
@@ -1729,11 +1740,7 @@ int mfg_tool_update(mfg_tool *t, double tc, double dt) {
     launch_tool_update(g_lib.stream, t->tris, t->p_init_all, t->n_tris, tc, t->vel, t->boxed,
                        t->p_init_boxed, t->n_boxed);
   }
-  t->mesh_tc = tc;
-  for (int k = 0; k < 3; k++) {
-    t->bbmin[k] += dt * t->vel[k];
-    t->bbmax[k] += dt * t->vel[k];
-  }
+  advance_tool(t, tc, dt);
   return MFG_OK;
 }
 
@@ -1947,11 +1954,11 @@ int step_impl(mfg_leap_frog *lf, mfg_particles *p, mfg_grid *g, int record,
   }
   if (keep_last_sort(g, p)) {
     p->since_sort++;
-    permute(g, p, c, 1, IN_PLACE);
+    permute(g, p, c, 1, IN_PLACE, cs.list_n);
   } else {
     const bool apart = order_apart(p->N_init);
     sort_keys(g, p, blanking, apart);
-    permute(g, p, c, 1, apart ? FROM_ORDER : FROM_SCATTERED);
+    permute(g, p, c, 1, apart ? FROM_ORDER : FROM_SCATTERED, cs.list_n);
   }
   g->scanned = false;  // the permutation is applied: a later mfg_grid_sort hashes again
   // pair pass
@@ -1974,32 +1981,46 @@ int step_impl(mfg_leap_frog *lf, mfg_particles *p, mfg_grid *g, int record,
     launch_pair(s, p->N_init, p->st(), p->rec, p->nbr, p->nl_stride, p->count, c, p->cnt,
                 p->sums, p->sum_stride, trav, p->cs4, g_lib.opt.pair_block, !g->locked);
   }
-  {
-    ProfScope ps("particle_update");
-    launch_particle_update(s, p->N_init, p->st(), p->sums, p->sum_stride, p->poison, c, p->cnt);
-  }
-  // tools
+  // tools: their motion and boxes of this step
   ToolSet ts;
+  ToolMoves mv;
   std::memset(&ts, 0, sizeof(ts));
+  std::memset(&mv, 0, sizeof(mv));
   ts.n = n_tools;
   ts.record = record ? 1 : 0;
-  if (record) launch_zero_f32(s, forces->d, 3 * forces->n);
+  mv.t = t_current;
+  auto moves = [&](const mfg_tool *t, Tri *tris, const double *p_init, int n) {
+    if (n <= 0 || !tris) return;
+    mv.tris[mv.n] = tris;
+    mv.p_init[mv.n] = p_init;
+    mv.end[mv.n] = (mv.n > 0 ? mv.end[mv.n - 1] : 0) + n;
+    for (int a = 0; a < 3; a++) mv.vel[mv.n][a] = t->vel[a];
+    mv.n++;
+  };
   for (int k = 0; k < n_tools; k++) {
     mfg_tool *t = tools[k];
-    rc = mfg_tool_update(t, t_current, dt);
-    if (rc != MFG_OK) return rc;
+    if (t->n_boxed > 0) {
+      // the exhaustive search runs over the boxed copies too (grid-accelerated, same result)
+      if (t->algo != MFG_CONTACT_HASHED) moves(t, t->tris, t->p_init_all, t->n_tris);
+      moves(t, t->boxed, t->p_init_boxed, t->n_boxed);
+      advance_tool(t, t_current, dt);
+    }
     fill_tool_view(t, t_current, ts.t[k]);
+    if (search && ts.t[k].algo == MFG_CONTACT_EXHAUSTIVE) {
+      ts.t[k].slot = cs.slot + (size_t)k * p->N_init;
+      ts.t[k].res = cs.res;
+    }
   }
+  {
+    ProfScope ps("particle_update");
+    launch_particle_update(s, p->N_init, p->st(), p->sums, p->sum_stride, p->poison, c, p->cnt, ts, cs, mv);
+  }
+  if (record) launch_zero_f32(s, forces->d, 3 * forces->n);
   if (n_tools > 0)
     for (int a = 0; a < 3; a++) ts.fric_vel[a] = tools[0]->vel[a];
   if (search) {
     ProfScope ps("contact_search");
-    for (int k = 0; k < n_tools; k++)
-      if (ts.t[k].algo == MFG_CONTACT_EXHAUSTIVE) {
-        ts.t[k].slot = cs.slot + (size_t)k * p->N_init;
-        ts.t[k].res = cs.res;
-      }
-    launch_contact_search(s, p->st(), p->N_init, ts, p->cnt, cs);
+    launch_contact_search(s, p->st(), ts, cs);
   }
   {
     ProfScope ps("contact_bc");
@@ -2387,6 +2408,7 @@ void batch_launch_step(mfg_batch *b, int record) {
   }
   {
     ProfScope ps("batch_pair");
+    launch_batch_tools(s, b->L, record);
     launch_batch_pair(s, b->L);
   }
   {

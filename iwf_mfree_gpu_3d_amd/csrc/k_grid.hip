@@ -364,7 +364,10 @@ template <class RecT>
 __global__ void __launch_bounds__(BS)
     k_permute_predict(State src, State dst, unsigned n_init, int *order, const int *scattered,
                       const int *off, const int *key, int *key_sorted, const Counters *cnt, Consts c, int predict, RecT *rec,
-                      double4 *nl4, double2 *pse2, double4 *cs4, double *p_dbg, double *R_dbg) {
+                      double4 *nl4, double2 *pse2, double4 *cs4, double *p_dbg, double *R_dbg,
+                      unsigned *list_n) {
+  // the contact search's list, which the particle update fills, starts empty
+  if (list_n && blockIdx.x == 0 && threadIdx.x == 0) *list_n = 0u;
   permute_predict<RecT>(blockIdx.x, src, dst, n_init, order, scattered, off, key, key_sorted, cnt, c, predict, rec,
                         nl4, pse2, cs4, p_dbg, R_dbg);
 }
@@ -463,15 +466,15 @@ void launch_order(hipStream_t s, unsigned n_init, GridBuffers &gb) {
 void launch_permute_predict_ex(hipStream_t s, const State &src, const State &dst, unsigned n_init,
                                const GridBuffers &gb, const Counters *cnt, const Consts &c,
                                int predict, void *rec, double4 *nl4, double2 *pse2, double4 *cs4,
-                               double *p_dbg, double *R_dbg) {
+                               double *p_dbg, double *R_dbg, unsigned *list_n) {
   if (c.precision == MFG_FP64)
     hipLaunchKernelGGL(k_permute_predict<Rec64>, dim3(nblocks(n_init, BS)), dim3(BS), 0, s, src,
                        dst, n_init, gb.order, gb.scattered, gb.count, gb.key, gb.key_sorted, cnt, c, predict, (Rec64 *)rec,
-                       nl4, pse2, cs4, p_dbg, R_dbg);
+                       nl4, pse2, cs4, p_dbg, R_dbg, list_n);
   else
     hipLaunchKernelGGL(k_permute_predict<Rec32>, dim3(nblocks(n_init, BS)), dim3(BS), 0, s, src,
                        dst, n_init, gb.order, gb.scattered, gb.count, gb.key, gb.key_sorted, cnt, c, predict, (Rec32 *)rec,
-                       nl4, pse2, cs4, p_dbg, R_dbg);
+                       nl4, pse2, cs4, p_dbg, R_dbg, list_n);
 }
 
 void launch_cells_to_tables(hipStream_t s, const GridInfo &g, const int *offsets, int rothlin,

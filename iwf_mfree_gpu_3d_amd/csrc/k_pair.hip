@@ -532,9 +532,10 @@ struct PairSums {
   double vt[3], xt[3], Tl;
 };
 
-__device__ __forceinline__ void particle_update(const State &st, unsigned i, uint32_t fl,
+// x: the new position; false if the particle was invalidated
+__device__ __forceinline__ bool particle_update(const State &st, unsigned i, uint32_t fl,
                                                 const Consts &c, const PairSums &ps,
-                                                bool brook, double thermal_alpha) {
+                                                bool brook, double thermal_alpha, double (&x)[3]) {
   const bool tool = (fl & FL_TOOL) != 0;
   const double dt = c.dt, hdt = 0.5 * c.dt;
   double x0[3] = {st.x[i], st.y[i], st.z[i]};
@@ -590,10 +591,10 @@ __device__ __forceinline__ void particle_update(const State &st, unsigned i, uin
                  bad(nSt[4]) || bad(nSt[5]) || bad(nrho_t) || bad(nT_t);
   if (invalid) {
     st.flags[i] = fl | FL_BLANKED;
-    return;
+    return false;
   }
   // correct (src/leap_frog.cu:72-100)
-  double x[3], v[3], S[6];
+  double v[3], S[6];
 #pragma unroll
   for (int k = 0; k < 3; k++) {
     x[k] = x0[k] + dt * nxt[k];
@@ -611,6 +612,7 @@ __device__ __forceinline__ void particle_update(const State &st, unsigned i, uin
   for (int k = 0; k < 6; k++) st.S[k][i] = S[k];
   st.rho[i] = rho;
   st.T[i] = T;
+  return true;
 }
 
 // The pair kernels end by storing a particle's neighbour sums (SoA, PAIR_SUMS doubles per
@@ -636,11 +638,13 @@ __device__ __forceinline__ void store_sums(double *__restrict__ sums, size_t str
 }
 
 // Jaumann rate, continuity, momentum, advection, invalidation, leap-frog correction and the
-// Johnson-Cook radial return of every particle the pair pass summed (not blanked, in a cell)
+// Johnson-Cook radial return of every particle the pair pass summed (not blanked, in a cell), and its
+// entry in the contact search's list (list_n null: none)
 __device__ __forceinline__ void update_body(unsigned b, unsigned n_init, const State &st,
                                             const double *__restrict__ sums, size_t stride,
                                             const int *__restrict__ poison, const Consts &c,
-                                            const Counters *cnt) {
+                                            const Counters *cnt, const ToolSet &ts,
+                                            const ContactSearch &cs) {
   const unsigned i = b * blockDim.x + threadIdx.x;
   if (i >= cnt->N || i >= n_init) return;
   const uint32_t fl = st.flags[i];
@@ -665,12 +669,28 @@ __device__ __forceinline__ void update_body(unsigned b, unsigned n_init, const S
   const bool tool_nz = (fl & FL_TOOL_NZ) != 0;
   const double thermal_alpha = tool_nz ? c.alpha_tool : c.alpha_wp;
   const bool brook = c.heat == MFG_HEAT_BROOKSHAW && thermal_alpha != 0.;
-  particle_update(st, i, fl, c, ps, brook, thermal_alpha);
+  double x[3];
+  if (particle_update(st, i, fl, c, ps, brook, thermal_alpha, x) && cs.list_n && !(fl & FL_TOOL))
+    contact_list(i, v3(x[0], x[1], x[2]), n_init, ts, cs);
 }
+// The workgroups past the particles' move the tools' triangles, one a thread.  Both would be launches of
+// their own, and a third to clear the list's counter (the permutation does): at 8,000 particles 13 us
+// of launches against none measurable here, at 1M 17 against 2; 24 batched instances list 29 against 12.
 __global__ void __launch_bounds__(BSP)
     k_particle_update(unsigned n_init, State st, const double *__restrict__ sums, size_t stride,
-                      const int *__restrict__ poison, Consts c, const Counters *cnt) {
-  update_body(blockIdx.x, n_init, st, sums, stride, poison, c, cnt);
+                      const int *__restrict__ poison, Consts c, const Counters *cnt, ToolSet ts,
+                      ContactSearch cs, ToolMoves mv) {
+  const unsigned blocks = (n_init + blockDim.x - 1) / blockDim.x;
+  if (blockIdx.x < blocks) {
+    update_body(blockIdx.x, n_init, st, sums, stride, poison, c, cnt, ts, cs);
+    return;
+  }
+  const int k = (int)((blockIdx.x - blocks) * blockDim.x + threadIdx.x);
+  int first = 0;
+  for (int a = 0; a < mv.n; a++) {
+    if (k >= first && k < mv.end[a]) move_tri(mv.tris[a], mv.p_init[a], k - first, mv.t, mv.vel[a]);
+    first = mv.end[a];
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1859,7 +1879,9 @@ __global__ void __launch_bounds__(BSP, PAIR32_WAVES) kb_pair_rows(const Inst *in
 __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  update_body(b, d.n_init, d.buf[d.cur ^ 1], d.sums, d.sum_stride, d.poison, d.c, d.cnt);
+  ContactSearch cs = d.cs;
+  if (!d.search) cs.list_n = nullptr;
+  update_body(b, d.n_init, d.buf[d.cur ^ 1], d.sums, d.sum_stride, d.poison, d.c, d.cnt, d.ts, cs);
 }
 
 // The kernels of the single-instance step in the sorted visiting order; the PSE mode as
@@ -1898,13 +1920,15 @@ void launch_pair_order(hipStream_t s, unsigned n_init, const GridInfo &g, const 
 
 void launch_particle_update(hipStream_t s, unsigned n_init, const State &st, const double *sums,
                             size_t sstride, const int *poison, const Consts &c,
-                            const Counters *cnt) {
+                            const Counters *cnt, const ToolSet &ts, const ContactSearch &cs,
+                            const ToolMoves &mv) {
   // one wavefront per workgroup: the few wavefronts with particles in the Johnson-Cook solve run for
   // six iterations of 1.6 us and more while the others are done, and hold back only themselves (256
   // threads: 8,000 particles 25 us, now 19; 19,000 26, 22.5; 1M 172, 156; 64,000 27, 28)
   constexpr int BS = 64;
-  hipLaunchKernelGGL(k_particle_update, dim3(nb(n_init, BS)), dim3(BS), 0, s, n_init, st, sums,
-                     sstride, poison, c, cnt);
+  const unsigned blocks = nb(n_init, BS) + (mv.n > 0 ? nb(mv.end[mv.n - 1], BS) : 0);
+  hipLaunchKernelGGL(k_particle_update, dim3(blocks), dim3(BS), 0, s, n_init, st, sums, sstride, poison, c,
+                     cnt, ts, cs, mv);
 }
 
 }  // namespace mfg

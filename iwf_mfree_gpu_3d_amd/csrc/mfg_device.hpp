@@ -500,4 +500,37 @@ __device__ __forceinline__ bool ray_hit(const Tri &tr, V3 o, V3 dir, double &t) 
   return (t > EPS);
 }
 
+// ---- tool motion and the exhaustive contact's list ------------------------------------------
+// triangle k at time t: its vertices at time 0 plus v t (update_tool, src/tool_3d_gpu.cu:74-99)
+__device__ __forceinline__ void move_tri(Tri *tris, const double *p_init, int k, double t,
+                                         const double v[3]) {
+#pragma unroll
+  for (int q = 0; q < 3; q++)
+#pragma unroll
+    for (int a = 0; a < 3; a++) tris[k].p[q][a] = p_init[9 * k + 3 * q + a] + v[a] * t;
+}
+
+__device__ __forceinline__ bool in_tool_box(const ToolView &tv, V3 qp) {
+  return qp.x > tv.bbmin[0] && qp.x < tv.bbmax[0] && qp.y > tv.bbmin[1] && qp.y < tv.bbmax[1] &&
+         qp.z > tv.bbmin[2] && qp.z < tv.bbmax[2];
+}
+
+// lists particle i, eligible and at qp, for every active exhaustive tool whose box it is inside (the
+// same test as k_contact_bc) and remembers its entry
+__device__ __forceinline__ void contact_list(unsigned i, V3 qp, unsigned n_init, const ToolSet &ts,
+                                             const ContactSearch &cs) {
+  for (int k = 0; k < ts.n; k++) {
+    const ToolView &tv = ts.t[k];
+    if (!tv.active || tv.algo == MFG_CONTACT_HASHED || !tv.slot) continue;
+    if (!in_tool_box(tv, qp)) continue;
+    const unsigned pos = atomicAdd(cs.list_n, 1u);
+    int sl = -1;
+    if (pos < cs.cap) {
+      cs.list[pos] = make_int2((int)i, k);
+      sl = (int)pos;
+    }
+    cs.slot[(size_t)k * n_init + i] = sl;  // -1: searched per thread by k_contact_bc
+  }
+}
+
 }  // namespace mfg

@@ -209,12 +209,6 @@ void launch_pair_order(hipStream_t s, unsigned n_init, const GridInfo &g, const 
                        int *trav);
 // neighbour sums per particle written by the pair pass (SoA, sum_stride apart)
 constexpr int PAIR_SUM_COUNT = 25;
-// Jaumann, continuity, momentum, advection, invalidation, leap-frog correction and Johnson-Cook
-// radial return from the neighbour sums
-void launch_particle_update(hipStream_t s, unsigned n_init, const State &st, const double *sums,
-                            size_t sum_stride, const int *poison, const Consts &c,
-                            const Counters *cnt);
-
 // A field as the host holds it (w doubles per particle, particle-major) from the device's arrays:
 // element k of particle i is src[k][i], flags and integers turned into doubles
 enum { PACK_F64, PACK_FIXED, PACK_BLANKED, PACK_TOOL, PACK_I32, PACK_SYM6 };  // SYM6: src[0] holds 6 a particle
@@ -232,8 +226,8 @@ void launch_words_to_host(hipStream_t s, const void *src, void *pinned, unsigned
 void launch_tool_update(hipStream_t s, Tri *tris, const double *p_init, int n, double t,
                         const double vel[3], Tri *tris2 = nullptr, const double *p_init2 = nullptr,
                         int n2 = 0);
-// exhaustive contact, lane-parallel: list the (particle, tool) pairs inside a tool box, then one
-// wavefront per pair finds the closest triangle; k_contact_bc reads the results
+// exhaustive contact, lane-parallel: of the listed (particle, tool) pairs inside a tool box one
+// wavefront each finds the closest triangle; k_contact_bc reads the results
 struct ContactSearch {
   int2 *list;           // (particle, tool)
   unsigned *list_n;     // entries appended this step
@@ -241,8 +235,23 @@ struct ContactSearch {
   int *slot;            // n_init per tool: entry of the particle, -1 if not listed
   double *res;          // 6 doubles per entry
 };
-void launch_contact_search(hipStream_t s, const State &st, unsigned n_init, const ToolSet &ts,
-                           const Counters *cnt, const ContactSearch &cs);
+// Jaumann, continuity, momentum, advection, invalidation, leap-frog correction and Johnson-Cook
+// radial return from the neighbour sums.  In the same launch: the tools' triangles move (mv), and a
+// particle whose new place is inside a tool's box is listed for the search (cs.list_n null: none)
+struct ToolMoves {
+  Tri *tris[2 * MAX_TOOLS];
+  const double *p_init[2 * MAX_TOOLS];
+  int end[2 * MAX_TOOLS];  // triangles of the arrays up to and including this one
+  double vel[2 * MAX_TOOLS][3];
+  double t;
+  int n;                   // arrays
+};
+void launch_particle_update(hipStream_t s, unsigned n_init, const State &st, const double *sums,
+                            size_t sum_stride, const int *poison, const Consts &c,
+                            const Counters *cnt, const ToolSet &ts, const ContactSearch &cs,
+                            const ToolMoves &mv);
+
+void launch_contact_search(hipStream_t s, const State &st, const ToolSet &ts, const ContactSearch &cs);
 void launch_contact_bc(hipStream_t s, const State &st, unsigned n_init, const ToolSet &ts,
                        const Consts &c, const Counters *cnt, float *partials, int nblocks);
 void launch_force_reduce(hipStream_t s, const float *partials, int nblocks, int n_tools,
@@ -329,6 +338,7 @@ struct BatchLaunch {
 void launch_batch_sort(hipStream_t s, const BatchLaunch &L);
 void launch_batch_permute(hipStream_t s, const BatchLaunch &L);
 void launch_batch_pair(hipStream_t s, const BatchLaunch &L);
+void launch_batch_tools(hipStream_t s, const BatchLaunch &L, int record);
 void launch_batch_contact(hipStream_t s, const BatchLaunch &L, int record);
 
 // ---------------------------------------------------------------------------------------------
