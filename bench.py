@@ -404,7 +404,7 @@ def main():
                     help="served / batched forms: one launch per kernel over the instances of a precision "
                          "(batched) or each instance's own kernels on a stream pool (streams)")
     ap.add_argument("--cell-tile", type=int, default=0, choices=[0, 1, 2, 4, 8, 16],
-                    help="cells per wavefront of the neighbour pass (0 automatic)")
+                    help="cell tile (accepted, without effect)")
     ap.add_argument("--sort-interval", type=int, default=0,
                     help="opt-in: sort every k-th step of the single-instance runs (0 or 1: every step, "
                          "the reference's schedule; other values change the results)")

@@ -110,11 +110,8 @@ typedef struct {
                          16 (FP32 modes), or the sorted order when five x-rows of records fit in
                          2 MB (small instances: the strips would only add two launches), a
                          negative value the sorted order.  The sums do not depend on it. */
-  int cell_tile;      /* neighbour pass: consecutive grid cells each wavefront takes in turn (1, 2,
-                         4, 8 or 16; the tile's empty cells cost one ballot, not a workgroup);
-                         0 selects 1, or, where the grid has two or more cells per particle
-                         (wide margins around the block), 4 from 256k cells and 16 from 1M.
-                         Lists and sums do not depend on it. */
+  int cell_tile;      /* 0, 1, 2, 4, 8 or 16, without effect: the neighbour pass runs over the
+                         occupied cells alone, so empty ones need no grouping. */
   int sort_interval;  /* opt-in, no counterpart in the reference (which sorts every step,
                          src/leap_frog.cu:139-145): mfg_leap_frog_step sorts a particle set on
                          every k-th step only; in between, the particle order, the cell tables
@@ -345,9 +342,7 @@ int mfg_batch_add(mfg_batch *b, mfg_particles *p, mfg_grid *g, mfg_tool *const *
                   double dt, double t_current, int *slot);
 int mfg_batch_remove(mfg_batch *b, int slot);
 int mfg_batch_size(const mfg_batch *b);
-/* cells per wavefront of the batch's neighbour pass (1, 2, 4, 8, 16), as mfg_options.cell_tile for a
- * single step; 0 (the default): mfg_options.cell_tile, automatic over the whole batch when that
- * is 0 too.  Results do not depend on it. */
+/* 0, 1, 2, 4, 8 or 16, without effect, as mfg_options.cell_tile */
 int mfg_batch_set_cell_tile(mfg_batch *b, int cell_tile);
 int mfg_batch_get_time(const mfg_batch *b, int slot, double *t);
 int mfg_batch_step(mfg_batch *b, int n_steps, int record_forces, int use_graph);

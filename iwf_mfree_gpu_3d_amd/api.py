@@ -93,7 +93,7 @@ def set_options(cspm: bool = False, heat: int = MFG_HEAT_BROOKSHAW, single_sqrt:
     """Switches that are compile-time macros in the reference (src/types.h:32-108), the
     pair-pass kernel (MFG_PAIR_LIST; MFG_PAIR_TILED selects the same one), the pair pass's
     visiting order (strip width in grid columns; 0 default, negative the sorted order),
-    the neighbour pass's cell tile (cells per wavefront: 1, 2, 4, 8; 0 automatic), the opt-in
+    a cell tile (accepted, without effect: the neighbour pass takes the occupied cells), the opt-in
     re-sort interval (sort every k-th step on a locked, still grid; 0 or 1 every step, as the
     reference: other values change the neighbour lists and results) and the pair pass's
     workgroup size (64, 128, 256; 0 selects 256; the sums do not depend on it)."""
@@ -673,7 +673,7 @@ class batch:
             self.set_cell_tile(cell_tile)
 
     def set_cell_tile(self, cell_tile: int) -> None:
-        """Cells per wavefront of the neighbour pass (1, 2, 4, 8; 0 automatic)."""
+        """Accepted (0, 1, 2, 4, 8, 16), without effect: the neighbour pass takes the occupied cells."""
         check(_L().mfg_batch_set_cell_tile(self._h, int(cell_tile)))
 
     def __del__(self):

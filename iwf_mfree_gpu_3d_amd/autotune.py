@@ -2,8 +2,8 @@
 
 Every choice offered leaves results bit-identical, so the tuner only measures time:
 - the pair pass's visiting order (strip width in grid columns, or the sorted order);
-- the neighbour pass's cell tile (consecutive grid cells per wavefront: 1, 2, 4, 8, 16), which
-  decides how much an empty cell of a grid with wide margins costs;
+- a cell tile (1, 2, 4, 8, 16), kept for tables made before: the neighbour pass takes the occupied
+  cells, and every tile runs the same;
 - the pair pass's workgroup size (64, 128, 256 threads): every wavefront works alone, and
   smaller workgroups spread a small instance over more compute units.
 
@@ -35,7 +35,7 @@ from . import api
 # (pair pass, strip): 0 the library's default, -1 the sorted order
 CANDIDATES = ((api.MFG_PAIR_LIST, 0), (api.MFG_PAIR_LIST, -1), (api.MFG_PAIR_LIST, 8),
               (api.MFG_PAIR_LIST, 16))
-# cells per wavefront of the neighbour pass; 0 the library's automatic choice
+# cell tiles (without effect on the run); 0 the default
 TILES = (1, 2, 4, 8, 16)
 # threads per workgroup of the list pair pass; 0 the library's default (256)
 BLOCKS = (64, 128, 256)

@@ -245,7 +245,8 @@ struct mfg_grid {
   long nx = 0, ny = 0, nz = 0, num_cell = 0, max_cell = 0;
   int *count = nullptr;  // max_cell + 1: counts, then offsets
   int *hist = nullptr;
-  int *parts = nullptr;
+  int *occ = nullptr;
+  unsigned long long *parts = nullptr;
   int nparts_cap = 0;
   double *bbox_part = nullptr;
   std::vector<double> bbox_host;  // host copy of the bbox partials (sized at creation)
@@ -331,11 +332,13 @@ void free_particles(mfg_particles *p) {
 
 int grid_alloc(mfg_grid *g) {
   HIP_TRY(hipMalloc(&g->count, sizeof(int) * (g->max_cell + 1)));
+  HIP_TRY(hipMalloc(&g->occ, sizeof(int) * (g->max_cell + 1)));
+  HIP_TRY(hipMemsetAsync(g->occ, 0, sizeof(int) * (g->max_cell + 1), g_lib.stream));  // none before a sort
   HIP_TRY(hipMalloc(&g->hist, sizeof(int) * (g->max_cell + 1)));
   HIP_TRY(hipMemsetAsync(g->hist, 0, sizeof(int) * (g->max_cell + 1), g_lib.stream));
   HIP_TRY(hipStreamSynchronize(g_lib.stream));  // a sort may run on a stream set later
   g->nparts_cap = scan_tiles(g->max_cell, false) + 1;
-  HIP_TRY(hipMalloc(&g->parts, sizeof(int) * g->nparts_cap));
+  HIP_TRY(hipMalloc(&g->parts, sizeof(unsigned long long) * g->nparts_cap));
   HIP_TRY(hipMalloc(&g->bbox_part, sizeof(double) * 7 * 1024));
   g->bbox_host.assign(7 * 1024, 0.);
   return MFG_OK;
@@ -357,6 +360,7 @@ GridBuffers grid_buffers(mfg_grid *g, mfg_particles *p) {
   gb.order = p->order;
   gb.count = g->count;
   gb.hist = g->hist;
+  gb.occ = g->occ;
   gb.scattered = p->trav;
   gb.blk = p->blk;
   gb.blk2 = g->parts;
@@ -551,16 +555,15 @@ int contact_search_buffers(mfg_particles *p, int n_tools, ContactSearch &cs) {
 // stats: the pass may count its pairs (when counting is on, mfg_pair_stats_enable)
 int run_neighbours(mfg_grid *g, mfg_particles *p, const Consts &c, int want_pse, bool stats = true) {
   const GridInfo gi = g->info();
-  const int tile = resolve_cell_tile(g_lib.opt.cell_tile, gi.num_cell, p->N_init);
   if (!stats || !g_lib.count_pairs) {
     p->stat_n = 0;
-    launch_neighbours(g_lib.stream, gi, g->count, p->nl4, p->pse2, p->st().h, p->st().flags, c,
+    launch_neighbours(g_lib.stream, p->N_init, gi, g->count, g->occ, p->nl4, p->pse2, p->st().h, p->st().flags, c,
                       p->nbr, p->nl_stride, p->count, p->st().T_t, p->cnt, want_pse, nullptr,
-                      p->poison, tile);
+                      p->poison);
     HIP_TRY(hipGetLastError());
     return MFG_OK;
   }
-  const int nb = neighbour_blocks(gi, tile);
+  const int nb = neighbour_blocks(gi, p->N_init);
   if (nb > p->stat_cap) {
     if (p->stat_part) (void)hipFree(p->stat_part);
     p->stat_part = nullptr;
@@ -570,9 +573,9 @@ int run_neighbours(mfg_grid *g, mfg_particles *p, const Consts &c, int want_pse,
     p->stat_cap = nb;
   }
   p->stat_n = nb;
-  launch_neighbours(g_lib.stream, gi, g->count, p->nl4, p->pse2, p->st().h, p->st().flags, c,
+  launch_neighbours(g_lib.stream, p->N_init, gi, g->count, g->occ, p->nl4, p->pse2, p->st().h, p->st().flags, c,
                     p->nbr, p->nl_stride, p->count, p->st().T_t, p->cnt, want_pse, p->stat_part,
-                    p->poison, tile);
+                    p->poison);
   HIP_TRY(hipGetLastError());
   return MFG_OK;
 }
@@ -1355,7 +1358,7 @@ int mfg_grid_create_unlocked(int kind, long max_cell, int num_part, mfg_grid **o
 int mfg_grid_destroy(mfg_grid *g) {
   if (!g) return MFG_OK;
   if (g_lib.ready) (void)hipStreamSynchronize(g_lib.stream);
-  void *ptrs[] = {g->count, g->hist, g->parts, g->bbox_part};
+  void *ptrs[] = {g->count, g->hist, g->occ, g->parts, g->bbox_part};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   delete g;
@@ -2200,7 +2203,7 @@ struct mfg_batch {
   };
   std::vector<Member> members;
   int precision = -1, pse = -1;
-  int cell_tile = 0;   // neighbour pass cells per wavefront; 0: the library option, else automatic
+  int cell_tile = 0;   // accepted, without effect
   bool dirty = true;   // the device descriptors and maps must be rebuilt before the next step
   int table_record = -1;
   Inst *d_inst = nullptr;
@@ -2344,15 +2347,11 @@ int batch_build(mfg_batch *b, int record) {
   std::vector<unsigned> maps(N_MAPS * map_len, 0u);
   BatchGrid *grids[N_MAPS] = {&b->L.tiles, &b->L.one, &b->L.parts,
                               &b->L.pairs8, &b->L.nbrs8, &b->L.tools, &b->L.search};
-  // cell tile of the batched neighbour pass: by the cells per particle of the whole batch
-  long cells = 0, parts = 0, most = 0;
+  long parts = 0, most = 0;
   for (const mfg_batch::Member &m : b->members) {
-    cells += m.g->num_cell;
-    most = std::max(most, (long)m.g->num_cell);
     parts += m.p->N_init;
+    most = std::max(most, (long)m.g->num_cell);
   }
-  const int tile = resolve_cell_tile(b->cell_tile ? b->cell_tile : g_lib.opt.cell_tile, cells,
-                                     (unsigned)std::min<long>(parts, 0xffffffffL));
   b->L.scan_alone = most <= SCAN_ALONE;
   b->L.ordered = order_apart(parts);
   for (int i = 0; i < n; i++) {
@@ -2366,7 +2365,7 @@ int batch_build(mfg_batch *b, int record) {
         1u,
         nblk,
         round8((unsigned)pair_blocks(m.p->N_init, 256)),
-        round8((unsigned)neighbour_blocks(gi, tile)),
+        (unsigned)neighbour_blocks(gi, m.p->N_init),
         (unsigned)std::max<size_t>(1, m.tools.size()),
         m.search ? std::min(BATCH_SEARCH_BLOCKS, std::max(1u, nblk)) : 0u};
     for (int k = 0; k < N_MAPS; k++) maps[k * map_len + i + 1] = maps[k * map_len + i] + blocks[k];
@@ -2387,7 +2386,6 @@ int batch_build(mfg_batch *b, int record) {
   b->L.n = n;
   b->L.precision = b->precision;
   b->L.pse = b->pse;
-  b->L.cell_tile = tile;
   b->L.brook = 0;
   for (const mfg_batch::Member &m : b->members)
     if (m.c.heat == MFG_HEAT_BROOKSHAW) b->L.brook = 1;
@@ -2537,7 +2535,6 @@ int mfg_batch_set_cell_tile(mfg_batch *b, int cell_tile) {
   if (cell_tile != 0 && cell_tile != 1 && cell_tile != 2 && cell_tile != 4 && cell_tile != 8 &&
       cell_tile != 16)
     return fail(MFG_ERR_ARG, "cell tile %d (0, 1, 2, 4, 8 or 16)", cell_tile);
-  if (cell_tile != b->cell_tile) b->dirty = true;
   b->cell_tile = cell_tile;
   return MFG_OK;
 }

@@ -32,34 +32,35 @@ constexpr int BS = 256;  // threads per block of the particle passes
 constexpr int SCAN_ITEMS = SCAN_TILE / BS;
 constexpr int SCAN_NT = 1024;  // threads of a tile without tile sums
 
-__device__ __forceinline__ int wave_incl_scan(int v) {
+template <class T>
+__device__ __forceinline__ T wave_incl_scan(T v) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    int t = __shfl_up(v, o, 64);
+    const T t = __shfl_up(v, o, 64);
     if (lane >= o) v += t;
   }
   return v;
 }
 
-// exclusive scan across a block of NT threads; lds must hold NT/64 + 1 ints
-template <int NT>
-__device__ __forceinline__ int block_excl_scan(int v, int *lds, int &total) {
+// exclusive scan across a block of NT threads; lds must hold NT/64 + 1 values
+template <int NT, class T>
+__device__ __forceinline__ T block_excl_scan(T v, T *lds, T &total) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  int incl = wave_incl_scan(v);
+  const T incl = wave_incl_scan(v);
   if (lane == 63) lds[wid] = incl;
   __syncthreads();
   if (threadIdx.x == 0) {
-    int acc = 0;
+    T acc = 0;
     for (int w = 0; w < NT / 64; w++) {
-      int t = lds[w];
+      const T t = lds[w];
       lds[w] = acc;
       acc += t;
     }
     lds[NT / 64] = acc;
   }
   __syncthreads();
-  int r = incl - v + lds[wid];
+  const T r = incl - v + lds[wid];
   total = lds[NT / 64];
   __syncthreads();
   return r;
@@ -152,31 +153,41 @@ __device__ __forceinline__ void load_items(const int *a, long k, long n, int (&v
   }
 }
 
+// Particles in the low and occupied cells in the high 32 bits: one scan gives both the offsets and the
+// occupied cells' places in their list
+typedef unsigned long long CellSum;
+__device__ __forceinline__ CellSum cell_sum(int count) {
+  return (CellSum)count | ((CellSum)(count > 0) << 32);
+}
+
 // tile reduction of the cell counts
-__device__ __forceinline__ void scan_reduce(unsigned b, const int *hist, long n, int *part) {
-  __shared__ int lds[BS / 64 + 1];
-  int v[SCAN_ITEMS], s = 0;
+__device__ __forceinline__ void scan_reduce(unsigned b, const int *hist, long n, CellSum *part) {
+  __shared__ CellSum lds[BS / 64 + 1];
+  int v[SCAN_ITEMS];
+  CellSum s = 0;
   load_items<SCAN_ITEMS>(hist, (long)b * SCAN_TILE + (long)threadIdx.x * SCAN_ITEMS, n, v);
 #pragma unroll
-  for (int q = 0; q < SCAN_ITEMS; q++) s += v[q];
-  int total;
+  for (int q = 0; q < SCAN_ITEMS; q++) s += cell_sum(v[q]);
+  CellSum total;
   block_excl_scan<BS>(s, lds, total);
   if (threadIdx.x == 0) part[b] = total;
 }
-__global__ void __launch_bounds__(BS) k_scan_reduce(const int *hist, long n, int *part) {
+__global__ void __launch_bounds__(BS) k_scan_reduce(const int *hist, long n, CellSum *part) {
   scan_reduce(blockIdx.x, hist, n, part);
 }
 
-// The offsets of tile b's cells (NT threads, ITEMS cells each), and with the last tile the totals.  A
-// tile's base is the sum of all before it: of the tile sums, or without them (part null: SCAN_ALONE)
-// of the counts themselves, eight loads of a thread in flight (26,000 cells: 6.7 us, 62,000: 7.4; the
-// two launches 4.6 and 4.8 and the gap between).
+// The offsets of tile b's cells (NT threads, ITEMS cells each), its occupied cells in the list of all
+// (ascending; occ[n]: how many), and with the last tile the totals.  A tile's base is the sum of all
+// before it: of the tile sums, or without them (part null: SCAN_ALONE) of the counts themselves, eight
+// loads of a thread in flight (26,000 cells: 6.7 us, 62,000: 7.4; the two launches 4.6 and 4.8 and the
+// gap between).
 template <int NT, int ITEMS>
-__device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, const int *part, int *off,
-                                           unsigned n_init, Counters *cnt) {
-  __shared__ int lds[NT / 64 + 1];
+__device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, const CellSum *part, int *off,
+                                           int *occ, unsigned n_init, Counters *cnt) {
+  __shared__ CellSum lds[NT / 64 + 1];
   const long base = ((long)b * NT + threadIdx.x) * ITEMS;
-  int v[ITEMS], s = 0, before = 0, total, prefix;
+  int v[ITEMS];
+  CellSum s = 0, before = 0, total, prefix;
   load_items<ITEMS>(hist, base, n, v);
   if (part) {
     for (unsigned k = threadIdx.x; k < b; k += NT) before += part[k];
@@ -186,25 +197,28 @@ __device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, 
 #pragma unroll 8
     for (unsigned k = 0; k < b * (ITEMS / 4); k++) {
       const int4 x = h[(size_t)k * NT];
-      before += x.x + x.y + x.z + x.w;
+      before += cell_sum(x.x) + cell_sum(x.y) + cell_sum(x.z) + cell_sum(x.w);
     }
   }
 #pragma unroll
-  for (int q = 0; q < ITEMS; q++) s += v[q];
+  for (int q = 0; q < ITEMS; q++) s += cell_sum(v[q]);
   block_excl_scan<NT>(before, lds, prefix);
-  int o = prefix + block_excl_scan<NT>(s, lds, total);
+  const CellSum first = prefix + block_excl_scan<NT>(s, lds, total);
   if (threadIdx.x == 0 && (long)(b + 1) * NT * ITEMS >= n) {  // the last tile
-    off[n] = prefix + total;
-    cnt->N = (unsigned)(prefix + total);
-    cnt->n_blank_key = n_init - (unsigned)(prefix + total);
+    const unsigned N = (unsigned)(prefix + total);
+    off[n] = (int)N;
+    occ[n] = (int)((prefix + total) >> 32);
+    cnt->N = N;
+    cnt->n_blank_key = n_init - N;
     cnt->candidates = 0ull;
     cnt->pairs = 0ull;
   }
-  int w[ITEMS];
+  int w[ITEMS], o = (int)(unsigned)first, place = (int)(first >> 32);
 #pragma unroll
   for (int q = 0; q < ITEMS; q++) {
     w[q] = o;
     o += v[q];
+    if (v[q] > 0) occ[place++] = (int)(base + q);
   }
   if (base + ITEMS <= n) {
 #pragma unroll
@@ -216,9 +230,9 @@ __device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, 
   }
 }
 template <int NT, int ITEMS>
-__global__ void __launch_bounds__(NT) k_scan_cells(const int *hist, long n, const int *part, int *off,
-                                                   unsigned n_init, Counters *cnt) {
-  scan_cells<NT, ITEMS>(blockIdx.x, hist, n, part, off, n_init, cnt);
+__global__ void __launch_bounds__(NT) k_scan_cells(const int *hist, long n, const CellSum *part, int *off,
+                                                   int *occ, unsigned n_init, Counters *cnt) {
+  scan_cells<NT, ITEMS>(blockIdx.x, hist, n, part, off, occ, n_init, cnt);
 }
 
 // particles to their cells (order: an INT_MAX key's particle at its final place, the others in any
@@ -444,12 +458,12 @@ void launch_scan_cells(hipStream_t s, const GridInfo &g, GridBuffers &gb, unsign
   const dim3 tiles((unsigned)scan_tiles(g.num_cell, alone));
   if (alone) {
     hipLaunchKernelGGL((k_scan_cells<SCAN_NT, SCAN_TILE_ALONE / SCAN_NT>), tiles, dim3(SCAN_NT), 0, s, gb.hist, g.num_cell,
-                       (const int *)nullptr, gb.count, n_init, cnt);
+                       (const CellSum *)nullptr, gb.count, gb.occ, n_init, cnt);
     return;
   }
   hipLaunchKernelGGL(k_scan_reduce, tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2);
   hipLaunchKernelGGL((k_scan_cells<BS, SCAN_ITEMS>), tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2,
-                     gb.count, n_init, cnt);
+                     gb.count, gb.occ, n_init, cnt);
 }
 
 void launch_scatter(hipStream_t s, unsigned n_init, const GridInfo &g, GridBuffers &gb,
@@ -510,8 +524,8 @@ template <int NT, int ITEMS>
 __global__ void __launch_bounds__(NT) kb_scan_cells(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  scan_cells<NT, ITEMS>(b, d.gb.hist, d.g.num_cell, NT == BS ? d.gb.blk2 : nullptr, d.gb.count, d.n_init,
-                        d.cnt);
+  scan_cells<NT, ITEMS>(b, d.gb.hist, d.g.num_cell, NT == BS ? d.gb.blk2 : nullptr, d.gb.count, d.gb.occ,
+                        d.n_init, d.cnt);
 }
 
 __global__ void __launch_bounds__(BS) kb_scatter(const Inst *in, BatchMap m) {

@@ -26,6 +26,7 @@
 // 1M it runs at 18 TB/s of record reads from the L2s; vector units busy half of the time, the L1 and
 // LDS paths about two thirds, at two waves per SIMD (45 FP64 sums a lane; compiled for three it
 // spills and is slower).
+#include <algorithm>
 #include <type_traits>
 
 #include "mfg_device.hpp"
@@ -135,13 +136,10 @@ __device__ __forceinline__ double exp_finish(const ExpPart &e) {
 // 0.74 ms, 65k FP64 131 -> 99 us: a group of four against 64 candidates took 211 vector instructions
 // and 28 LDS reads with its particles' data in LDS, a branch per particle and the candidates listed
 // in LDS beforehand; now 181 and 2 (+ 4 table reads), the listing included.
-// Cells (wavefronts) per workgroup.  One: cells differ in particles and candidates, and the
-// waves of a larger workgroup wait for its slowest cell at the end (the statistics sum) while
-// holding their slots; measured 12-14 % slower with four.
-#ifndef NB_WAVES_PER_BLOCK
-#define NB_WAVES_PER_BLOCK 1
-#endif
-constexpr int NB_WAVES = NB_WAVES_PER_BLOCK;
+// Cells (wavefronts) per workgroup: neighbouring cells on one compute unit share most of their
+// candidates in its L1.  1M cut, FP64 / FP32: one 0.91 / 0.75 ms, two 0.83 / 0.68, three 0.83 / 0.66,
+// four 0.84 / 0.66, eight 0.90 / 0.71; 24 batched wedges 0.54, 0.52, 0.53, 0.54, 0.61.
+constexpr int NB_WAVES = 3;
 constexpr int NB_BLOCK = 64 * NB_WAVES;
 #ifndef NB_GROUP_SIZE
 #define NB_GROUP_SIZE 4
@@ -393,20 +391,22 @@ __device__ __forceinline__ int cell_ranges(const GridInfo &g, const int *__restr
 }
 
 // minimum waves per SIMD the kernel is compiled for (register budget): FP64 PSE 6, the others 7;
-// 1M single-grain cut FP64 0.94 ms (5 waves 0.98, 4 waves 0.98), FP32 0.74 (6 waves 0.77, 5 waves
-// 0.76)
+// 1M single-grain cut FP64 0.83 ms (5 waves 0.88), FP32 0.66 (8 waves 0.78)
 #ifndef NB_WAVES_FP64_PSE
 #define NB_WAVES_FP64_PSE 6
 #endif
 #ifndef NB_WAVES_OTHER
 #define NB_WAVES_OTHER 7
 #endif
-// body of workgroup b of nb (the single-instance kernel and the batched one below); each wavefront
-// takes CPW consecutive cells in turn (the cell tile), so that an empty cell costs two loads
-// rather than a workgroup where the grid has wide margins around the block
-template <int PSE_MODE, int CPW>
+// Body of workgroup b of nb (the single-instance kernel and the batched one below): each wavefront takes
+// one cell of the occupied ones (occ, ascending; the scan of the sort lists them), each XCD one
+// contiguous eighth of the list.  The launch is sized for the most cells the particles can occupy, not
+// for the grid: its margins around the block are three quarters of the cells of a wedge cut.  Against
+// a wavefront for every cell: 8,000 particles 27 -> 13 us, 19,000 35 -> 18, 64,000 with PSE 100 -> 65;
+// 24 batched wedges, where a wavefront took 16 cells in turn, 0.77 -> 0.53 ms.
+template <int PSE_MODE>
 __device__ __forceinline__ void cell_neighbours(
-    unsigned b, unsigned nb, const GridInfo &g, const int *__restrict__ off,
+    unsigned b, const GridInfo &g, const int *__restrict__ off, const int *__restrict__ occ,
     const double4 *__restrict__ nl4, const double2 *__restrict__ pse2,
     const double *__restrict__ h, const uint32_t *__restrict__ flags, const Consts &c,
     int *__restrict__ nbr, int cap, int *__restrict__ count, double *__restrict__ T_t,
@@ -420,7 +420,10 @@ __device__ __forceinline__ void cell_neighbours(
     if (threadIdx.x < 64) s_exp[threadIdx.x] = EXP2_J64[threadIdx.x];
     __syncthreads();
   }
-  const long c0 = ((long)xcd_map(b, nb) * NB_WAVES + w) * CPW;
+  // workgroups x, x + 8, ... (XCD x) take the list's groups of NB_WAVES cells from x per on
+  const unsigned n_occ = min((unsigned)occ[g.num_cell], (unsigned)g.num_cell);
+  const unsigned groups = (n_occ + NB_WAVES - 1) / NB_WAVES;
+  const unsigned per = (groups + 7) / 8, slot = b >> 3, at = ((b & 7) * per + slot) * NB_WAVES + w;
   unsigned long long n_cand = 0, n_pair = 0;
   // the particles [s, e) of one cell against its stencil's candidates
   auto do_cell = [&](const long c_, const int s, const int e) {
@@ -458,31 +461,18 @@ __device__ __forceinline__ void cell_neighbours(
     cell_lists<PSE_MODE>(s, e, T, lane, fetch, nl4, pse2, h, flags, c, nbr, cap, count,
                          T_t, cnt, poison, s_exp, n_cand, n_pair);
   };
-  if constexpr (CPW == 1) {
-    const int s = c0 < g.num_cell ? off[c0] : 0;
-    const int e = c0 < g.num_cell ? off[c0 + 1] : 0;
-    if (s < e) do_cell(c0, s, e);
-  } else {
-    // the tile's cell offsets in one load, lane q holding off[c0 + q] (off[num_cell] = N), and
-    // the occupied cells as a ballot: empty cells cost nothing further
-    const int o = (lane <= CPW && c0 + lane <= g.num_cell) ? off[c0 + lane] : 0;
-    const int o_next = __shfl_down(o, 1, 64);
-    unsigned long long occ = __ballot(lane < CPW && c0 + lane < g.num_cell && o_next > o);
-    while (occ) {
-      const int q = __builtin_ctzll(occ);  // ascending cells, as the single-cell form visits them
-      occ &= occ - 1;
-      wave_lds_sync();  // the previous cell's lanes are done with this wave's LDS
-      do_cell(c0 + q, __builtin_amdgcn_readlane(o, q), __builtin_amdgcn_readlane(o, q + 1));
-    }
+  if (slot < per && at < n_occ) {
+    const int cell = occ[at];
+    do_cell(cell, off[cell], off[cell + 1]);
   }
-  // candidate / pair totals of this workgroup (work accounting of the roofline figures); a null
-  // stat_part skips them
+  if (!stat_part) return;
+  // candidate / pair totals of this workgroup (work accounting of the roofline figures)
   if (lane == 0) {
     s_stat[w][0] = n_cand;
     s_stat[w][1] = n_pair;
   }
   __syncthreads();
-  if (threadIdx.x == 0 && stat_part) {
+  if (threadIdx.x == 0) {
     unsigned long long a = 0, bb = 0;
 #pragma unroll
     for (int k = 0; k < NB_WAVES; k++) {
@@ -493,36 +483,17 @@ __device__ __forceinline__ void cell_neighbours(
     stat_part[2 * b + 1] = bb;
   }
 }
-// waves per SIMD: one fewer for a PSE sum over a tile of several cells (the tile's loop state
-// would otherwise spill)
-template <int PSE_MODE, int CPW>
+template <int PSE_MODE>
 __global__ void __launch_bounds__(NB_BLOCK)
-    __attribute__((amdgpu_waves_per_eu((PSE_MODE == 1 ? NB_WAVES_FP64_PSE : NB_WAVES_OTHER) -
-                                       (PSE_MODE != 0 && CPW > 1 ? 2 : 0))))
-    k_cell_neighbours(GridInfo g, const int *__restrict__ off, const double4 *__restrict__ nl4,
+    __attribute__((amdgpu_waves_per_eu(PSE_MODE == 1 ? NB_WAVES_FP64_PSE : NB_WAVES_OTHER)))
+    k_cell_neighbours(GridInfo g, const int *__restrict__ off, const int *__restrict__ occ,
+                      const double4 *__restrict__ nl4,
                       const double2 *__restrict__ pse2, const double *__restrict__ h,
                       const uint32_t *__restrict__ flags, Consts c, int *__restrict__ nbr, int cap,
                       int *__restrict__ count, double *__restrict__ T_t, Counters *cnt,
                       unsigned long long *__restrict__ stat_part, int *__restrict__ poison) {
-  cell_neighbours<PSE_MODE, CPW>(blockIdx.x, gridDim.x, g, off, nl4, pse2, h, flags, c, nbr, cap,
-                                 count, T_t, cnt, stat_part, poison);
-}
-
-// launches kernel template K<PSE mode, cell tile> for run-time values of both
-template <template <int, int> class Launch, class... A>
-void dispatch_neighbours(int mode, int cpw, A &&...a) {
-#define MFG_NB_CPW(P)                                          \
-  switch (cpw) {                                               \
-    case 1: Launch<P, 1>::run(a...); break;                    \
-    case 2: Launch<P, 2>::run(a...); break;                    \
-    case 4: Launch<P, 4>::run(a...); break;                    \
-    case 8: Launch<P, 8>::run(a...); break;                    \
-    default: Launch<P, 16>::run(a...); break;                  \
-  }
-  if (mode == 0) { MFG_NB_CPW(0) }
-  else if (mode == 1) { MFG_NB_CPW(1) }
-  else { MFG_NB_CPW(2) }
-#undef MFG_NB_CPW
+  cell_neighbours<PSE_MODE>(blockIdx.x, g, off, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t, cnt,
+                            stat_part, poison);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1761,40 +1732,25 @@ __global__ void __launch_bounds__(BS, PAIR32_WAVES)
 // ---------------------------------------------------------------------------------------------
 static inline unsigned nb(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-int neighbour_blocks(const GridInfo &g, int cell_tile) {
-  const long per = (long)NB_WAVES * cell_tile;
-  return (int)((g.num_cell + per - 1) / per);
+// a multiple of 8 workgroups: eight equal shares of the list
+int neighbour_blocks(const GridInfo &g, unsigned n_init) {
+  const long cells = std::min<long>(g.num_cell, n_init);
+  return (int)((cells + 8 * NB_WAVES - 1) / (8 * NB_WAVES)) * 8;
 }
 
-// Automatic: one cell per wavefront unless the grid is both sparse (two or more cells per
-// particle) and large, where empty cells would dominate the launch: 4 cells from 256k cells, 16
-// from 1M (measured: a single 8k-particle wedge cut or a 30k grain runs fastest with one cell
-// per wavefront, a batch of 256 wedge cuts (44M cells, 3.25 per particle) with 16)
-int resolve_cell_tile(int option, long num_cell, unsigned n_init) {
-  if (option == 1 || option == 2 || option == 4 || option == 8 || option == 16) return option;
-  if (num_cell < 2 * (long)n_init || num_cell < (1L << 18)) return 1;
-  return num_cell >= (1L << 20) ? 16 : 4;
-}
-
-template <int P, int CPW>
-struct SingleNeighbours {
-  static void run(hipStream_t s, const GridInfo &g, const int *offsets, const double4 *nl4,
-                  const double2 *pse2, const double *h, const uint32_t *flags, const Consts &c,
-                  int *nbr, int cap, int *count, double *T_t, Counters *cnt,
-                  unsigned long long *stat_part, int *poison) {
-    hipLaunchKernelGGL((k_cell_neighbours<P, CPW>), dim3(neighbour_blocks(g, CPW)),
-                       dim3(NB_BLOCK), 0, s, g, offsets, nl4, pse2, h, flags, c, nbr, cap, count,
-                       T_t, cnt, stat_part, poison);
-  }
-};
-
-void launch_neighbours(hipStream_t s, const GridInfo &g, const int *offsets, const double4 *nl4,
+void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const int *offsets,
+                       const int *occ, const double4 *nl4,
                        const double2 *pse2, const double *h, const uint32_t *flags,
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
-                       int want_pse, unsigned long long *stat_part, int *poison, int cell_tile) {
-  const int mode = !want_pse ? 0 : c.precision == MFG_FP64 ? 1 : 2;
-  dispatch_neighbours<SingleNeighbours>(mode, cell_tile, s, g, offsets, nl4, pse2, h, flags, c,
-                                        nbr, cap, count, T_t, cnt, stat_part, poison);
+                       int want_pse, unsigned long long *stat_part, int *poison) {
+  auto launch = [&](auto mode_c) {
+    hipLaunchKernelGGL((k_cell_neighbours<decltype(mode_c)::value>), dim3(neighbour_blocks(g, n_init)),
+                       dim3(NB_BLOCK), 0, s, g, offsets, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t,
+                       cnt, stat_part, poison);
+  };
+  if (!want_pse) launch(std::integral_constant<int, 0>{});
+  else if (c.precision == MFG_FP64) launch(std::integral_constant<int, 1>{});
+  else launch(std::integral_constant<int, 2>{});
 }
 
 int pair_blocks(unsigned n_init, int block) { return (int)nb((long)n_init * PAIR_LANES, block); }
@@ -1837,28 +1793,18 @@ void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *re
 // ---------------------------------------------------------------------------------------------
 // fewer waves per SIMD than the single-instance kernel (FP64 PSE 5, FP32 PSE 6, no PSE 7): the
 // instance lookup and descriptor take the registers that would otherwise spill
-template <int PSE_MODE, int CPW>
+template <int PSE_MODE>
 __global__ void __launch_bounds__(NB_BLOCK)
-    __attribute__((amdgpu_waves_per_eu((PSE_MODE == 1 ? NB_WAVES_FP64_PSE - 1
-                                        : PSE_MODE == 2 ? NB_WAVES_OTHER - 2
-                                                        : NB_WAVES_OTHER - 1) -
-                                       (PSE_MODE != 0 && CPW > 1 ? 2 : 0))))
+    __attribute__((amdgpu_waves_per_eu(PSE_MODE == 1   ? NB_WAVES_FP64_PSE - 1
+                                       : PSE_MODE == 2 ? NB_WAVES_OTHER - 2
+                                                       : NB_WAVES_OTHER - 1)))
     kb_cell_neighbours(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
   const State &st = d.buf[d.cur ^ 1];
-  cell_neighbours<PSE_MODE, CPW>(b, nb, d.g, d.gb.count, d.nl4, d.pse2, st.h, st.flags, d.c,
-                                 d.nbr, d.nl_stride, d.count, st.T_t, d.cnt, nullptr, d.poison);
+  cell_neighbours<PSE_MODE>(b, d.g, d.gb.count, d.gb.occ, d.nl4, d.pse2, st.h, st.flags, d.c, d.nbr,
+                            d.nl_stride, d.count, st.T_t, d.cnt, nullptr, d.poison);
 }
-
-
-template <int P, int CPW>
-struct BatchNeighbours {
-  static void run(hipStream_t s, const BatchLaunch &L) {
-    hipLaunchKernelGGL((kb_cell_neighbours<P, CPW>), dim3(L.nbrs8.blocks), dim3(NB_BLOCK), 0, s,
-                       L.inst, L.nbrs8.m);
-  }
-};
 
 template <bool BROOK>
 __global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair_sums(const Inst *in, BatchMap m) {
@@ -1888,8 +1834,13 @@ __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchM
 // run_neighbours picks it.  One Brookshaw instance selects the kernel with its sum for all: the
 // others' sums are the same in both.
 void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
-  const int mode = !L.pse ? 0 : L.precision == MFG_FP64 ? 1 : 2;
-  dispatch_neighbours<BatchNeighbours>(mode, L.cell_tile, s, L);
+  auto neighbours = [&](auto mode_c) {
+    hipLaunchKernelGGL((kb_cell_neighbours<decltype(mode_c)::value>), dim3(L.nbrs8.blocks), dim3(NB_BLOCK), 0,
+                       s, L.inst, L.nbrs8.m);
+  };
+  if (!L.pse) neighbours(std::integral_constant<int, 0>{});
+  else if (L.precision == MFG_FP64) neighbours(std::integral_constant<int, 1>{});
+  else neighbours(std::integral_constant<int, 2>{});
   const dim3 gp(L.pairs8.blocks), bp(BSP);
   auto launch = [&](auto brook_c) {
     constexpr bool BROOK = decltype(brook_c)::value;

@@ -159,7 +159,8 @@ struct GridBuffers {
   int *count;        // num_cell + 1: exclusive offsets of the cells
   int *hist;         // num_cell particle counts of a sort under way; zero between sorts
   int *blk;          // per-block blanked counts
-  int *blk2;         // scan scratch
+  unsigned long long *blk2;  // scan scratch
+  int *occ;          // occupied cells, ascending; [num_cell]: how many
   int nblk;          // blocks of the hash kernel
 };
 
@@ -184,14 +185,13 @@ void launch_bbox_reduce(hipStream_t s, const State &st, const Counters *cnt, uns
 // neighbour lists (+ PSE heat) for every cell; stat_part gets 2 totals (candidates, pairs) per
 // workgroup, neighbour_blocks(g) workgroups; poison[p] = 1 when a candidate of particle p holds a
 // non-finite record (nl4.w == 2), which the reference's sums carry into p's rates
-// cell_tile: consecutive cells per wavefront (1, 2, 4 or 8; resolve_cell_tile turns the option,
-// 0 for automatic, into one of them)
-int neighbour_blocks(const GridInfo &g, int cell_tile);
-int resolve_cell_tile(int option, long num_cell, unsigned n_init);
-void launch_neighbours(hipStream_t s, const GridInfo &g, const int *offsets, const double4 *nl4,
+// occ: the occupied cells (GridBuffers)
+int neighbour_blocks(const GridInfo &g, unsigned n_init);
+void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const int *offsets,
+                       const int *occ, const double4 *nl4,
                        const double2 *pse2, const double *h, const uint32_t *flags,
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
-                       int want_pse, unsigned long long *stat_part, int *poison, int cell_tile);
+                       int want_pse, unsigned long long *stat_part, int *poison);
 // pair pass (neighbour sums), four lanes per particle; pair_blocks: its workgroups of `block` threads
 // (64, 128 or 256).  ordered: FP64 sums in the reference's order of evaluation, to the bit (unlocked
 // grids), one lane per particle.  cs4: FP32 modes only
@@ -324,7 +324,6 @@ struct BatchLaunch {
   int n;
   int precision, pse;
   int brook;         // an instance conducts heat by Brookshaw's form
-  int cell_tile;     // cells per wavefront of the neighbour pass
   int ordered;       // order_apart
   int scan_alone;    // no instance has more than SCAN_ALONE cells
   BatchGrid tiles;   // scan tiles of the cell counts

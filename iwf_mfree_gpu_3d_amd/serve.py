@@ -206,7 +206,7 @@ def serve(requests: list, hbm_budget: float = 250e9, steps_per_round: int = 5, o
     result (the error counters are sticky, so the check at the end covers every step).
     `max_neighbours`: neighbour-list capacity of the instances (0: the library default).
     `mode`: "batched" or "streams" (see the module notes); `use_graph`: batched rounds replay a
-    captured step; `cell_tile`: cells per wavefront of the batches' neighbour pass (0 automatic).
+    captured step; `cell_tile`: accepted, without effect.
     `streams`: size of the stream pool the instances are spread over.  `tuning`: an
     autotune.Table; "streams": each instance runs with its bucket's (pair pass, strip, cell tile),
     "batched": each precision's batch with its cell tile (None: the library defaults).  Returns

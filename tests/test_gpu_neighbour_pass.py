@@ -15,9 +15,10 @@ from iwf_mfree_gpu_3d_amd import _lib, api
 pytestmark = pytest.mark.gpu
 
 H, MASS, RHO0, ALPHA = 7.5e-4, 5e-10, 4.43, 3e-8
-# particles, edge of the box they fill in cells: from one particle to 1,500 candidates of one cell
+# particles, edge of the box they fill in cells: from one particle to 1,500 candidates of one cell, and
+# 300 particles among 216,000 cells
 CLOUDS = [(1, 1.0), (2, 1.0), (3, 0.9), (5, 0.9), (9, 0.9), (63, 2.5), (64, 2.5), (65, 2.5), (127, 3.0), (128, 3.0),
-          (129, 4.5), (700, 4.5), (833, 4.9), (1500, 4.9), (400, 11.0)]
+          (129, 4.5), (700, 4.5), (833, 4.9), (1500, 4.9), (400, 11.0), (300, 60.0)]
 
 
 def setup(n, box, precision, cap, heat):
