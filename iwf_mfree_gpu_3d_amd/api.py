@@ -212,7 +212,7 @@ class particle_gpu:
         w = _L().mfg_field_width(field)
         if w <= 0:
             raise MfgError(_lib.MFG_ERR_ARG, f"unknown field {field}")
-        out = np.zeros(self.N_init * w)
+        out = np.empty(self.N_init * w)  # the call below writes every element or raises
         check(_L().mfg_particle_gpu_download(self._h, field, _dptr(out)))
         return out.reshape(self.N_init, w) if w > 1 else out
 

@@ -603,10 +603,11 @@ int check_counters(mfg_particles *p) {
 
 // A field of every particle to host memory, interleaved by the device.  Fields of up to STAGE_BYTES:
 // the kernel writes them and the counters into the set's pinned buffer, one launch and one wait (a
-// copy command takes 60 us however small: 8,000 positions 394 -> 24 us).  Larger ones go
+// copy command takes 60 us however small: 8,000 positions 394 -> 24 us; 1.4 MB of stresses 111 us this
+// way, 204 the other; 4.8 MB 327 and 375, too little for pinned memory of that size per set).  Larger ones go
 // through the pair-sum array (free between two calls: the pair pass writes it and the update of the
 // same call reads it) straight into the caller's memory.
-constexpr size_t STAGE_BYTES = (size_t)1 << 20;
+constexpr size_t STAGE_BYTES = (size_t)4 << 20;
 int download_field(mfg_particles *p, const PackField &f, double *host) {
   std::lock_guard<std::mutex> lock(p->stage_use);
   hipStream_t s = g_lib.stream;

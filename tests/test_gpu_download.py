@@ -1,5 +1,5 @@
-"""Fields of every particle to host memory at both sides of the staged size (1 MB: 14,563 symmetric
-tensors, 43,690 vectors, 131,072 scalars): what was uploaded comes back, element for element.  Copies
+"""Fields of every particle to host memory at both sides of the staged size (4 MB: 58,254 symmetric
+tensors, 174,762 vectors, 524,288 scalars): what was uploaded comes back, element for element.  Copies
 only, so exact; flags come back as the value class they were set to."""
 import numpy as np
 import pytest
@@ -12,7 +12,7 @@ F64 = {1: ("F_H", "F_RHO", "F_EPS_PL", "F_EPS_PL_DOT", "F_T", "F_RHO_T", "F_T_T"
        3: ("F_POS", "F_VEL", "F_VEL_BC", "F_FC", "F_FT", "F_POS_T", "F_VEL_T"), 9: ("F_S", "F_S_T")}
 
 
-@pytest.mark.parametrize("n", [1, 3, 255, 257, 14563, 14564, 43690, 43691, 131072, 131073])
+@pytest.mark.parametrize("n", [1, 3, 255, 257, 14563, 58254, 58255, 174762, 174763, 524288, 524289])
 def test_fields_come_back(hip_device, n):
     rng = np.random.default_rng(n)
     api.reset_globals()
