@@ -2355,6 +2355,10 @@ int batch_build(mfg_batch *b, int record) {
   }
   b->L.scan_alone = most <= SCAN_ALONE;
   b->L.ordered = order_apart(parts);
+  // FP64 sums depend on the lanes in their last bits: each instance has those it has alone
+  b->L.pair_lanes = b->precision == MFG_FP64 ? 0 : pair_lanes(b->precision, parts);
+  if (b->precision == MFG_FP64)
+    for (const mfg_batch::Member &m : b->members) b->L.pair_lanes |= pair_lanes(MFG_FP64, m.p->N_init);
   for (int i = 0; i < n; i++) {
     const mfg_batch::Member &m = b->members[i];
     host[i] = batch_inst(m, record);
@@ -2365,7 +2369,8 @@ int batch_build(mfg_batch *b, int record) {
         (unsigned)scan_tiles(gi.num_cell, b->L.scan_alone),
         1u,
         nblk,
-        round8((unsigned)pair_blocks(m.p->N_init, 256)),
+        round8((unsigned)pair_blocks(
+            m.p->N_init, b->precision == MFG_FP64 ? pair_lanes(MFG_FP64, m.p->N_init) : b->L.pair_lanes, 256)),
         (unsigned)neighbour_blocks(gi, m.p->N_init),
         (unsigned)std::max<size_t>(1, m.tools.size()),
         m.search ? std::min(BATCH_SEARCH_BLOCKS, std::max(1u, nblk)) : 0u};

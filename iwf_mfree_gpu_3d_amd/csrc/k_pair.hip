@@ -690,16 +690,15 @@ struct PairScale {
   double k1, fac, mass, eps;
 };
 
-// adds up the partial sums of the four lanes of a particle; every lane gets the total
-__device__ __forceinline__ double quad_sum(double v) {
-  auto dpp = [](double a, auto ctrl) {
-    const long long b = __builtin_bit_cast(long long, a);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, decltype(ctrl)::value, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), decltype(ctrl)::value, 0xf, 0xf, true);
-    return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-  };
-  v += dpp(v, std::integral_constant<int, 0xb1>{});  // quad_perm 1,0,3,2
-  v += dpp(v, std::integral_constant<int, 0x4e>{});  // quad_perm 2,3,0,1
+// adds up the partial sums of a particle's lanes (4 or 16, aligned); every lane gets the total
+template <int LANES>
+__device__ __forceinline__ double lanes_sum(double v) {
+  if (LANES == 16) {
+    v += dpp64<0x140>(v);  // row_mirror: the other eight of a row
+    v += dpp64<0x141>(v);  // row_half_mirror: the other quad of eight lanes
+  }
+  v += dpp64<0xb1>(v);  // quad_perm 1,0,3,2
+  v += dpp64<0x4e>(v);  // quad_perm 2,3,0,1
   return v;
 }
 
@@ -1096,11 +1095,10 @@ __device__ __forceinline__ void wave_sync_lds() {
 }
 
 // Four lanes (a quad) per particle: lane s of the quad takes neighbours s, s + 4, ... of the list
-// and the quad adds up its four partial sums at the end (quad_sum).  A wavefront holds 16 particles,
+// and the quad adds up its four partial sums at the end (lanes_sum).  A wavefront holds 16 particles,
 // so 8,000 particles fill 500 wavefronts instead of 125, the longest list of a wavefront is that of
 // 16 particles, not 64, and the four neighbours a quad holds at a time are mostly consecutive
-// records.
-constexpr int PAIR_LANES = 4;
+// records.  Small sets take 16 lanes (lanes64).
 
 // The gather.  Each lane of a quad needs one record per step; the quad loads its four records
 // together, straight into LDS (buffer_load_dwordx4 ... lds writes lane l's 16 bytes at 16 l of the
@@ -1156,16 +1154,16 @@ struct QuadGather {
   }
 };
 
-template <bool BROOK, int BS>
+// LANES: lanes of a particle, 4 or 16 (lanes64); area: QuadGather::AREA bytes a wavefront
+template <bool BROOK, int LANES, int BS>
 __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_init, const State &st,
                                           const Rec64 *__restrict__ rec,
                                           const int *__restrict__ nbr, int stride,
                                           const int *__restrict__ count, const Consts &c,
                                           const Counters *cnt, double *__restrict__ sums,
-                                          size_t sstride, const int *__restrict__ trav) {
+                                          size_t sstride, const int *__restrict__ trav, char *area) {
   typedef QuadGather<Rec64> Gather;
-  __shared__ __align__(16) char s_area[BS / 64][Gather::AREA];
-  const unsigned t = xcd_map(b, nb) * (BS / PAIR_LANES) + threadIdx.x / PAIR_LANES;
+  const unsigned t = xcd_map(b, nb) * (BS / LANES) + threadIdx.x / LANES;
   const unsigned N = cnt->N;
   const bool in_range = t < N && t < n_init;
   const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
@@ -1174,20 +1172,20 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
   const unsigned ic = act ? i : 0u;
   // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int s = lane & (PAIR_LANES - 1);
+  const int s = lane & (LANES - 1);
   const int nl = act ? count[i] : 0;
-  int steps = (nl + PAIR_LANES - 1) / PAIR_LANES;
+  int steps = (nl + LANES - 1) / LANES;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
   steps = __builtin_amdgcn_readfirstlane(steps);
   const int *row = nbr + (size_t)ic * stride + s;
-  // neighbour s + 4 k of the list; past its end the particle itself, which is loaded and not used
-  auto index = [&](int k) -> int { return s + 4 * k < nl ? row[4 * k] : (int)ic; };
+  // neighbour s + LANES k of the list; past its end the particle itself, which is loaded and not used
+  auto index = [&](int k) -> int { return s + LANES * k < nl ? row[LANES * k] : (int)ic; };
   const Pair64<BROOK> P(c, rec[ic]);
   const bool tool_i = (fl & FL_TOOL) != 0, tool_nz = (fl & FL_TOOL_NZ) != 0;
   const bool brook = BROOK && c.heat == MFG_HEAT_BROOKSHAW && (tool_nz ? c.alpha_tool : c.alpha_wp) != 0.;
   PairAcc acc = {};
-  const Gather g(rec, n_init, s_area[w], lane);
+  const Gather g(rec, n_init, area + w * Gather::AREA, lane);
   if (steps > 0) {
     g.issue(index(0));
     int jn = steps > 1 ? index(1) : 0;
@@ -1200,25 +1198,25 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
         g.issue(jn);
         if (k + 2 < steps) jn = index(k + 2);
       }
-      if (s + 4 * k < nl) P.term(acc, rj, !tool_i);
+      if (s + LANES * k < nl) P.term(acc, rj, !tool_i);
     }
   }
   if (!act) return;
 #pragma unroll
   for (int k = 0; k < 3; k++) {
-    acc.W[k] = quad_sum(acc.W[k]);
-    acc.F[k] = quad_sum(acc.F[k]);
-    acc.V[k] = quad_sum(acc.V[k]);
-    acc.X[k] = quad_sum(acc.X[k]);
+    acc.W[k] = lanes_sum<LANES>(acc.W[k]);
+    acc.F[k] = lanes_sum<LANES>(acc.F[k]);
+    acc.V[k] = lanes_sum<LANES>(acc.V[k]);
+    acc.X[k] = lanes_sum<LANES>(acc.X[k]);
 #pragma unroll
-    for (int e = 0; e < 3; e++) acc.D[e][k] = quad_sum(acc.D[e][k]);
+    for (int e = 0; e < 3; e++) acc.D[e][k] = lanes_sum<LANES>(acc.D[e][k]);
 #pragma unroll
-    for (int e = 0; e < 6; e++) acc.M[e][k] = quad_sum(acc.M[e][k]);
+    for (int e = 0; e < 6; e++) acc.M[e][k] = lanes_sum<LANES>(acc.M[e][k]);
   }
 #pragma unroll
   for (int e = 0; e < 6; e++) {
-    acc.B[e] = quad_sum(acc.B[e]);
-    if (BROOK) acc.Q[e] = quad_sum(acc.Q[e]);
+    acc.B[e] = lanes_sum<LANES>(acc.B[e]);
+    if (BROOK) acc.Q[e] = lanes_sum<LANES>(acc.Q[e]);
   }
   if (s != 0) return;
   double A[6], R[6];
@@ -1233,14 +1231,15 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
 }
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
 // depend on it)
-template <bool BROOK, int BS>
+template <bool BROOK, int LANES, int BS>
 __global__ void __launch_bounds__(BS, PAIR_WAVES)
     k_pair_sums(unsigned n_init, State st, const Rec64 *__restrict__ rec,
                 const int *__restrict__ nbr, int stride, const int *__restrict__ count, Consts c,
                 const Counters *cnt, double *__restrict__ sums, size_t sstride,
                 const int *__restrict__ trav) {
-  pair_sums<BROOK, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
-                       sstride, trav);
+  __shared__ __align__(16) char s_area[(BS / 64) * QuadGather<Rec64>::AREA];
+  pair_sums<BROOK, LANES, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
+                              sstride, trav, s_area);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1435,10 +1434,11 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 // ---------------------------------------------------------------------------------------------
 // FP32 pair pass.  Every sum runs over the list in its order (the Kahan sums depend on it), first
 // the nine of B, then the 24 with the corrected gradient; so a sum is one lane's, and a lane per
-// particle would keep 25 of them.  Here a particle has four lanes, one in each row of 16 of its
-// wavefront: in step k the lane of row n forms all terms of neighbour 4 k + n, the rows exchange
-// them (spread: four registers in four instructions), and every lane then adds the four neighbours'
-// terms of its own quarter of the sums, in list order.
+// particle would keep 25 of them.  Here a particle has L lanes (four or, in small sets, eight: pair_lanes),
+// one in each of the L groups of consecutive lanes of its wavefront: in step k the lane of group n forms
+// all terms of neighbour L k + n, the groups exchange them (spread: for four, four registers in four
+// instructions), and every lane then adds the L neighbours' terms of its own share of the sums, in list
+// order.
 //
 // Against one lane per particle, the same sums to the bit: 19,000 particles 137 -> 59 us (300 wavefronts
 // of 100 steps, now 1,200 of 26), 255k with wide sums 396 -> 324 us, 1M 1.35 -> 1.25 ms.  At 1M the
@@ -1449,54 +1449,79 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 // exchanging them waits longer (1.86 ms).
 constexpr int PAIR32_WAVES = 4;
 
-// rows of 16 lanes: on return v[n] in row r holds what v[r] held in row n
-__device__ __forceinline__ void spread(float (&v)[4]) {
-  unsigned u[4];
+// L groups of 64 / L lanes (rows of 16 for four, half rows for eight): on return v[n] in group r holds
+// what v[r] held in group n
+template <int L>
+__device__ __forceinline__ void spread(float (&v)[L]) {
+  unsigned u[L];
 #pragma unroll
-  for (int r = 0; r < 4; r++) u[r] = __builtin_bit_cast(unsigned, v[r]);
-  auto a = __builtin_amdgcn_permlane32_swap(u[0], u[2], false, false);
-  auto b = __builtin_amdgcn_permlane32_swap(u[1], u[3], false, false);
-  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
-  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-  u[0] = c[0]; u[1] = c[1]; u[2] = d[0]; u[3] = d[1];
+  for (int r = 0; r < L; r++) u[r] = __builtin_bit_cast(unsigned, v[r]);
+  // exchange bit by bit of the group number: halves of the wavefront, rows, half rows
 #pragma unroll
-  for (int r = 0; r < 4; r++) v[r] = __builtin_bit_cast(float, u[r]);
+  for (int r = 0; r < L / 2; r++) {
+    const auto x = __builtin_amdgcn_permlane32_swap(u[r], u[r + L / 2], false, false);
+    u[r] = x[0];
+    u[r + L / 2] = x[1];
+  }
+#pragma unroll
+  for (int b = 0; b < L; b += L / 2)
+#pragma unroll
+    for (int r = b; r < b + L / 4; r++) {
+      const auto x = __builtin_amdgcn_permlane16_swap(u[r], u[r + L / 4], false, false);
+      u[r] = x[0];
+      u[r + L / 4] = x[1];
+    }
+  if constexpr (L == 8) {
+#pragma unroll
+    for (int r = 0; r < L; r += 2) {
+      const int a = (int)u[r], b = (int)u[r + 1];  // row_ror:8 into the upper, the lower half of a row
+      u[r] = (unsigned)__builtin_amdgcn_update_dpp(a, b, 0x128, 0xf, 0xc, false);
+      u[r + 1] = (unsigned)__builtin_amdgcn_update_dpp(b, a, 0x128, 0xf, 0x3, false);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < L; r++) v[r] = __builtin_bit_cast(float, u[r]);
 }
-// v[n] = x of row n, in every row
-__device__ __forceinline__ void rows_of(float x, float (&v)[4]) {
-  v[0] = v[1] = v[2] = v[3] = x;
+// v[n] = x of group n, in every group
+template <int L>
+__device__ __forceinline__ void rows_of(float x, float (&v)[L]) {
+#pragma unroll
+  for (int n = 0; n < L; n++) v[n] = x;
   spread(v);
 }
-__device__ __forceinline__ void rows_of(double x, double (&v)[4]) {
+template <int L>
+__device__ __forceinline__ void rows_of(double x, double (&v)[L]) {
   const uint64_t w = __builtin_bit_cast(uint64_t, x);
   const unsigned w0 = (unsigned)w, w1 = (unsigned)(w >> 32);
-  float lo[4], hi[4];
+  float lo[L], hi[L];
   rows_of(__builtin_bit_cast(float, w0), lo);
   rows_of(__builtin_bit_cast(float, w1), hi);
 #pragma unroll
-  for (int n = 0; n < 4; n++)
+  for (int n = 0; n < L; n++)
     v[n] = __builtin_bit_cast(double, ((uint64_t)__builtin_bit_cast(unsigned, hi[n]) << 32) |
                                           __builtin_bit_cast(unsigned, lo[n]));
 }
-// the lanes of the 16 particles for which row n's bit of m is set
+// the lanes of the particles for which group n's bit of m is set
+template <int L>
 __device__ __forceinline__ uint64_t row_mask(uint64_t m, int n) {
+  if constexpr (L == 8) return ((m >> (8 * n)) & 0xff) * 0x0101010101010101ull;
   const uint64_t r = (m >> (16 * n)) & 0xffff;
   const uint64_t h = r | (r << 16);
   return h | (h << 32);
 }
-// adds neighbours 0 .. 3 to M sums; m: the lanes whose own neighbour counts.  With all of them in, no
-// masks (a masked sum costs a fifth operation)
-template <int M, class Acc>
-__device__ __forceinline__ void add_rows(Acc (&a)[M], const float (&v)[M][4], uint64_t m) {
+// adds neighbours 0 .. L - 1 to M sums; m: the lanes whose own neighbour counts.  With all of them in,
+// no masks (a masked sum costs a fifth operation)
+template <int M, int L, class Acc>
+__device__ __forceinline__ void add_rows(Acc (&a)[M], const float (&v)[M][L], uint64_t m) {
   if (m == ~0ull) {
 #pragma unroll
-    for (int n = 0; n < 4; n++)
+    for (int n = 0; n < L; n++)
 #pragma unroll
       for (int q = 0; q < M; q++) a[q].add(v[q][n]);
   } else {
 #pragma unroll
-    for (int n = 0; n < 4; n++)
-      if (__builtin_amdgcn_inverse_ballot_w64(row_mask(m, n))) {
+    for (int n = 0; n < L; n++)
+      if (__builtin_amdgcn_inverse_ballot_w64(row_mask<L>(m, n))) {
 #pragma unroll
         for (int q = 0; q < M; q++) a[q].add(v[q][n]);
       }
@@ -1579,7 +1604,7 @@ struct EntryGather {
   }
 };
 
-template <class Acc, bool BROOK, int BS>
+template <class Acc, bool BROOK, int L, int BS>
 __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_init, const State &st,
                                           const Rec32 *__restrict__ rec, const int *__restrict__ nbr,
                                           int stride, const int *__restrict__ count, const Consts &c,
@@ -1590,8 +1615,10 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   __shared__ __align__(16) char s_area[BS / 64][AREA];
   // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n = lane >> 4;
-  const unsigned t = xcd_map(b, nb) * (BS / PAIR_LANES) + 16 * w + (lane & 15);
+  constexpr int PER = 64 / L;  // particles of a wavefront
+  constexpr int NB = 8 / L, NA = 20 / L;  // sums of a lane: B, and those without the viscous ones
+  const int n = lane / PER;
+  const unsigned t = xcd_map(b, nb) * (BS / L) + PER * w + lane % PER;
   const unsigned N = cnt->N;
   const bool in_range = t < N && t < n_init;
   const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
@@ -1599,23 +1626,23 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   const bool act = in_range && !(fl & FL_BLANKED);
   const unsigned ic = act ? i : 0u;
   const int nl = act ? count[i] : 0;
-  int steps = (nl + PAIR_LANES - 1) / PAIR_LANES;
+  int steps = (nl + L - 1) / L;
 #pragma unroll
-  for (int o = 8; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
+  for (int o = PER / 2; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
   steps = __builtin_amdgcn_readfirstlane(steps);
   const int *row = nbr + (size_t)ic * stride + n;
-  // neighbour 4 k + n of the list; past its end the particle itself, which is loaded and not used
-  auto index = [&](int k) -> int { return n + 4 * k < nl ? row[4 * k] : (int)ic; };
+  // neighbour L k + n of the list; past its end the particle itself, which is loaded and not used
+  auto index = [&](int k) -> int { return n + L * k < nl ? row[L * k] : (int)ic; };
   Pair32<BROOK> P(c, rec[ic]);
   const bool tool_i = P.ri.tool == 1.f, tool_nz = (fl & FL_TOOL_NZ) != 0;
   char *area = s_area[w];
   if (c.cspm && steps > 0) {
     const EntryGather g(cs4, n_init, lane);
     // the wide sums' terms have always been rounded so for all but every fourth neighbour
-    const bool x_first = std::is_same<Acc, AccWide>::value && n != 0;
-    Acc a2[2], a1[1];  // B[4 m + n] and, in every row, B[8]
-    a2[0].zero();
-    a2[1].zero();
+    const bool x_first = std::is_same<Acc, AccWide>::value && (n & 3) != 0;
+    Acc a2[NB], a1[1];  // B[L q + n] and, in every group, B[8]
+#pragma unroll
+    for (int q = 0; q < NB; q++) a2[q].zero();
     a1[0].zero();
     const int nb = (steps + CSPM_BLOCK - 1) / CSPM_BLOCK;
     int jn[CSPM_BLOCK];
@@ -1638,13 +1665,14 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
       for (int s = 0; s < CSPM_BLOCK; s++) {
         const double4 e = g.read(here + s * CSPM_STEP);
         const ToolVol tv = __builtin_bit_cast(ToolVol, e.w);
-        float B[9], v2[2][4], v1[1][4];
+        float B[9], v2[NB][L], v1[1][L];
         P.cspm_term(e, tv.vol, x_first, B);
-        const uint64_t m = __builtin_amdgcn_ballot_w64(n + 4 * (b * CSPM_BLOCK + s) < nl && !tool_nz && tv.tool != 1.f);
+        const uint64_t m = 
+            __builtin_amdgcn_ballot_w64(n + L * (b * CSPM_BLOCK + s) < nl && !tool_nz && tv.tool != 1.f);
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
+        for (int q = 0; q < NB; q++) {
 #pragma unroll
-          for (int r = 0; r < 4; r++) v2[q][r] = B[4 * q + r];
+          for (int r = 0; r < L; r++) v2[q][r] = B[L * q + r];
           spread(v2[q]);
         }
         rows_of(B[8], v1[0]);
@@ -1653,19 +1681,20 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
       }
     }
     wave_sync_lds();  // the area is free for the next walk
-    double B[9], r4[4];
+    double B[9], of[L];
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-      rows_of(a2[q].val(), r4);
+    for (int q = 0; q < NB; q++) {
+      rows_of(a2[q].val(), of);
 #pragma unroll
-      for (int r = 0; r < 4; r++) B[4 * q + r] = r4[r];
+      for (int r = 0; r < L; r++) B[L * q + r] = of[r];
     }
     B[8] = a1[0].val();
     P.invert(B);
   }
-  Acc a5[5], av[1], ah[1];
+  // slots L q + n of the 24 (Pair32::term): the first NA, and the last, with the viscous sums; heat
+  Acc am[NA], av[1], ah[1];
 #pragma unroll
-  for (int q = 0; q < 5; q++) a5[q].zero();
+  for (int q = 0; q < NA; q++) am[q].zero();
   av[0].zero();
   ah[0].zero();
   const RecGather g(rec, n_init, area, lane);
@@ -1682,50 +1711,52 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
         g.issue(jn);
         jn = index(k + 2);
       }
-      float v[24], v5[5][4], vv[1][4], heat = 0.f;
+      float v[24], vm[NA][L], vv[L], heat = 0.f;
       bool approach, hot = false;
       P.term(rj, v, approach, heat, hot);
-      const bool in_list = n + 4 * k < nl, mech = in_list && !tool_i && !(rj.tool == 1.f);
+      const bool in_list = n + L * k < nl, mech = in_list && !tool_i && !(rj.tool == 1.f);
       const uint64_t m = __builtin_amdgcn_ballot_w64(mech), mv = __builtin_amdgcn_ballot_w64(mech && approach);
 #pragma unroll
-      for (int q = 0; q < 5; q++) {
+      for (int q = 0; q < NA; q++) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) v5[q][r] = v[4 * q + r];
-        spread(v5[q]);
+        for (int r = 0; r < L; r++) vm[q][r] = v[L * q + r];
+        spread(vm[q]);
       }
 #pragma unroll
-      for (int r = 0; r < 4; r++) vv[0][r] = v[20 + r];
-      spread(vv[0]);
-      add_rows(a5, v5, m);
-      // rows 0 .. 2 hold the viscous sums, row 3 one of the velocity smoothing
+      for (int r = 0; r < L; r++) vv[r] = v[24 - L + r];
+      spread(vv);
+      add_rows(am, vm, m);
+      // the last slots: 20 .. 22 the viscous sums, 23 (and for eight lanes 16 .. 19) others
+      constexpr uint64_t VISC = L == 8 ? 0x00ffffff00000000ull : 0x0000ffffffffffffull;
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const uint64_t keep = (row_mask(mv, q) & 0x0000ffffffffffffull) | (row_mask(m, q) & 0xffff000000000000ull);
-        if (__builtin_amdgcn_inverse_ballot_w64(keep)) av[0].add(vv[0][q]);
+      for (int q = 0; q < L; q++) {
+        const uint64_t keep = (row_mask<L>(mv, q) & VISC) | (row_mask<L>(m, q) & ~VISC);
+        if (__builtin_amdgcn_inverse_ballot_w64(keep)) av[0].add(vv[q]);
       }
       if (BROOK) {
-        float vh[1][4];
+        float vh[1][L];
         rows_of(heat, vh[0]);
         add_rows(ah, vh, __builtin_amdgcn_ballot_w64(in_list && brook && hot));
       }
     }
   }
   if (!act) return;
-  // slots 4 q + n: vd 0 .. 8, sd 0 .. 8, xt 0, xt 1 | vt 0 .. 2, xt 2
+  // slots: vd 0 .. 8, sd 0 .. 8, xt 0, xt 1, vt 0 .. 2, xt 2
+  auto place = [](int s) { return s < 18 || s == 23 ? s : s < 20 ? s + 3 : s - 2; };
 #pragma unroll
-  for (int q = 0; q < 5; q++) sums[(4 * q + n + (q == 4 && n >= 2 ? 3 : 0)) * sstride + i] = a5[q].val();
-  sums[(n < 3 ? 18 + n : 23) * sstride + i] = av[0].val();
+  for (int q = 0; q < NA; q++) sums[place(L * q + n) * sstride + i] = am[q].val();
+  sums[place(24 - L + n) * sstride + i] = av[0].val();
   if (n == 0) sums[24 * sstride + i] = BROOK ? ah[0].val() : 0.;
 }
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
 // depend on it).  Small instances spread over more compute units with smaller workgroups.
-template <class Acc, bool BROOK, int BS>
+template <class Acc, bool BROOK, int L, int BS>
 __global__ void __launch_bounds__(BS, PAIR32_WAVES)
     k_pair_rows(unsigned n_init, State st, const Rec32 *__restrict__ rec,
                 const int *__restrict__ nbr, int stride, const int *__restrict__ count,
                 Consts c, const Counters *cnt, double *__restrict__ sums, size_t sstride,
                 const int *__restrict__ trav, const double4 *__restrict__ cs4) {
-  pair_rows<Acc, BROOK, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
+  pair_rows<Acc, BROOK, L, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
                             sstride, trav, cs4);
 }
 
@@ -1753,30 +1784,58 @@ void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const 
   else launch(std::integral_constant<int, 2>{});
 }
 
-int pair_blocks(unsigned n_init, int block) { return (int)nb((long)n_init * PAIR_LANES, block); }
+// Lanes per particle.  Few particles leave SIMDs without a wavefront, and a wavefront alone on its SIMD
+// waits at every step of its lists: more lanes shorten them.
+// FP64: 16 below 4,096 particles (one wavefront per SIMD then; 512 particles 18.5 -> 11.7 us), else 4.
+// Eight lanes would take 17 us at 8,000 particles against 22.5, but the order of the sums is part of the
+// result in their last bits, and with it a single-precision rounding of the Johnson-Cook solve turns
+// within 1,000 steps of the cut that four lanes follow the oracle through to 1e-10.
+__host__ __device__ static inline int lanes64(unsigned n) { return n < 4096 ? 16 : 4; }
+// FP32 (the same sums for either): 8 below 24k particles, else 4: 19,000 particles 50 us against 58,
+// 32,000 60 against 58, 255k 362 against 322.
+int pair_lanes(int precision, long particles) {
+  if (precision == MFG_FP64) return lanes64((unsigned)std::min<long>(particles, 0xffffffffL));
+  return particles < 24 * 1024 ? 8 : 4;
+}
+int pair_blocks(unsigned n_init, int lanes, int block) { return (int)nb((long)n_init * lanes, block); }
 
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
                  int nl_stride, const int *count, const Consts &c, const Counters *cnt,
                  double *sums, size_t sstride, const int *trav, const double4 *cs4, int block,
                  bool ordered) {
   const int bs = block == 64 || block == 128 ? block : BSP;
-  const dim3 blk(bs), grid((unsigned)pair_blocks(n_init, bs));
+  const int lanes = pair_lanes(c.precision, n_init);
+  const dim3 blk(bs), grid((unsigned)pair_blocks(n_init, lanes, bs));
   const bool brook = c.heat == MFG_HEAT_BROOKSHAW;
+  auto sums64 = [&](auto bs_c, auto brook_c) {
+    auto with = [&](auto lanes_c) {
+      hipLaunchKernelGGL((k_pair_sums<decltype(brook_c)::value, decltype(lanes_c)::value, decltype(bs_c)::value>),
+                         grid, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums,
+                         sstride, trav);
+    };
+    if (lanes == 4) with(std::integral_constant<int, 4>{});
+    else with(std::integral_constant<int, 16>{});
+  };
   auto launch = [&](auto bs_c, auto brook_c) {
     constexpr int BS = decltype(bs_c)::value;
     constexpr bool BROOK = decltype(brook_c)::value;
+    auto rows = [&](auto acc) {
+      if (lanes == 4)
+        hipLaunchKernelGGL((k_pair_rows<decltype(acc), BROOK, 4, BS>), grid, blk, 0, s, n_init, st,
+                           (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+      else
+        hipLaunchKernelGGL((k_pair_rows<decltype(acc), BROOK, 8, BS>), grid, blk, 0, s, n_init, st,
+                           (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+    };
     if (c.precision == MFG_FP32_KAHAN)
-      hipLaunchKernelGGL((k_pair_rows<AccKahan, BROOK, BS>), grid, blk, 0, s, n_init, st, (const Rec32 *)rec,
-                         nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+      rows(AccKahan{});
     else if (c.precision == MFG_FP32_WIDE)
-      hipLaunchKernelGGL((k_pair_rows<AccWide, BROOK, BS>), grid, blk, 0, s, n_init, st, (const Rec32 *)rec,
-                         nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+      rows(AccWide{});
     else if (ordered)  // one lane per particle
       hipLaunchKernelGGL(k_pair_ordered<BS>, dim3(nb(n_init, bs)), blk, 0, s, n_init, st, (const Rec64 *)rec,
                          nbr, nl_stride, count, c, cnt, sums, sstride, trav);
     else
-      hipLaunchKernelGGL((k_pair_sums<BROOK, BS>), grid, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr,
-                         nl_stride, count, c, cnt, sums, sstride, trav);
+      sums64(bs_c, brook_c);
   };
   auto sized = [&](auto bs_c) {
     if (brook) launch(bs_c, std::true_type{});
@@ -1806,20 +1865,23 @@ __global__ void __launch_bounds__(NB_BLOCK)
                             d.nl_stride, d.count, st.T_t, d.cnt, nullptr, d.poison);
 }
 
-template <bool BROOK>
+// the instances that have LANES lanes a particle alone: the sums depend on it in their last bits
+template <bool BROOK, int LANES>
 __global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair_sums(const Inst *in, BatchMap m) {
+  __shared__ __align__(16) char s_area[(BSP / 64) * QuadGather<Rec64>::AREA];
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  pair_sums<BROOK, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec64 *)d.rec, d.nbr,
-                        d.nl_stride, d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr);
+  if (lanes64(d.n_init) != LANES) return;
+  pair_sums<BROOK, LANES, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec64 *)d.rec, d.nbr, d.nl_stride,
+                               d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, s_area);
 }
 
-template <class Acc, bool BROOK>
+template <class Acc, bool BROOK, int L>
 __global__ void __launch_bounds__(BSP, PAIR32_WAVES) kb_pair_rows(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  pair_rows<Acc, BROOK, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
-                             d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, d.cs4);
+  pair_rows<Acc, BROOK, L, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
+                                d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, d.cs4);
 }
 
 __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchMap m) {
@@ -1842,14 +1904,26 @@ void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
   else if (L.precision == MFG_FP64) neighbours(std::integral_constant<int, 1>{});
   else neighbours(std::integral_constant<int, 2>{});
   const dim3 gp(L.pairs8.blocks), bp(BSP);
+  auto sums64 = [&](auto brook_c) {
+    constexpr bool BROOK = decltype(brook_c)::value;
+    if (L.pair_lanes & 4) hipLaunchKernelGGL((kb_pair_sums<BROOK, 4>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    if (L.pair_lanes & 16) hipLaunchKernelGGL((kb_pair_sums<BROOK, 16>), gp, bp, 0, s, L.inst, L.pairs8.m);
+  };
+  auto rows = [&](auto acc, auto brook_c) {
+    constexpr bool BROOK = decltype(brook_c)::value;
+    if (L.pair_lanes == 4)
+      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 4>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    else
+      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 8>), gp, bp, 0, s, L.inst, L.pairs8.m);
+  };
   auto launch = [&](auto brook_c) {
     constexpr bool BROOK = decltype(brook_c)::value;
     if (L.precision == MFG_FP64)
-      hipLaunchKernelGGL(kb_pair_sums<BROOK>, gp, bp, 0, s, L.inst, L.pairs8.m);
+      sums64(brook_c);
     else if (L.precision == MFG_FP32_KAHAN)
-      hipLaunchKernelGGL((kb_pair_rows<AccKahan, BROOK>), gp, bp, 0, s, L.inst, L.pairs8.m);
+      rows(AccKahan{}, brook_c);
     else
-      hipLaunchKernelGGL((kb_pair_rows<AccWide, BROOK>), gp, bp, 0, s, L.inst, L.pairs8.m);
+      rows(AccWide{}, brook_c);
   };
   if (L.brook) launch(std::true_type{});
   else launch(std::false_type{});

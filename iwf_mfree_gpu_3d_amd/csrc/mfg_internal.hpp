@@ -192,10 +192,11 @@ void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const 
                        const double2 *pse2, const double *h, const uint32_t *flags,
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
                        int want_pse, unsigned long long *stat_part, int *poison);
-// pair pass (neighbour sums), four lanes per particle; pair_blocks: its workgroups of `block` threads
-// (64, 128 or 256).  ordered: FP64 sums in the reference's order of evaluation, to the bit (unlocked
-// grids), one lane per particle.  cs4: FP32 modes only
-int pair_blocks(unsigned n_init, int block);
+// pair pass (neighbour sums); pair_lanes: lanes per particle in a launch over so many; pair_blocks: its
+// workgroups of `block` threads (64, 128 or 256).  ordered: FP64 sums in the reference's order of
+// evaluation, to the bit (unlocked grids), one lane per particle.  cs4: FP32 modes only
+int pair_lanes(int precision, long particles);
+int pair_blocks(unsigned n_init, int lanes, int block);
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
                  int nl_stride, const int *count, const Consts &c, const Counters *cnt,
                  double *sums, size_t sum_stride, const int *trav, const double4 *cs4, int block,
@@ -324,6 +325,7 @@ struct BatchLaunch {
   int n;
   int precision, pse;
   int brook;         // an instance conducts heat by Brookshaw's form
+  int pair_lanes;    // lanes per particle of the pair pass; FP64: those of all instances, or-ed
   int ordered;       // order_apart
   int scan_alone;    // no instance has more than SCAN_ALONE cells
   BatchGrid tiles;   // scan tiles of the cell counts

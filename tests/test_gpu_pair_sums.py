@@ -1,7 +1,7 @@
-"""The pair pass (four lanes per particle, one walk over the list) against plain numpy.
+"""The pair pass (4, 8 or 16 lanes per particle, one walk over the list) against plain numpy.
 
-Small clouds whose particle counts and list lengths straddle the pass's units: four lanes per
-particle, 16 particles per wavefront, 64 per workgroup; lists of 0 to 8 neighbours and long ones,
+Small clouds whose particle counts and list lengths straddle the pass's units: 4 to 16 lanes per
+particle, 4 to 16 particles per wavefront, 16 to 64 per workgroup; lists of 0 to 8 neighbours and long ones,
 odd capacities.  Tool particles (their volume and mechanics left out, their temperature not) and
 unequal smoothing lengths are among them; unlocked grids take the ordered sums.  The reference is the brute-force
 sum over all pairs in numpy's 64 bits, B inverted per particle, the corrected gradient used pair by
@@ -137,3 +137,51 @@ def test_pair_sums_against_all_pairs(hip_device, precision, locked, heat, cspm, 
             scale = np.abs(b).max()
             err = np.abs(a - b).max() / scale if scale > 0 else np.abs(a).max()
             assert err <= tol, (n, spread, name, err)
+
+
+def many_clouds(n, spread, total, precision):
+    """Copies of a cloud too far apart to meet, `total` particles; (inputs, fields by id)."""
+    copies = -(-total // n)
+    one = cloud(n, 900 + n, spread)
+    step = np.ptp(one["pos"][:, 0]) + 8 * DX
+    c = {k: np.concatenate([v] * copies)[:total] for k, v in one.items()}
+    c["pos"] = c["pos"] + np.repeat(np.arange(copies) * step, n)[:total, None] * [1.0, 0.0, 0.0]
+    alphas = constants(_lib.MFG_HEAT_BROOKSHAW, True, False, c["h"].max(), 0)
+    p = api.particle_gpu(c["pos"], c["vel"], c["rho"], c["T"], c["h"], None, c["tool"], c["S9"], precision=precision)
+    g = api.grid_gpu_green(total, c["pos"].min(0) - DX, c["pos"].max(0) + DX, float(c["h"].max()))
+    g.sort(p)
+    place = np.argsort(p.download(_lib.F_ID).astype(int))
+    api.material_eos(p)
+    api.interactions_monaghan(p, g)
+    got = [p.download(f)[place] for f in (_lib.F_POS_T, _lib.F_VEL_T, _lib.F_V_DER, _lib.F_S_DER, _lib.F_T_T)]
+    return c, alphas, got
+
+
+@pytest.mark.parametrize("total", [4095, 4096])
+def test_fp64_lanes(hip_device, total):
+    """Both sides of the size where 16 lanes a particle become 4: the first and the last cloud against
+    all pairs."""
+    for n, spread in ((65, 1.0), (257, 1.0), (515, 2.2)):
+        c, alphas, got = many_clouds(n, spread, total, _lib.MFG_FP64)
+        for lo in (0, (total - 1) // n * n):
+            part = slice(lo, min(lo + n, total))
+            ref = reference({k: v[part] for k, v in c.items()}, _lib.MFG_HEAT_BROOKSHAW, True, False, alphas)
+            for name, a, b in zip(("x_t", "v_t", "v_der", "S_der", "T_t"), got, ref):
+                a = a[part]
+                if name in ("x_t", "v_t"):
+                    a = a * (c["tool"][part] == 0)[:, None]
+                scale = np.abs(b).max()
+                err = np.abs(a - b).max() / scale if scale > 0 else np.abs(a).max()
+                assert err <= 1e-12, (n, lo, name, err)
+
+
+@pytest.mark.parametrize("precision", [_lib.MFG_FP32_KAHAN, _lib.MFG_FP32_WIDE], ids=["kahan", "wide"])
+def test_fp32_lanes_give_the_same_sums(hip_device, precision):
+    """Both sides of the size where 8 lanes a particle become 4: every particle that the two sets share
+    with all its neighbours has the same sums, to the bit."""
+    for n, spread in ((65, 1.0), (257, 1.0), (515, 2.2)):
+        _, _, small = many_clouds(n, spread, 24 * 1024 - 1, precision)
+        _, _, large = many_clouds(n, spread, 24 * 1024, precision)
+        whole = (24 * 1024 - 1) // n * n
+        for a, b in zip(small, large):
+            assert np.array_equal(a[:whole], b[:whole]), (n, spread)
