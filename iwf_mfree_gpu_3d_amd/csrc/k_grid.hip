@@ -179,8 +179,8 @@ __global__ void __launch_bounds__(BS) k_scan_reduce(const int *hist, long n, Cel
 // The offsets of tile b's cells (NT threads, ITEMS cells each), its occupied cells in the list of all
 // (ascending; occ[n]: how many), and with the last tile the totals.  A tile's base is the sum of all
 // before it: of the tile sums, or without them (part null: SCAN_ALONE) of the counts themselves, eight
-// loads of a thread in flight (26,000 cells: 6.7 us, 62,000: 7.4; the two launches 4.6 and 4.8 and the
-// gap between).
+// loads of a thread in flight (26,000 cells: 8.4 us, 62,000: 9.3, of which the list of occupied cells
+// 1.8; in two launches 4.6 and 4.8, the gap between them, and the list).
 template <int NT, int ITEMS>
 __device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, const CellSum *part, int *off,
                                            int *occ, unsigned n_init, Counters *cnt) {

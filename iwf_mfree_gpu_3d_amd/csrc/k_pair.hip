@@ -19,13 +19,13 @@
 // Precision: FP64 throughout, or (FP32 modes) the relative position in FP64, the pair arithmetic in
 // FP32 and every neighbour sum compensated; the particle update stays FP64.
 //
-// The FP64 pair pass at 1M particles (single-grain cut, about 103 neighbours each): 2.07 -> 0.98 ms
-// against one lane per particle with a walk of its own for B and the
-// reference's order of evaluation (385 vector instructions per neighbour step and 110 of the B walk,
-// now 150 and none); 8,000 particles 198 -> 22 us (125 wavefronts of 100 steps, now 500 of 26).  At
-// 1M it runs at 18 TB/s of record reads from the L2s; vector units busy half of the time, the L1 and
-// LDS paths about two thirds, at two waves per SIMD (45 FP64 sums a lane; compiled for three it
-// spills and is slower).
+// The FP64 pair pass at 1M particles (single-grain cut, about 103 neighbours each): 2.07 -> 0.98-1.02
+// ms against one lane per particle with a walk of its own for B and the reference's order of evaluation
+// (385 vector instructions per neighbour step and 110 of the B walk, now 150 and none); 8,000
+// particles 198 -> 22 us (125 wavefronts of 100 steps, now 500 of 26).  At 1M it runs at 18 TB/s of
+// record reads from the L2s; vector units busy half of the time, the L1 and LDS paths about two
+// thirds, at two waves per SIMD (45 FP64 sums a lane; compiled for three it spills: 4.15 ms).
+// Workgroups of 512 threads: 1.10 ms.
 #include <algorithm>
 #include <type_traits>
 
@@ -1154,6 +1154,41 @@ struct QuadGather {
   }
 };
 
+// What a lane needs to begin its walk.  Of a particle past N or blanked it is loaded like any other (the
+// arrays hold n_init) and not used, so that the loads go out together; N, the flags, the list's length
+// and its first entry waited for one another: 512 particles 11.7 -> 10.3 us, 8,000 22.6 -> 21.9, 1M FP32
+// 1.25 -> 1.23 ms, 24 batched wedges 1.26 -> 1.22 ms.  An entry is read inside its row, however short.
+template <int F>
+struct PairHead {
+  unsigned i;   // the particle, below n_init
+  uint32_t fl;  // its flags, FL_BLANKED past N
+  bool act;
+  int nl;
+  int j[F];  // neighbours q0, q0 + dq, ... of the list; past its end the particle itself
+  __device__ __forceinline__ PairHead(unsigned t, unsigned n_init, const State &st, const Counters *cnt,
+                                      const int *__restrict__ trav, const int *__restrict__ nbr, int stride,
+                                      const int *__restrict__ count, int q0, int dq) {
+    const unsigned N = cnt->N;
+    i = min(t, n_init - 1);
+    if (trav) i = min((unsigned)trav[i], n_init - 1);  // trav holds no particles past N
+    uint32_t f = st.flags[i];
+    int n = count[i];
+    const int *row = nbr + (size_t)i * stride;
+#pragma unroll
+    for (int k = 0; k < F; k++) j[k] = row[min(q0 + k * dq, stride - 1)];
+    // the loads stay together and ahead of what their results decide
+    asm volatile("" : "+v"(f), "+v"(n));
+#pragma unroll
+    for (int k = 0; k < F; k++) asm volatile("" : "+v"(j[k]));
+    const bool in_range = t < N && t < n_init;
+    fl = in_range ? f : FL_BLANKED;
+    act = in_range && !(f & FL_BLANKED);
+    nl = act ? n : 0;
+#pragma unroll
+    for (int k = 0; k < F; k++) j[k] = q0 + k * dq < nl ? j[k] : (int)i;
+  }
+};
+
 // LANES: lanes of a particle, 4 or 16 (lanes64); area: QuadGather::AREA bytes a wavefront
 template <bool BROOK, int LANES, int BS>
 __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_init, const State &st,
@@ -1164,16 +1199,14 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
                                           size_t sstride, const int *__restrict__ trav, char *area) {
   typedef QuadGather<Rec64> Gather;
   const unsigned t = xcd_map(b, nb) * (BS / LANES) + threadIdx.x / LANES;
-  const unsigned N = cnt->N;
-  const bool in_range = t < N && t < n_init;
-  const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
-  const uint32_t fl = in_range ? st.flags[i] : FL_BLANKED;
-  const bool act = in_range && !(fl & FL_BLANKED);
-  const unsigned ic = act ? i : 0u;
   // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int s = lane & (LANES - 1);
-  const int nl = act ? count[i] : 0;
+  const PairHead<1> hd(t, n_init, st, cnt, trav, nbr, stride, count, s, LANES);
+  const unsigned i = hd.i, ic = hd.i;
+  const uint32_t fl = hd.fl;
+  const bool act = hd.act;
+  const int nl = hd.nl, j0 = hd.j[0];
   int steps = (nl + LANES - 1) / LANES;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
@@ -1187,7 +1220,7 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
   PairAcc acc = {};
   const Gather g(rec, n_init, area + w * Gather::AREA, lane);
   if (steps > 0) {
-    g.issue(index(0));
+    g.issue(j0);
     int jn = steps > 1 ? index(1) : 0;
     for (int k = 0; k < steps; k++) {
       __builtin_amdgcn_s_waitcnt(0);  // this step's records are in LDS
@@ -1441,7 +1474,7 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 // order.
 //
 // Against one lane per particle, the same sums to the bit: 19,000 particles 137 -> 59 us (300 wavefronts
-// of 100 steps, now 1,200 of 26), 255k with wide sums 396 -> 324 us, 1M 1.35 -> 1.25 ms.  At 1M the
+// of 100 steps, now 1,200 of 26), 255k with wide sums 396 -> 324 us, 1M 1.35 -> 1.23 ms.  At 1M the
 // vector units are full: 424 instructions per 64 pairs, the exchanges and the transcendentals counting
 // double and fourfold; one lane per particle needs 345 but runs at the pace of its list reads (each
 // lane walks its own row: 1.42 ms).  115 registers: four waves per SIMD (three: 1.25 ms; five spill).
@@ -1619,13 +1652,11 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   constexpr int NB = 8 / L, NA = 20 / L;  // sums of a lane: B, and those without the viscous ones
   const int n = lane / PER;
   const unsigned t = xcd_map(b, nb) * (BS / L) + PER * w + lane % PER;
-  const unsigned N = cnt->N;
-  const bool in_range = t < N && t < n_init;
-  const unsigned i = in_range && trav ? (unsigned)trav[t] : t;
-  const uint32_t fl = in_range ? st.flags[i] : FL_BLANKED;
-  const bool act = in_range && !(fl & FL_BLANKED);
-  const unsigned ic = act ? i : 0u;
-  const int nl = act ? count[i] : 0;
+  const PairHead<2> hd(t, n_init, st, cnt, trav, nbr, stride, count, n, L);
+  const unsigned i = hd.i, ic = hd.i;
+  const uint32_t fl = hd.fl;
+  const bool act = hd.act;
+  const int nl = hd.nl, j0 = hd.j[0], j1 = hd.j[1];
   int steps = (nl + L - 1) / L;
 #pragma unroll
   for (int o = PER / 2; o > 0; o >>= 1) steps = max(steps, __shfl_xor(steps, o, 64));
@@ -1647,7 +1678,8 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
     const int nb = (steps + CSPM_BLOCK - 1) / CSPM_BLOCK;
     int jn[CSPM_BLOCK];
 #pragma unroll
-    for (int s = 0; s < CSPM_BLOCK; s++) g.issue(index(s), area + s * CSPM_STEP);
+    for (int s = 0; s < CSPM_BLOCK; s++)
+      g.issue(s == 0 ? j0 : s == 1 ? j1 : index(s), area + s * CSPM_STEP);
 #pragma unroll
     for (int s = 0; s < CSPM_BLOCK; s++) jn[s] = index(CSPM_BLOCK + s);
     for (int b = 0; b < nb; b++) {
@@ -1700,8 +1732,8 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   const RecGather g(rec, n_init, area, lane);
   const bool brook = BROOK && (tool_nz ? c.alpha_tool : c.alpha_wp) != 0.;
   if (steps > 0) {
-    g.issue(index(0));
-    int jn = index(1);
+    g.issue(j0);
+    int jn = j1;
     for (int k = 0; k < steps; k++) {
       __builtin_amdgcn_s_waitcnt(0);  // this step's records are in LDS
       const Rec32 rj = g.read();
