@@ -581,7 +581,7 @@ int run_neighbours(mfg_grid *g, mfg_particles *p, const Consts &c, int want_pse,
 }
 
 // N and the device's errors from the pinned mirror (its copy has arrived)
-int judge_counters(mfg_particles *p) {
+int counters_status(mfg_particles *p) {
   p->N_host = p->cnt_h->N;
   if (p->cnt_h->err_capacity)
     return fail(MFG_ERR_CAPACITY, "a particle has %d neighbours, list capacity is %d",
@@ -598,7 +598,7 @@ int check_counters(mfg_particles *p) {
   launch_words_to_host(g_lib.stream, p->cnt, p->cnt_h, sizeof(Counters) / 4);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(g_lib.stream));
-  return judge_counters(p);
+  return counters_status(p);
 }
 
 // A field of every particle to host memory, interleaved by the device.  Fields of up to STAGE_BYTES:
@@ -624,7 +624,7 @@ int download_field(mfg_particles *p, const PackField &f, double *host) {
     launch_pack_field(s, f, p->N_init, p->stage, p->cnt, p->cnt_h);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s));
-    const int rc = judge_counters(p);
+    const int rc = counters_status(p);
     if (rc == MFG_OK) std::memcpy(host, p->stage, bytes);
     return rc;
   }
