@@ -1087,6 +1087,33 @@ __global__ void __launch_bounds__(BSP)
 // A 16-byte piece of a record (the unit of the cooperative gathers through LDS below).
 typedef unsigned piece16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) void glb_void;
+
+// A record array for the gathers: 16 bytes of every lane at record j, byte off + line, go to LDS.  A
+// buffer descriptor's stride is the record size, so the load unit forms index x stride + offset; an
+// index beyond n_rec reads zeros instead of faulting.  It forms them in 32 bits: an array of more than
+// 4 GiB (22.4M FP64 records, 38.3M FP32) is read by 64-bit addresses (FAR), two vector instructions a
+// load more, which at that size costs nothing (23.4M particles of 92 neighbours FP64 23.6 ms, 39.3M FP32
+// 42.8, with 32-bit offsets and wrong records 23.6 and 43.0).
+template <class Rec, bool FAR>
+struct RecordArray {
+  __amdgpu_buffer_rsrc_t rsrc;
+  // word 3: the untyped 32-bit data format the load-to-LDS path needs on gfx9-family parts
+  __device__ __forceinline__ RecordArray(const Rec *rec, unsigned n_rec)
+      : rsrc(__builtin_amdgcn_make_buffer_rsrc((void *)rec, (short)sizeof(Rec), (int)n_rec, 0x00020000)) {}
+  __device__ __forceinline__ void load(int j, int off, int line, char *lds) const {
+    __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)lds, 16, j, off, line, 0, 0);
+  }
+};
+template <class Rec>
+struct RecordArray<Rec, true> {
+  const char *rec;
+  __device__ __forceinline__ RecordArray(const Rec *r, unsigned) : rec((const char *)r) {}
+  __device__ __forceinline__ void load(int j, int off, int line, char *lds) const {
+    __builtin_amdgcn_global_load_lds((glb_void *)(rec + (uint64_t)(unsigned)j * sizeof(Rec) + off + line),
+                                     (lds_void *)lds, 16, 0, 0);
+  }
+};
 
 __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1104,13 +1131,12 @@ __device__ __forceinline__ void wave_sync_lds() {
 // together, straight into LDS (buffer_load_dwordx4 ... lds writes lane l's 16 bytes at 16 l of the
 // load's 1 KB block).  Load (r, line) of a step fetches 64-byte line `line` of the record of lane r
 // of every quad, one 64-byte line per quad: one L1 access each, where a lane loading its own record
-// makes one per 16-byte piece.  The index of lane r reaches the quad by a quad permutation, and the
-// buffer descriptor's stride is the record size, so the load unit forms index x stride + offset; an
-// index beyond n_rec reads zeros instead of faulting.  Lane e of the quad fetches piece (e + r) mod 4
+// makes one per 16-byte piece.  The index of lane r reaches the quad by a quad permutation.  Lane e of
+// the quad fetches piece (e + r) mod 4
 // of the line, so piece p of lane s's record lies in slot (p - s) mod 4 of its quad's 64 bytes in
 // block (s, line): the four lanes of a quad read four different slots, and the 16-byte reads of any
 // two (or four) quads fall on distinct banks.
-template <class Rec, int LINES = sizeof(Rec) / 64>
+template <class Rec, bool FAR, int LINES = sizeof(Rec) / 64>
 struct QuadGather {
   static constexpr int P = 4 * LINES;  // LINES: lines of a record fetched, from its first
   static constexpr int AREA = 4 * LINES * 1024;
@@ -1118,13 +1144,12 @@ struct QuadGather {
   struct Pieces {
     piece16 p[P];
   };
-  __amdgpu_buffer_rsrc_t rsrc;
+  RecordArray<Rec, FAR> array;
   char *area;
   int off[4];  // byte offset within a line of the piece this lane fetches, per record r
   int rd[4];   // LDS offset of piece p of line 0 of this lane's record
-  __device__ __forceinline__ QuadGather(const Rec *rec, unsigned n_rec, char *lds, int lane) : area(lds) {
-    // word 3: the untyped 32-bit data format the load-to-LDS path needs on gfx9-family parts
-    rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)rec, (short)sizeof(Rec), (int)n_rec, 0x00020000);
+  __device__ __forceinline__ QuadGather(const Rec *rec, unsigned n_rec, char *lds, int lane)
+      : array(rec, n_rec), area(lds) {
     const int s = lane & 3;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
@@ -1141,9 +1166,7 @@ struct QuadGather {
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int l = 0; l < LINES; l++)
-        __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + (r * LINES + l) * 1024),
-                                                    16, jr[r], off[r], 64 * l, 0, 0);
+      for (int l = 0; l < LINES; l++) array.load(jr[r], off[r], 64 * l, area + (r * LINES + l) * 1024);
   }
   // this lane's record, once the loads have arrived
   __device__ __forceinline__ Pieces read() const {
@@ -1190,14 +1213,14 @@ struct PairHead {
 };
 
 // LANES: lanes of a particle, 4 or 16 (lanes64); area: QuadGather::AREA bytes a wavefront
-template <bool BROOK, int LANES, int BS>
+template <bool BROOK, int LANES, int BS, bool FAR>
 __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_init, const State &st,
                                           const Rec64 *__restrict__ rec,
                                           const int *__restrict__ nbr, int stride,
                                           const int *__restrict__ count, const Consts &c,
                                           const Counters *cnt, double *__restrict__ sums,
                                           size_t sstride, const int *__restrict__ trav, char *area) {
-  typedef QuadGather<Rec64> Gather;
+  typedef QuadGather<Rec64, FAR> Gather;
   const unsigned t = xcd_map(b, nb) * (BS / LANES) + threadIdx.x / LANES;
   // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1264,14 +1287,14 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
 }
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
 // depend on it)
-template <bool BROOK, int LANES, int BS>
+template <bool BROOK, int LANES, int BS, bool FAR>
 __global__ void __launch_bounds__(BS, PAIR_WAVES)
     k_pair_sums(unsigned n_init, State st, const Rec64 *__restrict__ rec,
                 const int *__restrict__ nbr, int stride, const int *__restrict__ count, Consts c,
                 const Counters *cnt, double *__restrict__ sums, size_t sstride,
                 const int *__restrict__ trav) {
-  __shared__ __align__(16) char s_area[(BS / 64) * QuadGather<Rec64>::AREA];
-  pair_sums<BROOK, LANES, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
+  __shared__ __align__(16) char s_area[(BS / 64) * QuadGather<Rec64, FAR>::AREA];
+  pair_sums<BROOK, LANES, BS, FAR>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
                               sstride, trav, s_area);
 }
 
@@ -1397,8 +1420,8 @@ struct PairOrdered64 {
 };
 
 // walks the list of a lane with record gathers of LINES lines; step(k, pieces) for k < nl
-template <int LINES, class Step>
-__device__ __forceinline__ void ordered_walk(const QuadGather<Rec64, LINES> &g, const int *row, int nl,
+template <bool FAR, int LINES, class Step>
+__device__ __forceinline__ void ordered_walk(const QuadGather<Rec64, FAR, LINES> &g, const int *row, int nl,
                                              int nmax, int ic, Step &&step) {
   typedef int iv4 __attribute__((ext_vector_type(4)));
   if (nmax <= 0) return;
@@ -1425,13 +1448,13 @@ __device__ __forceinline__ void ordered_walk(const QuadGather<Rec64, LINES> &g, 
   }
 }
 
-template <int BS>
+template <int BS, bool FAR>
 __global__ void __launch_bounds__(BS, PAIR_WAVES)
     k_pair_ordered(unsigned n_init, State st, const Rec64 *__restrict__ rec,
                    const int *__restrict__ nbr, int stride, const int *__restrict__ count, Consts c,
                    const Counters *cnt, double *__restrict__ sums, size_t sstride,
                    const int *__restrict__ trav) {
-  typedef QuadGather<Rec64> Gather;
+  typedef QuadGather<Rec64, FAR> Gather;
   __shared__ __align__(16) char s_area[BS / 64][Gather::AREA];
   const unsigned t = xcd_map(blockIdx.x, gridDim.x) * BS + threadIdx.x;
   const bool in_range = t < cnt->N && t < n_init;
@@ -1449,7 +1472,7 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
   nmax = __builtin_amdgcn_readfirstlane(nmax);
   if (c.cspm) {
     // x, y, z, h, T, vol, c, tool: the record's first line
-    ordered_walk(QuadGather<Rec64, 1>(rec, n_init, s_area[w], lane), row, P.cspm_sum() ? nl : 0,
+    ordered_walk(QuadGather<Rec64, FAR, 1>(rec, n_init, s_area[w], lane), row, P.cspm_sum() ? nl : 0,
                  nmax, (int)ic, [&](const auto &pc) {
                    struct Line {
                      double x, y, z, h, T, vol, c, tool;
@@ -1480,7 +1503,8 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 // lane walks its own row: 1.42 ms).  115 registers: four waves per SIMD (three: 1.25 ms; five spill).
 // The index of a lane's next neighbour is one 4-byte read two steps ahead: reading them by fours and
 // exchanging them waits longer (1.86 ms).
-constexpr int PAIR32_WAVES = 4;
+// (FAR: three, its addresses take the registers that would otherwise spill.)
+constexpr int pair32_waves(bool far) { return far ? 3 : 4; }
 
 // L groups of 64 / L lanes (rows of 16 for four, half rows for eight): on return v[n] in group r holds
 // what v[r] held in group n
@@ -1564,21 +1588,19 @@ __device__ __forceinline__ void add_rows(Acc (&a)[M], const float (&v)[M][L], ui
 // The records of a step: 64 in LDS one after the other (record of lane L at 112 L), as seven 1 KB
 // blocks: load q fetches piece g = 64 q + lane of that image (record g / 7, piece g mod 7), so every
 // lane loads and no piece is fetched twice.  At the 112-byte stride the 16-byte reads of a lane's own
-// record fall on distinct banks for the lanes one read phase serves.  The buffer descriptor's stride
-// is the record size: the load unit forms index x stride + offset, and an index beyond n_rec reads
-// zeros instead of faulting.
+// record fall on distinct banks for the lanes one read phase serves.
+template <bool FAR>
 struct RecGather {
   static constexpr int P = 7, AREA = P * 1024;
   static_assert(sizeof(Rec32) == 16 * P, "FP32 record image");
   struct Pieces {
     piece16 p[P];
   };
-  __amdgpu_buffer_rsrc_t rsrc;
+  RecordArray<Rec32, FAR> array;
   char *area;
   int src[P], off[P], lane;
-  __device__ __forceinline__ RecGather(const Rec32 *rec, unsigned n_rec, char *lds, int l) : area(lds), lane(l) {
-    // word 3: the untyped 32-bit data format the load-to-LDS path needs on gfx9-family parts
-    rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)rec, (short)sizeof(Rec32), (int)n_rec, 0x00020000);
+  __device__ __forceinline__ RecGather(const Rec32 *rec, unsigned n_rec, char *lds, int l)
+      : array(rec, n_rec), area(lds), lane(l) {
 #pragma unroll
     for (int q = 0; q < P; q++) {
       const int g = 64 * q + lane, r = g / P;
@@ -1591,9 +1613,7 @@ struct RecGather {
 #pragma unroll
     for (int q = 0; q < P; q++) jm[q] = __builtin_amdgcn_ds_bpermute(src[q], j);
 #pragma unroll
-    for (int q = 0; q < P; q++)
-      __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + 1024 * q), 16, jm[q], off[q], 0,
-                                                  0, 0);
+    for (int q = 0; q < P; q++) array.load(jm[q], off[q], 0, area + 1024 * q);
   }
   __device__ __forceinline__ Rec32 read() const {
     Pieces pc;
@@ -1607,14 +1627,14 @@ struct RecGather {
 // 16-byte reads of 16 consecutive lanes fall on distinct bank groups.  The terms are light, so the
 // walk holds CSPM_BLOCK steps in LDS while the next CSPM_BLOCK load.
 constexpr int CSPM_BLOCK = 2, CSPM_STEP = 64 * 32, CSPM_AREA = 2 * CSPM_BLOCK * CSPM_STEP;
+template <bool FAR>
 struct EntryGather {
   struct Pieces {
     piece16 p[2];
   };
-  __amdgpu_buffer_rsrc_t rsrc;
+  RecordArray<double4, FAR> array;
   int src[2], off[2], rd[2];
-  __device__ __forceinline__ EntryGather(const double4 *cs4, unsigned n_rec, int lane) {
-    rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)cs4, (short)sizeof(double4), (int)n_rec, 0x00020000);
+  __device__ __forceinline__ EntryGather(const double4 *cs4, unsigned n_rec, int lane) : array(cs4, n_rec) {
 #pragma unroll
     for (int q = 0; q < 2; q++) {
       const int g = 64 * q + lane, r = g >> 1;
@@ -1626,8 +1646,7 @@ struct EntryGather {
   __device__ __forceinline__ void issue(int j, char *area) const {
 #pragma unroll
     for (int q = 0; q < 2; q++)
-      __builtin_amdgcn_struct_ptr_buffer_load_lds(rsrc, (lds_void *)(area + 1024 * q), 16,
-                                                  __builtin_amdgcn_ds_bpermute(src[q], j), off[q], 0, 0, 0);
+      array.load(__builtin_amdgcn_ds_bpermute(src[q], j), off[q], 0, area + 1024 * q);
   }
   __device__ __forceinline__ double4 read(const char *area) const {
     Pieces pc;
@@ -1637,14 +1656,14 @@ struct EntryGather {
   }
 };
 
-template <class Acc, bool BROOK, int L, int BS>
+template <class Acc, bool BROOK, int L, int BS, bool FAR>
 __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_init, const State &st,
                                           const Rec32 *__restrict__ rec, const int *__restrict__ nbr,
                                           int stride, const int *__restrict__ count, const Consts &c,
                                           const Counters *cnt, double *__restrict__ sums,
                                           size_t sstride, const int *__restrict__ trav,
                                           const double4 *__restrict__ cs4) {
-  constexpr int AREA = CSPM_AREA > RecGather::AREA ? CSPM_AREA : RecGather::AREA;
+  constexpr int AREA = CSPM_AREA > RecGather<FAR>::AREA ? CSPM_AREA : RecGather<FAR>::AREA;
   __shared__ __align__(16) char s_area[BS / 64][AREA];
   // the wave index as a scalar: the scalar unit forms the LDS destinations of the loads
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1668,7 +1687,7 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   const bool tool_i = P.ri.tool == 1.f, tool_nz = (fl & FL_TOOL_NZ) != 0;
   char *area = s_area[w];
   if (c.cspm && steps > 0) {
-    const EntryGather g(cs4, n_init, lane);
+    const EntryGather<FAR> g(cs4, n_init, lane);
     // the wide sums' terms have always been rounded so for all but every fourth neighbour
     const bool x_first = std::is_same<Acc, AccWide>::value && (n & 3) != 0;
     Acc a2[NB], a1[1];  // B[L q + n] and, in every group, B[8]
@@ -1729,7 +1748,7 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   for (int q = 0; q < NA; q++) am[q].zero();
   av[0].zero();
   ah[0].zero();
-  const RecGather g(rec, n_init, area, lane);
+  const RecGather<FAR> g(rec, n_init, area, lane);
   const bool brook = BROOK && (tool_nz ? c.alpha_tool : c.alpha_wp) != 0.;
   if (steps > 0) {
     g.issue(j0);
@@ -1782,13 +1801,13 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
 }
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not
 // depend on it).  Small instances spread over more compute units with smaller workgroups.
-template <class Acc, bool BROOK, int L, int BS>
-__global__ void __launch_bounds__(BS, PAIR32_WAVES)
+template <class Acc, bool BROOK, int L, int BS, bool FAR>
+__global__ void __launch_bounds__(BS, pair32_waves(FAR))
     k_pair_rows(unsigned n_init, State st, const Rec32 *__restrict__ rec,
                 const int *__restrict__ nbr, int stride, const int *__restrict__ count,
                 Consts c, const Counters *cnt, double *__restrict__ sums, size_t sstride,
                 const int *__restrict__ trav, const double4 *__restrict__ cs4) {
-  pair_rows<Acc, BROOK, L, BS>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
+  pair_rows<Acc, BROOK, L, BS, FAR>(blockIdx.x, gridDim.x, n_init, st, rec, nbr, stride, count, c, cnt, sums,
                             sstride, trav, cs4);
 }
 
@@ -1830,6 +1849,10 @@ int pair_lanes(int precision, long particles) {
   return particles < 24 * 1024 ? 8 : 4;
 }
 int pair_blocks(unsigned n_init, int lanes, int block) { return (int)nb((long)n_init * lanes, block); }
+// whether the record array is beyond the gathers' 32-bit offsets (RecordArray)
+bool pair_far(int precision, unsigned n_init) {
+  return (uint64_t)n_init * (precision == MFG_FP64 ? sizeof(Rec64) : sizeof(Rec32)) > 1ull << 32;
+}
 
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
                  int nl_stride, const int *count, const Consts &c, const Counters *cnt,
@@ -1838,36 +1861,38 @@ void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *re
   const int bs = block == 64 || block == 128 ? block : BSP;
   const int lanes = pair_lanes(c.precision, n_init);
   const dim3 blk(bs), grid((unsigned)pair_blocks(n_init, lanes, bs));
-  const bool brook = c.heat == MFG_HEAT_BROOKSHAW;
-  auto sums64 = [&](auto bs_c, auto brook_c) {
-    auto with = [&](auto lanes_c) {
-      hipLaunchKernelGGL((k_pair_sums<decltype(brook_c)::value, decltype(lanes_c)::value, decltype(bs_c)::value>),
-                         grid, blk, 0, s, n_init, st, (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums,
-                         sstride, trav);
-    };
-    if (lanes == 4) with(std::integral_constant<int, 4>{});
-    else with(std::integral_constant<int, 16>{});
-  };
+  const bool brook = c.heat == MFG_HEAT_BROOKSHAW, far = pair_far(c.precision, n_init);
+  constexpr std::false_type NEAR{};
+  constexpr std::true_type FAR{};
   auto launch = [&](auto bs_c, auto brook_c) {
     constexpr int BS = decltype(bs_c)::value;
     constexpr bool BROOK = decltype(brook_c)::value;
-    auto rows = [&](auto acc) {
-      if (lanes == 4)
-        hipLaunchKernelGGL((k_pair_rows<decltype(acc), BROOK, 4, BS>), grid, blk, 0, s, n_init, st,
-                           (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
-      else
-        hipLaunchKernelGGL((k_pair_rows<decltype(acc), BROOK, 8, BS>), grid, blk, 0, s, n_init, st,
-                           (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav, cs4);
+    auto sums64 = [&](auto lanes_c, auto far_c) {
+      hipLaunchKernelGGL((k_pair_sums<BROOK, decltype(lanes_c)::value, BS, decltype(far_c)::value>), grid, blk, 0, s,
+                         n_init, st, (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
     };
-    if (c.precision == MFG_FP32_KAHAN)
-      rows(AccKahan{});
-    else if (c.precision == MFG_FP32_WIDE)
-      rows(AccWide{});
-    else if (ordered)  // one lane per particle
-      hipLaunchKernelGGL(k_pair_ordered<BS>, dim3(nb(n_init, bs)), blk, 0, s, n_init, st, (const Rec64 *)rec,
-                         nbr, nl_stride, count, c, cnt, sums, sstride, trav);
-    else
-      sums64(bs_c, brook_c);
+    auto ordered64 = [&](auto far_c) {  // one lane per particle
+      hipLaunchKernelGGL((k_pair_ordered<BS, decltype(far_c)::value>), dim3(nb(n_init, bs)), blk, 0, s, n_init, st,
+                         (const Rec64 *)rec, nbr, nl_stride, count, c, cnt, sums, sstride, trav);
+    };
+    auto rows = [&](auto acc) {
+      auto with = [&](auto lanes_c, auto far_c) {
+        hipLaunchKernelGGL((k_pair_rows<decltype(acc), BROOK, decltype(lanes_c)::value, BS, decltype(far_c)::value>),
+                           grid, blk, 0, s, n_init, st, (const Rec32 *)rec, nbr, nl_stride, count, c, cnt, sums,
+                           sstride, trav, cs4);
+      };
+      // a set beyond the 32-bit offsets is far too large for eight lanes
+      if (far) with(std::integral_constant<int, 4>{}, FAR);
+      else if (lanes == 4) with(std::integral_constant<int, 4>{}, NEAR);
+      else with(std::integral_constant<int, 8>{}, NEAR);
+    };
+    if (c.precision == MFG_FP32_KAHAN) rows(AccKahan{});
+    else if (c.precision == MFG_FP32_WIDE) rows(AccWide{});
+    else if (ordered && far) ordered64(FAR);
+    else if (ordered) ordered64(NEAR);
+    else if (far) sums64(std::integral_constant<int, 4>{}, FAR);
+    else if (lanes == 4) sums64(std::integral_constant<int, 4>{}, NEAR);
+    else sums64(std::integral_constant<int, 16>{}, NEAR);
   };
   auto sized = [&](auto bs_c) {
     if (brook) launch(bs_c, std::true_type{});
@@ -1898,21 +1923,21 @@ __global__ void __launch_bounds__(NB_BLOCK)
 }
 
 // the instances that have LANES lanes a particle alone: the sums depend on it in their last bits
-template <bool BROOK, int LANES>
+template <bool BROOK, int LANES, bool FAR>
 __global__ void __launch_bounds__(BSP, PAIR_WAVES) kb_pair_sums(const Inst *in, BatchMap m) {
-  __shared__ __align__(16) char s_area[(BSP / 64) * QuadGather<Rec64>::AREA];
+  __shared__ __align__(16) char s_area[(BSP / 64) * QuadGather<Rec64, FAR>::AREA];
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
   if (lanes64(d.n_init) != LANES) return;
-  pair_sums<BROOK, LANES, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec64 *)d.rec, d.nbr, d.nl_stride,
+  pair_sums<BROOK, LANES, BSP, FAR>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec64 *)d.rec, d.nbr, d.nl_stride,
                                d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, s_area);
 }
 
-template <class Acc, bool BROOK, int L>
-__global__ void __launch_bounds__(BSP, PAIR32_WAVES) kb_pair_rows(const Inst *in, BatchMap m) {
+template <class Acc, bool BROOK, int L, bool FAR>
+__global__ void __launch_bounds__(BSP, pair32_waves(FAR)) kb_pair_rows(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  pair_rows<Acc, BROOK, L, BSP>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
+  pair_rows<Acc, BROOK, L, BSP, FAR>(b, nb, d.n_init, d.buf[d.cur ^ 1], (const Rec32 *)d.rec, d.nbr, d.nl_stride,
                                 d.count, d.c, d.cnt, d.sums, d.sum_stride, nullptr, d.cs4);
 }
 
@@ -1938,15 +1963,20 @@ void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
   const dim3 gp(L.pairs8.blocks), bp(BSP);
   auto sums64 = [&](auto brook_c) {
     constexpr bool BROOK = decltype(brook_c)::value;
-    if (L.pair_lanes & 4) hipLaunchKernelGGL((kb_pair_sums<BROOK, 4>), gp, bp, 0, s, L.inst, L.pairs8.m);
-    if (L.pair_lanes & 16) hipLaunchKernelGGL((kb_pair_sums<BROOK, 16>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    if ((L.pair_lanes & 4) && L.pair_far)
+      hipLaunchKernelGGL((kb_pair_sums<BROOK, 4, true>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    else if (L.pair_lanes & 4)
+      hipLaunchKernelGGL((kb_pair_sums<BROOK, 4, false>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    if (L.pair_lanes & 16) hipLaunchKernelGGL((kb_pair_sums<BROOK, 16, false>), gp, bp, 0, s, L.inst, L.pairs8.m);
   };
   auto rows = [&](auto acc, auto brook_c) {
     constexpr bool BROOK = decltype(brook_c)::value;
-    if (L.pair_lanes == 4)
-      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 4>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    if (L.pair_far)
+      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 4, true>), gp, bp, 0, s, L.inst, L.pairs8.m);
+    else if (L.pair_lanes == 4)
+      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 4, false>), gp, bp, 0, s, L.inst, L.pairs8.m);
     else
-      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 8>), gp, bp, 0, s, L.inst, L.pairs8.m);
+      hipLaunchKernelGGL((kb_pair_rows<decltype(acc), BROOK, 8, false>), gp, bp, 0, s, L.inst, L.pairs8.m);
   };
   auto launch = [&](auto brook_c) {
     constexpr bool BROOK = decltype(brook_c)::value;

@@ -197,6 +197,7 @@ void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const 
 // evaluation, to the bit (unlocked grids), one lane per particle.  cs4: FP32 modes only
 int pair_lanes(int precision, long particles);
 int pair_blocks(unsigned n_init, int lanes, int block);
+bool pair_far(int precision, unsigned n_init);
 void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *rec, const int *nbr,
                  int nl_stride, const int *count, const Consts &c, const Counters *cnt,
                  double *sums, size_t sum_stride, const int *trav, const double4 *cs4, int block,
@@ -326,6 +327,7 @@ struct BatchLaunch {
   int precision, pse;
   int brook;         // an instance conducts heat by Brookshaw's form
   int pair_lanes;    // lanes per particle of the pair pass; FP64: those of all instances, or-ed
+  int pair_far;      // an instance's records are beyond the gathers' 32-bit offsets
   int ordered;       // order_apart
   int scan_alone;    // no instance has more than SCAN_ALONE cells
   BatchGrid tiles;   // scan tiles of the cell counts
