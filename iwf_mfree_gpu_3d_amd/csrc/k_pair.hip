@@ -857,8 +857,9 @@ struct Pair64 {
     const double d = __builtin_fma(ve * hs, hs, r2);
     const double inv = rcp64(rs * d);
     const double irs = inv * d;
-    const double mu = 0.5 * hs * __builtin_fmin(vr, 0.) * (inv * rs);
-    const double pi = mu * __builtin_fma(vb, mu, -va * (cs + j.c)) * irs;
+    // a pair that recedes has no viscosity, also where a sound speed is NaN (a negative density)
+    const double mu = 0.5 * hs * vr * (inv * rs);
+    const double pi = vr < 0. ? mu * __builtin_fma(vb, mu, -va * (cs + j.c)) * irs : 0.;
     const double xw = val * irs;
 #pragma unroll
     for (int k = 0; k < 3; k++) {

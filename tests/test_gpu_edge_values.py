@@ -1,0 +1,58 @@
+"""Particles whose own values lie outside the ordinary range, one step against the oracle: which particles of their
+neighbourhood the NaN/Inf guard (src/actions_gpu.cu:302-331) blanks, exactly, and the rates of the others there.
+
+- A negative density has no sound speed (NaN).  The viscosity takes it only where a pair approaches
+  (src/interactions_gpu.cu:411-423), so the neighbours that recede keep finite rates.
+
+Tolerances from the arithmetic: FP64 sums of about 100 terms of a few roundings each, 1e-11 of a field's norm;
+FP32 terms, 2^-24 each with a handful of operations and cancellation of the stress sum by up to ten, 1e-4.
+"""
+import numpy as np
+import pytest
+
+import helpers
+import oracle as O
+from iwf_mfree_gpu_3d_amd import _lib, api, scenes
+from test_gpu_parity import perturbed_scene, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def spoil(sc, what):
+    """The particles nearest to three points of the workpiece, spoiled; their indices."""
+    wp = np.flatnonzero(sc.tool_p == 0)
+    lo, hi = sc.pos[wp].min(0), sc.pos[wp].max(0)
+    at = [lo + f * (hi - lo) for f in (0.2, 0.5, 0.8)]
+    ks = [int(wp[np.argmin(np.linalg.norm(sc.pos[wp] - a, axis=1))]) for a in at]
+    if what == "negative density":
+        sc.rho[ks] *= -0.3
+    return ks
+
+
+@pytest.mark.parametrize("what", ["negative density"])
+@pytest.mark.parametrize("scale", [0.5, 1.0])  # about 1,000 and 8,000 particles: either lane count of the pair pass
+@pytest.mark.parametrize("precision,tol", [(_lib.MFG_FP64, 1e-11), (_lib.MFG_FP32_KAHAN, 1e-4), (_lib.MFG_FP32_WIDE, 1e-4)],
+                         ids=["fp64", "kahan", "wide"])
+def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, tol, scale, what):
+    sc = perturbed_scene(1, scale, 7)
+    ks = spoil(sc, what)
+    sim = helpers.oracle_from_scene(sc)
+    dt = sc.params.dt
+    sim.set_time(dt, dt)
+    parts, grid = scenes.setup_cut(sc, precision=precision)
+    api.global_time_current = dt
+    assert sim.run(1) == 0
+    scenes.run(api.leap_frog(sc.n, grid.num_cell()), parts, grid, 1)
+    og = np.argsort(parts.download(_lib.F_ID).astype(np.int64))
+    oo = np.argsort(sim.field(O.F_ID).astype(np.int64))
+    blanked = sim.field(O.F_BLANKED)[oo]
+    # inside the support, where pairs interact (the oracle also adds 0 * NaN for the rest of the stencil)
+    near = np.min([np.linalg.norm(sc.pos - sc.pos[k], axis=1) for k in ks], axis=0) < 1.99 * sc.params.h
+    np.testing.assert_array_equal(parts.download(_lib.F_BLANKED)[og][near], blanked[near])
+    keep = (blanked != 1.0) & near
+    if what == "negative density":
+        assert blanked[ks].all() and keep.sum() > 20, "the particles are blanked, neighbours that recede are not"
+    for f, of in [(_lib.F_POS_T, O.F_POS_T), (_lib.F_VEL_T, O.F_VEL_T), (_lib.F_RHO_T, O.F_RHO_T)]:
+        g, o = parts.download(f)[og][keep], sim.field(of)[oo][keep]
+        assert np.isfinite(g).all()
+        assert rel_err(g, o) < tol, (f, rel_err(g, o))
