@@ -1282,8 +1282,11 @@ __device__ __forceinline__ void pair_sums(unsigned b, unsigned nb, unsigned n_in
     A[e] = rec[i].A[e];
     R[e] = rec[i].R[e];
   }
+  // without neighbours the sums are zero, whatever the kernel's scale (infinite for h = 0)
+  PairScale scale = P.scale(c);
+  if (nl == 0) scale.k1 = scale.fac = 0.;
   PairSums ps;
-  finish_sums<BROOK>(c, acc, P.scale(c), A, R, tool_nz, brook, ps);
+  finish_sums<BROOK>(c, acc, scale, A, R, tool_nz, brook, ps);
   store_sums(sums, sstride, i, ps);
 }
 // BS: threads per workgroup (64, 128 or 256; each wavefront works alone, so the sums do not

@@ -3,6 +3,7 @@ neighbourhood the NaN/Inf guard (src/actions_gpu.cu:302-331) blanks, exactly, an
 
 - A negative density has no sound speed (NaN).  The viscosity takes it only where a pair approaches
   (src/interactions_gpu.cu:411-423), so the neighbours that recede keep finite rates.
+- A smoothing length of zero has an empty list and an infinite kernel; without neighbours every sum is zero.
 
 Tolerances from the arithmetic: FP64 sums of about 100 terms of a few roundings each, 1e-11 of a field's norm;
 FP32 terms, 2^-24 each with a handful of operations and cancellation of the stress sum by up to ten, 1e-4.
@@ -26,10 +27,12 @@ def spoil(sc, what):
     ks = [int(wp[np.argmin(np.linalg.norm(sc.pos[wp] - a, axis=1))]) for a in at]
     if what == "negative density":
         sc.rho[ks] *= -0.3
+    elif what == "no smoothing length":
+        sc.h[ks] = 0.0
     return ks
 
 
-@pytest.mark.parametrize("what", ["negative density"])
+@pytest.mark.parametrize("what", ["negative density", "no smoothing length"])
 @pytest.mark.parametrize("scale", [0.5, 1.0])  # about 1,000 and 8,000 particles: either lane count of the pair pass
 @pytest.mark.parametrize("precision,tol", [(_lib.MFG_FP64, 1e-11), (_lib.MFG_FP32_KAHAN, 1e-4), (_lib.MFG_FP32_WIDE, 1e-4)],
                          ids=["fp64", "kahan", "wide"])
@@ -52,6 +55,8 @@ def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, tol, scale, 
     keep = (blanked != 1.0) & near
     if what == "negative density":
         assert blanked[ks].all() and keep.sum() > 20, "the particles are blanked, neighbours that recede are not"
+    else:
+        assert keep[ks].all()
     for f, of in [(_lib.F_POS_T, O.F_POS_T), (_lib.F_VEL_T, O.F_VEL_T), (_lib.F_RHO_T, O.F_RHO_T)]:
         g, o = parts.download(f)[og][keep], sim.field(of)[oo][keep]
         assert np.isfinite(g).all()
