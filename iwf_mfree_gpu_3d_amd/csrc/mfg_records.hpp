@@ -61,6 +61,14 @@ __device__ __forceinline__ void emit_record(unsigned i, const double xh[3], doub
                  Sh[3] * rho21,       Sh[4] * rho21,       Sh[5] * rho21};
   double vol = c.i_mass / rhoh;
   double cs = sqrt_site(c.i_K / rhoh, c.single_sqrt);
+  if constexpr (sizeof(RecT) == sizeof(Rec64)) {
+    // The FP64 sums share one reciprocal between viscosity and XSPH.  A neighbour's NaN h belongs to the
+    // viscosity alone, which its sound speed carries as well; its own sums are NaN or infinite for h = 0
+    if (isnan(h)) {
+      cs = h;
+      h = 0.;
+    }
+  }
   store_rec<RecT>(rec, i, xh, h, vh, rhoh, A, R, Th, vol, cs, tool ? 1.0 : 0.0);
   if constexpr (sizeof(RecT) == sizeof(Rec32)) {  // what the FP32 CSPM sum reads of a neighbour
     struct {

@@ -4,6 +4,8 @@ neighbourhood the NaN/Inf guard (src/actions_gpu.cu:302-331) blanks, exactly, an
 - A negative density has no sound speed (NaN).  The viscosity takes it only where a pair approaches
   (src/interactions_gpu.cu:411-423), so the neighbours that recede keep finite rates.
 - A smoothing length of zero has an empty list and an infinite kernel; without neighbours every sum is zero.
+- A NaN smoothing length excludes no candidate (src/kernels.cuh:41), so the particle's rates are NaN; its
+  neighbours take it into their viscosity alone.
 
 Tolerances from the arithmetic: FP64 sums of about 100 terms of a few roundings each, 1e-11 of a field's norm;
 FP32 terms, 2^-24 each with a handful of operations and cancellation of the stress sum by up to ten, 1e-4.
@@ -29,10 +31,12 @@ def spoil(sc, what):
         sc.rho[ks] *= -0.3
     elif what == "no smoothing length":
         sc.h[ks] = 0.0
+    elif what == "NaN smoothing length":
+        sc.h[ks] = np.nan
     return ks
 
 
-@pytest.mark.parametrize("what", ["negative density", "no smoothing length"])
+@pytest.mark.parametrize("what", ["negative density", "no smoothing length", "NaN smoothing length"])
 @pytest.mark.parametrize("scale", [0.5, 1.0])  # about 1,000 and 8,000 particles: either lane count of the pair pass
 @pytest.mark.parametrize("precision,tol", [(_lib.MFG_FP64, 1e-11), (_lib.MFG_FP32_KAHAN, 1e-4), (_lib.MFG_FP32_WIDE, 1e-4)],
                          ids=["fp64", "kahan", "wide"])
@@ -42,7 +46,7 @@ def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, tol, scale, 
     sim = helpers.oracle_from_scene(sc)
     dt = sc.params.dt
     sim.set_time(dt, dt)
-    parts, grid = scenes.setup_cut(sc, precision=precision)
+    parts, grid = scenes.setup_cut(sc, precision=precision, max_neighbours=1024)  # a whole stencil
     api.global_time_current = dt
     assert sim.run(1) == 0
     scenes.run(api.leap_frog(sc.n, grid.num_cell()), parts, grid, 1)
@@ -53,7 +57,7 @@ def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, tol, scale, 
     near = np.min([np.linalg.norm(sc.pos - sc.pos[k], axis=1) for k in ks], axis=0) < 1.99 * sc.params.h
     np.testing.assert_array_equal(parts.download(_lib.F_BLANKED)[og][near], blanked[near])
     keep = (blanked != 1.0) & near
-    if what == "negative density":
+    if what != "no smoothing length":
         assert blanked[ks].all() and keep.sum() > 20, "the particles are blanked, neighbours that recede are not"
     else:
         assert keep[ks].all()
