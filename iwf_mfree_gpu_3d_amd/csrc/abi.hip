@@ -563,7 +563,7 @@ int run_neighbours(mfg_grid *g, mfg_particles *p, const Consts &c, int want_pse,
     HIP_TRY(hipGetLastError());
     return MFG_OK;
   }
-  const int nb = neighbour_blocks(gi, p->N_init);
+  const int nb = (int)neighbour_blocks(gi, p->N_init);
   if (nb > p->stat_cap) {
     if (p->stat_part) (void)hipFree(p->stat_part);
     p->stat_part = nullptr;
@@ -2353,6 +2353,15 @@ int batch_build(mfg_batch *b, int record) {
     parts += m.p->N_init;
     most = std::max(most, (long)m.g->num_cell);
   }
+  // a launch for all the cells, or equal shares of one until they are done
+  size_t nbr = 0;
+  b->L.nbr_blocks = 0;
+  for (const mfg_batch::Member &m : b->members) {
+    const unsigned blocks = neighbour_blocks(m.g->info(), m.p->N_init);
+    nbr += blocks;
+    b->L.nbr_blocks = std::max(b->L.nbr_blocks, blocks);
+  }
+  b->L.nbr_most = nbr <= NB_MOST_BLOCKS ? NB_MOST_BLOCKS : std::max(8u, NB_MOST_BLOCKS / n / 8 * 8);
   b->L.scan_alone = most <= SCAN_ALONE;
   b->L.ordered = order_apart(parts);
   // FP64 sums depend on the lanes in their last bits: each instance has those it has alone
@@ -2373,7 +2382,7 @@ int batch_build(mfg_batch *b, int record) {
         nblk,
         round8((unsigned)pair_blocks(
             m.p->N_init, b->precision == MFG_FP64 ? pair_lanes(MFG_FP64, m.p->N_init) : b->L.pair_lanes, 256)),
-        (unsigned)neighbour_blocks(gi, m.p->N_init),
+        std::min(neighbour_blocks(gi, m.p->N_init), b->L.nbr_most),
         (unsigned)std::max<size_t>(1, m.tools.size()),
         m.search ? std::min(BATCH_SEARCH_BLOCKS, std::max(1u, nblk)) : 0u};
     for (int k = 0; k < N_MAPS; k++) maps[k * map_len + i + 1] = maps[k * map_len + i] + blocks[k];

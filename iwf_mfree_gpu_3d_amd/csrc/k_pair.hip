@@ -404,7 +404,9 @@ __device__ __forceinline__ int cell_ranges(const GridInfo &g, const int *__restr
 // Body of workgroup b of nb (the single-instance kernel and the batched one below): each wavefront takes
 // one cell of the occupied ones (occ, ascending; the scan of the sort lists them), each XCD one
 // contiguous eighth of the list.  The launch is sized for the most cells the particles can occupy, not
-// for the grid: its margins around the block are three quarters of the cells of a wedge cut.  Against
+// for the grid: its margins around the block are three quarters of the cells of a wedge cut.  Where that
+// is more than a launch holds (NB_MOST_BLOCKS), further launches take the cells that follow (first: workgroups
+// of the launches before; a loop in the kernel spills: FP64 PSE 6 registers, then 14).  Against
 // a wavefront for every cell: 8,000 particles 27 -> 13 us, 19,000 35 -> 18, 64,000 with PSE 100 -> 65;
 // 24 batched wedges, where a wavefront took 16 cells in turn, 0.77 -> 0.53 ms.
 template <int PSE_MODE>
@@ -482,20 +484,20 @@ __device__ __forceinline__ void cell_neighbours(
       a += s_stat[k][0];
       bb += s_stat[k][1];
     }
-    stat_part[2 * b] = a;
-    stat_part[2 * b + 1] = bb;
+    stat_part[2 * (size_t)b] = a;
+    stat_part[2 * (size_t)b + 1] = bb;
   }
 }
 template <int PSE_MODE>
 __global__ void __launch_bounds__(NB_BLOCK)
     __attribute__((amdgpu_waves_per_eu(PSE_MODE == 1 ? NB_WAVES_FP64_PSE : NB_WAVES_OTHER)))
-    k_cell_neighbours(GridInfo g, const int *__restrict__ off, const int *__restrict__ occ,
+    k_cell_neighbours(unsigned first, GridInfo g, const int *__restrict__ off, const int *__restrict__ occ,
                       const double4 *__restrict__ nl4,
                       const double2 *__restrict__ pse2, const double *__restrict__ h,
                       const uint32_t *__restrict__ flags, Consts c, int *__restrict__ nbr, int cap,
                       int *__restrict__ count, double *__restrict__ T_t, Counters *cnt,
                       unsigned long long *__restrict__ stat_part, int *__restrict__ poison) {
-  cell_neighbours<PSE_MODE>(blockIdx.x, g, off, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t, cnt,
+  cell_neighbours<PSE_MODE>(first + blockIdx.x, g, off, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t, cnt,
                             stat_part, poison);
 }
 
@@ -1824,20 +1826,23 @@ __global__ void __launch_bounds__(BS, pair32_waves(FAR))
 static inline unsigned nb(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 // a multiple of 8 workgroups: eight equal shares of the list
-int neighbour_blocks(const GridInfo &g, unsigned n_init) {
+unsigned neighbour_blocks(const GridInfo &g, unsigned n_init) {
   const long cells = std::min<long>(g.num_cell, n_init);
-  return (int)((cells + 8 * NB_WAVES - 1) / (8 * NB_WAVES)) * 8;
+  return (unsigned)((cells + 8 * NB_WAVES - 1) / (8 * NB_WAVES) * 8);
 }
+static_assert((long)NB_MOST_BLOCKS * NB_BLOCK < 1L << 32, "a launch holds fewer than 2^32 threads");
 
 void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const int *offsets,
                        const int *occ, const double4 *nl4,
                        const double2 *pse2, const double *h, const uint32_t *flags,
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
                        int want_pse, unsigned long long *stat_part, int *poison) {
+  const unsigned blocks = neighbour_blocks(g, n_init);
   auto launch = [&](auto mode_c) {
-    hipLaunchKernelGGL((k_cell_neighbours<decltype(mode_c)::value>), dim3(neighbour_blocks(g, n_init)),
-                       dim3(NB_BLOCK), 0, s, g, offsets, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t,
-                       cnt, stat_part, poison);
+    for (unsigned first = 0; first < blocks; first += NB_MOST_BLOCKS)
+      hipLaunchKernelGGL((k_cell_neighbours<decltype(mode_c)::value>), dim3(std::min(blocks - first, NB_MOST_BLOCKS)),
+                         dim3(NB_BLOCK), 0, s, first, g, offsets, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t,
+                         cnt, stat_part, poison);
   };
   if (!want_pse) launch(std::integral_constant<int, 0>{});
   else if (c.precision == MFG_FP64) launch(std::integral_constant<int, 1>{});
@@ -1923,11 +1928,11 @@ __global__ void __launch_bounds__(NB_BLOCK)
     __attribute__((amdgpu_waves_per_eu(PSE_MODE == 1   ? NB_WAVES_FP64_PSE - 1
                                        : PSE_MODE == 2 ? NB_WAVES_OTHER - 2
                                                        : NB_WAVES_OTHER - 1)))
-    kb_cell_neighbours(const Inst *in, BatchMap m) {
+    kb_cell_neighbours(const Inst *in, BatchMap m, unsigned first) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
   const State &st = d.buf[d.cur ^ 1];
-  cell_neighbours<PSE_MODE>(b, d.g, d.gb.count, d.gb.occ, d.nl4, d.pse2, st.h, st.flags, d.c, d.nbr,
+  cell_neighbours<PSE_MODE>(first + b, d.g, d.gb.count, d.gb.occ, d.nl4, d.pse2, st.h, st.flags, d.c, d.nbr,
                             d.nl_stride, d.count, st.T_t, d.cnt, nullptr, d.poison);
 }
 
@@ -1963,8 +1968,9 @@ __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchM
 // others' sums are the same in both.
 void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
   auto neighbours = [&](auto mode_c) {
-    hipLaunchKernelGGL((kb_cell_neighbours<decltype(mode_c)::value>), dim3(L.nbrs8.blocks), dim3(NB_BLOCK), 0,
-                       s, L.inst, L.nbrs8.m);
+    for (unsigned first = 0; first < L.nbr_blocks; first += L.nbr_most)
+      hipLaunchKernelGGL((kb_cell_neighbours<decltype(mode_c)::value>), dim3(L.nbrs8.blocks), dim3(NB_BLOCK), 0,
+                         s, L.inst, L.nbrs8.m, first);
   };
   if (!L.pse) neighbours(std::integral_constant<int, 0>{});
   else if (L.precision == MFG_FP64) neighbours(std::integral_constant<int, 1>{});

@@ -183,10 +183,11 @@ void launch_bbox_reduce(hipStream_t s, const State &st, const Counters *cnt, uns
                         double *partials, int nblocks);
 
 // neighbour lists (+ PSE heat) for every cell; stat_part gets 2 totals (candidates, pairs) per
-// workgroup, neighbour_blocks(g) workgroups; poison[p] = 1 when a candidate of particle p holds a
+// workgroup, neighbour_blocks of them; poison[p] = 1 when a candidate of particle p holds a
 // non-finite record (nl4.w == 2), which the reference's sums carry into p's rates
 // occ: the occupied cells (GridBuffers)
-int neighbour_blocks(const GridInfo &g, unsigned n_init);
+unsigned neighbour_blocks(const GridInfo &g, unsigned n_init);
+constexpr unsigned NB_MOST_BLOCKS = 1u << 24;  // of one launch
 void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const int *offsets,
                        const int *occ, const double4 *nl4,
                        const double2 *pse2, const double *h, const uint32_t *flags,
@@ -335,6 +336,7 @@ struct BatchLaunch {
   BatchGrid parts;   // N_init particles, 256 per workgroup
   BatchGrid pairs8;  // pair-pass workgroups, padded to a multiple of 8 (XCD-ordered kernels)
   BatchGrid nbrs8;   // neighbour-pass workgroups, padded to a multiple of 8
+  unsigned nbr_blocks, nbr_most;  // the largest instance's, and how many of them one launch takes
   BatchGrid tools;   // one workgroup per tool (at least one per instance)
   BatchGrid search;  // lane-parallel contact search workgroups
 };

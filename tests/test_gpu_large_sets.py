@@ -1,5 +1,5 @@
-"""Sets whose arrays are beyond 32-bit offsets: FP64 records of 192 bytes pass 4 GiB at 22.4M particles, FP32 records
-of 112 at 38.3M.
+"""Sets beyond 32-bit offsets and launches: FP64 records of 192 bytes pass 4 GiB at 22.4M particles, FP32 records of
+112 at 38.3M; a wavefront for each of 67.1M occupied cells passes the 2^32 threads of a launch.
 
 A cubic lattice of spacing 1 with a support between 1 and sqrt(2): every particle has its up to six lattice
 neighbours, visited in the same order everywhere, and the velocity field v = L x of constant L does not depend on
@@ -20,9 +20,10 @@ TRACE = -2e-3 + 3e-3
 
 def lattice(n1, precision, locked=True):
     n, h = n1 ** 3, 0.675
-    ax = np.arange(n1, dtype=float)
-    pos = np.zeros((n, 4))
-    pos[:, 0], pos[:, 1], pos[:, 2] = np.repeat(ax, n1 * n1), np.tile(np.repeat(ax, n1), n1), np.tile(ax, n1 * n1)
+    pos = np.zeros((n1, n1, n1, 4))
+    for k in range(3):
+        pos[..., k] = np.arange(n1, dtype=float).reshape([-1 if a == k else 1 for a in range(3)])
+    pos = pos.reshape(n, 4)
     vel = pos * [0.0, -2e-3, 3e-3, 0.0]
     api.reset_globals()
     api.constants_reset()
@@ -42,6 +43,16 @@ def lattice(n1, precision, locked=True):
     return p, g
 
 
+def check_planes(p, n1):
+    rho_t = np.empty(n1 ** 3)
+    rho_t[p.download(_lib.F_ID).astype(np.int64)] = p.download(_lib.F_RHO_T)
+    planes = rho_t.reshape(n1, -1)
+    bad = np.flatnonzero((planes[1:-1] != planes[1]).any(1)) + 1
+    assert len(bad) == 0, (len(bad), bad[:3])
+    # in FP32 the planes are to be right, not only alike
+    assert np.abs(rho_t / -TRACE - 1.0).max() <= (1e-10 if p.precision == _lib.MFG_FP64 else 1e-2)
+
+
 @pytest.mark.parametrize("form", ["step", "unlocked", "batch"])
 @pytest.mark.parametrize("precision,n1", [(_lib.MFG_FP64, 290), (_lib.MFG_FP32_KAHAN, 344), (_lib.MFG_FP32_WIDE, 344)],
                          ids=["fp64", "kahan", "wide"])
@@ -55,12 +66,22 @@ def test_records_beyond_4_gib(hip_device, precision, n1, form):
         b.step()
     else:
         api.leap_frog(p.N_init, g.num_cell()).step(p, g)
-    rho_t = np.empty(n1 ** 3)
-    rho_t[p.download(_lib.F_ID).astype(np.int64)] = p.download(_lib.F_RHO_T)
-    planes = rho_t.reshape(n1, -1)
-    bad = np.flatnonzero((planes[1:-1] != planes[1]).any(1)) + 1
-    assert len(bad) == 0, (len(bad), bad[:3])
-    if precision == _lib.MFG_FP64:
-        assert np.abs(rho_t / -TRACE - 1.0).max() <= 1e-10
-    else:  # the planes are right, not only alike
-        assert np.abs(rho_t / -TRACE - 1.0).max() <= 1e-2
+    check_planes(p, n1)
+
+
+@pytest.mark.parametrize("form", ["step", "batch"])
+def test_more_cells_than_a_launch_holds(hip_device, form):
+    """68.4M particles (409 a side) in 2.9 cells each."""
+    p, g = lattice(409, _lib.MFG_FP32_KAHAN)
+    api.pair_stats_enable(form == "step")
+    try:
+        if form == "batch":
+            b = api.batch()
+            b.add(p, g)
+            b.step()
+        else:
+            api.leap_frog(p.N_init, g.num_cell()).step(p, g)
+            assert p.pair_stats()[1] == 6 * 409 ** 2 * 408
+        check_planes(p, 409)
+    finally:
+        api.pair_stats_enable(False)
