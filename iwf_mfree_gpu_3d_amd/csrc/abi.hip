@@ -2368,8 +2368,11 @@ int batch_build(mfg_batch *b, int record) {
   b->L.pair_lanes = b->precision == MFG_FP64 ? 0 : pair_lanes(b->precision, parts);
   if (b->precision == MFG_FP64)
     for (const mfg_batch::Member &m : b->members) b->L.pair_lanes |= pair_lanes(MFG_FP64, m.p->N_init);
-  b->L.pair_far = 0;
-  for (const mfg_batch::Member &m : b->members) b->L.pair_far |= pair_far(b->precision, m.p->N_init);
+  b->L.pair_far = b->L.nbr_far = 0;
+  for (const mfg_batch::Member &m : b->members) {
+    b->L.pair_far |= pair_far(b->precision, m.p->N_init);
+    b->L.nbr_far |= neighbours_far(m.p->N_init);
+  }
   for (int i = 0; i < n; i++) {
     const mfg_batch::Member &m = b->members[i];
     host[i] = batch_inst(m, record);

@@ -409,7 +409,7 @@ __device__ __forceinline__ int cell_ranges(const GridInfo &g, const int *__restr
 // of the launches before; a loop in the kernel spills: FP64 PSE 6 registers, then 14).  Against
 // a wavefront for every cell: 8,000 particles 27 -> 13 us, 19,000 35 -> 18, 64,000 with PSE 100 -> 65;
 // 24 batched wedges, where a wavefront took 16 cells in turn, 0.77 -> 0.53 ms.
-template <int PSE_MODE>
+template <int PSE_MODE, bool FAR>
 __device__ __forceinline__ void cell_neighbours(
     unsigned b, const GridInfo &g, const int *__restrict__ off, const int *__restrict__ occ,
     const double4 *__restrict__ nl4, const double2 *__restrict__ pse2,
@@ -457,10 +457,12 @@ __device__ __forceinline__ void cell_neighbours(
       const int q = b0 + lane;
       NbCand cd;
       cd.j = q < T ? d + q : s;
-      // byte offsets of 32 bits: a particle takes over 2 KB of device memory, so all are below 2^27
-      cd.pj = *(const double4 *)((const char *)nl4 + (unsigned)cd.j * 32u);
+      // byte offsets of 32 bits up to 2^27 particles (neighbours_far): 64 bits cost 1M FP64 with PSE 0.79 ->
+      // 0.83 ms, 65k 63 -> 66 us
+      typedef std::conditional_t<FAR, uint64_t, unsigned> Offset;
+      cd.pj = *(const double4 *)((const char *)nl4 + (Offset)(unsigned)cd.j * 32u);
       cd.tr = make_double2(0., 1.);
-      if (PSE_MODE) cd.tr = *(const double2 *)((const char *)pse2 + (unsigned)cd.j * 16u);
+      if (PSE_MODE) cd.tr = *(const double2 *)((const char *)pse2 + (Offset)(unsigned)cd.j * 16u);
       return cd;
     };
     cell_lists<PSE_MODE>(s, e, T, lane, fetch, nl4, pse2, h, flags, c, nbr, cap, count,
@@ -488,7 +490,7 @@ __device__ __forceinline__ void cell_neighbours(
     stat_part[2 * (size_t)b + 1] = bb;
   }
 }
-template <int PSE_MODE>
+template <int PSE_MODE, bool FAR>
 __global__ void __launch_bounds__(NB_BLOCK)
     __attribute__((amdgpu_waves_per_eu(PSE_MODE == 1 ? NB_WAVES_FP64_PSE : NB_WAVES_OTHER)))
     k_cell_neighbours(unsigned first, GridInfo g, const int *__restrict__ off, const int *__restrict__ occ,
@@ -497,7 +499,7 @@ __global__ void __launch_bounds__(NB_BLOCK)
                       const uint32_t *__restrict__ flags, Consts c, int *__restrict__ nbr, int cap,
                       int *__restrict__ count, double *__restrict__ T_t, Counters *cnt,
                       unsigned long long *__restrict__ stat_part, int *__restrict__ poison) {
-  cell_neighbours<PSE_MODE>(first + blockIdx.x, g, off, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t, cnt,
+  cell_neighbours<PSE_MODE, FAR>(first + blockIdx.x, g, off, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t, cnt,
                             stat_part, poison);
 }
 
@@ -1830,6 +1832,7 @@ unsigned neighbour_blocks(const GridInfo &g, unsigned n_init) {
   const long cells = std::min<long>(g.num_cell, n_init);
   return (unsigned)((cells + 8 * NB_WAVES - 1) / (8 * NB_WAVES) * 8);
 }
+bool neighbours_far(unsigned n_init) { return n_init > 1u << 27; }
 static_assert((long)NB_MOST_BLOCKS * NB_BLOCK < 1L << 32, "a launch holds fewer than 2^32 threads");
 
 void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const int *offsets,
@@ -1838,11 +1841,15 @@ void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const 
                        const Consts &c, int *nbr, int cap, int *count, double *T_t, Counters *cnt,
                        int want_pse, unsigned long long *stat_part, int *poison) {
   const unsigned blocks = neighbour_blocks(g, n_init);
-  auto launch = [&](auto mode_c) {
+  auto launch_as = [&](auto mode_c, auto far_c) {
     for (unsigned first = 0; first < blocks; first += NB_MOST_BLOCKS)
-      hipLaunchKernelGGL((k_cell_neighbours<decltype(mode_c)::value>), dim3(std::min(blocks - first, NB_MOST_BLOCKS)),
-                         dim3(NB_BLOCK), 0, s, first, g, offsets, occ, nl4, pse2, h, flags, c, nbr, cap, count, T_t,
-                         cnt, stat_part, poison);
+      hipLaunchKernelGGL((k_cell_neighbours<decltype(mode_c)::value, decltype(far_c)::value>),
+                         dim3(std::min(blocks - first, NB_MOST_BLOCKS)), dim3(NB_BLOCK), 0, s, first, g, offsets, occ,
+                         nl4, pse2, h, flags, c, nbr, cap, count, T_t, cnt, stat_part, poison);
+  };
+  auto launch = [&](auto mode_c) {
+    if (neighbours_far(n_init)) launch_as(mode_c, std::true_type{});
+    else launch_as(mode_c, std::false_type{});
   };
   if (!want_pse) launch(std::integral_constant<int, 0>{});
   else if (c.precision == MFG_FP64) launch(std::integral_constant<int, 1>{});
@@ -1923,7 +1930,7 @@ void launch_pair(hipStream_t s, unsigned n_init, const State &st, const void *re
 // ---------------------------------------------------------------------------------------------
 // fewer waves per SIMD than the single-instance kernel (FP64 PSE 5, FP32 PSE 6, no PSE 7): the
 // instance lookup and descriptor take the registers that would otherwise spill
-template <int PSE_MODE>
+template <int PSE_MODE, bool FAR>
 __global__ void __launch_bounds__(NB_BLOCK)
     __attribute__((amdgpu_waves_per_eu(PSE_MODE == 1   ? NB_WAVES_FP64_PSE - 1
                                        : PSE_MODE == 2 ? NB_WAVES_OTHER - 2
@@ -1932,7 +1939,7 @@ __global__ void __launch_bounds__(NB_BLOCK)
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
   const State &st = d.buf[d.cur ^ 1];
-  cell_neighbours<PSE_MODE>(first + b, d.g, d.gb.count, d.gb.occ, d.nl4, d.pse2, st.h, st.flags, d.c, d.nbr,
+  cell_neighbours<PSE_MODE, FAR>(first + b, d.g, d.gb.count, d.gb.occ, d.nl4, d.pse2, st.h, st.flags, d.c, d.nbr,
                             d.nl_stride, d.count, st.T_t, d.cnt, nullptr, d.poison);
 }
 
@@ -1967,10 +1974,14 @@ __global__ void __launch_bounds__(BSP) kb_particle_update(const Inst *in, BatchM
 // run_neighbours picks it.  One Brookshaw instance selects the kernel with its sum for all: the
 // others' sums are the same in both.
 void launch_batch_pair(hipStream_t s, const BatchLaunch &L) {
-  auto neighbours = [&](auto mode_c) {
+  auto neighbours_as = [&](auto mode_c, auto far_c) {
     for (unsigned first = 0; first < L.nbr_blocks; first += L.nbr_most)
-      hipLaunchKernelGGL((kb_cell_neighbours<decltype(mode_c)::value>), dim3(L.nbrs8.blocks), dim3(NB_BLOCK), 0,
-                         s, L.inst, L.nbrs8.m, first);
+      hipLaunchKernelGGL((kb_cell_neighbours<decltype(mode_c)::value, decltype(far_c)::value>), dim3(L.nbrs8.blocks),
+                         dim3(NB_BLOCK), 0, s, L.inst, L.nbrs8.m, first);
+  };
+  auto neighbours = [&](auto mode_c) {
+    if (L.nbr_far) neighbours_as(mode_c, std::true_type{});
+    else neighbours_as(mode_c, std::false_type{});
   };
   if (!L.pse) neighbours(std::integral_constant<int, 0>{});
   else if (L.precision == MFG_FP64) neighbours(std::integral_constant<int, 1>{});

@@ -188,6 +188,7 @@ void launch_bbox_reduce(hipStream_t s, const State &st, const Counters *cnt, uns
 // occ: the occupied cells (GridBuffers)
 unsigned neighbour_blocks(const GridInfo &g, unsigned n_init);
 constexpr unsigned NB_MOST_BLOCKS = 1u << 24;  // of one launch
+bool neighbours_far(unsigned n_init);  // whether the candidate entries are beyond 32-bit offsets
 void launch_neighbours(hipStream_t s, unsigned n_init, const GridInfo &g, const int *offsets,
                        const int *occ, const double4 *nl4,
                        const double2 *pse2, const double *h, const uint32_t *flags,
@@ -337,6 +338,7 @@ struct BatchLaunch {
   BatchGrid pairs8;  // pair-pass workgroups, padded to a multiple of 8 (XCD-ordered kernels)
   BatchGrid nbrs8;   // neighbour-pass workgroups, padded to a multiple of 8
   unsigned nbr_blocks, nbr_most;  // the largest instance's, and how many of them one launch takes
+  int nbr_far;       // neighbours_far of an instance
   BatchGrid tools;   // one workgroup per tool (at least one per instance)
   BatchGrid search;  // lane-parallel contact search workgroups
 };

@@ -1,5 +1,6 @@
 """Sets beyond 32-bit offsets and launches: FP64 records of 192 bytes pass 4 GiB at 22.4M particles, FP32 records of
-112 at 38.3M; a wavefront for each of 67.1M occupied cells passes the 2^32 threads of a launch.
+112 at 38.3M, the neighbour pass's candidates of 32 bytes at 134.2M; a wavefront for each of 67.1M occupied cells
+passes the 2^32 threads of a launch.
 
 A cubic lattice of spacing 1 with a support between 1 and sqrt(2): every particle has its up to six lattice
 neighbours, visited in the same order everywhere, and the velocity field v = L x of constant L does not depend on
@@ -69,10 +70,10 @@ def test_records_beyond_4_gib(hip_device, precision, n1, form):
     check_planes(p, n1)
 
 
-@pytest.mark.parametrize("form", ["step", "batch"])
-def test_more_cells_than_a_launch_holds(hip_device, form):
-    """68.4M particles (409 a side) in 2.9 cells each."""
-    p, g = lattice(409, _lib.MFG_FP32_KAHAN)
+@pytest.mark.parametrize("n1,form", [(409, "step"), (409, "batch"), (513, "step"), (513, "batch")])
+def test_more_cells_than_a_launch_holds(hip_device, n1, form):
+    """68.4M particles (409 a side) in 3.3 cells each, and 135M, whose candidates are beyond 4 GiB."""
+    p, g = lattice(n1, _lib.MFG_FP32_KAHAN)
     api.pair_stats_enable(form == "step")
     try:
         if form == "batch":
@@ -81,7 +82,7 @@ def test_more_cells_than_a_launch_holds(hip_device, form):
             b.step()
         else:
             api.leap_frog(p.N_init, g.num_cell()).step(p, g)
-            assert p.pair_stats()[1] == 6 * 409 ** 2 * 408
-        check_planes(p, 409)
+            assert p.pair_stats()[1] == 6 * n1 ** 2 * (n1 - 1)
+        check_planes(p, n1)
     finally:
         api.pair_stats_enable(False)
