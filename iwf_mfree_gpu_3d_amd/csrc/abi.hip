@@ -75,6 +75,18 @@ struct Lib {
 Lib g_lib;
 thread_local std::string g_err;
 
+// Pinned memory of the downloads, made at mfg_init: two chunks, one filled by the device while the host
+// empties the other.  Downloads of several threads take turns.  512 KB a chunk: 72 MB into fresh memory 5.1
+// ms, with 1 to 8 MB 5.4 to 6.0.
+constexpr size_t STAGE_CHUNK = 512 * 1024;
+struct Stage {
+  std::mutex use;
+  char *mem = nullptr;
+  hipEvent_t done[2] = {nullptr, nullptr};
+  double *chunk(unsigned k) const { return (double *)(mem + (k & 1) * STAGE_CHUNK); }
+};
+Stage g_stage;
+
 // Work memory of the allocation-free step (mfg_leap_frog_step_noalloc): one array per GPU, held
 // until the process ends.  Host code never passes `scratch` itself to a kernel or copy (in host
 // code the name is a stand-in, not a device address); it uses the device address that mfg_init
@@ -216,9 +228,6 @@ struct mfg_particles {
   // leap-frog start-of-step copies (lazily allocated)
   double *vder = nullptr, *sder = nullptr, *nrm = nullptr, *x0 = nullptr;
   int *flag_d = nullptr;
-  double *stage = nullptr;  // pinned host buffer of small downloads (made by the first)
-  size_t stage_bytes = 0;
-  std::mutex stage_use;
   unsigned long long *stat_part = nullptr;  // per-workgroup (candidates, pairs) of the last list build
   int stat_cap = 0, stat_n = 0;
   // lane-parallel exhaustive contact search (lazily sized)
@@ -327,7 +336,6 @@ void free_particles(mfg_particles *p) {
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (p->cnt_h) (void)hipHostFree(p->cnt_h);
-  if (p->stage) (void)hipHostFree(p->stage);
 }
 
 int grid_alloc(mfg_grid *g) {
@@ -601,43 +609,32 @@ int check_counters(mfg_particles *p) {
   return counters_status(p);
 }
 
-// A field of every particle to host memory, interleaved by the device.  Fields of up to STAGE_BYTES:
-// the kernel writes them and the counters into the set's pinned buffer, one launch and one wait (a
-// copy command takes 60 us however small: 8,000 positions 394 -> 24 us; 1.4 MB of stresses 111 us this
-// way, 204 the other; 4.8 MB 327 and 375, too little for pinned memory of that size per set).  Larger ones go
-// through the pair-sum array (free between two calls: the pair pass writes it and the update of the
-// same call reads it) straight into the caller's memory.
-constexpr size_t STAGE_BYTES = (size_t)4 << 20;
+// A field of every particle to host memory, interleaved by the device: the kernel writes it into the
+// library's pinned chunks, the next chunk while the host copies one (a copy command takes 60 us however
+// small: 8,000 positions 394 -> 24 us; 24 MB into the caller's pageable memory 1.37 ms, 72 MB 6.7, so 0.83 and 5.0).  The
+// counters come with the first chunk; on an error of the queued steps nothing is written to `host`.
 int download_field(mfg_particles *p, const PackField &f, double *host) {
-  std::lock_guard<std::mutex> lock(p->stage_use);
+  std::lock_guard<std::mutex> lock(g_stage.use);
   hipStream_t s = g_lib.stream;
-  const size_t bytes = sizeof(double) * f.w * (size_t)p->N_init;
-  if (bytes <= STAGE_BYTES) {
-    if (bytes > p->stage_bytes) {
-      if (p->stage) (void)hipHostFree(p->stage);
-      p->stage = nullptr;
-      p->stage_bytes = 0;
-      const size_t want = std::min(STAGE_BYTES, sizeof(double) * 9 * (size_t)p->N_init);
-      HIP_TRY(hipHostMalloc(&p->stage, want));
-      p->stage_bytes = want;
+  const unsigned N = p->N_init, per = (unsigned)(STAGE_CHUNK / (sizeof(double) * f.w)), chunks = (N + per - 1) / per;
+  auto count = [&](unsigned k) { return std::min(per, N - k * per); };
+  for (unsigned k = 0; k <= chunks; k++) {
+    if (k < chunks) {
+      launch_pack_field(s, f, k * per, count(k), g_stage.chunk(k), k == 0 ? p->cnt : nullptr, p->cnt_h);
+      HIP_TRY(hipGetLastError());
+      HIP_TRY(hipEventRecord(g_stage.done[k & 1], s));
     }
-    launch_pack_field(s, f, p->N_init, p->stage, p->cnt, p->cnt_h);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));
-    const int rc = counters_status(p);
-    if (rc == MFG_OK) std::memcpy(host, p->stage, bytes);
-    return rc;
+    if (k == 0) continue;
+    HIP_TRY(hipEventSynchronize(g_stage.done[(k - 1) & 1]));
+    if (k == 1) {
+      const int rc = counters_status(p);
+      if (rc != MFG_OK) {
+        HIP_TRY(hipStreamSynchronize(s));  // the second chunk is the next caller's too
+        return rc;
+      }
+    }
+    std::memcpy(host + (size_t)(k - 1) * per * f.w, g_stage.chunk(k - 1), sizeof(double) * f.w * (size_t)count(k - 1));
   }
-  const void *dev = f.src[0];
-  if (f.w != 1 || f.kind != PACK_F64) {
-    launch_pack_field(s, f, p->N_init, p->sums, nullptr, nullptr);
-    HIP_TRY(hipGetLastError());
-    dev = p->sums;
-  }
-  const int rc = check_counters(p);
-  if (rc != MFG_OK) return rc;
-  HIP_TRY(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
   return MFG_OK;
 }
 
@@ -804,6 +801,9 @@ int mfg_init(int device) {
     if (!ptr) return fail(MFG_ERR_HIP, "no device address for the step's work memory");
     g_scratch = (unsigned char *)ptr;
   }
+  HIP_TRY(hipHostMalloc(&g_stage.mem, 2 * STAGE_CHUNK));
+  for (hipEvent_t &e : g_stage.done)
+    HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem));
   const char *lane_contact = std::getenv("MFG_LANE_CONTACT");
   g_lib.opt_contact_search = !(lane_contact && lane_contact[0] == '0');
   g_lib.device = device;

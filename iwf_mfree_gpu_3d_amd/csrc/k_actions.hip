@@ -239,13 +239,13 @@ __global__ void __launch_bounds__(BA) k_act_sums(State st, const Counters *cnt, 
 // One thread per element of the host's layout.  The host-side interleave that it replaces went over the
 // field once per component (S at 1M particles: 14.5 ms, now the copy's 5).
 template <int W>
-__global__ void __launch_bounds__(BA) k_pack_field(PackField f, unsigned n, double *out,
+__global__ void __launch_bounds__(BA) k_pack_field(PackField f, unsigned first, unsigned n, double *out,
                                                    const Counters *cnt, Counters *cnt_h) {
   if (cnt && blockIdx.x == 0 && threadIdx.x == 0) *cnt_h = *cnt;
   const size_t e = (size_t)blockIdx.x * BA + threadIdx.x;
   if (e >= (size_t)n * W) return;
-  const unsigned i = (unsigned)(e / W);
-  const int k = (int)(e - (size_t)i * W);
+  const unsigned q0 = (unsigned)(e / W), i = first + q0;
+  const int k = (int)(e - (size_t)q0 * W);
   const void *src = f.src[0];
 #pragma unroll
   for (int q = 1; q < W; q++) src = k == q ? f.src[q] : src;
@@ -324,12 +324,12 @@ void launch_act_sums(hipStream_t s, const State &st, unsigned n_init, const Coun
                      poison);
 }
 
-void launch_pack_field(hipStream_t s, const PackField &f, unsigned n, double *out, const Counters *cnt,
-                       Counters *cnt_h) {
+void launch_pack_field(hipStream_t s, const PackField &f, unsigned first, unsigned n, double *out,
+                       const Counters *cnt, Counters *cnt_h) {
   const dim3 g(nba((long)n * f.w)), b(BA);
-  if (f.w == 1) hipLaunchKernelGGL(k_pack_field<1>, g, b, 0, s, f, n, out, cnt, cnt_h);
-  else if (f.w == 3) hipLaunchKernelGGL(k_pack_field<3>, g, b, 0, s, f, n, out, cnt, cnt_h);
-  else hipLaunchKernelGGL(k_pack_field<9>, g, b, 0, s, f, n, out, cnt, cnt_h);
+  if (f.w == 1) hipLaunchKernelGGL(k_pack_field<1>, g, b, 0, s, f, first, n, out, cnt, cnt_h);
+  else if (f.w == 3) hipLaunchKernelGGL(k_pack_field<3>, g, b, 0, s, f, first, n, out, cnt, cnt_h);
+  else hipLaunchKernelGGL(k_pack_field<9>, g, b, 0, s, f, first, n, out, cnt, cnt_h);
 }
 
 void launch_words_to_host(hipStream_t s, const void *src, void *pinned, unsigned n_words) {

@@ -220,9 +220,10 @@ struct PackField {
   const void *src[9];
   int w, kind;
 };
-// out may be pinned host memory; cnt, if given, goes to cnt_h (pinned) in the same launch
-void launch_pack_field(hipStream_t s, const PackField &f, unsigned n, double *out, const Counters *cnt,
-                       Counters *cnt_h);
+// n particles from `first` on; out may be pinned host memory; cnt, if given, goes to cnt_h (pinned) in the
+// same launch
+void launch_pack_field(hipStream_t s, const PackField &f, unsigned first, unsigned n, double *out,
+                       const Counters *cnt, Counters *cnt_h);
 // a few words to pinned host memory: a kernel's store arrives in 6 us, a copy command's in 60
 void launch_words_to_host(hipStream_t s, const void *src, void *pinned, unsigned n_words);
 
