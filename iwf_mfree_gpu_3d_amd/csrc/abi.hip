@@ -254,7 +254,7 @@ struct mfg_grid {
   long nx = 0, ny = 0, nz = 0, num_cell = 0, max_cell = 0;
   int *count = nullptr;  // max_cell + 1: counts, then offsets
   int *hist = nullptr;
-  int *occ = nullptr;
+  int *occ = nullptr;    // in hist's allocation
   unsigned long long *parts = nullptr;
   int nparts_cap = 0;
   double *bbox_part = nullptr;
@@ -299,8 +299,6 @@ struct mfg_tool {
 struct mfg_tool_forces {
   unsigned n = 0;
   float *d = nullptr;
-  float *h = nullptr;  // pinned, what get_host reads
-  std::mutex h_use;
 };
 
 struct mfg_leap_frog {
@@ -340,11 +338,12 @@ void free_particles(mfg_particles *p) {
 
 int grid_alloc(mfg_grid *g) {
   HIP_TRY(hipMalloc(&g->count, sizeof(int) * (g->max_cell + 1)));
-  HIP_TRY(hipMalloc(&g->occ, sizeof(int) * (g->max_cell + 1)));
-  HIP_TRY(hipMemsetAsync(g->occ, 0, sizeof(int) * (g->max_cell + 1), g_lib.stream));  // none before a sort
-  HIP_TRY(hipMalloc(&g->hist, sizeof(int) * (g->max_cell + 1)));
-  HIP_TRY(hipMemsetAsync(g->hist, 0, sizeof(int) * (g->max_cell + 1), g_lib.stream));
-  HIP_TRY(hipStreamSynchronize(g_lib.stream));  // a sort may run on a stream set later
+  // no particles counted and no cells occupied before a sort; one array, cleared and waited for at once (a
+  // sort may run on a stream set later)
+  HIP_TRY(hipMalloc(&g->hist, 2 * sizeof(int) * (g->max_cell + 1)));
+  g->occ = g->hist + g->max_cell + 1;
+  HIP_TRY(hipMemsetAsync(g->hist, 0, 2 * sizeof(int) * (g->max_cell + 1), g_lib.stream));
+  HIP_TRY(hipStreamSynchronize(g_lib.stream));
   g->nparts_cap = scan_tiles(g->max_cell, false) + 1;
   HIP_TRY(hipMalloc(&g->parts, sizeof(unsigned long long) * g->nparts_cap));
   HIP_TRY(hipMalloc(&g->bbox_part, sizeof(double) * 7 * 1024));
@@ -1359,7 +1358,7 @@ int mfg_grid_create_unlocked(int kind, long max_cell, int num_part, mfg_grid **o
 int mfg_grid_destroy(mfg_grid *g) {
   if (!g) return MFG_OK;
   if (g_lib.ready) (void)hipStreamSynchronize(g_lib.stream);
-  void *ptrs[] = {g->count, g->hist, g->occ, g->parts, g->bbox_part};
+  void *ptrs[] = {g->count, g->hist, g->parts, g->bbox_part};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   delete g;
@@ -1754,9 +1753,8 @@ int mfg_tool_forces_create(unsigned n, mfg_tool_forces **out) {
   if (!out || n == 0 || n > MAX_TOOLS) return fail(MFG_ERR_ARG, "tool forces for %u tools (max %d)", n, MAX_TOOLS);
   mfg_tool_forces *f = new mfg_tool_forces();
   f->n = n;
-  if (hipMalloc(&f->d, sizeof(float) * 3 * n) != hipSuccess ||
-      hipHostMalloc(&f->h, sizeof(float) * 3 * n) != hipSuccess) {
-    mfg_tool_forces_destroy(f);
+  if (hipMalloc(&f->d, sizeof(float) * 3 * n) != hipSuccess) {
+    delete f;
     return fail(MFG_ERR_NOMEM, "tool forces");
   }
   (void)hipMemsetAsync(f->d, 0, sizeof(float) * 3 * n, g_lib.stream);
@@ -1766,7 +1764,6 @@ int mfg_tool_forces_create(unsigned n, mfg_tool_forces **out) {
 int mfg_tool_forces_destroy(mfg_tool_forces *f) {
   if (!f) return MFG_OK;
   if (f->d) (void)hipFree(f->d);
-  if (f->h) (void)hipHostFree(f->h);
   delete f;
   return MFG_OK;
 }
@@ -1779,11 +1776,11 @@ int mfg_tool_forces_reset(mfg_tool_forces *f) {
 int mfg_tool_forces_get_host(mfg_tool_forces *f, float *xyz) {
   NEED_LIB();
   if (!f || !xyz) return fail(MFG_ERR_ARG, "null argument");
-  std::lock_guard<std::mutex> lock(f->h_use);
-  launch_words_to_host(g_lib.stream, f->d, f->h, 3 * f->n);
+  std::lock_guard<std::mutex> lock(g_stage.use);
+  launch_words_to_host(g_lib.stream, f->d, g_stage.chunk(0), 3 * f->n);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(g_lib.stream));
-  std::memcpy(xyz, f->h, sizeof(float) * 3 * f->n);
+  std::memcpy(xyz, g_stage.chunk(0), sizeof(float) * 3 * f->n);
   return MFG_OK;
 }
 
