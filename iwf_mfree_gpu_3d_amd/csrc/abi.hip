@@ -1160,7 +1160,11 @@ int mfg_particle_gpu_download(mfg_particles *p, int f, double *host) {
   const size_t n = padded(N);
   const State &st = p->st();
   hipStream_t s = g_lib.stream;
-  // errors of the queued steps surface here too
+  // errors of the queued steps surface here too, before an array that is missing
+  auto missing = [&](const char *what) {
+    const int rc = check_counters(p);
+    return rc != MFG_OK ? rc : fail(MFG_ERR_STATE, "%s", what);
+  };
   auto put1 = [&](const double *x) { return download_field(p, PackField{{x}, 1, PACK_F64}, host); };
   auto put3 = [&](const double *x, const double *y, const double *z) {
     return download_field(p, PackField{{x, y, z}, 3, PACK_F64}, host);
@@ -1196,25 +1200,21 @@ int mfg_particle_gpu_download(mfg_particles *p, int f, double *host) {
     case MFG_F_IDX: return put_u(p->order, PACK_I32);
     case MFG_F_S_DER:
     case MFG_F_V_DER: {
-      const int rc = check_counters(p);
-      if (rc != MFG_OK) return rc;
       const double *m = f == MFG_F_V_DER ? p->vder : p->sder;
-      if (!m) return fail(MFG_ERR_STATE, "no velocity gradient / stress divergence yet (interactions_monaghan computes them)");
+      if (!m)
+        return missing("no velocity gradient / stress divergence yet (interactions_monaghan computes them)");
       PackField pf{{}, 9, PACK_F64};
       for (int k = 0; k < 9; k++) pf.src[k] = m + k * n;
       return download_field(p, pf, host);
     }
-    case MFG_F_N: {
-      const int rc = check_counters(p);
-      if (rc != MFG_OK) return rc;
-      if (!p->nrm) return fail(MFG_ERR_STATE, "no contact normals yet (tool compute_contact_force writes them)");
+    case MFG_F_N:
+      if (!p->nrm) return missing("no contact normals yet (tool compute_contact_force writes them)");
       return put3(p->nrm, p->nrm + n, p->nrm + 2 * n);
-    }
     case MFG_F_P:
     case MFG_F_R: {
-      const int rc = check_counters(p);
-      if (rc != MFG_OK) return rc;
       if (!p->p_dbg) {
+        const int rc = check_counters(p);
+        if (rc != MFG_OK) return rc;
         // pressure and artificial stress live in the pair records; keep copies from now on
         if (hipMalloc(&p->p_dbg, sizeof(double) * n) != hipSuccess ||
             hipMalloc(&p->R_dbg, sizeof(double) * 6 * n) != hipSuccess)
