@@ -2,15 +2,15 @@
 
 Every choice offered leaves results bit-identical, so the tuner only measures time:
 - the pair pass's visiting order (strip width in grid columns, or the sorted order);
-- a cell tile (1, 2, 4, 8, 16), kept for tables made before: the neighbour pass takes the occupied
-  cells, and every tile runs the same;
+- a cell tile (1, 2, 4, 8, 16), kept for tables made before and for measures of the caller's own: the
+  library takes the occupied cells and runs every tile alike, so its own runs do not try them;
 - the pair pass's workgroup size (64, 128, 256 threads): every wavefront works alone, and
   smaller workgroups spread a small instance over more compute units.
 
 For instances on a stream pool (serve mode "streams"), `tune` picks per (bucket, precision) the
-visiting order first, then the cell tile with them, then the pair pass's workgroup size.  For batches (serve mode "batched") the cell
-tile is a property of the whole launch: `tune_batched` measures a throwaway batch of the first
-requests of each precision with every tile.
+visiting order first, then the pair pass's workgroup size with it.  For batches (serve mode "batched") the
+cell tile was the only choice of the whole launch: `tune_batched` has nothing left to measure, unless a
+measure of the caller's is given.
 
 The re-sort interval is offered only when the caller opts in (`sort_intervals`): the reference
 rebuilds its cell lists from a fresh sort every step (src/leap_frog.cu:139-145), and sorting on
@@ -121,13 +121,19 @@ def measure(req, candidate: tuple, steps: int = 6, warmup: int = 2) -> float:
         gc.collect()
 
 
-def tune(requests, candidates=CANDIDATES, tiles=TILES, steps: int = 6, warmup: int = 2, measure=measure,
+_own_runs = measure
+
+
+def tune(requests, candidates=CANDIDATES, tiles=None, steps: int = 6, warmup: int = 2, measure=measure,
          log=None, sort_intervals=(), blocks=BLOCKS) -> Table:
     """One representative request per (bucket, precision) among `requests` (the first seen):
     every form / order candidate measured on it with the automatic cell tile, then every cell
     tile with the fastest of those, then every pair-pass workgroup size, then (opt-in, results
     change) every re-sort interval in `sort_intervals` with the fastest of all the others; ties
-    go to the earlier candidate."""
+    go to the earlier candidate.  `tiles`: by default none for the library's own runs, whose times
+    would differ by noise alone, and TILES for another `measure`."""
+    if tiles is None:
+        tiles = () if measure is _own_runs else TILES
     table = Table()
     reps = {}
     for r in requests:
@@ -193,11 +199,19 @@ def measure_batch(requests, tile: int, steps: int = 4, warmup: int = 2) -> float
         gc.collect()
 
 
-def tune_batched(requests, tiles=TILES, sample: int = 16, steps: int = 4, warmup: int = 2,
+_own_batches = measure_batch
+
+
+def tune_batched(requests, tiles=None, sample: int = 16, steps: int = 4, warmup: int = 2,
                  measure=measure_batch, log=None, table: Table | None = None) -> Table:
     """The cell tile of each precision's batch: the first `sample` requests of the precision as a
-    throwaway batch, measured with every tile (ties: the smaller tile)."""
+    throwaway batch, measured with every tile (ties: the smaller tile).  `tiles` as in `tune`:
+    by default the library's own runs measure none and leave the table as it is."""
+    if tiles is None:
+        tiles = () if measure is _own_batches else TILES
     table = table or Table()
+    if not tiles:
+        return table
     by_prec = {}
     for r in requests:
         by_prec.setdefault(r.precision, []).append(r)

@@ -2201,7 +2201,6 @@ struct mfg_batch {
   };
   std::vector<Member> members;
   int precision = -1, pse = -1;
-  int cell_tile = 0;   // accepted, without effect
   bool dirty = true;   // the device descriptors and maps must be rebuilt before the next step
   int table_record = -1;
   Inst *d_inst = nullptr;
@@ -2552,7 +2551,6 @@ int mfg_batch_set_cell_tile(mfg_batch *b, int cell_tile) {
   if (cell_tile != 0 && cell_tile != 1 && cell_tile != 2 && cell_tile != 4 && cell_tile != 8 &&
       cell_tile != 16)
     return fail(MFG_ERR_ARG, "cell tile %d (0, 1, 2, 4, 8 or 16)", cell_tile);
-  b->cell_tile = cell_tile;
   return MFG_OK;
 }
 
