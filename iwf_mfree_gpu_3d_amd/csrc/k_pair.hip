@@ -1701,7 +1701,8 @@ __device__ __forceinline__ void pair_rows(unsigned b, unsigned nb, unsigned n_in
   char *area = s_area[w];
   if (c.cspm && steps > 0) {
     const EntryGather<FAR> g(cs4, n_init, lane);
-    // the wide sums' terms have always been rounded so for all but every fourth neighbour
+    // No numerical reason (either order errs alike): the one-lane kernel's unrolled walk rounded the terms so for
+    // all but every fourth neighbour, and results are to keep their bits (tests/golden/wide_pair_sums.npz)
     const bool x_first = std::is_same<Acc, AccWide>::value && (n & 3) != 0;
     Acc a2[NB], a1[1];  // B[L q + n] and, in every group, B[8]
 #pragma unroll
