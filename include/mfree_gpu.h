@@ -196,6 +196,8 @@ int mfg_particle_gpu_destroy(mfg_particles *p);
 /* host view of particle_gpu::N / N_init (synchronises) */
 int mfg_particle_gpu_counts(mfg_particles *p, unsigned *N, unsigned *N_init);
 int mfg_particle_gpu_precision(const mfg_particles *p);
+/* waits for the queued steps; nothing is written on an error.  Downloads of several threads take turns; one beside
+ * a thread that steps the set does not disturb the step */
 int mfg_particle_gpu_download(mfg_particles *p, int field, double *host);
 int mfg_particle_gpu_upload(mfg_particles *p, int field, const double *host);
 /* No counterpart in the reference (its particle_gpu lives as long as the process): a snapshot of

@@ -1317,7 +1317,9 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 // (src/interactions_gpu.cu:152-471).  An unlocked grid takes its origin and cell size from the
 // particles, to the last bit of the outermost position, so there the positions of every step must
 // round as the reference's do for its cell tables to be the reference's; the sums above differ from
-// these in the last bits.  On a locked grid nothing depends on those bits.
+// these in the last bits.  On a locked grid nothing depends on those bits.  B is summed from the records'
+// first 64-byte lines: from 32-byte entries of its own the pass took 3 % less (1M 1.98 against 1.92 ms, a step
+// 3.19 ms against 3.65 with the neighbour pass and the sort of that time).
 struct PairOrdered64 {
   Rec64 ri;
   bool tool_i, tool_nz, brook;
@@ -1509,8 +1511,8 @@ __global__ void __launch_bounds__(BS, PAIR_WAVES)
 // instructions), and every lane then adds the L neighbours' terms of its own share of the sums, in list
 // order.
 //
-// Against one lane per particle, the same sums to the bit: 19,000 particles 137 -> 59 us (300 wavefronts
-// of 100 steps, now 1,200 of 26), 255k with wide sums 396 -> 324 us, 1M 1.35 -> 1.23 ms.  At 1M the
+// Against one lane per particle, the same sums to the bit: 19,000 particles 137 -> 50 us (300 wavefronts
+// of 100 steps, now 2,400 of 13; with four lanes 59), 255k with wide sums 396 -> 324 us, 1M 1.35 -> 1.23 ms.  At 1M the
 // vector units are full: 424 instructions per 64 pairs, the exchanges and the transcendentals counting
 // double and fourfold; one lane per particle needs 345 but runs at the pace of its list reads (each
 // lane walks its own row: 1.42 ms).  115 registers: four waves per SIMD (three: 1.25 ms; five spill).

@@ -1,8 +1,8 @@
 // mfg_device.hpp -- per-particle device math of the SPH cutting step (FP64 unless noted).
 //
-// The files are compiled with -ffp-contract=off: every expression rounds exactly as written, so
-// the FP64 path evaluates the reference formulas in the reference's operation order; fused
-// multiply-adds are only used where they are spelled out (the pair sums and the PSE exponential).
+// The files are compiled with -ffp-contract=off: every expression rounds exactly as written, in the
+// reference's operation order but for the pair sums of locked grids (one walk, B^-1 at the end, over 4 or
+// 16 lanes) and the PSE sum, where fused multiply-adds and reciprocals are spelled out.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -13,8 +13,8 @@
 //   neighbour list: int32 nbr[i * cap + k] (row-major), count[i]
 //   neighbour sums: 25 doubles per particle (SoA), written by the pair pass and read by the
 //     per-particle update
-//   grid: key[N_init] (unsorted), key_sorted[N_init], order[N_init], cell counts / offsets
-//         [num_cell + 1], fill counters [num_cell]
+//   grid: key[N_init] (unsorted), key_sorted[N_init], order[N_init], cell offsets [num_cell + 1], counts of
+//         the sort under way [num_cell], list of the occupied cells [num_cell + 1]
 #pragma once
 
 #include <hip/hip_runtime.h>

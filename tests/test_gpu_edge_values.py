@@ -38,15 +38,18 @@ def spoil(sc, what):
 
 @pytest.mark.parametrize("what", ["negative density", "no smoothing length", "NaN smoothing length"])
 @pytest.mark.parametrize("scale", [0.5, 1.0])  # about 1,000 and 8,000 particles: either lane count of the pair pass
-@pytest.mark.parametrize("precision,tol", [(_lib.MFG_FP64, 1e-11), (_lib.MFG_FP32_KAHAN, 1e-4), (_lib.MFG_FP32_WIDE, 1e-4)],
-                         ids=["fp64", "kahan", "wide"])
-def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, tol, scale, what):
+@pytest.mark.parametrize("precision,locked,tol", [(_lib.MFG_FP64, True, 1e-11), (_lib.MFG_FP64, False, 1e-11),
+                                                  (_lib.MFG_FP32_KAHAN, True, 1e-4), (_lib.MFG_FP32_WIDE, True, 1e-4)],
+                         ids=["fp64", "fp64_unlocked", "kahan", "wide"])
+def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, locked, tol, scale, what):
     sc = perturbed_scene(1, scale, 7)
     ks = spoil(sc, what)
     sim = helpers.oracle_from_scene(sc)
     dt = sc.params.dt
     sim.set_time(dt, dt)
     parts, grid = scenes.setup_cut(sc, precision=precision, max_neighbours=1024)  # a whole stencil
+    if not locked:
+        grid = api.grid_gpu_green(4 * grid.num_cell() + 1000, sc.n)
     api.global_time_current = dt
     assert sim.run(1) == 0
     scenes.run(api.leap_frog(sc.n, grid.num_cell()), parts, grid, 1)
