@@ -345,7 +345,7 @@ int grid_alloc(mfg_grid *g) {
   HIP_TRY(hipMemsetAsync(g->hist, 0, 2 * sizeof(int) * (g->max_cell + 1), g_lib.stream));
   HIP_TRY(hipStreamSynchronize(g_lib.stream));
   g->nparts_cap = scan_tiles(g->max_cell, false) + 1;
-  HIP_TRY(hipMalloc(&g->parts, sizeof(unsigned long long) * g->nparts_cap));
+  HIP_TRY(hipMalloc(&g->parts, sizeof(unsigned long long) * (g->nparts_cap + g->nparts_cap / PREFIX_CHUNK + 1)));
   HIP_TRY(hipMalloc(&g->bbox_part, sizeof(double) * 7 * 1024));
   g->bbox_host.assign(7 * 1024, 0.);
   return MFG_OK;
@@ -371,6 +371,9 @@ GridBuffers grid_buffers(mfg_grid *g, mfg_particles *p) {
   gb.scattered = p->trav;
   gb.blk = p->blk;
   gb.blk2 = g->parts;
+  const int tiles = g->num_cell > SCAN_ALONE ? scan_tiles(g->num_cell, false) : 0;
+  gb.blk_chunk = p->nblk >= PREFIX_CHUNKS ? p->blk + p->nblk : nullptr;
+  gb.part_chunk = tiles >= PREFIX_CHUNKS ? g->parts + g->nparts_cap : nullptr;
   gb.nblk = p->nblk;
   return gb;
 }
@@ -992,7 +995,7 @@ int mfg_particle_gpu_create(unsigned N, const double *pos4, const double *vel4, 
       hipMalloc(&p->count, sizeof(int) * n) != hipSuccess || hipMalloc(&p->key, sizeof(int) * n) != hipSuccess ||
       hipMalloc(&p->key_sorted, sizeof(int) * n) != hipSuccess ||
       hipMalloc(&p->order, sizeof(int) * n) != hipSuccess ||
-      hipMalloc(&p->blk, sizeof(int) * (p->nblk + 1)) != hipSuccess ||
+      hipMalloc(&p->blk, sizeof(int) * (p->nblk + p->nblk / PREFIX_CHUNK + 1)) != hipSuccess ||
       hipMalloc(&p->cnt, sizeof(Counters)) != hipSuccess ||
       hipMalloc(&p->partials, sizeof(float) * MAX_TOOLS * 3 * p->contact_blocks) != hipSuccess ||
       hipMalloc(&p->flag_d, sizeof(int)) != hipSuccess ||
@@ -2369,9 +2372,11 @@ int batch_build(mfg_batch *b, int record) {
     b->L.pair_far |= pair_far(b->precision, m.p->N_init);
     b->L.nbr_far |= neighbours_far(m.p->N_init);
   }
+  b->L.sort_chunks = 0;
   for (int i = 0; i < n; i++) {
     const mfg_batch::Member &m = b->members[i];
     host[i] = batch_inst(m, record);
+    b->L.sort_chunks |= host[i].gb.blk_chunk || host[i].gb.part_chunk;
     host[i].ordered = b->L.ordered;
     const GridInfo gi = m.g->info();
     const unsigned nblk = (unsigned)m.p->nblk;

@@ -153,6 +153,35 @@ __device__ __forceinline__ void load_items(const int *a, long k, long n, int (&v
   }
 }
 
+// Block sums of a sort: a workgroup's base is the sum of those of all workgroups before it, which each adds
+// up itself.  From PREFIX_CHUNKS of them on also sums over PREFIX_CHUNK of them each are made (one workgroup of
+// CS_NT threads for both arrays), which keeps that linear: 68M particles of which every tenth is blanked 8.5 -> 0.5
+// ms of scatter, 549M cells 10.0 -> 1.6 ms of scan; 8M without blanked particles 6 us more.
+constexpr int CS_NT = 1024;
+template <class T>
+__device__ __forceinline__ void chunk_sums(const T *a, unsigned n, T *chunk) {
+  const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6, chunks = n / PREFIX_CHUNK;  // whole ones
+  for (unsigned c = w; c < chunks; c += CS_NT / 64) {
+    T s = 0;
+#pragma unroll
+    for (unsigned q = 0; q < PREFIX_CHUNK; q += 64) s += a[(size_t)c * PREFIX_CHUNK + q + lane];
+    s = wave_incl_scan(s);
+    if (lane == 63) chunk[c] = s;
+  }
+}
+// this thread's share of the sum of a[0 .. b) among NT
+template <int NT, class T>
+__device__ __forceinline__ T sum_before(const T *a, const T *chunk, unsigned b) {
+  T s = 0;
+  unsigned first = 0;
+  if (chunk) {
+    for (unsigned k = threadIdx.x; k < b / PREFIX_CHUNK; k += NT) s += chunk[k];
+    first = b / PREFIX_CHUNK * PREFIX_CHUNK;
+  }
+  for (unsigned k = first + threadIdx.x; k < b; k += NT) s += a[k];
+  return s;
+}
+
 // Particles in the low and occupied cells in the high 32 bits: one scan gives both the offsets and the
 // occupied cells' places in their list
 typedef unsigned long long CellSum;
@@ -176,21 +205,28 @@ __global__ void __launch_bounds__(BS) k_scan_reduce(const int *hist, long n, Cel
   scan_reduce(blockIdx.x, hist, n, part);
 }
 
+// the chunk sums that a sort needs
+__device__ __forceinline__ void sort_chunks(const GridBuffers &gb, unsigned tiles) {
+  if (gb.part_chunk) chunk_sums(gb.blk2, tiles, gb.part_chunk);
+  if (gb.blk_chunk) chunk_sums(gb.blk, (unsigned)gb.nblk, gb.blk_chunk);
+}
+__global__ void __launch_bounds__(CS_NT) k_sort_chunks(GridBuffers gb, unsigned tiles) { sort_chunks(gb, tiles); }
+
 // The offsets of tile b's cells (NT threads, ITEMS cells each), its occupied cells in the list of all
 // (ascending; occ[n]: how many), and with the last tile the totals.  A tile's base is the sum of all
 // before it: of the tile sums, or without them (part null: SCAN_ALONE) of the counts themselves, eight
 // loads of a thread in flight (26,000 cells: 8.4 us, 62,000: 9.3, of which the list of occupied cells
 // 1.8; in two launches 4.6 and 4.8, the gap between them, and the list).
 template <int NT, int ITEMS>
-__device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, const CellSum *part, int *off,
-                                           int *occ, unsigned n_init, Counters *cnt) {
+__device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, const CellSum *part,
+                                           const CellSum *chunk, int *off, int *occ, unsigned n_init, Counters *cnt) {
   __shared__ CellSum lds[NT / 64 + 1];
   const long base = ((long)b * NT + threadIdx.x) * ITEMS;
   int v[ITEMS];
   CellSum s = 0, before = 0, total, prefix;
   load_items<ITEMS>(hist, base, n, v);
   if (part) {
-    for (unsigned k = threadIdx.x; k < b; k += NT) before += part[k];
+    before = sum_before<NT>(part, chunk, b);
   } else {
     // b tiles of NT x ITEMS counts: ITEMS / 4 vectors a thread and tile
     const int4 *h = (const int4 *)hist + threadIdx.x;
@@ -230,16 +266,16 @@ __device__ __forceinline__ void scan_cells(unsigned b, const int *hist, long n, 
   }
 }
 template <int NT, int ITEMS>
-__global__ void __launch_bounds__(NT) k_scan_cells(const int *hist, long n, const CellSum *part, int *off,
-                                                   int *occ, unsigned n_init, Counters *cnt) {
-  scan_cells<NT, ITEMS>(blockIdx.x, hist, n, part, off, occ, n_init, cnt);
+__global__ void __launch_bounds__(NT) k_scan_cells(const int *hist, long n, const CellSum *part, const CellSum *chunk,
+                                                   int *off, int *occ, unsigned n_init, Counters *cnt) {
+  scan_cells<NT, ITEMS>(blockIdx.x, hist, n, part, chunk, off, occ, n_init, cnt);
 }
 
 // particles to their cells (order: an INT_MAX key's particle at its final place, the others in any
 // order within their cell), and the counts back to zero
 __device__ __forceinline__ void scatter(unsigned b, unsigned nb, unsigned n_init, long num_cell, const int *key,
                                         const int *off, const int *slot, int *hist, const int *blk,
-                                        const Counters *cnt, int *order) {
+                                        const int *chunk, const Counters *cnt, int *order) {
   __shared__ int lds[BS / 64 + 1];
   const unsigned i = b * BS + threadIdx.x;
   const int k = (i < n_init) ? key[i] : 0;
@@ -247,18 +283,17 @@ __device__ __forceinline__ void scatter(unsigned b, unsigned nb, unsigned n_init
   int total;
   const int rank = block_excl_scan<BS>(is_blank, lds, total);
   if (total > 0) {
-    int before = 0, prefix;
-    for (unsigned q = threadIdx.x; q < b; q += BS) before += blk[q];
-    block_excl_scan<BS>(before, lds, prefix);
+    int prefix;
+    block_excl_scan<BS>(sum_before<BS>(blk, chunk, b), lds, prefix);
     if (is_blank) order[(int)cnt->N + prefix + rank] = (int)i;
   }
   if (i < n_init && !is_blank) order[off[k] + slot[i]] = (int)i;
   for (long c = (long)i; c < num_cell; c += (long)nb * BS) hist[c] = 0;
 }
 __global__ void __launch_bounds__(BS) k_scatter(unsigned n_init, long num_cell, const int *key, const int *off,
-                                                const int *slot, int *hist, const int *blk,
+                                                const int *slot, int *hist, const int *blk, const int *chunk,
                                                 const Counters *cnt, int *order) {
-  scatter(blockIdx.x, gridDim.x, n_init, num_cell, key, off, slot, hist, blk, cnt, order);
+  scatter(blockIdx.x, gridDim.x, n_init, num_cell, key, off, slot, hist, blk, chunk, cnt, order);
 }
 
 // The place of the particle at scattered position t: by previous index among its cell's.
@@ -456,20 +491,21 @@ void launch_scan_cells(hipStream_t s, const GridInfo &g, GridBuffers &gb, unsign
                        Counters *cnt) {
   const bool alone = g.num_cell <= SCAN_ALONE;
   const dim3 tiles((unsigned)scan_tiles(g.num_cell, alone));
+  if (!alone) hipLaunchKernelGGL(k_scan_reduce, tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2);
+  if (gb.part_chunk || gb.blk_chunk) hipLaunchKernelGGL(k_sort_chunks, dim3(1), dim3(CS_NT), 0, s, gb, tiles.x);
   if (alone) {
     hipLaunchKernelGGL((k_scan_cells<SCAN_NT, SCAN_TILE_ALONE / SCAN_NT>), tiles, dim3(SCAN_NT), 0, s, gb.hist, g.num_cell,
-                       (const CellSum *)nullptr, gb.count, gb.occ, n_init, cnt);
+                       (const CellSum *)nullptr, (const CellSum *)nullptr, gb.count, gb.occ, n_init, cnt);
     return;
   }
-  hipLaunchKernelGGL(k_scan_reduce, tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2);
   hipLaunchKernelGGL((k_scan_cells<BS, SCAN_ITEMS>), tiles, dim3(BS), 0, s, gb.hist, g.num_cell, gb.blk2,
-                     gb.count, gb.occ, n_init, cnt);
+                     gb.part_chunk, gb.count, gb.occ, n_init, cnt);
 }
 
 void launch_scatter(hipStream_t s, unsigned n_init, const GridInfo &g, GridBuffers &gb,
                     Counters *cnt) {
   hipLaunchKernelGGL(k_scatter, dim3(gb.nblk), dim3(BS), 0, s, n_init, g.num_cell, gb.key, gb.count,
-                     gb.order, gb.hist, gb.blk, cnt, gb.scattered);
+                     gb.order, gb.hist, gb.blk, gb.blk_chunk, cnt, gb.scattered);
 }
 
 void launch_order(hipStream_t s, unsigned n_init, GridBuffers &gb) {
@@ -520,19 +556,25 @@ __global__ void __launch_bounds__(BS) kb_scan_reduce(const Inst *in, BatchMap m)
   scan_reduce(b, d.gb.hist, d.g.num_cell, d.gb.blk2);
 }
 
+__global__ void __launch_bounds__(CS_NT) kb_sort_chunks(const Inst *in, BatchMap m) {
+  unsigned b, nb;
+  const Inst &d = in[batch_locate(m, b, nb)];
+  sort_chunks(d.gb, (unsigned)((d.g.num_cell + SCAN_TILE - 1) / SCAN_TILE));
+}
+
 template <int NT, int ITEMS>
 __global__ void __launch_bounds__(NT) kb_scan_cells(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  scan_cells<NT, ITEMS>(b, d.gb.hist, d.g.num_cell, NT == BS ? d.gb.blk2 : nullptr, d.gb.count, d.gb.occ,
-                        d.n_init, d.cnt);
+  scan_cells<NT, ITEMS>(b, d.gb.hist, d.g.num_cell, NT == BS ? d.gb.blk2 : nullptr, d.gb.part_chunk, d.gb.count,
+                        d.gb.occ, d.n_init, d.cnt);
 }
 
 __global__ void __launch_bounds__(BS) kb_scatter(const Inst *in, BatchMap m) {
   unsigned b, nb;
   const Inst &d = in[batch_locate(m, b, nb)];
-  scatter(b, nb, d.n_init, d.g.num_cell, d.gb.key, d.gb.count, d.gb.order, d.gb.hist, d.gb.blk, d.cnt,
-          d.gb.scattered);
+  scatter(b, nb, d.n_init, d.g.num_cell, d.gb.key, d.gb.count, d.gb.order, d.gb.hist, d.gb.blk,
+          d.gb.blk_chunk, d.cnt, d.gb.scattered);
 }
 
 __global__ void __launch_bounds__(BS) kb_order(const Inst *in, BatchMap m) {
@@ -553,11 +595,12 @@ __global__ void __launch_bounds__(BS) kb_permute_predict(const Inst *in, BatchMa
 // hash + blanking, scan and scatter of every instance, as sort_keys does for one
 void launch_batch_sort(hipStream_t s, const BatchLaunch &L) {
   hipLaunchKernelGGL(kb_blank_hash_count, dim3(L.parts.blocks), dim3(BS), 0, s, L.inst, L.parts.m);
+  if (!L.scan_alone) hipLaunchKernelGGL(kb_scan_reduce, dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
+  if (L.sort_chunks) hipLaunchKernelGGL(kb_sort_chunks, dim3(L.one.blocks), dim3(CS_NT), 0, s, L.inst, L.one.m);
   if (L.scan_alone) {
     hipLaunchKernelGGL((kb_scan_cells<SCAN_NT, SCAN_TILE_ALONE / SCAN_NT>), dim3(L.tiles.blocks), dim3(SCAN_NT), 0, s,
                        L.inst, L.tiles.m);
   } else {
-    hipLaunchKernelGGL(kb_scan_reduce, dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
     hipLaunchKernelGGL((kb_scan_cells<BS, SCAN_ITEMS>), dim3(L.tiles.blocks), dim3(BS), 0, s, L.inst, L.tiles.m);
   }
   hipLaunchKernelGGL(kb_scatter, dim3(L.parts.blocks), dim3(BS), 0, s, L.inst, L.parts.m);

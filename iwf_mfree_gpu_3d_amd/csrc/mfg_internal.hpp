@@ -159,7 +159,9 @@ struct GridBuffers {
   int *count;        // num_cell + 1: exclusive offsets of the cells
   int *hist;         // num_cell particle counts of a sort under way; zero between sorts
   int *blk;          // per-block blanked counts
-  unsigned long long *blk2;  // scan scratch
+  unsigned long long *blk2;  // tile sums of the scan
+  int *blk_chunk;            // sums over PREFIX_CHUNK of blk and of blk2; null below PREFIX_CHUNKS blocks,
+  unsigned long long *part_chunk;  // tiles
   int *occ;          // occupied cells, ascending; [num_cell]: how many
   int nblk;          // blocks of the hash kernel
 };
@@ -176,6 +178,7 @@ void launch_order(hipStream_t s, unsigned n_init, GridBuffers &gb);
 constexpr int SCAN_TILE = 256 * 16, SCAN_TILE_ALONE = 1024 * 4;
 constexpr long SCAN_ALONE = 128 * 1024;
 int scan_tiles(long num_cell, bool alone);
+constexpr int PREFIX_CHUNK = 256, PREFIX_CHUNKS = 16 * 1024;
 bool order_apart(long particles);  // whether a step runs launch_order
 void launch_cells_to_tables(hipStream_t s, const GridInfo &g, const int *offsets, int rothlin,
                             int *start, int *end);
@@ -333,6 +336,7 @@ struct BatchLaunch {
   int pair_far;      // an instance's records are beyond the gathers' 32-bit offsets
   int ordered;       // order_apart
   int scan_alone;    // no instance has more than SCAN_ALONE cells
+  int sort_chunks;   // an instance needs blk_chunk or part_chunk
   BatchGrid tiles;   // scan tiles of the cell counts
   BatchGrid one;     // one workgroup per instance
   BatchGrid parts;   // N_init particles, 256 per workgroup
