@@ -2334,7 +2334,7 @@ int batch_build(mfg_batch *b, int record) {
     HIP_TRY(hipMalloc(&b->d_inst, sizeof(Inst) * (size_t)n));
     b->inst_cap = n;
   }
-  constexpr int N_MAPS = 7;
+  constexpr int N_MAPS = 8;
   const size_t map_len = (size_t)n + 1;
   if (N_MAPS * map_len > b->maps_cap) {
     if (b->d_maps) (void)hipFree(b->d_maps);
@@ -2345,7 +2345,7 @@ int batch_build(mfg_batch *b, int record) {
   }
   std::vector<Inst> host(n);
   std::vector<unsigned> maps(N_MAPS * map_len, 0u);
-  BatchGrid *grids[N_MAPS] = {&b->L.tiles, &b->L.one, &b->L.parts,
+  BatchGrid *grids[N_MAPS] = {&b->L.tiles, &b->L.one, &b->L.parts, &b->L.scatter,
                               &b->L.pairs8, &b->L.nbrs8, &b->L.tools, &b->L.search};
   long parts = 0, most = 0;
   for (const mfg_batch::Member &m : b->members) {
@@ -2384,6 +2384,7 @@ int batch_build(mfg_batch *b, int record) {
         (unsigned)scan_tiles(gi.num_cell, b->L.scan_alone),
         1u,
         nblk,
+        (unsigned)scatter_blocks(m.p->N_init, gi.num_cell),
         round8((unsigned)pair_blocks(
             m.p->N_init, b->precision == MFG_FP64 ? pair_lanes(MFG_FP64, m.p->N_init) : b->L.pair_lanes, 256)),
         std::min(neighbour_blocks(gi, m.p->N_init), b->L.nbr_most),

@@ -178,6 +178,7 @@ void launch_order(hipStream_t s, unsigned n_init, GridBuffers &gb);
 constexpr int SCAN_TILE = 256 * 16, SCAN_TILE_ALONE = 1024 * 4;
 constexpr long SCAN_ALONE = 128 * 1024;
 int scan_tiles(long num_cell, bool alone);
+int scatter_blocks(unsigned n_init, long num_cell);
 constexpr int PREFIX_CHUNK = 256, PREFIX_CHUNKS = 16 * 1024;
 bool order_apart(long particles);  // whether a step runs launch_order
 void launch_cells_to_tables(hipStream_t s, const GridInfo &g, const int *offsets, int rothlin,
@@ -340,6 +341,7 @@ struct BatchLaunch {
   BatchGrid tiles;   // scan tiles of the cell counts
   BatchGrid one;     // one workgroup per instance
   BatchGrid parts;   // N_init particles, 256 per workgroup
+  BatchGrid scatter; // scatter_blocks
   BatchGrid pairs8;  // pair-pass workgroups, padded to a multiple of 8 (XCD-ordered kernels)
   BatchGrid nbrs8;   // neighbour-pass workgroups, padded to a multiple of 8
   unsigned nbr_blocks, nbr_most;  // the largest instance's, and how many of them one launch takes
