@@ -288,7 +288,8 @@ __device__ __forceinline__ void cell_lists(int s, int e, int T, int lane, Fetch 
       if (TAIL) in_chunk = __builtin_amdgcn_ballot_w64(valid);
       const unsigned long long cand_ok = __builtin_amdgcn_ballot_w64(pj.w == 0.) & in_chunk;
       bad |= __builtin_amdgcn_ballot_w64(pj.w == 2.) & in_chunk;
-      if (PSE_MODE && TAIL) tr.y = valid ? tr.y : 0.;  // masked lanes add zero
+      // masked lanes add zero, also where the record they hold is of an infinite temperature
+      if (PSE_MODE && TAIL) tr = valid ? tr : make_double2(0., 0.);
       float try_f = 0.f;
       if (PSE_MODE == 2) try_f = (float)tr.y;
       // lapl_pse (src/kernels.cuh:71-92) times (T_j - T_i) m / rho_j

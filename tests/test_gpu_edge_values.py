@@ -68,3 +68,31 @@ def test_guard_blanks_what_the_oracle_blanks(hip_device, precision, locked, tol,
         g, o = parts.download(f)[og][keep], sim.field(of)[oo][keep]
         assert np.isfinite(g).all()
         assert rel_err(g, o) < tol, (f, rel_err(g, o))
+
+
+@pytest.mark.parametrize("precision", [_lib.MFG_FP64, _lib.MFG_FP32_KAHAN], ids=["fp64", "fp32"])
+def test_infinite_temperature_heats_to_infinity(hip_device, precision):
+    """The PSE rate of a particle beside one of infinite temperature is infinite, not NaN (a chunk of candidates has
+    unused lanes, which are to add nothing)."""
+    h, n = 7.5e-4, 70
+    rng = np.random.default_rng(5)
+    api.reset_globals()
+    api.constants_reset()
+    api.set_options(cspm=False, heat=_lib.MFG_HEAT_PSE, single_sqrt=False)
+    phys = api.make_phys_constants()
+    phys.rho0, phys.K, phys.G, phys.mass = 4.43, 1.2, 0.4, 5e-10
+    trml = api.make_trml_constants()
+    trml.cp, trml.k, trml.alpha, trml.T_init = 5e-6, 7e-13, 3e-8, 300.0
+    api.actions_setup_physical_constants(phys)
+    api.interactions_setup_physical_constants(phys)
+    api.interactions_setup_thermal_constants_workpiece(trml)
+    pos = rng.uniform(0.0, h, (n, 3))  # one cell's stencil
+    T = np.full(n, 300.0)
+    T[0] = np.inf
+    p = api.particle_gpu(pos, None, np.full(n, 4.43), T, np.full(n, h), None, None, None, precision=precision)
+    g = api.grid_gpu_green(n, pos.min(0), pos.max(0), h)
+    g.sort(p)
+    hot = p.download(_lib.F_ID) == 0
+    api.interactions_heat_pse(p, g)
+    rate = p.download(_lib.F_T_T)
+    assert np.isnan(rate[hot]).all() and (rate[~hot] == np.inf).all()
